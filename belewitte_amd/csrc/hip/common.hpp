@@ -50,6 +50,22 @@ int device_cus();
 
 // -------------------------------------------------------- device side
 
+// The block of vertices (of n equal blocks) that workgroup b takes.
+// Workgroups go to the eight XCDs round robin, and the degrees of an R-MAT
+// graph in its generated order follow the bits of the vertex id (each zero
+// bit makes a vertex about three times heavier), so block b for workgroup b
+// gives one XCD 2.5 to 3.4 times its share of the edges (scales 16 to 21,
+// 256-vertex blocks).  Each run of eight blocks is rotated by the sum of the
+// octal digits of its index instead: no low bit of the id stays tied to an
+// XCD (1.02 to 1.14 times the share at scales 19 to 21).  A bijection; the
+// last, incomplete run keeps its order.
+__device__ __forceinline__ uint32_t spread_block(uint32_t b, uint32_t n)
+{
+    const uint32_t q = b >> 3;
+    if ((q << 3) + 8 > n) return b;
+    return (q << 3) | ((b + q + (q >> 3) + (q >> 6) + (q >> 9) + (q >> 12) + (q >> 15)) & 7u);
+}
+
 __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v)
 {
     // xor butterfly over the 64 lanes; every lane ends with the total.

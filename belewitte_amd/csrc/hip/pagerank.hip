@@ -6,9 +6,9 @@
 // pr/deg, the double/float base terms of the two consolidate kernels.  The
 // mapping is MI355X's own:
 //   - pull forms: a workgroup stages its rows' in-edge contributions in LDS
-//     in rounds of 2048, gathered with every load in flight; rows with more
-//     than 256 in-edges are summed one wave each, longest first, in the
-//     same launch (the pull plan).  vertex-pull and vertex-pull-nodiv keep
+//     in rounds of 2048, gathered with every load in flight; long rows are
+//     summed one wave or one workgroup each in the same launch (the pull
+//     plan).  vertex-pull and vertex-pull-nodiv keep
 //     the reference's sequential FP32 sum in CSR order, bit for bit; the
 //     _warp forms combine lane-strided partials by shuffles where the
 //     reference adds them atomically.  The dividing forms gather
@@ -339,7 +339,7 @@ __global__ __launch_bounds__(1024) void pr_vertex_push_kernel(uint64_t V, const 
 constexpr uint32_t kPullRows = 256;
 constexpr uint32_t kPullChunk = 2048;
 constexpr uint32_t kPullPerThread = kPullChunk / kPullRows;
-constexpr uint32_t kSumBatch = 32;     // LDS reads in flight in a row's sequential sum
+constexpr uint32_t kSumBatch = 32;     // LDS reads in flight in a short row's sequential sum
 constexpr uint32_t kStrideBatch = 8;   // the same for a lane of a virtual warp
 
 // The contribution one in-edge from u brings: pr[u] / deg[u] for the
@@ -352,6 +352,33 @@ __device__ __forceinline__ float pull_contribution(const float *__restrict__ pr,
     if constexpr (DIV == 1) return pr[u] / static_cast<float>(deg[u]);
     else if constexpr (DIV == 2) return pr[u] / static_cast<float>(static_cast<int32_t>(deg[u]));
     else return pr[u];
+}
+
+// Inclusive prefix sum over the wave by DPP row shifts and row broadcasts.
+template<int kCtrl, int kRowMask, bool kBound>
+__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t v)
+{
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), kCtrl, kRowMask, 0xF, kBound));
+}
+
+__device__ __forceinline__ uint32_t wave_prefix_sum(uint32_t x)
+{
+    x += dpp_or_zero<0x111, 0xF, true>(x);
+    x += dpp_or_zero<0x112, 0xF, true>(x);
+    x += dpp_or_zero<0x114, 0xF, true>(x);
+    x += dpp_or_zero<0x118, 0xF, true>(x);
+    x += dpp_or_zero<0x142, 0xA, false>(x);
+    x += dpp_or_zero<0x143, 0xC, false>(x);
+    return x;
+}
+
+__device__ __forceinline__ uint64_t wave_prefix_sum(uint64_t x)
+{
+    for (int o = 1; o < kWave; o <<= 1) {
+        const uint64_t y = __shfl_up(static_cast<unsigned long long>(x), static_cast<unsigned>(o), kWave);
+        if (static_cast<int>(__lane_id()) >= o) x += y;
+    }
+    return x;
 }
 
 // The pull iteration of pagerank/vertex_pull.cu:16-30, vertex_pull_nodiv.cu,
@@ -371,56 +398,97 @@ __device__ __forceinline__ float pull_contribution(const float *__restrict__ pr,
 // adds them atomically, in no fixed order.  Rows go round-robin to the
 // virtual warps; a round boundary cuts at most one row, whose partials the
 // owning warp carries to the next round.
+//
+// Rows with more than long_degree in-edges are summed elsewhere
+// (pull_long_rows).  The rounds run over the other rows' edges only: a
+// compacted position c is the edge e0 + c + the long rows' edges before it,
+// found among the workgroup's few long rows by binary search.  (Rounds over
+// the stored edges that jumped from long row to long row held up R-MAT's
+// first workgroups, where long and short rows alternate: at scale 20, edge
+// factor 16, the short rows alone took 246 us per launch and 162 us since;
+// spread_block took the whole launch from 192 to 137 us, the splits below to
+// 113: 142 G gathers/s, where a table of the size of one XCD's L2 allows
+// between 76 (16 MiB) and 216 (2 MiB).)
+template<typename Off>
 struct PullShortLds {
     float vals[2][kPullChunk];
-    uint64_t rowOff[kPullRows + 1];
+    Off rowC[kPullRows + 1];  // compacted position of each row's first edge
+    Off lpos[kPullRows];      // per long row: the compacted position it stands before,
+    Off lskip[kPullRows];     // and the edges of the long rows up to and including it
+    Off wsum[kPullRows / kWave];
+    uint32_t wlong[kPullRows / kWave];
 };
 
 template<int DIV, int W, typename Off>
-__device__ __forceinline__ void pull_short_rows(uint32_t block, PullShortLds &lds, uint64_t V,
+__device__ __forceinline__ void pull_short_rows(uint32_t block, PullShortLds<Off> &lds, uint64_t V,
                                                 const Off *__restrict__ roff, const uint32_t *__restrict__ rcols,
                                                 const uint32_t *__restrict__ deg, const float *__restrict__ pr,
                                                 float *np, uint64_t long_degree)
 {
     auto &vals = lds.vals;
-    auto &rowOff = lds.rowOff;
+    const Off *rowC = lds.rowC;
     constexpr uint32_t kWarps = kPullRows / W;
-    const uint32_t t = threadIdx.x;
+    const uint32_t t = threadIdx.x, wv = t / kWave;
     const uint64_t r0 = static_cast<uint64_t>(block) * kPullRows;
     const uint32_t nrows = static_cast<uint32_t>(V - r0 < kPullRows ? V - r0 : kPullRows);
-    for (uint32_t i = t; i <= nrows; i += kPullRows) rowOff[i] = static_cast<uint64_t>(roff[r0 + i]);
-    __syncthreads();
-    const uint64_t e0 = rowOff[0], e1 = rowOff[nrows];
     const uint32_t warp = t / W, lane = t % W;
-    auto is_long = [&](uint32_t i) { return rowOff[i + 1] - rowOff[i] > long_degree; };
-
-    // Rows with more than long_degree in-edges are summed by
-    // pr_pull_long_kernel; a round starting inside one jumps to its end.
-    auto skip_long = [&](uint64_t c) {
-        while (c < e1) {
-            uint32_t lo = 0, hi = nrows - 1;  // the row holding edge c: last row starting at or before it
-            while (lo < hi) {
-                const uint32_t m = (lo + hi + 1) / 2;
-                if (rowOff[m] <= c) lo = m;
-                else hi = m - 1;
-            }
-            if (!is_long(lo)) break;
-            c = rowOff[lo + 1];
+    const Off e0 = roff[r0];
+    Off rs = 0, re = 0;
+    if (t < nrows) {
+        rs = roff[r0 + t];
+        re = roff[r0 + t + 1];
+    }
+    const bool isLong = static_cast<uint64_t>(re - rs) > long_degree;
+    const Off len = isLong ? Off{0} : static_cast<Off>(re - rs);
+    const Off incl = wave_prefix_sum(len);
+    const uint64_t longs = __ballot(isLong);
+    if ((t & (kWave - 1)) == kWave - 1) {
+        lds.wsum[wv] = incl;
+        lds.wlong[wv] = static_cast<uint32_t>(__popcll(longs));
+    }
+    __syncthreads();
+    Off before = incl - len, total = 0;
+    uint32_t nlong = 0;
+    uint32_t li = static_cast<uint32_t>(__popcll(longs & ((1ull << (t & (kWave - 1))) - 1ull)));
+#pragma unroll
+    for (uint32_t w = 0; w < kPullRows / kWave; w++) {
+        if (w < wv) {
+            before += lds.wsum[w];
+            li += lds.wlong[w];
         }
-        return c;
+        total += lds.wsum[w];
+        nlong += lds.wlong[w];
+    }
+    lds.rowC[t] = before;
+    if (t == kPullRows - 1) lds.rowC[kPullRows] = total;
+    if (isLong) {
+        lds.lpos[li] = before;
+        lds.lskip[li] = re - e0 - before;
+    }
+    // Rows without in-edges get an empty sum.
+    if (t < nrows && rs == re) np[r0 + t] = 0.0f;
+    __syncthreads();
+    auto edge_of = [&](Off c) {
+        uint32_t lo = 0, hi = nlong;  // the long rows standing before position c
+        while (lo < hi) {
+            const uint32_t m = (lo + hi) / 2;
+            if (lds.lpos[m] <= c) lo = m + 1;
+            else hi = m;
+        }
+        return static_cast<Off>(e0 + c + (lo ? lds.lskip[lo - 1] : Off{0}));
     };
 
     // Loads of one round into registers; stored to LDS after the previous
     // round's sums, so those sums overlap the gathers' latency.  The loads
-    // are unconditional (indices past the round repeat its last edge) so
+    // are unconditional (positions past the round repeat its last edge) so
     // that all column loads, then all gathers, are in flight together.
     float reg[kPullPerThread];
-    auto gather = [&](uint64_t c0, uint64_t c1) {
+    auto gather = [&](Off c0, Off c1) {
         uint32_t u[kPullPerThread];
 #pragma unroll
         for (uint32_t k = 0; k < kPullPerThread; k++) {
-            const uint64_t e = c0 + k * kPullRows + t;
-            u[k] = rcols[e < c1 ? e : c1 - 1];
+            const Off c = c0 + k * kPullRows + t;
+            u[k] = rcols[edge_of(c < c1 ? c : c1 - 1)];
         }
 #pragma unroll
         for (uint32_t k = 0; k < kPullPerThread; k++) reg[k] = pull_contribution<DIV>(pr, deg, u[k]);
@@ -430,29 +498,23 @@ __device__ __forceinline__ void pull_short_rows(uint32_t block, PullShortLds &ld
         for (uint32_t k = 0; k < kPullPerThread; k++) vals[buf][k * kPullRows + t] = reg[k];
     };
 
-    // Rows without in-edges get an empty sum.
-    for (uint32_t i = t; i < nrows; i += kPullRows)
-        if (rowOff[i] == rowOff[i + 1]) np[r0 + i] = 0.0f;
-
     float carry = 0.0f;  // partial of this lane's row cut by the round boundary
-    uint64_t c0 = skip_long(e0);
-    uint64_t c1 = c0 + kPullChunk < e1 ? c0 + kPullChunk : e1;
-    if (c0 < e1) {
+    Off c0 = 0, c1 = min(static_cast<Off>(kPullChunk), total);
+    if (c0 < total) {
         gather(c0, c1);
         stage(0);
     }
     __syncthreads();
     int buf = 0;
-    while (c0 < e1) {
-        const uint64_t n0 = skip_long(c1);
-        const uint64_t n1 = n0 + kPullChunk < e1 ? n0 + kPullChunk : e1;
-        if (n0 < e1) gather(n0, n1);
+    while (c0 < total) {
+        const Off n0 = c1, n1 = c1 + min(static_cast<Off>(kPullChunk), static_cast<Off>(total - c1));
+        if (n0 < total) gather(n0, n1);
         const float *v = vals[buf];
         if constexpr (W == 1) {
             // Thread t owns row t.
-            if (t < nrows && !is_long(t)) {
-                const uint64_t s = rowOff[t], e = rowOff[t + 1];
-                const uint64_t lo = s > c0 ? s : c0, hi = e < c1 ? e : c1;
+            {
+                const Off s = rowC[t], e = rowC[t + 1];
+                const Off lo = s > c0 ? s : c0, hi = e < c1 ? e : c1;
                 if (lo < hi) {
                     // In CSR order; the LDS reads of a batch are issued
                     // together, the adds stay sequential.
@@ -477,25 +539,25 @@ __device__ __forceinline__ void pull_short_rows(uint32_t block, PullShortLds &ld
             uint32_t lo = 0, hi = nrows;
             while (lo < hi) {
                 const uint32_t m = (lo + hi) / 2;
-                if (rowOff[m + 1] <= c0) lo = m + 1;
+                if (rowC[m + 1] <= c0) lo = m + 1;
                 else hi = m;
             }
             const uint32_t ra = lo;
             hi = nrows;
             while (lo < hi) {
                 const uint32_t m = (lo + hi) / 2;
-                if (rowOff[m] < c1) lo = m + 1;
+                if (rowC[m] < c1) lo = m + 1;
                 else hi = m;
             }
             const uint32_t rb = lo;  // rows [ra, rb) overlap the round
             const uint32_t first = ra + (warp + kWarps - ra % kWarps) % kWarps;
             for (uint32_t i = first; i < rb; i += kWarps) {
-                const uint64_t s = rowOff[i], e = rowOff[i + 1];
-                if (s == e || is_long(i)) continue;
-                const uint64_t a = s > c0 ? s : c0, b = e < c1 ? e : c1;
+                const Off s = rowC[i], e = rowC[i + 1];
+                if (s == e) continue;
+                const Off a = s > c0 ? s : c0, b = e < c1 ? e : c1;
                 // Lane l takes the row positions congruent to l modulo W.
-                const uint64_t p0 = a - s;
-                uint32_t j = static_cast<uint32_t>(a - c0) + static_cast<uint32_t>((lane + W - p0 % W) % W);
+                const uint32_t p0 = static_cast<uint32_t>((a - s) % W);
+                uint32_t j = static_cast<uint32_t>(a - c0) + (lane + W - p0) % W;
                 const uint32_t end = static_cast<uint32_t>(b - c0);
                 float part = (a == s) ? 0.0f : carry;
                 for (; j + (kStrideBatch - 1) * W < end; j += kStrideBatch * W) {
@@ -516,7 +578,7 @@ __device__ __forceinline__ void pull_short_rows(uint32_t block, PullShortLds &ld
                 }
             }
         }
-        if (n0 < e1) stage(buf ^ 1);
+        if (n0 < total) stage(buf ^ 1);
         __syncthreads();
         c0 = n0;
         c1 = n1;
@@ -524,100 +586,294 @@ __device__ __forceinline__ void pull_short_rows(uint32_t block, PullShortLds &ld
     }
 }
 
-// Rows with more than long_degree in-edges, one wave per row (listed by
-// the pull plan), so that the hubs of a skewed graph are summed side by
-// side rather than one after another by the workgroup owning their rows.
-// The wave gathers kLongRound contributions per round (8 per lane, all in
-// flight together).  SEQ: lane 0 adds them in CSR order through LDS, the
-// reference's sequential sum bit for bit.  Otherwise (the _warp variants)
-// lane l keeps the partial of the positions congruent to l modulo 64 and
-// the partials meet in a shuffle tree -- the reference's per-lane partials
-// and atomic adds in another, equally valid order.
-constexpr uint32_t kLongWaves = 4;
-constexpr uint32_t kLongPerLane = 8;
-constexpr uint32_t kLongRound = kWave * kLongPerLane;
+// ------------------------------------- sequential FP32 sums in parallel
+//
+// The reference adds a row's contributions one after another in FP32, and
+// vertex-pull and vertex-pull-nodiv keep that sum bit for bit.  Written as
+// a loop it is one dependent add per in-edge, and the longest rows of an
+// R-MAT graph hold up the whole iteration (scale 20, edge factor 16: a row
+// of 39585).  The same bits come out of a parallel sum: while the running sum stays in one binade [2^k, 2^(k+1)) it is an
+// integer m of units u = 2^(k-23), and adding x >= 0 rounds to
+// m + rne(x / u), where x's rounded quotient depends on m only when x / u
+// is exactly halfway between two integers, and then only on m's parity.  So
+// a group of values maps the parity p of the incoming m to an increment
+// d[p], and such maps compose associatively.  The lanes hold consecutive
+// values; a wave scan of their maps gives every lane's m, the first lane
+// whose m leaves the binade (m >= 2^24) is added value by value, and the
+// scan goes on behind it in the new binade.  A sum leaves its binade at most
+// once per doubling, so the scans are about as many as the rounds.
+// Values that are negative or NaN, and a running sum that is zero,
+// subnormal or not finite, are added value by value too.
 
-struct PullLongLds {
-    float vals[kLongWaves][2][kLongRound];
+__device__ __forceinline__ float lane_f32(float x, int l)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
+}
+
+constexpr int kSeqPerLane = 8;
+constexpr uint32_t kSeqLimit = 1u << 24;  // m at which a sum has left its binade
+
+// The increment of m (units 2^(e - 150) for a sum with exponent field e) by
+// a lane's values, for an even and an odd incoming m.
+struct SeqMap {
+    uint32_t d0, d1;
 };
 
+__device__ __forceinline__ bool seq_normal(uint32_t bits)
+{
+    const uint32_t e = bits >> 23;  // the sign bit makes it >= 256
+    return e >= 1 && e <= 254;
+}
+
+// The inclusive scan over the wave of the lanes' maps for the incoming sum's
+// exponent field e; lanes below `first` add nothing.  Each value's quotient
+// is capped at 2^24 and each lane's increment at 2^25: past the cap the sum
+// has left the binade anyway, and 64 capped increments fit 32 bits.
+__device__ __forceinline__ SeqMap seq_scan(const float (&x)[kSeqPerLane], uint32_t e, uint32_t first)
+{
+    const uint32_t lane = __lane_id();
+    uint32_t q[kSeqPerLane];
+    uint32_t ties = 0, sum = 0;
+#pragma unroll
+    for (int k = 0; k < kSeqPerLane; k++) {
+        const float y = fminf(ldexpf(x[k], 150 - static_cast<int>(e)), 16777216.0f);
+        const float f = floorf(y), r = y - f;  // exact
+        q[k] = static_cast<uint32_t>(f) + (r > 0.5f ? 1u : 0u);
+        ties |= (r == 0.5f ? 1u : 0u) << k;
+        sum += q[k];
+    }
+    const bool live = lane >= first;
+    if (__ballot(live && ties != 0) == 0) {
+        const uint32_t d = wave_prefix_sum(live ? min(sum, 1u << 25) : 0u);
+        return SeqMap{d, d};
+    }
+    SeqMap m{0, 0};
+    if (live) {
+#pragma unroll
+        for (int k = 0; k < kSeqPerLane; k++) {
+            const uint32_t tie = (ties >> k) & 1u;
+            m.d0 += q[k] + (tie & ((m.d0 + q[k]) & 1u));
+            m.d1 += q[k] + (tie & ((m.d1 + q[k] + 1u) & 1u));
+        }
+        m.d0 = min(m.d0, 1u << 25);
+        m.d1 = min(m.d1, 1u << 25);
+    }
+    for (int o = 1; o < kWave; o <<= 1) {
+        // the lanes before this one first: p -> a[p], then this one's map at
+        // the parity p + a[p]
+        const uint32_t a0 = __shfl_up(m.d0, static_cast<unsigned>(o), kWave);
+        const uint32_t a1 = __shfl_up(m.d1, static_cast<unsigned>(o), kWave);
+        if (static_cast<int>(lane) >= o)
+            m = SeqMap{a0 + ((a0 & 1u) ? m.d1 : m.d0), a1 + ((a1 & 1u) ? m.d0 : m.d1)};
+    }
+    return m;
+}
+
+// acc after adding the wave's 512 values one by one in lane order, each
+// lane's kSeqPerLane in theirs.  acc is the same in every lane, and every
+// lane takes part.
+__device__ __forceinline__ float seq_add_wave(float acc, const float (&x)[kSeqPerLane])
+{
+    bool plain = true;
+#pragma unroll
+    for (int k = 0; k < kSeqPerLane; k++) plain = plain && x[k] >= 0.0f;
+    const bool allPlain = __ballot(!plain) == 0;
+    uint32_t first = 0;
+    while (first < kWave) {
+        const uint32_t bits = __builtin_amdgcn_readfirstlane(__float_as_uint(acc));
+        uint32_t serial = first;  // the lane to add value by value
+        if (allPlain && seq_normal(bits)) {
+            const uint32_t m = (bits & 0x7FFFFFu) | 0x800000u;
+            const SeqMap f = seq_scan(x, bits >> 23, first);
+            const uint32_t incl = (m & 1u) ? f.d1 : f.d0;
+            const uint64_t over = __ballot(m + incl >= kSeqLimit);
+            serial = over ? static_cast<uint32_t>(__builtin_ctzll(over)) : kWave;
+            const uint32_t before =
+                serial ? static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), static_cast<int>(serial) - 1)) : 0u;
+            acc = __uint_as_float((bits & 0xFF800000u) | ((m + before) & 0x7FFFFFu));
+            if (serial == kWave) return acc;
+        }
+#pragma unroll
+        for (int k = 0; k < kSeqPerLane; k++) acc += lane_f32(x[k], static_cast<int>(serial));
+        first = serial + 1;
+    }
+    return acc;
+}
+
+// Rows with more than long_degree in-edges (listed by the pull plan), so
+// that the hubs of a skewed graph are summed side by side rather than one
+// after another by the workgroup owning their rows: one wave per row, or a
+// whole workgroup for a row of more than kHugeDegree in-edges, whose four
+// waves gather 2048 contributions per round where one wave's 512 would leave
+// the row waiting on the latency of its rounds.  SEQ: the sum is the
+// reference's sequential one, bit for bit (seq_add_wave).  Otherwise (the
+// _warp variants) each lane keeps a partial and the partials meet in a
+// tree -- the reference's per-lane partials and atomic adds in another,
+// equally valid order.
+constexpr uint32_t kLongWaves = 4;
+constexpr uint32_t kLongPerLane = kSeqPerLane;
+constexpr uint32_t kLongRound = kWave * kLongPerLane;
+constexpr uint32_t kHugeRound = kLongWaves * kLongRound;
+
+// Rows listed by the pull plan.
+struct RowList {
+    const uint32_t *rows = nullptr;
+    uint32_t n = 0;
+};
+
+struct PullLongLds {
+    float vals[kLongWaves][kLongRound];  // a wave's round, or the four waves' parts of a workgroup's
+    uint32_t d0[kLongWaves], d1[kLongWaves], plain[kLongWaves];
+    float sums[kLongWaves];
+};
+
+// The contributions of in-edges c0 + k * stride + t (k < kLongPerLane) of a
+// row ending at e, all in flight together; 0 past the end (adding it
+// changes no sum: the running sum is never -0).
+template<int DIV>
+__device__ __forceinline__ void long_gather(float (&x)[kLongPerLane], uint64_t c0, uint64_t e, uint32_t t,
+                                            uint32_t stride, const uint32_t *__restrict__ rcols,
+                                            const uint32_t *__restrict__ deg, const float *__restrict__ pr)
+{
+    uint32_t u[kLongPerLane];
+#pragma unroll
+    for (uint32_t k = 0; k < kLongPerLane; k++) {
+        const uint64_t j = c0 + k * stride + t;
+        u[k] = rcols[j < e ? j : e - 1];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kLongPerLane; k++) {
+        const uint64_t j = c0 + k * stride + t;
+        const float v = pull_contribution<DIV>(pr, deg, u[k]);
+        x[k] = j < e ? v : 0.0f;
+    }
+}
+
+// The lane's kSeqPerLane consecutive values of a staged round.
+__device__ __forceinline__ void seq_values(float (&y)[kSeqPerLane], const float *v)
+{
+    const float4 *v4 = reinterpret_cast<const float4 *>(v + __lane_id() * kSeqPerLane);
+    const float4 a = v4[0], b = v4[1];
+    y[0] = a.x, y[1] = a.y, y[2] = a.z, y[3] = a.w;
+    y[4] = b.x, y[5] = b.y, y[6] = b.z, y[7] = b.w;
+}
+
 template<int DIV, bool SEQ, typename Off>
-__device__ __forceinline__ void pull_long_rows(uint32_t block, PullLongLds &lds, const uint32_t *__restrict__ rows,
-                                               uint32_t nrows, const Off *__restrict__ roff,
+__device__ __forceinline__ void pull_huge_row(uint32_t row, PullLongLds &lds, const Off *__restrict__ roff,
+                                              const uint32_t *__restrict__ rcols, const uint32_t *__restrict__ deg,
+                                              const float *__restrict__ pr, float *np)
+{
+    const uint32_t t = threadIdx.x, wv = t / kWave, lane = t & (kWave - 1);
+    const uint64_t s = static_cast<uint64_t>(roff[row]), e = static_cast<uint64_t>(roff[row + 1]);
+    float x[kLongPerLane];
+    if constexpr (!SEQ) {
+        float part = 0.0f;
+        for (uint64_t c0 = s; c0 < e; c0 += kHugeRound) {
+            long_gather<DIV>(x, c0, e, t, kPullRows, rcols, deg, pr);
+#pragma unroll
+            for (uint32_t k = 0; k < kLongPerLane; k++) part += x[k];
+        }
+        part = wave_sum_f32(part);
+        if (lane == 0) lds.sums[wv] = part;
+        __syncthreads();
+        if (t == 0) {
+            float total = 0.0f;
+            for (uint32_t w = 0; w < kLongWaves; w++) total += lds.sums[w];
+            np[row] = total;
+        }
+    } else {
+        float *flat = lds.vals[0];
+        float acc = 0.0f;  // the same in every thread
+        long_gather<DIV>(x, s, e, t, kPullRows, rcols, deg, pr);
+        for (uint64_t c0 = s; c0 < e; c0 += kHugeRound) {
+#pragma unroll
+            for (uint32_t k = 0; k < kLongPerLane; k++) flat[k * kPullRows + t] = x[k];
+            __syncthreads();
+            // The next round's gathers run under this round's sums.
+            if (c0 + kHugeRound < e) long_gather<DIV>(x, c0 + kHugeRound, e, t, kPullRows, rcols, deg, pr);
+            float y[kSeqPerLane];
+            seq_values(y, lds.vals[wv]);
+            // Each wave's map in the binade of the round's incoming sum.
+            const uint32_t bits = __builtin_amdgcn_readfirstlane(__float_as_uint(acc));
+            bool plain = true;
+#pragma unroll
+            for (int k = 0; k < kSeqPerLane; k++) plain = plain && y[k] >= 0.0f;
+            const bool allPlain = __ballot(!plain) == 0 && seq_normal(bits);
+            SeqMap f{0, 0};
+            if (allPlain) f = seq_scan(y, bits >> 23, 0);
+            if (lane == kWave - 1) {
+                lds.d0[wv] = f.d0;
+                lds.d1[wv] = f.d1;
+                lds.plain[wv] = allPlain ? 1u : 0u;
+            }
+            __syncthreads();
+            uint32_t m = (bits & 0x7FFFFFu) | 0x800000u;
+            bool stays = true;
+#pragma unroll
+            for (uint32_t w = 0; w < kLongWaves; w++) {
+                m += (m & 1u) ? lds.d1[w] : lds.d0[w];
+                stays = stays && lds.plain[w] && m < kSeqLimit;
+                m = min(m, kSeqLimit);
+            }
+            if (stays) {
+                acc = __uint_as_float((bits & 0xFF800000u) | (m & 0x7FFFFFu));
+            } else {
+                // Every wave adds the four parts in order: the same sum in all.
+                for (uint32_t w = 0; w < kLongWaves; w++) {
+                    seq_values(y, lds.vals[w]);
+                    acc = seq_add_wave(acc, y);
+                }
+            }
+            __syncthreads();  // the staged round and the maps have been read
+        }
+        if (t == 0) np[row] = acc;
+    }
+}
+
+template<int DIV, bool SEQ, typename Off>
+__device__ __forceinline__ void pull_long_rows(uint32_t block, PullLongLds &lds, RowList huge, RowList longs,
+                                               const Off *__restrict__ roff,
                                                const uint32_t *__restrict__ rcols, const uint32_t *__restrict__ deg,
                                                const float *__restrict__ pr, float *np)
 {
-    auto &vals = lds.vals;
+    if (block < huge.n) {
+        pull_huge_row<DIV, SEQ>(huge.rows[block], lds, roff, rcols, deg, pr, np);
+        return;
+    }
     const uint32_t wv = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-    const uint32_t i = block * kLongWaves + wv;
-    if (i >= nrows) return;
-    const uint32_t row = rows[i];
+    const uint32_t i = (block - huge.n) * kLongWaves + wv;
+    if (i >= longs.n) return;
+    const uint32_t row = longs.rows[i];
     const uint64_t s = static_cast<uint64_t>(roff[row]), e = static_cast<uint64_t>(roff[row + 1]);
     float x[kLongPerLane];
-    auto gather = [&](uint64_t c0) {
-        uint32_t u[kLongPerLane];
-#pragma unroll
-        for (uint32_t k = 0; k < kLongPerLane; k++) {
-            const uint64_t j = c0 + k * kWave + lane;
-            u[k] = rcols[j < e ? j : e - 1];
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < kLongPerLane; k++) {
-            const uint64_t j = c0 + k * kWave + lane;
-            x[k] = j < e ? pull_contribution<DIV>(pr, deg, u[k]) : 0.0f;
-        }
-    };
     if constexpr (!SEQ) {
         float part = 0.0f;
         for (uint64_t c0 = s; c0 < e; c0 += kLongRound) {
-            gather(c0);
+            long_gather<DIV>(x, c0, e, lane, kWave, rcols, deg, pr);
 #pragma unroll
             for (uint32_t k = 0; k < kLongPerLane; k++) part += x[k];
         }
         part = wave_sum_f32(part);
         if (lane == 0) np[row] = part;
     } else {
+        float *v = lds.vals[wv];
         float acc = 0.0f;
-        int buf = 0;
-        gather(s);
-#pragma unroll
-        for (uint32_t k = 0; k < kLongPerLane; k++) vals[wv][0][k * kWave + lane] = x[k];
+        long_gather<DIV>(x, s, e, lane, kWave, rcols, deg, pr);
         for (uint64_t c0 = s; c0 < e; c0 += kLongRound) {
-            const uint64_t c1 = c0 + kLongRound < e ? c0 + kLongRound : e;
-            if (c1 < e) gather(c1);
-            // The staged round is visible to lane 0 once the wave's LDS
-            // writes are ordered before its reads.
+#pragma unroll
+            for (uint32_t k = 0; k < kLongPerLane; k++) v[k * kWave + lane] = x[k];
+            if (c0 + kLongRound < e) long_gather<DIV>(x, c0 + kLongRound, e, lane, kWave, rcols, deg, pr);
+            // The wave's LDS writes ordered before its reads, and the reads
+            // before the next round's writes.
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-            if (lane == 0) {
-                // In CSR order, four values per 16-byte LDS read.
-                const float *v = vals[wv][buf];
-                const float4 *v4 = reinterpret_cast<const float4 *>(v);
-                const uint32_t n = static_cast<uint32_t>(c1 - c0);
-                uint32_t q = 0;
-                for (; 4 * (q + kSumBatch / 4) <= n; q += kSumBatch / 4) {
-                    float4 y[kSumBatch / 4];
-#pragma unroll
-                    for (uint32_t k = 0; k < kSumBatch / 4; k++) y[k] = v4[q + k];
-#pragma unroll
-                    for (uint32_t k = 0; k < kSumBatch / 4; k++) {
-                        acc += y[k].x;
-                        acc += y[k].y;
-                        acc += y[k].z;
-                        acc += y[k].w;
-                    }
-                }
-                for (uint32_t j = 4 * q; j < n; j++) acc += v[j];
-            }
+            float y[kSeqPerLane];
+            seq_values(y, v);
+            acc = seq_add_wave(acc, y);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-            if (c1 < e) {
-#pragma unroll
-                for (uint32_t k = 0; k < kLongPerLane; k++) vals[wv][buf ^ 1][k * kWave + lane] = x[k];
-            }
-            buf ^= 1;
         }
         if (lane == 0) np[row] = acc;
     }
@@ -641,39 +897,63 @@ __global__ __launch_bounds__(256) void pr_contrib_kernel(uint64_t V, const uint3
 }
 
 // One launch of a pull iteration: workgroups [0, long_blocks) sum the long
-// rows (longest first, so the biggest hub starts at once), the others one
-// block of kPullRows rows each.
+// rows (the longest first, so that they start at once), the others one block
+// of kPullRows rows each.
 template<int DIV, int W, typename Off>
 __global__ __launch_bounds__(kPullRows) void pr_pull_kernel(uint64_t V, const Off *__restrict__ roff,
                                                              const uint32_t *__restrict__ rcols,
                                                              const uint32_t *__restrict__ deg,
                                                              const float *__restrict__ pr, float *np,
-                                                             uint64_t long_degree, const uint32_t *__restrict__ rows,
-                                                             uint32_t nlong, uint32_t long_blocks)
+                                                             uint64_t long_degree, RowList huge, RowList longs,
+                                                             uint32_t long_blocks)
 {
     static_assert(kLongWaves * kWave == kPullRows, "both parts use the same workgroup");
     __shared__ union alignas(16) {
-        PullShortLds s;
+        PullShortLds<Off> s;
         PullLongLds l;
     } lds;
     if (blockIdx.x < long_blocks)
-        pull_long_rows<DIV, W == 1, Off>(blockIdx.x, lds.l, rows, nlong, roff, rcols, deg, pr, np);
+        pull_long_rows<DIV, W == 1, Off>(blockIdx.x, lds.l, huge, longs, roff, rcols, deg, pr, np);
     else
-        pull_short_rows<DIV, W, Off>(blockIdx.x - long_blocks, lds.s, V, roff, rcols, deg, pr, np, long_degree);
+        pull_short_rows<DIV, W, Off>(spread_block(blockIdx.x - long_blocks, gridDim.x - long_blocks), lds.s, V, roff,
+                                     rcols, deg, pr, np, long_degree);
 }
 
-// The long rows of a reverse CSR: rows whose in-degree exceeds `threshold`
-// (appended in any order).
+// The long rows of a reverse CSR, rows whose in-degree exceeds `threshold`:
+// those past `huge` from the front of rows[0, cap), the others from its
+// back, in any order; count[0] and count[1] of them.  A workgroup takes
+// 1024 consecutive vertices and reserves its slots with one atomic per list.
+constexpr uint32_t kListRows = 1024;
+
 template<typename Off>
-__global__ void pr_long_rows_kernel(uint64_t V, const Off *__restrict__ roff, uint64_t threshold, uint2 *rows,
-                                    uint32_t *count)
+__global__ __launch_bounds__(256) void pr_long_rows_kernel(uint64_t V, const Off *__restrict__ roff,
+                                                           uint64_t threshold, uint64_t huge, uint64_t cap,
+                                                           uint32_t *rows, uint32_t *count)
 {
-    const uint64_t stride = static_cast<uint64_t>(blockDim.x) * gridDim.x;
-    for (uint64_t v = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; v < V; v += stride) {
-        const uint64_t d = static_cast<uint64_t>(roff[v + 1]) - static_cast<uint64_t>(roff[v]);
-        if (d > threshold)
-            rows[atomicAdd(count, 1u)] = make_uint2(static_cast<uint32_t>(v), d > 0xFFFFFFFFull ? 0xFFFFFFFFu
-                                                                                             : static_cast<uint32_t>(d));
+    __shared__ uint32_t n[2], base[2];
+    if (threadIdx.x < 2) n[threadIdx.x] = 0;
+    __syncthreads();
+    constexpr int kPer = kListRows / 256;
+    uint32_t pos[kPer];
+    int list[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const uint64_t v = static_cast<uint64_t>(blockIdx.x) * kListRows + k * 256 + threadIdx.x;
+        list[k] = -1;
+        if (v < V) {
+            const uint64_t d = static_cast<uint64_t>(roff[v + 1]) - static_cast<uint64_t>(roff[v]);
+            if (d > threshold) list[k] = d > huge ? 0 : 1;
+        }
+        if (list[k] >= 0) pos[k] = atomicAdd(&n[list[k]], 1u);
+    }
+    __syncthreads();
+    if (threadIdx.x < 2 && n[threadIdx.x]) base[threadIdx.x] = atomicAdd(&count[threadIdx.x], n[threadIdx.x]);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const uint32_t v = static_cast<uint32_t>(static_cast<uint64_t>(blockIdx.x) * kListRows + k * 256 + threadIdx.x);
+        if (list[k] == 0) rows[base[0] + pos[k]] = v;
+        if (list[k] == 1) rows[cap - 1 - (base[1] + pos[k])] = v;
     }
 }
 
@@ -972,17 +1252,17 @@ extern "C" int bw_pr_vertex_push(uint64_t V, const void *off, int32_t ob, const 
 template<int DIV, int W>
 static int launch_pull(uint64_t V, const void *roff, int32_t ob, const uint32_t *rcols, const uint32_t *deg,
                        const float *pr, float *np, hipStream_t s, uint64_t long_degree = ~0ull,
-                       const uint32_t *long_rows = nullptr, uint32_t nlong = 0)
+                       RowList huge = {}, RowList longs = {})
 {
     const uint64_t blocks = (V + kPullRows - 1) / kPullRows;
     if (blocks > 0x7FFFFFFFull) return fail(BW_HIP_ERR_ARG, "too many vertices for the pull kernel");
     return with_offsets(roff, ob, [&](auto *o) {
         using Off = std::remove_const_t<std::remove_pointer_t<decltype(o)>>;
-        const uint32_t long_blocks = (nlong + kLongWaves - 1) / kLongWaves;
+        const uint64_t long_blocks = static_cast<uint64_t>(huge.n) + (longs.n + kLongWaves - 1) / kLongWaves;
         if (blocks + long_blocks > 0x7FFFFFFFull) return fail(BW_HIP_ERR_ARG, "too many vertices for the pull kernel");
         hipLaunchKernelGGL((pr_pull_kernel<DIV, W, Off>), dim3(static_cast<uint32_t>(blocks + long_blocks)),
-                           dim3(kPullRows), 0, s, V, o, rcols, deg, pr, np, nlong ? long_degree : ~0ull, long_rows,
-                           nlong, long_blocks);
+                           dim3(kPullRows), 0, s, V, o, rcols, deg, pr, np, long_degree, huge, longs,
+                           static_cast<uint32_t>(long_blocks));
         BW_LAUNCH_CHECK();
         return BW_HIP_OK;
     });
@@ -999,15 +1279,19 @@ static int pull_entry(uint64_t V, const void *roff, int32_t ob, const uint32_t *
 
 // Rows with more in-edges than this are summed one wave each
 // (pull_long_rows): beyond it, one thread's sequential sum of a row would
-// hold up the workgroup owning it.
-constexpr uint64_t kLongDegree = 256;
+// hold up the workgroup owning it (R-MAT scale 20, edge factor 16: a pull
+// launch takes 137 us with a split at 64, 119 at 128, 139 at 256).
+constexpr uint64_t kLongDegree = 128;
+// Rows with more in-edges than this get a whole workgroup (pull_huge_row;
+// the same launch: 120 us with a split at 2048, 119 at 4096, 113 at 8192).
+constexpr uint64_t kHugeDegree = 8192;
 
 struct bw_pr_pull_plan {
     uint64_t V = 0;
     const void *roff = nullptr;
     int32_t ob = 4;
     uint32_t *rows = nullptr;
-    uint32_t nlong = 0;
+    RowList huge, longs;       // rows past kHugeDegree, and the others past kLongDegree
     float *contrib = nullptr;  // per-vertex contributions of the dividing variants
     ~bw_pr_pull_plan()
     {
@@ -1038,41 +1322,25 @@ extern "C" int bw_pr_pull_plan_create(bw_pr_pull_plan **out, uint64_t V, const v
             BW_HIP_CHECK(hipStreamSynchronize(s));
         }
         // At most E / (kLongDegree + 1) rows can exceed the threshold; the
-        // count lives in the slot after them.
+        // two counts live in the slots after them.
         const uint64_t cap = E / (kLongDegree + 1);
+        const uint64_t blocks = (V + kListRows - 1) / kListRows;
+        if (blocks > 0x7FFFFFFFull) return fail(BW_HIP_ERR_ARG, "too many vertices for the pull plan");
         if (cap) {
-            // (row, degree) pairs appended on the device, then ordered by
-            // decreasing degree on the host (once per plan), so the longest
-            // rows are dispatched first.
-            uint2 *pairs = nullptr;
-            BW_HIP_CHECK(hipMalloc(&pairs, sizeof(uint2) * (cap + 1)));
-            struct Free {
-                void *p;
-                ~Free() { (void)hipFree(p); }
-            } free_pairs{pairs};
-            uint32_t *count = reinterpret_cast<uint32_t *>(pairs + cap);
-            BW_TRY(bw_hip_fill_u32(count, 0u, 1, s));
-            uint32_t block = 256, grid = 0;
-            BW_TRY(resolve_geometry(nullptr, V, block, grid));
+            BW_HIP_CHECK(hipMalloc(&plan->rows, sizeof(uint32_t) * (cap + 2)));
+            uint32_t *count = plan->rows + cap;
+            BW_TRY(bw_hip_fill_u32(count, 0u, 2, s));
             BW_TRY(with_offsets(roff, ob, [&](auto *o) {
-                hipLaunchKernelGGL(pr_long_rows_kernel, dim3(grid), dim3(block), 0, s, V, o, kLongDegree, pairs,
-                                   count);
+                hipLaunchKernelGGL(pr_long_rows_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(256), 0, s, V, o,
+                                   kLongDegree, kHugeDegree, cap, plan->rows, count);
                 BW_LAUNCH_CHECK();
                 return BW_HIP_OK;
             }));
-            BW_HIP_CHECK(hipMemcpyAsync(&plan->nlong, count, 4, hipMemcpyDeviceToHost, s));
+            uint32_t n[2] = {0, 0};
+            BW_HIP_CHECK(hipMemcpyAsync(n, count, sizeof n, hipMemcpyDeviceToHost, s));
             BW_HIP_CHECK(hipStreamSynchronize(s));
-            if (plan->nlong) {
-                std::vector<uint2> h(plan->nlong);
-                BW_HIP_CHECK(hipMemcpy(h.data(), pairs, sizeof(uint2) * h.size(), hipMemcpyDeviceToHost));
-                std::sort(h.begin(), h.end(), [](const uint2 &a, const uint2 &b) {
-                    return a.y > b.y || (a.y == b.y && a.x < b.x);
-                });
-                std::vector<uint32_t> rows(h.size());
-                for (size_t k = 0; k < h.size(); k++) rows[k] = h[k].x;
-                BW_HIP_CHECK(hipMalloc(&plan->rows, sizeof(uint32_t) * rows.size()));
-                BW_HIP_CHECK(hipMemcpy(plan->rows, rows.data(), sizeof(uint32_t) * rows.size(), hipMemcpyHostToDevice));
-            }
+            plan->huge = RowList{plan->rows, n[0]};
+            plan->longs = RowList{plan->rows + (cap - n[1]), n[1]};
         }
     }
     if (V) BW_HIP_CHECK(hipMalloc(&plan->contrib, sizeof(float) * V));
@@ -1089,7 +1357,7 @@ extern "C" int bw_pr_pull_plan_destroy(bw_pr_pull_plan *plan)
 extern "C" int bw_pr_pull_plan_info(const bw_pr_pull_plan *plan, uint32_t *long_rows)
 {
     if (!plan) return fail(BW_HIP_ERR_ARG, "plan is NULL");
-    if (long_rows) *long_rows = plan->nlong;
+    if (long_rows) *long_rows = plan->huge.n + plan->longs.n;
     return BW_HIP_OK;
 }
 
@@ -1104,8 +1372,7 @@ extern "C" int bw_pr_pull_iteration(const bw_pr_pull_plan *plan, int32_t variant
     hipStream_t s = stream_of(cfg);
     const void *ro = plan->roff;
     const int32_t ob = plan->ob;
-    const uint32_t *lr = plan->rows;
-    const uint32_t nl = plan->nlong;
+    const RowList huge = plan->huge, longs = plan->longs;
     if (variant != BW_PR_VERTEX_PULL && variant != BW_PR_VERTEX_PULL_NODIV && variant != BW_PR_VERTEX_PULL_WARP &&
         variant != BW_PR_VERTEX_PULL_WARP_NODIV)
         return fail(BW_HIP_ERR_ARG, "bw_pr_pull_iteration takes the four pull variants");
@@ -1124,13 +1391,13 @@ extern "C" int bw_pr_pull_iteration(const bw_pr_pull_plan *plan, int32_t variant
         pr = plan->contrib;
     }
     switch (W) {
-    case 1: return launch_pull<0, 1>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, lr, nl);
-    case 2: return launch_pull<0, 2>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, lr, nl);
-    case 4: return launch_pull<0, 4>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, lr, nl);
-    case 8: return launch_pull<0, 8>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, lr, nl);
-    case 16: return launch_pull<0, 16>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, lr, nl);
-    case 32: return launch_pull<0, 32>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, lr, nl);
-    default: return launch_pull<0, 64>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, lr, nl);
+    case 1: return launch_pull<0, 1>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, huge, longs);
+    case 2: return launch_pull<0, 2>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, huge, longs);
+    case 4: return launch_pull<0, 4>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, huge, longs);
+    case 8: return launch_pull<0, 8>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, huge, longs);
+    case 16: return launch_pull<0, 16>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, huge, longs);
+    case 32: return launch_pull<0, 32>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, huge, longs);
+    default: return launch_pull<0, 64>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, huge, longs);
     }
 }
 
