@@ -106,6 +106,36 @@ __device__ __forceinline__ double block_sum_f64(double v, double *lds)
     return t;
 }
 
+// Sum of n (residual, dangling) partials in a fixed order: thread t adds
+// partials t, t + kThreads, ...; then a fixed tree.  Results in thread 0.
+template<int kThreads>
+__device__ __forceinline__ void reduce_partials(const double2 *p, uint32_t n, double &r, double &g, double (*red)[2])
+{
+    r = 0.0;
+    g = 0.0;
+    for (uint32_t i = threadIdx.x; i < n; i += kThreads) {
+        const double2 t = p[i];
+        r += t.x;
+        g += t.y;
+    }
+    r = wave_sum_f64(r);
+    g = wave_sum_f64(g);
+    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+    if (lane == 0) {
+        red[wid][0] = r;
+        red[wid][1] = g;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        r = 0.0;
+        g = 0.0;
+        for (int w = 0; w < kThreads / kWave; w++) {
+            r += red[w][0];
+            g += red[w][1];
+        }
+    }
+}
+
 // Frontier counters: the four Reduction strategies of bfs/bfs.hpp:32-116,
 // with wave64 in place of the 32-wide warp.
 template<int R>

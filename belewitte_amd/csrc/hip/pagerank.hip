@@ -158,6 +158,34 @@ __global__ __launch_bounds__(1024) void pr_struct_edge_list_kernel(uint64_t E, c
     for (uint64_t i = done + gid; i < E; i += stride) push_edge<REV>(edges[2 * i], edges[2 * i + 1], deg, pr, np);
 }
 
+// A PageRank run's iteration launches reduce the (residual, dangling mass)
+// partials of the launch before them in one extra workgroup, their last: a
+// launch of its own would cost more than the reduction.
+struct ReducePrev {
+    const double2 *part = nullptr;  // NULL: no extra workgroup
+    uint32_t n = 0;
+    double *resid = nullptr;
+    double *dangl = nullptr;
+};
+
+struct ReduceLds {
+    double red[16][2];
+};
+
+// Whether this workgroup is the extra one; it has done the reduction then.
+template<int kThreads>
+__device__ __forceinline__ bool reduce_prev(const ReducePrev &p, ReduceLds &lds)
+{
+    if (!p.part || blockIdx.x != gridDim.x - 1) return false;
+    double r, g;
+    reduce_partials<kThreads>(p.part, p.n, r, g, lds.red);
+    if (threadIdx.x == 0) {
+        *p.resid = r;
+        *p.dangl = g;
+    }
+    return true;
+}
+
 // ------------------------------------------------- reverse edge lists
 
 constexpr uint32_t kSegThreads = 256;
@@ -196,8 +224,10 @@ __global__ __launch_bounds__(kSegThreads) void pr_rev_segmented_kernel(uint64_t 
                                                                        const uint32_t *__restrict__ b,
                                                                        const uint32_t *__restrict__ deg,
                                                                        const float *__restrict__ pr, float *np,
-                                                                       int vec)
+                                                                       int vec, ReducePrev prev)
 {
+    __shared__ ReduceLds red;
+    if (reduce_prev<kSegThreads>(prev, red)) return;
     __shared__ uint32_t firstKeys[kSegThreads], lastKeys[kSegThreads];
     __shared__ float sums[kSegThreads];
     __shared__ float waveTotal[kSegThreads / kWave];
@@ -905,17 +935,20 @@ __global__ __launch_bounds__(kPullRows) void pr_pull_kernel(uint64_t V, const Of
                                                              const uint32_t *__restrict__ deg,
                                                              const float *__restrict__ pr, float *np,
                                                              uint64_t long_degree, RowList huge, RowList longs,
-                                                             uint32_t long_blocks)
+                                                             uint32_t long_blocks, ReducePrev prev)
 {
     static_assert(kLongWaves * kWave == kPullRows, "both parts use the same workgroup");
     __shared__ union alignas(16) {
         PullShortLds<Off> s;
         PullLongLds l;
+        ReduceLds r;
     } lds;
+    if (reduce_prev<kPullRows>(prev, lds.r)) return;
+    const uint32_t blocks = gridDim.x - (prev.part ? 1u : 0u);
     if (blockIdx.x < long_blocks)
         pull_long_rows<DIV, W == 1, Off>(blockIdx.x, lds.l, huge, longs, roff, rcols, deg, pr, np);
     else
-        pull_short_rows<DIV, W, Off>(spread_block(blockIdx.x - long_blocks, gridDim.x - long_blocks), lds.s, V, roff,
+        pull_short_rows<DIV, W, Off>(spread_block(blockIdx.x - long_blocks, blocks - long_blocks), lds.s, V, roff,
                                      rcols, deg, pr, np, long_degree);
 }
 
@@ -1050,23 +1083,126 @@ __global__ __launch_bounds__(1024) void pr_dangling_kernel(uint64_t V, const uin
     if (threadIdx.x == 0 && t != 0.0) add_f64(out, t);
 }
 
-__global__ void pr_init_kernel(uint64_t V, float *pr, float *np, const uint32_t *deg, int predivide)
+// What bw_pr_run does between two iterations' sums, in one pass over the
+// vertices: consolidateRank / consolidateRankNoDiv (the arithmetic of
+// pr_consolidate_kernel), the contributions the next iteration gathers
+// (pr_contrib_kernel) and the dangling mass of the new ranks
+// (pr_dangling_kernel).  Each workgroup leaves its (residual, dangling mass)
+// in part[]; the next launch's extra workgroup adds them up in a fixed
+// order, where one atomic per workgroup on one address took most of a pass
+// (R-MAT scale 20: consolidate 11.0 us, contributions 5.4 us, now 8.1 us
+// together; 20 bytes per vertex are 4.3 us of HBM).
+struct FinishArgs {
+    uint64_t V;
+    const uint32_t *deg;      // out-degrees
+    float *pr;
+    float *np;                // the sums
+    float *contrib;           // NULL: nothing gathers contributions
+    const double *dangling;   // UNIFORM: the mass of the ranks just gathered
+    double2 *part;
+    int not_last, nodiv, mode;
+    int zero_np;              // the next sums are added to np
+    int int_degree;           // contributions divide by the degree read as int (vertex_pull_warp.cu:40)
+};
+
+constexpr uint32_t kFinishThreads = 256;
+constexpr uint32_t kFinishVerts = 4 * kFinishThreads;  // per workgroup and step
+constexpr uint32_t kFinishGrid = 4096;                 // most workgroups (and partials)
+
+__device__ __forceinline__ float contribution_of(float rank, uint32_t d, int int_degree)
 {
-    const uint64_t stride = static_cast<uint64_t>(blockDim.x) * gridDim.x;
-    // pagerank/pagerank.cpp:88: 1.0f / vertex_count.
-    const float init = 1.0f / static_cast<float>(V);
-    for (uint64_t v = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; v < V; v += stride) {
-        float x = init;
-        if (predivide && deg[v] != 0) x = init / static_cast<float>(deg[v]);
-        pr[v] = x;
-        np[v] = 0.0f;
+    if (d == 0) return 0.0f;
+    return int_degree ? rank / static_cast<float>(static_cast<int32_t>(d)) : rank / static_cast<float>(d);
+}
+
+// The workgroup's partial, in a fixed order.
+__device__ __forceinline__ void store_partial(double2 *part, double resid, double dangl, ReduceLds &lds)
+{
+    resid = wave_sum_f64(resid);
+    dangl = wave_sum_f64(dangl);
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        lds.red[threadIdx.x / kWave][0] = resid;
+        lds.red[threadIdx.x / kWave][1] = dangl;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double r = 0.0, g = 0.0;
+        for (uint32_t w = 0; w < kFinishThreads / kWave; w++) {
+            r += lds.red[w][0];
+            g += lds.red[w][1];
+        }
+        part[blockIdx.x] = make_double2(r, g);
     }
 }
 
-__global__ void zero_f64_kernel(double *p, uint64_t n)
+__global__ __launch_bounds__(kFinishThreads) void pr_finish_kernel(FinishArgs a)
 {
-    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.0;
+    __shared__ ReduceLds red;
+    const double d = static_cast<double>(kDamp);
+    const double D = a.mode == BW_PR_DANGLING_UNIFORM ? *a.dangling : 0.0;
+    const float baseF = (1.0f - kDamp) / static_cast<float>(a.V);
+    const double baseD = (1.0 - d) / static_cast<double>(a.V);
+    double resid = 0.0, dangl = 0.0;
+    for (uint64_t b0 = static_cast<uint64_t>(blockIdx.x) * kFinishVerts; b0 < a.V;
+         b0 += static_cast<uint64_t>(gridDim.x) * kFinishVerts) {
+        float acc[4], old[4];
+        uint32_t dv[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint64_t v = b0 + k * kFinishThreads + threadIdx.x;
+            const uint64_t w = v < a.V ? v : a.V - 1;
+            acc[k] = a.np[w];
+            old[k] = a.pr[w];
+            dv[k] = a.deg[w];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint64_t v = b0 + k * kFinishThreads + threadIdx.x;
+            if (v >= a.V) continue;
+            float nr;
+            if (a.mode == BW_PR_DANGLING_DROP) {
+                if (a.nodiv) nr = __builtin_fmaf(kDamp, acc[k], baseF);
+                else nr = static_cast<float>(baseD + static_cast<double>(kDamp * acc[k]));
+            } else {
+                nr = static_cast<float>(baseD + d * (static_cast<double>(acc[k]) + D / static_cast<double>(a.V)));
+            }
+            double oldRank = static_cast<double>(old[k]);
+            if (a.nodiv && a.mode == BW_PR_DANGLING_UNIFORM && dv[k] != 0) oldRank *= static_cast<double>(dv[k]);
+            resid += fabs(static_cast<double>(nr) - oldRank);
+            if (dv[k] == 0) dangl += static_cast<double>(nr);
+            a.pr[v] = (a.nodiv && dv[k] != 0 && a.not_last) ? nr / static_cast<float>(dv[k]) : nr;
+            if (a.contrib && a.not_last) a.contrib[v] = contribution_of(nr, dv[k], a.int_degree);
+            if (a.zero_np) a.np[v] = 0.0f;
+        }
+    }
+    store_partial(a.part, resid, dangl, red);
+}
+
+// The initial ranks (1/V, pagerank/pagerank.cpp:88), divided by the
+// out-degree when the nodiv variants start so, their contributions and the
+// dangling mass partials; np starts at zero.
+__global__ __launch_bounds__(kFinishThreads) void pr_start_kernel(FinishArgs a, int predivide)
+{
+    __shared__ ReduceLds red;
+    const float init = 1.0f / static_cast<float>(a.V);
+    double dangl = 0.0;
+    for (uint64_t v = static_cast<uint64_t>(blockIdx.x) * kFinishThreads + threadIdx.x; v < a.V;
+         v += static_cast<uint64_t>(gridDim.x) * kFinishThreads) {
+        const uint32_t d = a.deg[v];
+        a.pr[v] = (predivide && d != 0) ? init / static_cast<float>(d) : init;
+        if (a.contrib) a.contrib[v] = contribution_of(init, d, a.int_degree);
+        a.np[v] = 0.0f;
+        if (d == 0) dangl += static_cast<double>(init);
+    }
+    store_partial(a.part, 0.0, dangl, red);
+}
+
+// The reduction of an extra workgroup as a launch: after the last iteration,
+// and before a pass over the vertices when no launch went before it.
+__global__ __launch_bounds__(256) void pr_reduce_prev_kernel(ReducePrev p)
+{
+    __shared__ ReduceLds red;
+    (void)reduce_prev<256>(p, red);
 }
 
 // ------------------------------------------------------------ host glue
@@ -1188,13 +1324,13 @@ extern "C" int bw_pr_edge_list(uint64_t E, const uint32_t *in, const uint32_t *o
 // per 4096 edges (its fixed geometry; cfg's block and grid do not apply).
 template<bool AOS, bool PRE = false>
 static int launch_rev_segmented(uint64_t E, const uint32_t *a, const uint32_t *b, const uint32_t *deg,
-                                const float *pr, float *np, hipStream_t s)
+                                const float *pr, float *np, hipStream_t s, const ReducePrev &prev = {})
 {
     const uint64_t blocks = (E + kSegBlockEdges - 1) / kSegBlockEdges;
-    if (blocks > 0x7FFFFFFFull) return fail(BW_HIP_ERR_ARG, "too many edges for the reverse edge-list kernel");
+    if (blocks >= 0x7FFFFFFFull) return fail(BW_HIP_ERR_ARG, "too many edges for the reverse edge-list kernel");
     const int vec = aligned16(a) && (AOS || aligned16(b));
-    hipLaunchKernelGGL((pr_rev_segmented_kernel<AOS, PRE>), dim3(static_cast<uint32_t>(blocks)), dim3(kSegThreads),
-                       0, s, E, a, b, deg, pr, np, vec);
+    hipLaunchKernelGGL((pr_rev_segmented_kernel<AOS, PRE>), dim3(static_cast<uint32_t>(blocks) + (prev.part ? 1u : 0u)),
+                       dim3(kSegThreads), 0, s, E, a, b, deg, pr, np, vec, prev);
     BW_LAUNCH_CHECK();
     return BW_HIP_OK;
 }
@@ -1252,17 +1388,16 @@ extern "C" int bw_pr_vertex_push(uint64_t V, const void *off, int32_t ob, const 
 template<int DIV, int W>
 static int launch_pull(uint64_t V, const void *roff, int32_t ob, const uint32_t *rcols, const uint32_t *deg,
                        const float *pr, float *np, hipStream_t s, uint64_t long_degree = ~0ull,
-                       RowList huge = {}, RowList longs = {})
+                       RowList huge = {}, RowList longs = {}, const ReducePrev &prev = {})
 {
     const uint64_t blocks = (V + kPullRows - 1) / kPullRows;
     if (blocks > 0x7FFFFFFFull) return fail(BW_HIP_ERR_ARG, "too many vertices for the pull kernel");
     return with_offsets(roff, ob, [&](auto *o) {
         using Off = std::remove_const_t<std::remove_pointer_t<decltype(o)>>;
         const uint64_t long_blocks = static_cast<uint64_t>(huge.n) + (longs.n + kLongWaves - 1) / kLongWaves;
-        if (blocks + long_blocks > 0x7FFFFFFFull) return fail(BW_HIP_ERR_ARG, "too many vertices for the pull kernel");
-        hipLaunchKernelGGL((pr_pull_kernel<DIV, W, Off>), dim3(static_cast<uint32_t>(blocks + long_blocks)),
-                           dim3(kPullRows), 0, s, V, o, rcols, deg, pr, np, long_degree, huge, longs,
-                           static_cast<uint32_t>(long_blocks));
+        if (blocks + long_blocks >= 0x7FFFFFFFull) return fail(BW_HIP_ERR_ARG, "too many vertices for the pull kernel");
+        hipLaunchKernelGGL((pr_pull_kernel<DIV, W, Off>), dim3(static_cast<uint32_t>(blocks + long_blocks) + (prev.part ? 1u : 0u)), dim3(kPullRows), 0, s, V, o, rcols, deg, pr, np, long_degree, huge, longs,
+                           static_cast<uint32_t>(long_blocks), prev);
         BW_LAUNCH_CHECK();
         return BW_HIP_OK;
     });
@@ -1361,6 +1496,34 @@ extern "C" int bw_pr_pull_plan_info(const bw_pr_pull_plan *plan, uint32_t *long_
     return BW_HIP_OK;
 }
 
+static bool pull_variant(int32_t variant)
+{
+    return variant == BW_PR_VERTEX_PULL || variant == BW_PR_VERTEX_PULL_NODIV || variant == BW_PR_VERTEX_PULL_WARP ||
+           variant == BW_PR_VERTEX_PULL_WARP_NODIV;
+}
+
+// The sums of one pull iteration: np[v] = the sum of c over v's in-neighbours.
+static int pull_sums(const bw_pr_pull_plan *plan, int32_t variant, const uint32_t *rcols, const float *c, float *np,
+                     const bw_launch *cfg, const ReducePrev &prev)
+{
+    const uint64_t V = plan->V;
+    hipStream_t s = stream_of(cfg);
+    const void *ro = plan->roff;
+    const int32_t ob = plan->ob;
+    const RowList huge = plan->huge, longs = plan->longs;
+    uint32_t W = 1, C = 1;
+    if (variant == BW_PR_VERTEX_PULL_WARP || variant == BW_PR_VERTEX_PULL_WARP_NODIV) BW_TRY(warp_params(cfg, W, C));
+    switch (W) {
+    case 1: return launch_pull<0, 1>(V, ro, ob, rcols, nullptr, c, np, s, kLongDegree, huge, longs, prev);
+    case 2: return launch_pull<0, 2>(V, ro, ob, rcols, nullptr, c, np, s, kLongDegree, huge, longs, prev);
+    case 4: return launch_pull<0, 4>(V, ro, ob, rcols, nullptr, c, np, s, kLongDegree, huge, longs, prev);
+    case 8: return launch_pull<0, 8>(V, ro, ob, rcols, nullptr, c, np, s, kLongDegree, huge, longs, prev);
+    case 16: return launch_pull<0, 16>(V, ro, ob, rcols, nullptr, c, np, s, kLongDegree, huge, longs, prev);
+    case 32: return launch_pull<0, 32>(V, ro, ob, rcols, nullptr, c, np, s, kLongDegree, huge, longs, prev);
+    default: return launch_pull<0, 64>(V, ro, ob, rcols, nullptr, c, np, s, kLongDegree, huge, longs, prev);
+    }
+}
+
 extern "C" int bw_pr_pull_iteration(const bw_pr_pull_plan *plan, int32_t variant, const uint32_t *rcols,
                                     const uint32_t *deg, const float *pr, float *np, const bw_launch *cfg)
 {
@@ -1369,17 +1532,10 @@ extern "C" int bw_pr_pull_iteration(const bw_pr_pull_plan *plan, int32_t variant
     if (V == 0) return BW_HIP_OK;
     const bool div = variant == BW_PR_VERTEX_PULL || variant == BW_PR_VERTEX_PULL_WARP;
     if (!rcols || !pr || !np || (div && !deg)) return fail(BW_HIP_ERR_ARG, "NULL device pointer");
-    hipStream_t s = stream_of(cfg);
-    const void *ro = plan->roff;
-    const int32_t ob = plan->ob;
-    const RowList huge = plan->huge, longs = plan->longs;
-    if (variant != BW_PR_VERTEX_PULL && variant != BW_PR_VERTEX_PULL_NODIV && variant != BW_PR_VERTEX_PULL_WARP &&
-        variant != BW_PR_VERTEX_PULL_WARP_NODIV)
-        return fail(BW_HIP_ERR_ARG, "bw_pr_pull_iteration takes the four pull variants");
-    uint32_t W = 1, C = 1;
-    if (variant == BW_PR_VERTEX_PULL_WARP || variant == BW_PR_VERTEX_PULL_WARP_NODIV) BW_TRY(warp_params(cfg, W, C));
+    if (!pull_variant(variant)) return fail(BW_HIP_ERR_ARG, "bw_pr_pull_iteration takes the four pull variants");
     if (div) {
         // The dividing variants gather per-vertex contributions computed here.
+        hipStream_t s = stream_of(cfg);
         const uint64_t blocks = std::min<uint64_t>((V + 255) / 256, 8ull * device_cus());
         if (variant == BW_PR_VERTEX_PULL)
             hipLaunchKernelGGL(pr_contrib_kernel<false>, dim3(static_cast<uint32_t>(blocks)), dim3(256), 0, s, V, deg,
@@ -1390,15 +1546,7 @@ extern "C" int bw_pr_pull_iteration(const bw_pr_pull_plan *plan, int32_t variant
         BW_LAUNCH_CHECK();
         pr = plan->contrib;
     }
-    switch (W) {
-    case 1: return launch_pull<0, 1>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, huge, longs);
-    case 2: return launch_pull<0, 2>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, huge, longs);
-    case 4: return launch_pull<0, 4>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, huge, longs);
-    case 8: return launch_pull<0, 8>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, huge, longs);
-    case 16: return launch_pull<0, 16>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, huge, longs);
-    case 32: return launch_pull<0, 32>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, huge, longs);
-    default: return launch_pull<0, 64>(V, ro, ob, rcols, deg, pr, np, s, kLongDegree, huge, longs);
-    }
+    return pull_sums(plan, variant, rcols, pr, np, cfg, ReducePrev{});
 }
 
 extern "C" int bw_pr_vertex_pull(uint64_t V, const void *roff, int32_t ob, const uint32_t *rcols,
@@ -1519,14 +1667,14 @@ namespace {
 struct RunBuffers {
     uint32_t *deg = nullptr;
     float *np = nullptr;
-    float *contrib = nullptr;  // per-vertex contributions (reverse edge lists)
-    double *acc = nullptr;  // [iterations] residuals, then [iterations] dangling masses
+    float *contrib = nullptr;  // per-vertex contributions (the variants that gather them)
+    double *acc = nullptr;     // [iterations] residuals, [iterations + 1] dangling masses, one spare
+    double2 *part = nullptr;   // per workgroup of a pass over the vertices: (residual, dangling mass)
     ~RunBuffers()
     {
-        if (deg) (void)hipFree(deg);
-        if (np) (void)hipFree(np);
-        if (contrib) (void)hipFree(contrib);
-        if (acc) (void)hipFree(acc);
+        for (void *p : {static_cast<void *>(deg), static_cast<void *>(np), static_cast<void *>(contrib),
+                        static_cast<void *>(acc), static_cast<void *>(part)})
+            if (p) (void)hipFree(p);
     }
 };
 
@@ -1567,44 +1715,30 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
     }
 
     RunBuffers buf;
+    const uint64_t iters = static_cast<uint64_t>(std::max(iterations, 1));
+    const uint32_t passGrid = static_cast<uint32_t>(std::min<uint64_t>((V + kFinishVerts - 1) / kFinishVerts, kFinishGrid));
     BW_HIP_CHECK(hipMalloc(&buf.deg, sizeof(uint32_t) * V));
     BW_HIP_CHECK(hipMalloc(&buf.np, sizeof(float) * V));
-    const uint64_t nacc = 2 * static_cast<uint64_t>(std::max(iterations, 1));
-    BW_HIP_CHECK(hipMalloc(&buf.acc, sizeof(double) * nacc));
-    hipLaunchKernelGGL(zero_f64_kernel, dim3((nacc + 255) / 256), dim3(256), 0, s, buf.acc, nacc);
-    BW_LAUNCH_CHECK();
-    double *resid = buf.acc, *dang = buf.acc + std::max(iterations, 1);
+    BW_HIP_CHECK(hipMalloc(&buf.acc, sizeof(double) * (2 * iters + 2)));
+    BW_HIP_CHECK(hipMalloc(&buf.part, sizeof(double2) * passGrid));
+    if (!nodiv) BW_HIP_CHECK(hipMalloc(&buf.contrib, sizeof(float) * V));
+    double *resid = buf.acc, *dang = buf.acc + iters, *spare = buf.acc + 2 * iters + 1;
 
-    // Degrees once per run (pagerank/pagerank.cpp:102-112); the push
-    // variants have none in the reference and get them from the CSR only
-    // when UNIFORM mode needs the dangling vertices.
+    // Degrees once per run (pagerank/pagerank.cpp:102-112).  With the forward
+    // CSR resident, every variant's out-degrees come from its offsets: the
+    // same integers the variant's own degree kernel counts
+    // (pagerank/pagerank.cu:40-123), without an atomic per edge; the push
+    // variants, which have no degree kernel, read the same offsets.
     BW_TRY(bw_pr_zero_degrees(V, buf.deg, &cfg));
-    // With the forward CSR resident, every variant's out-degrees come from
-    // its offsets: the same integers the variant's own degree kernel counts
-    // (pagerank/pagerank.cu:40-123), without an atomic per edge.
-    const bool needDeg = !(variant == BW_PR_VERTEX_PUSH || variant == BW_PR_VERTEX_PUSH_WARP) ||
-                         mode == BW_PR_DANGLING_UNIFORM;
-    if (needDeg && g->offsets) {
+    if (g->offsets) {
         BW_TRY(bw_pr_degrees_csr(V, g->offsets, g->offset_bytes, buf.deg, &cfg));
     } else switch (variant) {
     case BW_PR_EDGE_LIST: BW_TRY(bw_pr_degrees_edge_list(E, g->el_in, buf.deg, &cfg)); break;
     case BW_PR_REV_EDGE_LIST: BW_TRY(bw_pr_degrees_edge_list(E, g->rel_out, buf.deg, &cfg)); break;
     case BW_PR_STRUCT_EDGE_LIST: BW_TRY(bw_pr_degrees_struct_edge_list(E, g->sel, 0, buf.deg, &cfg)); break;
     case BW_PR_REV_STRUCT_EDGE_LIST: BW_TRY(bw_pr_degrees_struct_edge_list(E, g->rsel, 1, buf.deg, &cfg)); break;
-    case BW_PR_VERTEX_PUSH:
-    case BW_PR_VERTEX_PUSH_WARP:
-        if (mode == BW_PR_DANGLING_UNIFORM) BW_TRY(bw_pr_degrees_csr(V, g->offsets, g->offset_bytes, buf.deg, &cfg));
-        break;
     default:
         BW_TRY(bw_pr_degrees_rev_csr(V, g->rev_offsets, g->offset_bytes, g->rev_cols, buf.deg, &cfg));
-    }
-
-    {
-        uint32_t block, grid;
-        BW_TRY(resolve_geometry(nullptr, V, block, grid));
-        hipLaunchKernelGGL(pr_init_kernel, dim3(grid), dim3(block), 0, s, V, ranks, buf.np, buf.deg,
-                           (nodiv && mode == BW_PR_DANGLING_UNIFORM) ? 1 : 0);
-        BW_LAUNCH_CHECK();
     }
 
     // The push forms scatter through a binned layout (propagation blocking)
@@ -1627,83 +1761,71 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
         if (st != BW_HIP_OK && st != BW_HIP_ERR_ARG) return st;
     }
 
-    // The pull forms split off their long rows (one wave each) once per run.
+    // The pull forms split off their long rows once per run.
     bw_pr_pull_plan *pull = nullptr;
     struct PullGuard {
         bw_pr_pull_plan *&p;
         ~PullGuard() { bw_pr_pull_plan_destroy(p); }
     } pull_guard{pull};
-    if (variant == BW_PR_VERTEX_PULL || variant == BW_PR_VERTEX_PULL_NODIV || variant == BW_PR_VERTEX_PULL_WARP ||
-        variant == BW_PR_VERTEX_PULL_WARP_NODIV)
+    if (pull_variant(variant)) {
+        if (!g->rev_cols) return fail(BW_HIP_ERR_ARG, "NULL device pointer");
         BW_TRY(bw_pr_pull_plan_create(&pull, V, g->rev_offsets, g->offset_bytes, s));
+    }
 
+    FinishArgs fin{};
+    fin.V = V;
+    fin.deg = buf.deg;
+    fin.pr = ranks;
+    fin.np = buf.np;
+    fin.contrib = buf.contrib;
+    fin.part = buf.part;
+    fin.nodiv = nodiv;
+    fin.mode = mode;
+    fin.zero_np = pull == nullptr;  // a pull iteration stores every row's sum
+    fin.int_degree = variant == BW_PR_VERTEX_PULL_WARP;
+    hipLaunchKernelGGL(pr_start_kernel, dim3(passGrid), dim3(kFinishThreads), 0, s, fin,
+                       (nodiv && mode == BW_PR_DANGLING_UNIFORM) ? 1 : 0);
+    BW_LAUNCH_CHECK();
+
+    // Per iteration the sums, whose launch also reduces the partials of the
+    // pass before it, and one pass over the vertices.
     for (int32_t it = 1; it <= iterations; it++) {
-        if (mode == BW_PR_DANGLING_UNIFORM) BW_TRY(bw_pr_dangling_mass(V, buf.deg, ranks, &dang[it - 1], &cfg));
+        const ReducePrev prev{buf.part, passGrid, it > 1 ? &resid[it - 2] : spare, &dang[it - 1]};
+        bool reduced = false;  // the sums' launch reduced `prev`
         if (pull) {
-            BW_TRY(bw_pr_pull_iteration(pull, variant, g->rev_cols, buf.deg, ranks, buf.np, &cfg));
-            BW_TRY(bw_pr_consolidate(V, buf.deg, ranks, buf.np, iterations > it, nodiv, mode,
-                                     mode == BW_PR_DANGLING_UNIFORM ? &dang[it - 1] : nullptr, &resid[it - 1], &cfg));
-            continue;
-        }
-        if (variant == BW_PR_REV_EDGE_LIST || variant == BW_PR_REV_STRUCT_EDGE_LIST) {
-            // One gather per edge: each source's contribution computed once.
-            if (!buf.contrib) BW_HIP_CHECK(hipMalloc(&buf.contrib, sizeof(float) * V));
-            const uint64_t blocks = std::min<uint64_t>((V + 255) / 256, 8ull * device_cus());
-            hipLaunchKernelGGL(pr_contrib_kernel<false>, dim3(static_cast<uint32_t>(blocks)), dim3(256), 0, s, V,
-                               buf.deg, ranks, buf.contrib);
-            BW_LAUNCH_CHECK();
-            if (E) {
-                if (variant == BW_PR_REV_EDGE_LIST)
-                    BW_TRY((launch_rev_segmented<false, true>(E, g->rel_in, g->rel_out, nullptr, buf.contrib, buf.np,
-                                                              s)));
-                else
-                    BW_TRY((launch_rev_segmented<true, true>(E, g->rsel, nullptr, nullptr, buf.contrib, buf.np, s)));
-            }
-            const bool useDeg = nodiv || mode == BW_PR_DANGLING_UNIFORM;
-            BW_TRY(bw_pr_consolidate(V, useDeg ? buf.deg : nullptr, ranks, buf.np, iterations > it, nodiv, mode,
-                                     mode == BW_PR_DANGLING_UNIFORM ? &dang[it - 1] : nullptr, &resid[it - 1], &cfg));
-            continue;
-        }
-        if (scatter) {
+            BW_TRY(pull_sums(pull, variant, g->rev_cols, nodiv ? ranks : buf.contrib, buf.np, &cfg, prev));
+            reduced = true;
+        } else if (E && variant == BW_PR_REV_EDGE_LIST) {
+            BW_TRY((launch_rev_segmented<false, true>(E, g->rel_in, g->rel_out, nullptr, buf.contrib, buf.np, s,
+                                                      prev)));
+            reduced = true;
+        } else if (E && variant == BW_PR_REV_STRUCT_EDGE_LIST) {
+            BW_TRY((launch_rev_segmented<true, true>(E, g->rsel, nullptr, nullptr, buf.contrib, buf.np, s, prev)));
+            reduced = true;
+        } else if (scatter) {
             BW_TRY(bw_pr_scatter_iteration(scatter, buf.deg, ranks, buf.np, s));
-            const bool useDeg = nodiv || mode == BW_PR_DANGLING_UNIFORM;
-            BW_TRY(bw_pr_consolidate(V, useDeg ? buf.deg : nullptr, ranks, buf.np, iterations > it, nodiv, mode,
-                                     mode == BW_PR_DANGLING_UNIFORM ? &dang[it - 1] : nullptr, &resid[it - 1], &cfg));
-            continue;
-        }
-        switch (variant) {
-        case BW_PR_EDGE_LIST: BW_TRY(bw_pr_edge_list(E, g->el_in, g->el_out, buf.deg, ranks, buf.np, &cfg)); break;
-        case BW_PR_REV_EDGE_LIST:
-            BW_TRY(bw_pr_rev_edge_list(E, g->rel_in, g->rel_out, buf.deg, ranks, buf.np, &cfg));
-            break;
-        case BW_PR_STRUCT_EDGE_LIST: BW_TRY(bw_pr_struct_edge_list(E, g->sel, buf.deg, ranks, buf.np, &cfg)); break;
-        case BW_PR_REV_STRUCT_EDGE_LIST:
-            BW_TRY(bw_pr_rev_struct_edge_list(E, g->rsel, buf.deg, ranks, buf.np, &cfg));
-            break;
-        case BW_PR_VERTEX_PUSH:
+        } else if (variant == BW_PR_EDGE_LIST) {
+            BW_TRY(bw_pr_edge_list(E, g->el_in, g->el_out, buf.deg, ranks, buf.np, &cfg));
+        } else if (variant == BW_PR_STRUCT_EDGE_LIST) {
+            BW_TRY(bw_pr_struct_edge_list(E, g->sel, buf.deg, ranks, buf.np, &cfg));
+        } else if (variant == BW_PR_VERTEX_PUSH) {
             BW_TRY(bw_pr_vertex_push(V, g->offsets, g->offset_bytes, g->cols, ranks, buf.np, &cfg));
-            break;
-        case BW_PR_VERTEX_PUSH_WARP:
+        } else if (variant == BW_PR_VERTEX_PUSH_WARP) {
             BW_TRY(bw_pr_vertex_push_warp(V, g->offsets, g->offset_bytes, g->cols, ranks, buf.np, &cfg));
-            break;
-        case BW_PR_VERTEX_PULL:
-            BW_TRY(bw_pr_vertex_pull(V, g->rev_offsets, g->offset_bytes, g->rev_cols, buf.deg, ranks, buf.np, &cfg));
-            break;
-        case BW_PR_VERTEX_PULL_NODIV:
-            BW_TRY(bw_pr_vertex_pull_nodiv(V, g->rev_offsets, g->offset_bytes, g->rev_cols, ranks, buf.np, &cfg));
-            break;
-        case BW_PR_VERTEX_PULL_WARP:
-            BW_TRY(bw_pr_vertex_pull_warp(V, g->rev_offsets, g->offset_bytes, g->rev_cols, buf.deg, ranks, buf.np,
-                                          &cfg));
-            break;
-        case BW_PR_VERTEX_PULL_WARP_NODIV:
-            BW_TRY(bw_pr_vertex_pull_warp_nodiv(V, g->rev_offsets, g->offset_bytes, g->rev_cols, ranks, buf.np,
-                                                &cfg));
-            break;
         }
-        const bool useDeg = nodiv || mode == BW_PR_DANGLING_UNIFORM;
-        BW_TRY(bw_pr_consolidate(V, useDeg ? buf.deg : nullptr, ranks, buf.np, iterations > it, nodiv, mode,
-                                 mode == BW_PR_DANGLING_UNIFORM ? &dang[it - 1] : nullptr, &resid[it - 1], &cfg));
+        if (!reduced) {
+            hipLaunchKernelGGL(pr_reduce_prev_kernel, dim3(1), dim3(256), 0, s, prev);
+            BW_LAUNCH_CHECK();
+        }
+        fin.not_last = iterations > it;
+        fin.dangling = &dang[it - 1];
+        hipLaunchKernelGGL(pr_finish_kernel, dim3(passGrid), dim3(kFinishThreads), 0, s, fin);
+        BW_LAUNCH_CHECK();
+    }
+    if (iterations > 0) {
+        const ReducePrev prev{buf.part, passGrid, &resid[iterations - 1], spare};
+        hipLaunchKernelGGL(pr_reduce_prev_kernel, dim3(1), dim3(256), 0, s, prev);
+        BW_LAUNCH_CHECK();
     }
     if (resid_host && iterations > 0) {
         BW_HIP_CHECK(hipMemcpyAsync(resid_host, resid, sizeof(double) * iterations, hipMemcpyDeviceToHost, s));

@@ -172,36 +172,6 @@ __device__ __forceinline__ void block_kahan(float &s, float &c, float (*wsum)[2]
     }
 }
 
-// Sum of n (residual, dangling) partials in a fixed order: thread t adds
-// partials t, t + kThreads, ...; then a fixed tree.  Results in thread 0.
-template<int kThreads = kBlock>
-__device__ __forceinline__ void reduce_partials(const double2 *p, uint32_t n, double &r, double &g, double (*red)[2])
-{
-    r = 0.0;
-    g = 0.0;
-    for (uint32_t i = threadIdx.x; i < n; i += kThreads) {
-        const double2 t = p[i];
-        r += t.x;
-        g += t.y;
-    }
-    r = wave_sum_f64(r);
-    g = wave_sum_f64(g);
-    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
-    if (lane == 0) {
-        red[wid][0] = r;
-        red[wid][1] = g;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        r = 0.0;
-        g = 0.0;
-        for (int w = 0; w < kThreads / kWave; w++) {
-            r += red[w][0];
-            g += red[w][1];
-        }
-    }
-}
-
 // The last workgroup reduces the previous launch's partials; the others
 // take pieces b, b + (gridDim.x - 1), ...
 template<uint32_t kHot>
@@ -212,7 +182,7 @@ __global__ __launch_bounds__(kBlock) void pr_pieces_kernel(IterArgs a)
     __shared__ float hot[kHot > 0 ? kHot : 1];
     if (blockIdx.x == gridDim.x - 1) {
         double r, g;
-        reduce_partials(a.prev, a.nprev, r, g, red);
+        reduce_partials<kBlock>(a.prev, a.nprev, r, g, red);
         if (threadIdx.x == 0) {
             *a.resid_out = r;
             *a.dangl_out = g;
@@ -945,7 +915,7 @@ __global__ __launch_bounds__(kBlock) void pr_reduce_kernel(const double2 *p, uin
 {
     __shared__ double red[kBlock / kWave][2];
     double r, g;
-    reduce_partials(p, n, r, g, red);
+    reduce_partials<kBlock>(p, n, r, g, red);
     if (threadIdx.x == 0) {
         *resid_out = r;
         *dangl_out = g;
