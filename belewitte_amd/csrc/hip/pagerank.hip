@@ -23,6 +23,7 @@
 //     workgroup on a grid of two workgroups per CU.
 
 #include "common.hpp"
+#include "pagerank_scatter.hpp"
 
 #include <algorithm>
 #include <memory>
@@ -156,34 +157,6 @@ __global__ __launch_bounds__(1024) void pr_struct_edge_list_kernel(uint64_t E, c
         done = E2 * 2;
     }
     for (uint64_t i = done + gid; i < E; i += stride) push_edge<REV>(edges[2 * i], edges[2 * i + 1], deg, pr, np);
-}
-
-// A PageRank run's iteration launches reduce the (residual, dangling mass)
-// partials of the launch before them in one extra workgroup, their last: a
-// launch of its own would cost more than the reduction.
-struct ReducePrev {
-    const double2 *part = nullptr;  // NULL: no extra workgroup
-    uint32_t n = 0;
-    double *resid = nullptr;
-    double *dangl = nullptr;
-};
-
-struct ReduceLds {
-    double red[16][2];
-};
-
-// Whether this workgroup is the extra one; it has done the reduction then.
-template<int kThreads>
-__device__ __forceinline__ bool reduce_prev(const ReducePrev &p, ReduceLds &lds)
-{
-    if (!p.part || blockIdx.x != gridDim.x - 1) return false;
-    double r, g;
-    reduce_partials<kThreads>(p.part, p.n, r, g, lds.red);
-    if (threadIdx.x == 0) {
-        *p.resid = r;
-        *p.dangl = g;
-    }
-    return true;
 }
 
 // ------------------------------------------------- reverse edge lists
@@ -1106,8 +1079,11 @@ struct FinishArgs {
 };
 
 constexpr uint32_t kFinishThreads = 256;
-constexpr uint32_t kFinishVerts = 4 * kFinishThreads;  // per workgroup and step
-constexpr uint32_t kFinishGrid = 4096;                 // most workgroups (and partials)
+constexpr uint32_t kFinishGrid = 4096;  // most workgroups (and partials)
+
+// Vertices per thread and step: four, whose loads are in flight together;
+// one where each vertex's sum is a chain of its own.
+constexpr int finish_per_thread(bool gathered) { return gathered ? 1 : 4; }
 
 __device__ __forceinline__ float contribution_of(float rank, uint32_t d, int int_degree)
 {
@@ -1135,7 +1111,9 @@ __device__ __forceinline__ void store_partial(double2 *part, double resid, doubl
     }
 }
 
-__global__ __launch_bounds__(kFinishThreads) void pr_finish_kernel(FinishArgs a)
+// GATHERED: the sums are the scatter layout's partials, not np.
+template<bool GATHERED>
+__global__ __launch_bounds__(kFinishThreads) void pr_finish_kernel(FinishArgs a, ScatterSums sums)
 {
     __shared__ ReduceLds red;
     const double d = static_cast<double>(kDamp);
@@ -1143,20 +1121,21 @@ __global__ __launch_bounds__(kFinishThreads) void pr_finish_kernel(FinishArgs a)
     const float baseF = (1.0f - kDamp) / static_cast<float>(a.V);
     const double baseD = (1.0 - d) / static_cast<double>(a.V);
     double resid = 0.0, dangl = 0.0;
-    for (uint64_t b0 = static_cast<uint64_t>(blockIdx.x) * kFinishVerts; b0 < a.V;
-         b0 += static_cast<uint64_t>(gridDim.x) * kFinishVerts) {
-        float acc[4], old[4];
-        uint32_t dv[4];
+    constexpr int kPer = finish_per_thread(GATHERED);
+    for (uint64_t b0 = static_cast<uint64_t>(blockIdx.x) * kPer * kFinishThreads; b0 < a.V;
+         b0 += static_cast<uint64_t>(gridDim.x) * kPer * kFinishThreads) {
+        float acc[kPer], old[kPer];
+        uint32_t dv[kPer];
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
+        for (int k = 0; k < kPer; k++) {
             const uint64_t v = b0 + k * kFinishThreads + threadIdx.x;
             const uint64_t w = v < a.V ? v : a.V - 1;
-            acc[k] = a.np[w];
             old[k] = a.pr[w];
             dv[k] = a.deg[w];
+            acc[k] = GATHERED ? sums.row_sum(static_cast<uint32_t>(w)) : a.np[w];
         }
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
+        for (int k = 0; k < kPer; k++) {
             const uint64_t v = b0 + k * kFinishThreads + threadIdx.x;
             if (v >= a.V) continue;
             float nr;
@@ -1716,11 +1695,10 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
 
     RunBuffers buf;
     const uint64_t iters = static_cast<uint64_t>(std::max(iterations, 1));
-    const uint32_t passGrid = static_cast<uint32_t>(std::min<uint64_t>((V + kFinishVerts - 1) / kFinishVerts, kFinishGrid));
     BW_HIP_CHECK(hipMalloc(&buf.deg, sizeof(uint32_t) * V));
     BW_HIP_CHECK(hipMalloc(&buf.np, sizeof(float) * V));
     BW_HIP_CHECK(hipMalloc(&buf.acc, sizeof(double) * (2 * iters + 2)));
-    BW_HIP_CHECK(hipMalloc(&buf.part, sizeof(double2) * passGrid));
+    BW_HIP_CHECK(hipMalloc(&buf.part, sizeof(double2) * kFinishGrid));
     if (!nodiv) BW_HIP_CHECK(hipMalloc(&buf.contrib, sizeof(float) * V));
     double *resid = buf.acc, *dang = buf.acc + iters, *spare = buf.acc + 2 * iters + 1;
 
@@ -1781,7 +1759,10 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
     fin.part = buf.part;
     fin.nodiv = nodiv;
     fin.mode = mode;
-    fin.zero_np = pull == nullptr;  // a pull iteration stores every row's sum
+    const bool gathered = scatter && scatter_gathers(scatter);
+    const uint64_t passVerts = static_cast<uint64_t>(finish_per_thread(gathered)) * kFinishThreads;
+    const uint32_t passGrid = static_cast<uint32_t>(std::min<uint64_t>((V + passVerts - 1) / passVerts, kFinishGrid));
+    fin.zero_np = !pull && !gathered;  // these store every row's sum
     fin.int_degree = variant == BW_PR_VERTEX_PULL_WARP;
     hipLaunchKernelGGL(pr_start_kernel, dim3(passGrid), dim3(kFinishThreads), 0, s, fin,
                        (nodiv && mode == BW_PR_DANGLING_UNIFORM) ? 1 : 0);
@@ -1802,6 +1783,9 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
         } else if (E && variant == BW_PR_REV_STRUCT_EDGE_LIST) {
             BW_TRY((launch_rev_segmented<true, true>(E, g->rsel, nullptr, nullptr, buf.contrib, buf.np, s, prev)));
             reduced = true;
+        } else if (gathered) {
+            BW_TRY(scatter_gather(scatter, buf.contrib, prev, s));
+            reduced = true;
         } else if (scatter) {
             BW_TRY(bw_pr_scatter_iteration(scatter, buf.deg, ranks, buf.np, s));
         } else if (variant == BW_PR_EDGE_LIST) {
@@ -1819,7 +1803,12 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
         }
         fin.not_last = iterations > it;
         fin.dangling = &dang[it - 1];
-        hipLaunchKernelGGL(pr_finish_kernel, dim3(passGrid), dim3(kFinishThreads), 0, s, fin);
+        if (gathered)
+            hipLaunchKernelGGL(pr_finish_kernel<true>, dim3(passGrid), dim3(kFinishThreads), 0, s, fin,
+                               scatter_sums(scatter));
+        else
+            hipLaunchKernelGGL(pr_finish_kernel<false>, dim3(passGrid), dim3(kFinishThreads), 0, s, fin,
+                               ScatterSums{});
         BW_LAUNCH_CHECK();
     }
     if (iterations > 0) {

@@ -6,7 +6,9 @@
 // at about 21 G/s, and at 4.6-7.3 G/s when many edges of an R-MAT graph hit
 // the same hub, so the edge loop cannot get near the HBM roofline that way.
 //
-// Here one iteration is two launches over a layout built once per run:
+// Here one iteration is two launches over a layout built once per run
+// (one, over another layout, for a graph of at most kGatherMaxV vertices:
+// see scatter_gather_kernel):
 //   1. bin: each workgroup streams a fixed range of 8192 edges in their
 //      stored order (source-grouped), computes each edge's contribution,
 //      sorts (destination row within its partition, contribution) by
@@ -21,6 +23,7 @@
 // fixed order either; each row's FP64 partial is rounded once to FP32.
 
 #include "common.hpp"
+#include "pagerank_scatter.hpp"
 
 #include <algorithm>
 #include <memory>
@@ -37,6 +40,22 @@ constexpr uint32_t kBinBaseEdges = 8192;    // edges per bin workgroup (scaled u
 constexpr uint32_t kAccThreads = 512;
 constexpr uint32_t kChunkEdges = 1u << 17;  // most edges one accumulate workgroup sums
 constexpr uint64_t kMaxLayout = 1ull << 25; // partitions x bin workgroups
+// The gathered layout (see scatter_gather_kernel): graphs whose
+// contributions fit an XCD's 4 MB L2.  us per iteration, gathered against
+// binned values: R-MAT, edge factor 16, scale 16 10 / 95, 18 21 / 84, 20
+// 47 / 158, 21 98 / 320, 22 276 / 656; but on uniform graphs past that size
+// the gathers miss the L2 (Erdos-Renyi, edge factor 4, 2^22 vertices
+// 239 / 156, 2^24 1192 / 854), and a bound on sizes has to hold for both.
+constexpr uint64_t kGatherMaxV = 1ull << 20;
+// Its partitions: the smallest power of two of rows, from 2^8 on, that gives
+// at most kGatherParts of them, cut into chunks of E / kGatherChunks edges
+// (at least kGatherMinEdges), so that a few workgroups per CU have work and
+// no partition of hubs holds one up (2^13-row partitions and chunks of 2^17
+// edges left 35 workgroups at 200003 vertices and 3.2 M edges).
+constexpr uint32_t kGatherParts = 1024;
+constexpr uint32_t kGatherMinLog = 8;
+constexpr uint64_t kGatherChunks = 1024;
+constexpr uint64_t kGatherMinEdges = 2048;
 
 // -------------------------------------------------------- edge sources
 
@@ -45,6 +64,8 @@ constexpr uint64_t kMaxLayout = 1ull << 25; // partitions x bin workgroups
 // of its out-edges.
 struct EdgeListSrc {
     const uint32_t *in, *out;
+    __device__ __forceinline__ float contribution(uint32_t s, const uint32_t *__restrict__ deg,
+                                                 const float *__restrict__ pr) const { return value(s, deg, pr); }
     __device__ __forceinline__ void edge(uint64_t e, uint32_t &s, uint32_t &d) const { s = in[e], d = out[e]; }
     // pagerank/edgelist.cu:15-21: pr[src] / deg[src], zero without out-edges.
     __device__ __forceinline__ float value(uint32_t s, const uint32_t *__restrict__ deg,
@@ -56,6 +77,8 @@ struct EdgeListSrc {
 };
 struct StructSrc {
     const uint32_t *pairs;
+    __device__ __forceinline__ float contribution(uint32_t s, const uint32_t *__restrict__ deg,
+                                                 const float *__restrict__ pr) const { return value(s, deg, pr); }
     __device__ __forceinline__ void edge(uint64_t e, uint32_t &s, uint32_t &d) const
     {
         s = pairs[2 * e], d = pairs[2 * e + 1];
@@ -80,6 +103,11 @@ struct CsrSrc {
         const uint64_t n = static_cast<uint64_t>(off[s + 1]) - static_cast<uint64_t>(off[s]);
         return pr[s] / static_cast<float>(static_cast<uint32_t>(n));
     }
+    __device__ __forceinline__ float contribution(uint32_t s, const uint32_t *__restrict__ deg,
+                                                 const float *__restrict__ pr) const
+    {
+        return off[s + 1] != off[s] ? value(s, deg, pr) : 0.0f;
+    }
 };
 
 // src[e] = the CSR row holding edge e, one wave per row.
@@ -100,7 +128,8 @@ __global__ void expand_sources_kernel(uint64_t V, const Off *__restrict__ off, u
 // (partition-major: counts[p * nb + blk]).
 template<typename Src>
 __global__ __launch_bounds__(kBinThreads) void scatter_count_kernel(Src src, uint64_t E, uint32_t per_block,
-                                                                    uint32_t parts, uint32_t nb, uint32_t *counts)
+                                                                    uint32_t parts, uint32_t rows_log, uint32_t nb,
+                                                                    uint32_t *counts)
 {
     __shared__ uint32_t hist[kMaxParts];
     for (uint32_t p = threadIdx.x; p < parts; p += kBinThreads) hist[p] = 0;
@@ -110,7 +139,7 @@ __global__ __launch_bounds__(kBinThreads) void scatter_count_kernel(Src src, uin
     for (uint64_t e = b0 + threadIdx.x; e < b1; e += kBinThreads) {
         uint32_t s, d;
         src.edge(e, s, d);
-        atomicAdd(&hist[d >> kRowsLog], 1u);
+        atomicAdd(&hist[d >> rows_log], 1u);
     }
     __syncthreads();
     for (uint32_t p = threadIdx.x; p < parts; p += kBinThreads)
@@ -371,6 +400,114 @@ __global__ __launch_bounds__(kAccThreads) void scatter_accumulate_kernel(const C
     }
 }
 
+// ------------------------------------------------- gathered layout
+
+// A graph whose contributions (4 bytes per vertex) stay in an XCD's L2 needs
+// no values in its bins: the layout holds each bin's (source, row) pairs and
+// an iteration gathers the sources' contributions instead of writing and
+// reading a value per edge (200003 vertices, 3.2 M edges: bin 22 us and
+// accumulate 77 us, now 11 us; the pairs alone are 19 MB, 4 us of HBM).
+// Slots follow the edges' stored order block by block, so the sources of
+// neighbouring slots are close.
+struct PlaceOut {
+    const uint32_t *base;  // [nb][parts] first slot of each (workgroup, partition)
+    uint32_t *src;         // [E] source
+    uint16_t *row;         // [E] destination row within its partition
+    uint32_t parts;
+    uint32_t rows_log;
+};
+
+// The bins' (source, row) pairs, once per layout: a workgroup takes the
+// edges it counted and hands out its slots of each bin by LDS atomics.
+template<typename Src>
+__global__ __launch_bounds__(kBinThreads) void scatter_place_kernel(Src src, uint64_t E, uint32_t per_block,
+                                                                    PlaceOut o)
+{
+    __shared__ uint32_t cursor[kMaxParts];
+    const uint32_t *b = o.base + static_cast<uint64_t>(blockIdx.x) * o.parts;
+    for (uint32_t p = threadIdx.x; p < o.parts; p += kBinThreads) cursor[p] = b[p];
+    __syncthreads();
+    const uint64_t b0 = static_cast<uint64_t>(blockIdx.x) * per_block;
+    const uint64_t b1 = b0 + per_block < E ? b0 + per_block : E;
+    const uint32_t mask = (1u << o.rows_log) - 1u;
+    for (uint64_t e0 = b0 + threadIdx.x; e0 < b1; e0 += kBinBatch * kBinThreads) {
+        uint32_t s[kBinBatch], d[kBinBatch];
+#pragma unroll
+        for (uint32_t k = 0; k < kBinBatch; k++) {
+            const uint64_t e = e0 + k * kBinThreads;
+            src.edge(e < b1 ? e : b1 - 1, s[k], d[k]);
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kBinBatch; k++) {
+            if (e0 + k * kBinThreads >= b1) continue;
+            const uint32_t slot = atomicAdd(&cursor[d[k] >> o.rows_log], 1u);
+            o.src[slot] = s[k];
+            o.row[slot] = static_cast<uint16_t>(d[k] & mask);
+        }
+    }
+}
+
+// Sums of one chunk of one partition's bin in FP64, written whole to the
+// chunk's slot of partials.  kGatherBatch gathers per thread in flight.
+constexpr uint32_t kGatherThreads = 512;
+constexpr uint32_t kGatherBatch = 8;
+
+struct GatherArgs {
+    const Chunk *chunks;
+    const uint32_t *src;
+    const uint16_t *row;
+    const float *contrib;
+    double *partials;  // [chunk][rows]
+    uint32_t nchunks;
+    uint32_t rows;
+};
+
+__global__ __launch_bounds__(kGatherThreads) void scatter_gather_kernel(GatherArgs a, ReducePrev prev)
+{
+    extern __shared__ double acc[];  // a.rows
+    __shared__ ReduceLds red;
+    if (reduce_prev<kGatherThreads>(prev, red)) return;
+    const Chunk ch = a.chunks[blockIdx.x];
+    for (uint32_t i = threadIdx.x; i < a.rows; i += kGatherThreads) acc[i] = 0.0;
+    __syncthreads();
+    for (uint32_t j0 = ch.begin + threadIdx.x; j0 < ch.end; j0 += kGatherBatch * kGatherThreads) {
+        uint32_t s[kGatherBatch];
+        uint32_t r[kGatherBatch];
+        float c[kGatherBatch];
+#pragma unroll
+        for (uint32_t k = 0; k < kGatherBatch; k++) {
+            const uint32_t j = min(j0 + k * kGatherThreads, ch.end - 1);
+            s[k] = a.src[j];
+            r[k] = a.row[j];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kGatherBatch; k++) c[k] = a.contrib[s[k]];
+#pragma unroll
+        for (uint32_t k = 0; k < kGatherBatch; k++)
+            if (j0 + k * kGatherThreads < ch.end) atomicAdd(&acc[r[k]], static_cast<double>(c[k]));
+    }
+    __syncthreads();
+    double *out = a.partials + static_cast<uint64_t>(blockIdx.x) * a.rows;
+    for (uint32_t i = threadIdx.x; i < a.rows; i += kGatherThreads) out[i] = acc[i];
+}
+
+// c[v] = what a source sends along each of its out-edges.
+template<typename Src>
+__global__ __launch_bounds__(256) void scatter_contrib_kernel(Src src, uint64_t V, const uint32_t *__restrict__ deg,
+                                                              const float *__restrict__ pr, float *c)
+{
+    for (uint64_t v = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; v < V;
+         v += static_cast<uint64_t>(gridDim.x) * blockDim.x)
+        c[v] = src.contribution(static_cast<uint32_t>(v), deg, pr);
+}
+
+// np[v] += its row's sum.
+__global__ __launch_bounds__(256) void scatter_add_kernel(uint64_t V, ScatterSums sums, float *np)
+{
+    const uint64_t v = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (v < V) np[v] += sums.row_sum(static_cast<uint32_t>(v));
+}
+
 }  // namespace
 }  // namespace bw
 
@@ -381,15 +518,21 @@ struct bw_pr_scatter {
     uint64_t V = 0, E = 0;
     const void *a = nullptr, *b = nullptr;
     int32_t ob = 4;
-    uint32_t parts = 0, nb = 0, per_block = 0, nchunks = 0;
-    uint32_t *base = nullptr, *src = nullptr;
+    uint32_t parts = 0, rows_log = 0, nb = 0, per_block = 0, nchunks = 0;
+    bool gather = false;        // the bins hold (source, row) pairs, not (value, row)
+    uint32_t *base = nullptr;
+    uint32_t *src = nullptr;    // CSR: each edge's source; gather: each slot's
     uint16_t *row = nullptr;
-    float *val = nullptr;
+    float *val = nullptr;       // not gather: each slot's contribution
     Chunk *chunks = nullptr;
+    float *contrib = nullptr;   // gather: contributions of bw_pr_scatter_iteration
+    double *partials = nullptr; // gather: one vector of row sums per chunk
+    uint32_t *chunk_base = nullptr;  // gather: each partition's first chunk
     ~bw_pr_scatter()
     {
         for (void *p : {static_cast<void *>(base), static_cast<void *>(src), static_cast<void *>(row),
-                        static_cast<void *>(val), static_cast<void *>(chunks)})
+                        static_cast<void *>(val), static_cast<void *>(chunks), static_cast<void *>(contrib),
+                        static_cast<void *>(partials), static_cast<void *>(chunk_base)})
             if (p) (void)hipFree(p);
     }
 };
@@ -402,6 +545,19 @@ int with_off(const void *off, int32_t ob, F &&f)
     if (ob == 4) return f(static_cast<const uint32_t *>(off));
     if (ob == 8) return f(static_cast<const uint64_t *>(off));
     return fail(BW_HIP_ERR_ARG, "offset_bytes must be 4 or 8");
+}
+
+// f(source) for the stored form of a layout; `expanded` holds a CSR's edges' sources.
+template<typename F>
+int with_source(int32_t kind, const void *a, const void *b, int32_t ob, const uint32_t *expanded, F &&f)
+{
+    if (kind == BW_PR_SCATTER_EDGE_LIST)
+        return f(EdgeListSrc{static_cast<const uint32_t *>(a), static_cast<const uint32_t *>(b)});
+    if (kind == BW_PR_SCATTER_STRUCT) return f(StructSrc{static_cast<const uint32_t *>(a)});
+    return with_off(a, ob, [&](auto *off) {
+        using Off = std::remove_const_t<std::remove_pointer_t<decltype(off)>>;
+        return f(CsrSrc<Off>{off, static_cast<const uint32_t *>(b), expanded});
+    });
 }
 
 // Temporary device buffers of the layout build.
@@ -453,7 +609,13 @@ extern "C" int bw_pr_scatter_create(bw_pr_scatter **out, int32_t kind, uint64_t 
     if (!a || (kind != BW_PR_SCATTER_STRUCT && !b)) return fail(BW_HIP_ERR_ARG, "NULL device pointer");
     if (kind == BW_PR_SCATTER_CSR && offset_bytes != 4 && offset_bytes != 8)
         return fail(BW_HIP_ERR_ARG, "offset_bytes must be 4 or 8");
-    const uint64_t parts = (V + kRows - 1) >> kRowsLog;
+    const bool gather = V <= kGatherMaxV;
+    uint32_t rows_log = kRowsLog;
+    if (gather) {
+        rows_log = kGatherMinLog;
+        while (rows_log < kRowsLog && ((V - 1) >> rows_log) >= kGatherParts) rows_log++;
+    }
+    const uint64_t parts = ((V - 1) >> rows_log) + 1;
     if (parts > kMaxParts || E > 0xFFFFFFFFull)
         return fail(BW_HIP_ERR_ARG, "graph too large for the scatter layout (at most 2^25 vertices and "
                                     "2^32 - 1 edges)");
@@ -466,6 +628,7 @@ extern "C" int bw_pr_scatter_create(bw_pr_scatter **out, int32_t kind, uint64_t 
 
     auto sc = std::make_unique<bw_pr_scatter>();
     sc->kind = kind, sc->V = V, sc->E = E, sc->a = a, sc->b = b, sc->ob = offset_bytes;
+    sc->gather = gather, sc->rows_log = rows_log;
     sc->parts = static_cast<uint32_t>(parts), sc->nb = static_cast<uint32_t>(nb);
     sc->per_block = static_cast<uint32_t>(per);
     const uint64_t cells = parts * nb;
@@ -475,27 +638,38 @@ extern "C" int bw_pr_scatter_create(bw_pr_scatter **out, int32_t kind, uint64_t 
     BW_TRY(tmp.alloc(pos, cells));
     BW_HIP_CHECK(hipMalloc(&sc->base, sizeof(uint32_t) * cells));
     BW_HIP_CHECK(hipMalloc(&sc->row, sizeof(uint16_t) * E));
-    BW_HIP_CHECK(hipMalloc(&sc->val, sizeof(float) * E));
+    if (gather) {
+        BW_HIP_CHECK(hipMalloc(&sc->src, sizeof(uint32_t) * E));
+        BW_HIP_CHECK(hipMalloc(&sc->contrib, sizeof(float) * V));
+    } else {
+        BW_HIP_CHECK(hipMalloc(&sc->val, sizeof(float) * E));
+    }
+    uint32_t *csr_src = nullptr;  // a CSR's edges expanded
 
     if (kind == BW_PR_SCATTER_EDGE_LIST) {
         EdgeListSrc src{static_cast<const uint32_t *>(a), static_cast<const uint32_t *>(b)};
         hipLaunchKernelGGL(scatter_count_kernel<EdgeListSrc>, dim3(sc->nb), dim3(kBinThreads), 0, s, src, E,
-                           sc->per_block, sc->parts, sc->nb, counts);
+                           sc->per_block, sc->parts, sc->rows_log, sc->nb, counts);
     } else if (kind == BW_PR_SCATTER_STRUCT) {
         StructSrc src{static_cast<const uint32_t *>(a)};
         hipLaunchKernelGGL(scatter_count_kernel<StructSrc>, dim3(sc->nb), dim3(kBinThreads), 0, s, src, E,
-                           sc->per_block, sc->parts, sc->nb, counts);
+                           sc->per_block, sc->parts, sc->rows_log, sc->nb, counts);
     } else {
-        BW_HIP_CHECK(hipMalloc(&sc->src, sizeof(uint32_t) * E));
+        if (gather) {
+            BW_TRY(tmp.alloc(csr_src, E));
+        } else {
+            BW_HIP_CHECK(hipMalloc(&sc->src, sizeof(uint32_t) * E));
+            csr_src = sc->src;
+        }
         BW_TRY(with_off(a, offset_bytes, [&](auto *o) {
             using Off = std::remove_const_t<std::remove_pointer_t<decltype(o)>>;
             uint32_t block = 256, grid = 0;
             BW_TRY(resolve_geometry(nullptr, V * kWave, block, grid));
-            hipLaunchKernelGGL(expand_sources_kernel<Off>, dim3(grid), dim3(block), 0, s, V, o, sc->src);
+            hipLaunchKernelGGL(expand_sources_kernel<Off>, dim3(grid), dim3(block), 0, s, V, o, csr_src);
             BW_LAUNCH_CHECK();
-            CsrSrc<Off> src{o, static_cast<const uint32_t *>(b), sc->src};
+            CsrSrc<Off> src{o, static_cast<const uint32_t *>(b), csr_src};
             hipLaunchKernelGGL(scatter_count_kernel<CsrSrc<Off>>, dim3(sc->nb), dim3(kBinThreads), 0, s, src, E,
-                               sc->per_block, sc->parts, sc->nb, counts);
+                               sc->per_block, sc->parts, sc->rows_log, sc->nb, counts);
             return BW_HIP_OK;
         }));
     }
@@ -517,20 +691,61 @@ extern "C" int bw_pr_scatter_create(bw_pr_scatter **out, int32_t kind, uint64_t 
     BW_HIP_CHECK(hipStreamSynchronize(s));
     starts[parts] = static_cast<uint32_t>(E);
     std::vector<Chunk> chunks;
+    std::vector<uint32_t> chunk_base(parts + 1, 0);
+    uint64_t per_chunk = kChunkEdges;
+    if (gather) {
+        const uint64_t want = (E + kGatherChunks - 1) / kGatherChunks;
+        per_chunk = std::min<uint64_t>(std::max<uint64_t>(want, kGatherMinEdges), kChunkEdges);
+    }
     for (uint32_t p = 0; p < parts; p++) {
+        chunk_base[p] = static_cast<uint32_t>(chunks.size());
         const uint32_t b0 = starts[p], b1 = starts[p + 1];
         if (b0 == b1) continue;
-        const uint32_t whole = (b1 - b0) <= kChunkEdges ? 1u : 0u;
-        for (uint32_t c = b0; c < b1; c += kChunkEdges)
-            chunks.push_back(Chunk{p, c, std::min(b1, c + kChunkEdges), whole});
+        const uint32_t whole = (b1 - b0) <= per_chunk ? 1u : 0u;
+        for (uint64_t c = b0; c < b1; c += per_chunk)
+            chunks.push_back(Chunk{p, static_cast<uint32_t>(c), static_cast<uint32_t>(std::min<uint64_t>(b1, c + per_chunk)),
+                                   whole});
     }
+    chunk_base[parts] = static_cast<uint32_t>(chunks.size());
     sc->nchunks = static_cast<uint32_t>(chunks.size());
     BW_HIP_CHECK(hipMalloc(&sc->chunks, sizeof(Chunk) * std::max<size_t>(chunks.size(), 1)));
     if (!chunks.empty())
         BW_HIP_CHECK(hipMemcpy(sc->chunks, chunks.data(), sizeof(Chunk) * chunks.size(), hipMemcpyHostToDevice));
+    if (gather) {
+        BW_HIP_CHECK(hipMalloc(&sc->partials, (sizeof(double) << rows_log) * std::max<size_t>(chunks.size(), 1)));
+        BW_HIP_CHECK(hipMalloc(&sc->chunk_base, sizeof(uint32_t) * (parts + 1)));
+        BW_HIP_CHECK(hipMemcpy(sc->chunk_base, chunk_base.data(), sizeof(uint32_t) * (parts + 1), hipMemcpyHostToDevice));
+        const PlaceOut o{sc->base, sc->src, sc->row, sc->parts, rows_log};
+        BW_TRY(with_source(kind, a, b, offset_bytes, csr_src, [&](auto src) {
+            hipLaunchKernelGGL(scatter_place_kernel<decltype(src)>, dim3(sc->nb), dim3(kBinThreads), 0, s, src, E,
+                               sc->per_block, o);
+            return BW_HIP_OK;
+        }));
+        BW_LAUNCH_CHECK();
+        BW_HIP_CHECK(hipStreamSynchronize(s));
+    }
     *out = sc.release();
     return BW_HIP_OK;
 }
+
+namespace bw {
+
+bool scatter_gathers(const bw_pr_scatter *sc) { return sc->gather; }
+
+ScatterSums scatter_sums(const bw_pr_scatter *sc) { return ScatterSums{sc->partials, sc->chunk_base, sc->rows_log}; }
+
+int scatter_gather(const bw_pr_scatter *sc, const float *contrib, const ReducePrev &prev, hipStream_t s)
+{
+    const uint32_t grid = sc->nchunks + (prev.part ? 1u : 0u);
+    if (!grid) return BW_HIP_OK;
+    const GatherArgs a{sc->chunks, sc->src, sc->row, contrib, sc->partials, sc->nchunks, 1u << sc->rows_log};
+    hipLaunchKernelGGL(scatter_gather_kernel, dim3(grid), dim3(kGatherThreads), sizeof(double) << sc->rows_log, s, a,
+                       prev);
+    BW_LAUNCH_CHECK();
+    return BW_HIP_OK;
+}
+
+}  // namespace bw
 
 extern "C" int bw_pr_scatter_destroy(bw_pr_scatter *sc)
 {
@@ -544,8 +759,21 @@ extern "C" int bw_pr_scatter_iteration(const bw_pr_scatter *sc, const uint32_t *
     if (!sc || !pr || !np) return fail(BW_HIP_ERR_ARG, "bw_pr_scatter_iteration: invalid argument");
     if (sc->kind != BW_PR_SCATTER_CSR && !deg) return fail(BW_HIP_ERR_ARG, "edge-list scatter needs the degrees");
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (sc->gather) {
+        const uint32_t blocks = static_cast<uint32_t>((sc->V + 255) / 256);
+        BW_TRY(with_source(sc->kind, sc->a, sc->b, sc->ob, nullptr, [&](auto src) {
+            hipLaunchKernelGGL(scatter_contrib_kernel<decltype(src)>, dim3(blocks), dim3(256), 0, s, src, sc->V, deg, pr,
+                               sc->contrib);
+            return BW_HIP_OK;
+        }));
+        BW_LAUNCH_CHECK();
+        BW_TRY(scatter_gather(sc, sc->contrib, ReducePrev{}, s));
+        hipLaunchKernelGGL(scatter_add_kernel, dim3(blocks), dim3(256), 0, s, sc->V, scatter_sums(sc), np);
+        BW_LAUNCH_CHECK();
+        return BW_HIP_OK;
+    }
     BinOut o{sc->base, sc->row, sc->val, sc->parts, sc->per_block};
-    auto bin = [&](auto src) {
+    BW_TRY(with_source(sc->kind, sc->a, sc->b, sc->ob, sc->src, [&](auto src) {
         using Src = decltype(src);
         if (sc->per_block == kBinBaseEdges)
             hipLaunchKernelGGL(scatter_bin_staged_kernel<Src>, dim3(sc->nb), dim3(kStagedThreads), 0, s, src, sc->E,
@@ -554,17 +782,7 @@ extern "C" int bw_pr_scatter_iteration(const bw_pr_scatter *sc, const uint32_t *
             hipLaunchKernelGGL(scatter_bin_kernel<Src>, dim3(sc->nb), dim3(kBinThreads), 0, s, src, sc->E, deg, pr,
                                o);
         return BW_HIP_OK;
-    };
-    if (sc->kind == BW_PR_SCATTER_EDGE_LIST) {
-        bin(EdgeListSrc{static_cast<const uint32_t *>(sc->a), static_cast<const uint32_t *>(sc->b)});
-    } else if (sc->kind == BW_PR_SCATTER_STRUCT) {
-        bin(StructSrc{static_cast<const uint32_t *>(sc->a)});
-    } else {
-        BW_TRY(with_off(sc->a, sc->ob, [&](auto *off) {
-            using Off = std::remove_const_t<std::remove_pointer_t<decltype(off)>>;
-            return bin(CsrSrc<Off>{off, static_cast<const uint32_t *>(sc->b), sc->src});
-        }));
-    }
+    }));
     BW_LAUNCH_CHECK();
     if (sc->nchunks) {
         hipLaunchKernelGGL(scatter_accumulate_kernel, dim3(sc->nchunks), dim3(kAccThreads), 0, s, sc->chunks, sc->row,

@@ -368,10 +368,11 @@ int bw_pr_pull_iteration(const bw_pr_pull_plan *plan, int32_t variant,
  * pagerank/edgelist.cu:3-23, struct_edgelist.cu:3-24, vertex_push.cu:3-31,
  * vertex_push_warp.cu:4-49).  Those add each edge's contribution to
  * new_pr[destination] with a global atomic; here a layout built once per
- * graph (bw_pr_scatter_create: one pass over the destinations and a scan,
- * 6 bytes of bins per edge) lets one iteration bin every (destination,
- * contribution) by partition of 8192 rows and sum each partition in LDS
- * (FP64), writing each row once per chunk of its bin.  Sums are added in a
+ * graph (bw_pr_scatter_create: passes over the destinations and a scan, 6
+ * bytes per edge) groups the edges by partition of destination rows, and one
+ * iteration sums each partition in LDS (FP64): from the sources'
+ * contributions where these fit an XCD's L2 (at most 2^20 vertices), else
+ * from bins of contributions it writes first.  Sums are added in a
  * different order than the reference's atomics, which have no fixed order
  * either.  Source kinds: the forward EdgeList (a = in[], b = out[]), the
  * forward StructEdgeList (a = the (in, out) pairs, b unused) or the forward
