@@ -63,25 +63,49 @@ __device__ __forceinline__ uint32_t row_of(const uint32_t *roff, uint32_t lo, ui
     return lo;
 }
 
+// The rows of a step's edges [a, b): the range [r0, r1] of rows they fall
+// into, whose offsets go to LDS when they fit, so that the binary search of
+// each edge's row reads LDS (R-MAT scale 20, 16 M edges: 134 us for a pass
+// over the rows with the offsets read through the caches, 102 with LDS).
+constexpr uint32_t kStagedRows = 4096;
+
+struct RowSearch {
+    uint32_t range[2];
+    uint32_t off[kStagedRows + 1];
+};
+
+// Every thread of the workgroup; the previous step's searches may still run.
+__device__ __forceinline__ void row_search_begin(RowSearch &lds, uint32_t V, const uint32_t *roff, uint32_t a,
+                                                 uint32_t b)
+{
+    __syncthreads();
+    if (threadIdx.x < 2) lds.range[threadIdx.x] = row_of(roff, 0, V - 1, threadIdx.x ? b - 1 : a);
+    __syncthreads();
+    const uint32_t r0 = lds.range[0], n = lds.range[1] - r0 + 1;
+    if (n <= kStagedRows)
+        for (uint32_t i = threadIdx.x; i < n; i += kThreads) lds.off[i] = roff[r0 + i];
+    __syncthreads();
+}
+
+__device__ __forceinline__ uint32_t row_search(const RowSearch &lds, const uint32_t *roff, uint32_t e)
+{
+    const uint32_t r0 = lds.range[0], n = lds.range[1] - r0 + 1;
+    if (n > kStagedRows) return row_of(roff, r0, lds.range[1], e);
+    return r0 + row_of(lds.off, 0, n - 1, e);
+}
+
 // rows[e] = row of reverse edge e; bad = 1 if a column is out of range.
 __global__ __launch_bounds__(kThreads) void plan_rows_kernel(uint32_t V, uint32_t E, const uint32_t *roff,
                                                              const uint32_t *rcols, uint32_t *rows, uint32_t *bad)
 {
-    __shared__ uint32_t range[2];
+    __shared__ RowSearch lds;
     for (uint64_t e0 = static_cast<uint64_t>(blockIdx.x) * kEdgesPerStep; e0 < E;
          e0 += static_cast<uint64_t>(gridDim.x) * kEdgesPerStep) {
         const uint32_t a = static_cast<uint32_t>(e0);
         const uint32_t b = static_cast<uint32_t>(std::min<uint64_t>(e0 + kEdgesPerStep, E));
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const uint32_t r0 = row_of(roff, 0, V - 1, a);
-            range[0] = r0;
-            range[1] = row_of(roff, r0, V - 1, b - 1);
-        }
-        __syncthreads();
-        const uint32_t r0 = range[0], r1 = range[1];
+        row_search_begin(lds, V, roff, a, b);
         for (uint32_t e = a + threadIdx.x; e < b; e += kThreads) {
-            rows[e] = row_of(roff, r0, r1, e);
+            rows[e] = row_search(lds, roff, e);
             if (rcols[e] >= V) *bad = 1u;
         }
     }
@@ -169,10 +193,13 @@ __global__ void plan_bounds_kernel(uint32_t V, uint32_t L, uint32_t K, const uin
 // work (vertices x chunks of the partition + pairs) past kBlockWork.  (The
 // host builder also closes a block whose distinct target partitions would
 // pass kMaxRuns; that never happens, since a plan has at most kMaxRuns
-// partitions.)  One wave: lane j holds the pair count of vertex base + j,
-// and the greedy walks them with wave-uniform state.  Writes each vertex's
-// block (local to the partition) and, at k << L + b, block b's (first
-// vertex, end vertex, pairs, 0); plan_block_runs_kernel fills in the runs.
+// partitions.)  A block's work is perVertex x vertices + pairs, and pbase
+// holds the prefix sums of the pairs, so the end of the block from v0 is the
+// last e whose work fits: one wave finds it by probing 64 vertices at a time
+// (a walk over the vertices took 1.54 ms at R-MAT scale 20, 30 us now).
+// Writes each vertex's block (local to the partition) and, at k << L + b,
+// block b's (first vertex, end vertex, pairs, 0); plan_block_runs_kernel
+// fills in the runs.
 __global__ __launch_bounds__(64) void plan_cut_kernel(uint32_t V, uint32_t L, const uint32_t *pbase,
                                                       const uint32_t *chunk_base, uint32_t *block_local,
                                                       uint4 *pblocks, uint32_t *nblocks)
@@ -181,31 +208,27 @@ __global__ __launch_bounds__(64) void plan_cut_kernel(uint32_t V, uint32_t L, co
     const uint32_t vBeg = k << L;
     const uint32_t vEnd = static_cast<uint32_t>(std::min<uint64_t>(static_cast<uint64_t>(vBeg) + (1u << L), V));
     const uint64_t perVertex = std::max<uint32_t>(1, chunk_base[k + 1] - chunk_base[k]);
-    uint32_t nb = 0, v0 = vBeg, npairs = 0;
-    uint64_t work = 0;
-    auto close_block = [&](uint32_t end) {
-        if (lane == 0) pblocks[vBeg + nb] = make_uint4(v0, end, npairs, 0u);
-        nb++;
-        v0 = end;
-        work = 0;
-        npairs = 0;
-    };
-    for (uint32_t base = vBeg; base < vEnd; base += 64) {
-        const uint32_t s = base + lane, cnt = std::min(64u, vEnd - base);
-        const uint32_t n = s < vEnd ? pbase[s + 1] - pbase[s] : 0u;
-        uint32_t mine = 0;  // the block of vertex s
-        for (uint32_t j = 0; j < cnt; j++) {
-            const uint32_t sj = base + j, nj = __builtin_amdgcn_readlane(n, j);
-            if (sj - v0 >= kBlockVerts) close_block(sj);
-            const uint64_t w = perVertex + nj;
-            if (sj > v0 && work + w > kBlockWork) close_block(sj);
-            npairs += nj;
-            work += w;
-            if (lane == j) mine = nb;
+    uint32_t nb = 0;
+    for (uint32_t v0 = vBeg; v0 < vEnd; nb++) {
+        const uint32_t p0 = pbase[v0];
+        auto fits = [&](uint32_t e) {
+            return e - v0 <= 1 || perVertex * (e - v0) + (pbase[e] - p0) <= kBlockWork;
+        };
+        // The largest e in [lo, hi] that fits; lo = v0 + 1 does.  The work
+        // grows with e, so the lanes that fit are the first ones.
+        uint32_t lo = v0 + 1, hi = std::min(v0 + kBlockVerts, vEnd);
+        while (lo < hi) {
+            const uint32_t step = (hi - lo + 63) / 64;
+            const uint32_t e = std::min(lo + (lane + 1) * step, hi);
+            const uint32_t n = static_cast<uint32_t>(__popcll(__ballot(fits(e))));
+            const uint32_t next = std::min(lo + n * step, hi);
+            if (n < 64) hi = std::min(lo + (n + 1) * step, hi) - 1;  // lane n's e does not fit
+            lo = next;
         }
-        if (s < vEnd) block_local[s] = mine;
+        if (lane == 0) pblocks[vBeg + nb] = make_uint4(v0, lo, pbase[lo] - p0, 0u);
+        for (uint32_t v = v0 + lane; v < lo; v += 64) block_local[v] = nb;
+        v0 = lo;
     }
-    close_block(vEnd);
     if (lane == 0) nblocks[k] = nb;
 }
 
@@ -799,31 +822,42 @@ __global__ __launch_bounds__(kThreads) void relabel_degrees_kernel(uint32_t V, c
     }
 }
 
-// key[j] = (new row << 32) | new column, for new edge j (rows found by
-// binary search over the new offsets within each workgroup's range).
+// New edge j's row and mapped column: as one key (row << 32) | column, or
+// apart.
 __global__ __launch_bounds__(kThreads) void relabel_edges_kernel(uint32_t V, uint32_t E, const uint32_t *off,
                                                                  const uint32_t *cols, const uint32_t *order,
                                                                  const uint32_t *perm, const uint32_t *noff,
-                                                                 uint64_t *key)
+                                                                 uint64_t *key, uint32_t *row, uint32_t *col)
 {
-    __shared__ uint32_t range[2];
+    __shared__ RowSearch lds;
     for (uint64_t e0 = static_cast<uint64_t>(blockIdx.x) * kEdgesPerStep; e0 < E;
          e0 += static_cast<uint64_t>(gridDim.x) * kEdgesPerStep) {
         const uint32_t a = static_cast<uint32_t>(e0);
         const uint32_t b = static_cast<uint32_t>(std::min<uint64_t>(e0 + kEdgesPerStep, E));
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const uint32_t r0 = row_of(noff, 0, V - 1, a);
-            range[0] = r0;
-            range[1] = row_of(noff, r0, V - 1, b - 1);
-        }
-        __syncthreads();
-        const uint32_t r0 = range[0], r1 = range[1];
+        row_search_begin(lds, V, noff, a, b);
         for (uint32_t j = a + threadIdx.x; j < b; j += kThreads) {
-            const uint32_t i = row_of(noff, r0, r1, j);
+            const uint32_t i = row_search(lds, noff, j);
             const uint32_t old = off[order[i]] + (j - noff[i]);
-            key[j] = (static_cast<uint64_t>(i) << 32) | perm[cols[old]];
+            const uint32_t c = perm[cols[old]];
+            if (key) {
+                key[j] = (static_cast<uint64_t>(i) << 32) | c;
+            } else {
+                row[j] = i;
+                col[j] = c;
+            }
         }
+    }
+}
+
+// bad = 1 unless the sorted columns hold each vertex v at its positions
+// [roff[v], roff[v + 1]).
+__global__ __launch_bounds__(kThreads) void relabel_check_kernel(uint32_t V, const uint32_t *roff,
+                                                                 const uint32_t *scol, uint32_t *bad)
+{
+    for (uint64_t v = static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x; v < V;
+         v += static_cast<uint64_t>(gridDim.x) * kThreads) {
+        const uint32_t b = roff[v], e = roff[v + 1];
+        if (b < e && (scol[b] != v || scol[e - 1] != v)) *bad = 1u;
     }
 }
 
@@ -834,26 +868,82 @@ __global__ __launch_bounds__(kThreads) void relabel_cols_kernel(uint32_t E, cons
         ncols[j] = static_cast<uint32_t>(key[j]);
 }
 
+// A permuted direction's offsets.
+hipError_t relabel_offsets(Scratch &sc, uint32_t V, const uint32_t *off, const uint32_t *order, uint32_t *noff,
+                           hipStream_t s)
+{
+    uint32_t *ndeg = sc.get<uint32_t>(static_cast<uint64_t>(V) + 1);
+    if (!ndeg) return hipErrorOutOfMemory;
+    hipLaunchKernelGGL(relabel_degrees_kernel, dim3(grid_for(static_cast<uint64_t>(V) + 1)), dim3(kThreads), 0, s, V,
+                       off, order, ndeg);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = exclusive_scan(sc, ndeg, noff, static_cast<uint64_t>(V) + 1, s);
+    return e;
+}
+
+// Both directions of a directed graph from its forward lists: the permuted
+// lists stably sorted by column are the reverse lists (rows ascending within
+// each column), and those stably sorted by row are the forward lists
+// (columns ascending within each row).  Two sorts by a 20-bit vertex id at
+// scale 20, three passes of 8 bytes each, where sorting each direction by
+// (row, column) took seven passes of an 8-byte key each (1.47 ms, 0.81
+// now).  `transposed` tells whether the in-degrees are those of the reverse
+// lists given; if not these are no transpose and nothing is to be used.
+int relabel_both(Scratch &sc, uint32_t V, uint32_t E, const uint32_t *off, const uint32_t *cols, const uint32_t *roff,
+                 const uint32_t *order, const uint32_t *perm, uint32_t *noff, uint32_t *ncols, uint32_t *nroff,
+                 uint32_t *nrcols, hipStream_t s, bool &transposed, std::string &err)
+{
+    uint32_t *row = sc.get<uint32_t>(E), *col = sc.get<uint32_t>(E), *scol = sc.get<uint32_t>(E);
+    uint32_t *bad = sc.get<uint32_t>(1), hbad = 0;
+    if (!row || !col || !scol || !bad) {
+        err = "device allocation of the relabel failed";
+        return BW_HIP_ERR_NOMEM;
+    }
+    hipError_t e = relabel_offsets(sc, V, off, order, noff, s);
+    if (e == hipSuccess) e = relabel_offsets(sc, V, roff, order, nroff, s);
+    if (e == hipSuccess) e = hipMemsetAsync(bad, 0, sizeof(uint32_t), s);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(relabel_edges_kernel, dim3(grid_for(E, kEdgesPerStep)), dim3(kThreads), 0, s, V, E, off,
+                           cols, order, perm, noff, nullptr, row, col);
+        e = hipGetLastError();
+    }
+    const uint32_t bits = bits_for(V - 1);
+    if (e == hipSuccess)
+        e = sort_pairs(sc, static_cast<const uint32_t *>(col), scol, static_cast<const uint32_t *>(row), nrcols, E,
+                       bits, s);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(relabel_check_kernel, dim3(grid_for(V)), dim3(kThreads), 0, s, V, nroff, scol, bad);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess)
+        e = sort_pairs(sc, static_cast<const uint32_t *>(nrcols), row, static_cast<const uint32_t *>(scol), ncols, E,
+                       bits, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(&hbad, bad, sizeof hbad, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) {
+        err = std::string("relabel: ") + hipGetErrorString(e);
+        return e == hipErrorOutOfMemory ? BW_HIP_ERR_NOMEM : BW_HIP_ERR_RUNTIME;
+    }
+    transposed = !hbad;
+    return BW_HIP_OK;
+}
+
 // One stored direction: rows permuted by `order`, columns mapped by `perm`
 // and sorted within each row.
 int relabel_direction(Scratch &sc, uint32_t V, uint32_t E, const uint32_t *off, const uint32_t *cols,
                       const uint32_t *order, const uint32_t *perm, uint32_t *noff, uint32_t *ncols, hipStream_t s,
                       std::string &err)
 {
-    uint32_t *ndeg = sc.get<uint32_t>(static_cast<uint64_t>(V) + 1);
     uint64_t *key = sc.get<uint64_t>(E);
     uint64_t *skey = sc.get<uint64_t>(E);
-    if (!ndeg || !key || !skey) {
+    if (!key || !skey) {
         err = "device allocation of the relabel failed";
         return BW_HIP_ERR_NOMEM;
     }
-    hipLaunchKernelGGL(relabel_degrees_kernel, dim3(grid_for(static_cast<uint64_t>(V) + 1)), dim3(kThreads), 0, s, V,
-                       off, order, ndeg);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = exclusive_scan(sc, ndeg, noff, static_cast<uint64_t>(V) + 1, s);
+    hipError_t e = relabel_offsets(sc, V, off, order, noff, s);
     if (e == hipSuccess && E) {
         hipLaunchKernelGGL(relabel_edges_kernel, dim3(grid_for(E, kEdgesPerStep)), dim3(kThreads), 0, s, V, E, off,
-                           cols, order, perm, noff, key);
+                           cols, order, perm, noff, key, nullptr, nullptr);
         e = hipGetLastError();
         size_t bytes = 0;
         const uint32_t bits = 32 + bits_for(V - 1);
@@ -929,6 +1019,11 @@ int relabel_by_degree_device(uint32_t V, uint32_t E, const uint32_t *off, const 
     if (e != hipSuccess) {
         err = std::string("relabel: ") + hipGetErrorString(e);
         return e == hipErrorOutOfMemory ? BW_HIP_ERR_NOMEM : BW_HIP_ERR_RUNTIME;
+    }
+    if (roff && E) {
+        bool transposed = false;
+        BW_TRY(relabel_both(sc, V, E, off, cols, roff, order, perm, noff, ncols, nroff, nrcols, s, transposed, err));
+        if (transposed) return BW_HIP_OK;
     }
     BW_TRY(relabel_direction(sc, V, E, off, cols, order, perm, noff, ncols, s, err));
     if (roff) BW_TRY(relabel_direction(sc, V, E, roff, rcols, order, perm, nroff, nrcols, s, err));
