@@ -979,9 +979,11 @@ struct bw_pr_plan {
         uint16_t *psrc = nullptr;
         float *vals = nullptr, *partials = nullptr;
         double2 *part = nullptr;
+        void *slab = nullptr;  // the one allocation behind the arrays (device build)
         void release()
         {
-            for (void *p : {static_cast<void *>(codes), static_cast<void *>(tasks), static_cast<void *>(chunks),
+            if (slab) (void)hipFree(slab);
+            else for (void *p : {static_cast<void *>(codes), static_cast<void *>(tasks), static_cast<void *>(chunks),
                             static_cast<void *>(blocks), static_cast<void *>(chunk_base),
                             static_cast<void *>(run_flat), static_cast<void *>(run_bin), static_cast<void *>(psrc),
                             static_cast<void *>(vals), static_cast<void *>(partials), static_cast<void *>(part)})
@@ -1274,6 +1276,7 @@ int bin_device(bw_pr_plan *plan, uint32_t rows_log2, uint32_t chunk_tasks, bw_pr
     const int st = bins::build_plan_device(static_cast<const uint32_t *>(plan->roff), plan->rcols, plan->V, plan->E,
                                            rows_log2, chunk_tasks, nullptr, d, err);
     if (st != BW_HIP_OK) return fail(st, "binned PageRank plan: " + err);
+    nb.slab = d.slab;
     nb.codes = d.codes;
     nb.tasks = d.tasks;
     nb.chunks = d.chunks;
@@ -1282,8 +1285,9 @@ int bin_device(bw_pr_plan *plan, uint32_t rows_log2, uint32_t chunk_tasks, bw_pr
     nb.run_flat = d.run_flat;
     nb.run_bin = d.run_bin;
     nb.psrc = d.psrc;
-    if (alloc_bin_buffers(nb, rows_log2, d.pairs, d.slots, d.nblocks) != BW_HIP_OK)
-        return fail(BW_HIP_ERR_NOMEM, "device allocation of the binned PageRank buffers failed");
+    nb.vals = d.vals;
+    nb.partials = d.partials;
+    nb.part = d.part;
     nb.nchunks = d.nchunks;
     nb.nblocks = d.nblocks;
     nb.pairs = d.pairs;

@@ -401,27 +401,71 @@ __global__ __launch_bounds__(kThreads) void plan_zero16_kernel(uint64_t n, uint1
         p[i] = 0;
 }
 
-// Device allocations of one build, freed on every path out.
-struct Scratch {
-    std::vector<void *> ptrs;
+// Device scratch of one build, freed on every path out.  The arrays are cut
+// from a few large allocations: one of 16 MB or more costs about 280 us and
+// its release as much, whatever its size, so the thirty arrays of a plan took
+// longer than its kernels (R-MAT scale 20: 9.7 ms for 2.6 ms of kernels,
+// 2.1 ms now).  Everything runs on one stream, so space given back to a
+// mark may be handed out again at once.
+class Scratch {
+public:
+    // `guess`: bytes the build will need, at least about.
+    explicit Scratch(uint64_t guess) : slab_(std::min<uint64_t>(std::max<uint64_t>(guess, 1u << 20), kSlabMax)) {}
+    Scratch(const Scratch &) = delete;
+    Scratch &operator=(const Scratch &) = delete;
     ~Scratch()
     {
-        for (void *p : ptrs)
-            if (p) (void)hipFree(p);
+        for (const Slab &x : slabs_) (void)hipFree(x.p);
     }
+
     template<typename T>
     T *get(uint64_t n)
     {
-        void *p = nullptr;
-        if (hipMalloc(&p, sizeof(T) * std::max<uint64_t>(n, 1)) != hipSuccess) return nullptr;
-        ptrs.push_back(p);
-        return static_cast<T *>(p);
+        const uint64_t bytes = (sizeof(T) * std::max<uint64_t>(n, 1) + 255) & ~255ull;
+        while (cur_ < slabs_.size() && slabs_[cur_].size - used_ < bytes) {
+            cur_++;
+            used_ = 0;
+        }
+        if (cur_ == slabs_.size()) {
+            Slab x{nullptr, std::max(bytes, slab_)};
+            if (hipMalloc(&x.p, x.size) != hipSuccess) {
+                // The array alone may still fit.
+                (void)hipGetLastError();
+                x.size = bytes;
+                if (hipMalloc(&x.p, x.size) != hipSuccess) return nullptr;
+            }
+            slabs_.push_back(x);
+            used_ = 0;
+        }
+        T *out = reinterpret_cast<T *>(static_cast<char *>(slabs_[cur_].p) + used_);
+        used_ += bytes;
+        return out;
     }
-    void give_up(void *p)  // ownership moves to the caller
-    {
-        for (void *&q : ptrs)
-            if (q == p) q = nullptr;
-    }
+
+    // What was handed out since the mark is free again when it goes.
+    class Mark {
+    public:
+        explicit Mark(Scratch &s) : s_(s), cur_(s.cur_), used_(s.used_) {}
+        ~Mark() { s_.cur_ = cur_, s_.used_ = used_; }
+        Mark(const Mark &) = delete;
+        Mark &operator=(const Mark &) = delete;
+
+    private:
+        Scratch &s_;
+        size_t cur_;
+        uint64_t used_;
+    };
+
+private:
+    struct Slab {
+        void *p;
+        uint64_t size;
+    };
+    static constexpr uint64_t kSlabMax = 1ull << 30;
+    uint64_t slab_;
+    std::vector<Slab> slabs_;
+    size_t cur_ = 0;      // the slab being cut
+    uint64_t used_ = 0;   // bytes of it handed out
 };
 
 template<typename K, typename Vv>
@@ -431,6 +475,7 @@ hipError_t sort_pairs(Scratch &sc, const K *kin, K *kout, const Vv *vin, Vv *vou
     size_t bytes = 0;
     hipError_t e = rocprim::radix_sort_pairs(nullptr, bytes, kin, kout, vin, vout, n, 0, bits, s);
     if (e != hipSuccess) return e;
+    Scratch::Mark mark(sc);
     void *tmp = sc.get<uint8_t>(bytes);
     if (!tmp) return hipErrorOutOfMemory;
     return rocprim::radix_sort_pairs(tmp, bytes, kin, kout, vin, vout, n, 0, bits, s);
@@ -441,6 +486,7 @@ hipError_t exclusive_scan(Scratch &sc, const uint32_t *in, uint32_t *out, uint64
     size_t bytes = 0;
     hipError_t e = rocprim::exclusive_scan(nullptr, bytes, in, out, 0u, n, rocprim::plus<uint32_t>(), s);
     if (e != hipSuccess) return e;
+    Scratch::Mark mark(sc);
     void *tmp = sc.get<uint8_t>(bytes);
     if (!tmp) return hipErrorOutOfMemory;
     return rocprim::exclusive_scan(tmp, bytes, in, out, 0u, n, rocprim::plus<uint32_t>(), s);
@@ -450,12 +496,50 @@ hipError_t exclusive_scan(Scratch &sc, const uint32_t *in, uint32_t *out, uint64
 
 void release(DeviceBins &b)
 {
-    for (void *p : {static_cast<void *>(b.codes), static_cast<void *>(b.tasks), static_cast<void *>(b.chunks),
-                    static_cast<void *>(b.blocks), static_cast<void *>(b.chunk_base), static_cast<void *>(b.run_flat),
-                    static_cast<void *>(b.run_bin), static_cast<void *>(b.psrc)})
-        if (p) (void)hipFree(p);
+    if (b.slab) (void)hipFree(b.slab);
     b = DeviceBins();
 }
+
+namespace {
+
+// Lays the plan's arrays and its iteration's buffers out in one allocation.
+hipError_t alloc_outputs(DeviceBins &b, uint64_t max_tasks, uint32_t rows_log2)
+{
+    uint64_t total = 0;
+    auto place = [&total](uint64_t bytes) {
+        const uint64_t at = total;
+        total += (std::max<uint64_t>(bytes, 1) + 255) & ~255ull;
+        return at;
+    };
+    const uint64_t codes = place(sizeof(uint16_t) * b.ncodes), tasks = place(sizeof(uint4) * max_tasks);
+    const uint64_t chunks = place(sizeof(uint4) * static_cast<uint64_t>(b.slots));
+    const uint64_t blocks = place(sizeof(uint4) * static_cast<uint64_t>(b.nblocks));
+    const uint64_t chunk_base = place(sizeof(uint32_t) * (static_cast<uint64_t>(b.K) + 1));
+    const uint64_t run_flat = place(sizeof(uint32_t) * static_cast<uint64_t>(b.nruns));
+    const uint64_t run_bin = place(sizeof(uint32_t) * static_cast<uint64_t>(b.nruns));
+    const uint64_t psrc = place(sizeof(uint16_t) * static_cast<uint64_t>(b.pairs));
+    // 8 values of padding: the accumulate reads 8-pair windows from a lane's first pair
+    const uint64_t vals = place(sizeof(float) * (static_cast<uint64_t>(b.pairs) + 8));
+    const uint64_t partials = place((sizeof(float) << rows_log2) * std::max<uint64_t>(b.slots, 1));
+    const uint64_t part = place(sizeof(double2) * static_cast<uint64_t>(b.nblocks));
+    const hipError_t e = hipMalloc(&b.slab, total);
+    if (e != hipSuccess) return e;
+    char *p = static_cast<char *>(b.slab);
+    b.codes = reinterpret_cast<uint16_t *>(p + codes);
+    b.tasks = reinterpret_cast<uint4 *>(p + tasks);
+    b.chunks = reinterpret_cast<uint4 *>(p + chunks);
+    b.blocks = reinterpret_cast<uint4 *>(p + blocks);
+    b.chunk_base = reinterpret_cast<uint32_t *>(p + chunk_base);
+    b.run_flat = reinterpret_cast<uint32_t *>(p + run_flat);
+    b.run_bin = reinterpret_cast<uint32_t *>(p + run_bin);
+    b.psrc = reinterpret_cast<uint16_t *>(p + psrc);
+    b.vals = reinterpret_cast<float *>(p + vals);
+    b.partials = reinterpret_cast<float *>(p + partials);
+    b.part = reinterpret_cast<double2 *>(p + part);
+    return hipSuccess;
+}
+
+}  // namespace
 
 int build_plan_device(const uint32_t *roff, const uint32_t *rcols, uint32_t V, uint32_t E, uint32_t L,
                       uint32_t chunk_tasks, hipStream_t s, DeviceBins &out, std::string &err)
@@ -479,7 +563,15 @@ int build_plan_device(const uint32_t *roff, const uint32_t *rcols, uint32_t V, u
         err = "too many partitions for the binned layout: raise rows_log2";
         return BW_HIP_ERR_ARG;
     }
-    Scratch sc;
+    // About 60 bytes an edge and 40 a vertex (more where sources reach many
+    // partitions: another slab then).
+    Scratch sc(60ull * E + 40ull * V + (4u << 20));
+    // The arrays to come back; on an error they go.
+    DeviceBins made;
+    struct Guard {
+        DeviceBins &b;
+        ~Guard() { release(b); }
+    } guard{made};
 #define PLAN_TRY(x)                                                                                     \
     do {                                                                                                \
         hipError_t e_ = (x);                                                                            \
@@ -651,19 +743,25 @@ int build_plan_device(const uint32_t *roff, const uint32_t *rcols, uint32_t V, u
         err = "internal error: run count";
         return BW_HIP_ERR_RUNTIME;
     }
-    uint16_t *psrc = sc.get<uint16_t>(U);
-    uint32_t *run_flat = sc.get<uint32_t>(static_cast<uint64_t>(nruns) + NB);
-    uint32_t *run_bin = sc.get<uint32_t>(static_cast<uint64_t>(nruns) + NB);
-    if (!psrc || !run_flat || !run_bin) {
+    made.K = K;
+    made.pairs = U;
+    made.slots = slots;
+    made.nchunks = slots;
+    made.nblocks = NB;
+    made.nruns = nruns + NB;
+    made.ncodes = std::max<uint64_t>(ep, 8);
+    if (alloc_outputs(made, static_cast<uint64_t>(slots) * kChunkWaves, L) != hipSuccess) {
         err = "device allocation of the plan failed";
         return BW_HIP_ERR_NOMEM;
     }
     hipLaunchKernelGGL(plan_runs_kernel, dim3(grid_for(U)), dim3(kThreads), 0, s, U, order, pair_src, pair_block,
-                       blocks, bin_index, run_start, run_scan, psrc, run_flat, run_bin);
+                       blocks, bin_index, run_start, run_scan, made.psrc, made.run_flat, made.run_bin);
     PLAN_TRY(hipGetLastError());
     hipLaunchKernelGGL(plan_terminators_kernel, dim3(grid_for(NB)), dim3(kThreads), 0, s, NB, blocks, pair_scan_b,
-                       bpairs, run_flat, run_bin);
+                       bpairs, made.run_flat, made.run_bin);
     PLAN_TRY(hipGetLastError());
+    PLAN_TRY(hipMemcpyAsync(made.blocks, blocks, sizeof(uint4) * NB, hipMemcpyDeviceToDevice, s));
+    PLAN_TRY(hipMemcpyAsync(made.chunk_base, chunk_base.data(), sizeof(uint32_t) * (K + 1), hipMemcpyHostToDevice, s));
 
     // 5. Edge codes in (partition, source, row) order.
     PLAN_ALLOC(epart, uint32_t, E);
@@ -674,22 +772,17 @@ int build_plan_device(const uint32_t *roff, const uint32_t *rcols, uint32_t V, u
     PLAN_ALLOC(code_scan, uint32_t, static_cast<uint64_t>(E) + 1);
     PLAN_ALLOC(dedge_start, uint32_t, static_cast<uint64_t>(K) + 1);
     PLAN_ALLOC(dustart, uint32_t, static_cast<uint64_t>(K) + 1);
-    const uint64_t ncodes = std::max<uint64_t>(ep, 8);
-    uint16_t *codes = sc.get<uint16_t>(ncodes);
-    if (!codes) {
-        err = "device allocation of the plan failed";
-        return BW_HIP_ERR_NOMEM;
-    }
     PLAN_TRY(hipMemcpyAsync(dedge_start, edge_start.data(), sizeof(uint32_t) * (K + 1), hipMemcpyHostToDevice, s));
     PLAN_TRY(hipMemcpyAsync(dustart, ustart.data(), sizeof(uint32_t) * (K + 1), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(plan_zero16_kernel, dim3(grid_for(ncodes)), dim3(kThreads), 0, s, ncodes, codes);
+    hipLaunchKernelGGL(plan_zero16_kernel, dim3(grid_for(made.ncodes)), dim3(kThreads), 0, s, made.ncodes,
+                       made.codes);
     PLAN_TRY(hipGetLastError());
     hipLaunchKernelGGL(plan_code_keys_kernel, dim3(grid_for(E)), dim3(kThreads), 0, s, E, L, frow, flag, epart, ecode);
     PLAN_TRY(hipGetLastError());
     PLAN_TRY(sort_pairs(sc, static_cast<const uint32_t *>(epart), spart, static_cast<const uint16_t *>(ecode), scode, E,
                         bits_for(K - 1), s));
     hipLaunchKernelGGL(plan_place_codes_kernel, dim3(grid_for(static_cast<uint64_t>(E) + 1)), dim3(kThreads), 0, s, E,
-                       spart, scode, dedge_start, dustart, codes, code_flag);
+                       spart, scode, dedge_start, dustart, made.codes, code_flag);
     PLAN_TRY(hipGetLastError());
     PLAN_TRY(exclusive_scan(sc, code_flag, code_scan, static_cast<uint64_t>(E) + 1, s));
 
@@ -747,40 +840,20 @@ int build_plan_device(const uint32_t *roff, const uint32_t *rcols, uint32_t V, u
     }
     std::stable_sort(chunks.begin(), chunks.end(), [](const Quad &a, const Quad &b) { return a.y - a.x > b.y - b.x; });
     static_assert(sizeof(Quad) == sizeof(uint4), "Quad and uint4 share a layout");
-    uint4 *dtasks = sc.get<uint4>(tasks.size());
-    uint4 *dchunks = sc.get<uint4>(chunks.size());
-    if (!dtasks || !dchunks) {
-        err = "device allocation of the plan failed";
-        return BW_HIP_ERR_NOMEM;
+    if (chunks.size() != slots) {
+        err = "internal error: chunk count";
+        return BW_HIP_ERR_RUNTIME;
     }
     if (!tasks.empty())
-        PLAN_TRY(hipMemcpyAsync(dtasks, tasks.data(), sizeof(uint4) * tasks.size(), hipMemcpyHostToDevice, s));
+        PLAN_TRY(hipMemcpyAsync(made.tasks, tasks.data(), sizeof(uint4) * tasks.size(), hipMemcpyHostToDevice, s));
     if (!chunks.empty())
-        PLAN_TRY(hipMemcpyAsync(dchunks, chunks.data(), sizeof(uint4) * chunks.size(), hipMemcpyHostToDevice, s));
+        PLAN_TRY(hipMemcpyAsync(made.chunks, chunks.data(), sizeof(uint4) * chunks.size(), hipMemcpyHostToDevice, s));
     PLAN_TRY(hipStreamSynchronize(s));
 #undef PLAN_TRY
 #undef PLAN_ALLOC
-
-    out.codes = codes;
-    out.tasks = dtasks;
-    out.chunks = dchunks;
-    out.blocks = blocks;
-    out.chunk_base = dchunk_base;
-    out.run_flat = run_flat;
-    out.run_bin = run_bin;
-    out.psrc = psrc;
-    for (void *p : {static_cast<void *>(codes), static_cast<void *>(dtasks), static_cast<void *>(dchunks),
-                    static_cast<void *>(blocks), static_cast<void *>(dchunk_base), static_cast<void *>(run_flat),
-                    static_cast<void *>(run_bin), static_cast<void *>(psrc)})
-        sc.give_up(p);
-    out.K = K;
-    out.pairs = U;
-    out.slots = slots;
-    out.nchunks = static_cast<uint32_t>(chunks.size());
-    out.nblocks = NB;
-    out.ntasks = static_cast<uint32_t>(tasks.size());
-    out.nruns = nruns + NB;
-    out.ncodes = ncodes;
+    made.ntasks = static_cast<uint32_t>(tasks.size());
+    out = made;
+    made = DeviceBins();  // the caller's now
     return BW_HIP_OK;
 }
 
@@ -893,6 +966,7 @@ int relabel_both(Scratch &sc, uint32_t V, uint32_t E, const uint32_t *off, const
                  const uint32_t *order, const uint32_t *perm, uint32_t *noff, uint32_t *ncols, uint32_t *nroff,
                  uint32_t *nrcols, hipStream_t s, bool &transposed, std::string &err)
 {
+    Scratch::Mark mark(sc);
     uint32_t *row = sc.get<uint32_t>(E), *col = sc.get<uint32_t>(E), *scol = sc.get<uint32_t>(E);
     uint32_t *bad = sc.get<uint32_t>(1), hbad = 0;
     if (!row || !col || !scol || !bad) {
@@ -934,6 +1008,7 @@ int relabel_direction(Scratch &sc, uint32_t V, uint32_t E, const uint32_t *off, 
                       const uint32_t *order, const uint32_t *perm, uint32_t *noff, uint32_t *ncols, hipStream_t s,
                       std::string &err)
 {
+    Scratch::Mark mark(sc);
     uint64_t *key = sc.get<uint64_t>(E);
     uint64_t *skey = sc.get<uint64_t>(E);
     if (!key || !skey) {
@@ -981,7 +1056,9 @@ int relabel_by_degree_device(uint32_t V, uint32_t E, const uint32_t *off, const 
                              const uint32_t *rcols, uint32_t *noff, uint32_t *ncols, uint32_t *nroff, uint32_t *nrcols,
                              uint32_t *perm_out, hipStream_t s, std::string &err)
 {
-    Scratch sc;
+    // About 32 bytes an edge (three edge arrays and a sort's temporaries; the
+    // keys of one direction take as much) and 40 a vertex.
+    Scratch sc(32ull * E + 40ull * V + (4u << 20));
     if (E) {  // every column must name a vertex before it indexes the permutation
         uint32_t *bad = sc.get<uint32_t>(1), hbad = 0;
         if (!bad || hipMemsetAsync(bad, 0, sizeof(uint32_t), s) != hipSuccess) {

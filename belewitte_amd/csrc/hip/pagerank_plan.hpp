@@ -13,12 +13,16 @@
 namespace bw {
 namespace bins {
 
-// Device arrays of a plan (owned by the caller after a successful build).
+// Device arrays of a plan and its iteration's buffers, cut from one
+// allocation (owned by the caller after a successful build).
 struct DeviceBins {
+    void *slab = nullptr;
     uint16_t *codes = nullptr;
     uint4 *tasks = nullptr, *chunks = nullptr, *blocks = nullptr;
     uint32_t *chunk_base = nullptr, *run_flat = nullptr, *run_bin = nullptr;
     uint16_t *psrc = nullptr;
+    float *vals = nullptr, *partials = nullptr;
+    double2 *part = nullptr;
     uint32_t K = 0, pairs = 0, slots = 0, nchunks = 0, nblocks = 0, ntasks = 0, nruns = 0;
     uint64_t ncodes = 0;
 };
