@@ -88,6 +88,33 @@ __device__ __forceinline__ float wave_sum_f32(float v)
     return v;
 }
 
+// Inclusive prefix sum over the wave by DPP row shifts and row broadcasts.
+template<int kCtrl, int kRowMask, bool kBound>
+__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t v)
+{
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), kCtrl, kRowMask, 0xF, kBound));
+}
+
+__device__ __forceinline__ uint32_t wave_prefix_sum(uint32_t x)
+{
+    x += dpp_or_zero<0x111, 0xF, true>(x);
+    x += dpp_or_zero<0x112, 0xF, true>(x);
+    x += dpp_or_zero<0x114, 0xF, true>(x);
+    x += dpp_or_zero<0x118, 0xF, true>(x);
+    x += dpp_or_zero<0x142, 0xA, false>(x);
+    x += dpp_or_zero<0x143, 0xC, false>(x);
+    return x;
+}
+
+__device__ __forceinline__ uint64_t wave_prefix_sum(uint64_t x)
+{
+    for (int o = 1; o < kWave; o <<= 1) {
+        const uint64_t y = __shfl_up(static_cast<unsigned long long>(x), static_cast<unsigned>(o), kWave);
+        if (static_cast<int>(__lane_id()) >= o) x += y;
+    }
+    return x;
+}
+
 // Block-wide sum of a double; result valid in thread 0.  `lds` holds one
 // slot per wave (16 for a 1024-thread block).
 __device__ __forceinline__ double block_sum_f64(double v, double *lds)
@@ -137,40 +164,71 @@ __device__ __forceinline__ void reduce_partials(const double2 *p, uint32_t n, do
 }
 
 // Frontier counters: the four Reduction strategies of bfs/bfs.hpp:32-116,
-// with wave64 in place of the 32-wide warp.
+// with wave64 in place of the 32-wide warp.  Each adds to a counter of the
+// workgroup in LDS -- per discovery, per thread, per wave or by the block --
+// and the workgroup adds that to the global counter once: atomics on one
+// address run one after another (the discoveries of the widest vertex-push
+// level of an R-MAT scale-16 search: 473 us with a global atomic each, 406
+// with this).
+// Every thread of the workgroup constructs and finalises its counter.
+__device__ __forceinline__ uint32_t *workgroup_count()
+{
+    __shared__ uint32_t count;
+    return &count;
+}
+
+struct WorkgroupCount {
+    __device__ __forceinline__ WorkgroupCount()
+    {
+        if (threadIdx.x == 0) *workgroup_count() = 0;
+        __syncthreads();
+    }
+    __device__ __forceinline__ void flush(uint32_t *frontier)
+    {
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const uint32_t total = *workgroup_count();
+            if (total) atomicAdd(frontier, total);
+        }
+    }
+};
+
 template<int R>
 struct FrontierCount;
 
 template<>
-struct FrontierCount<BW_RED_NORMAL> {
-    __device__ __forceinline__ void update(uint32_t *frontier)
-    { atomicAdd(frontier, 1u); }
-    __device__ __forceinline__ void finalise(uint32_t *) {}
+struct FrontierCount<BW_RED_NORMAL> : WorkgroupCount {
+    __device__ __forceinline__ void update() { atomicAdd(workgroup_count(), 1u); }
+    __device__ __forceinline__ void finalise(uint32_t *frontier) { flush(frontier); }
 };
 
 template<>
-struct FrontierCount<BW_RED_BULK> {
+struct FrontierCount<BW_RED_BULK> : WorkgroupCount {
     uint32_t count = 0;
-    __device__ __forceinline__ void update(uint32_t *) { count++; }
-    __device__ __forceinline__ void finalise(uint32_t *frontier)
-    { if (count) atomicAdd(frontier, count); }
-};
-
-template<>
-struct FrontierCount<BW_RED_WAVE> {
-    uint32_t count = 0;
-    __device__ __forceinline__ void update(uint32_t *) { count++; }
+    __device__ __forceinline__ void update() { count++; }
     __device__ __forceinline__ void finalise(uint32_t *frontier)
     {
-        uint32_t total = wave_sum_u32(count);
-        if ((threadIdx.x & (kWave - 1)) == 0 && total) atomicAdd(frontier, total);
+        if (count) atomicAdd(workgroup_count(), count);
+        flush(frontier);
+    }
+};
+
+template<>
+struct FrontierCount<BW_RED_WAVE> : WorkgroupCount {
+    uint32_t count = 0;
+    __device__ __forceinline__ void update() { count++; }
+    __device__ __forceinline__ void finalise(uint32_t *frontier)
+    {
+        const uint32_t total = wave_sum_u32(count);
+        if ((threadIdx.x & (kWave - 1)) == 0 && total) atomicAdd(workgroup_count(), total);
+        flush(frontier);
     }
 };
 
 template<>
 struct FrontierCount<BW_RED_BLOCK> {
     uint32_t count = 0;
-    __device__ __forceinline__ void update(uint32_t *) { count++; }
+    __device__ __forceinline__ void update() { count++; }
     __device__ __forceinline__ void finalise(uint32_t *frontier)
     {
         __shared__ uint32_t partial[1024 / kWave];

@@ -357,33 +357,6 @@ __device__ __forceinline__ float pull_contribution(const float *__restrict__ pr,
     else return pr[u];
 }
 
-// Inclusive prefix sum over the wave by DPP row shifts and row broadcasts.
-template<int kCtrl, int kRowMask, bool kBound>
-__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t v)
-{
-    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), kCtrl, kRowMask, 0xF, kBound));
-}
-
-__device__ __forceinline__ uint32_t wave_prefix_sum(uint32_t x)
-{
-    x += dpp_or_zero<0x111, 0xF, true>(x);
-    x += dpp_or_zero<0x112, 0xF, true>(x);
-    x += dpp_or_zero<0x114, 0xF, true>(x);
-    x += dpp_or_zero<0x118, 0xF, true>(x);
-    x += dpp_or_zero<0x142, 0xA, false>(x);
-    x += dpp_or_zero<0x143, 0xC, false>(x);
-    return x;
-}
-
-__device__ __forceinline__ uint64_t wave_prefix_sum(uint64_t x)
-{
-    for (int o = 1; o < kWave; o <<= 1) {
-        const uint64_t y = __shfl_up(static_cast<unsigned long long>(x), static_cast<unsigned>(o), kWave);
-        if (static_cast<int>(__lane_id()) >= o) x += y;
-    }
-    return x;
-}
-
 // The pull iteration of pagerank/vertex_pull.cu:16-30, vertex_pull_nodiv.cu,
 // vertex_pull_warp.cu:4-49 and vertex_pull_warp_nodiv.cu:4-47 for wave64:
 // a workgroup owns kPullRows consecutive rows of the reverse CSR and streams
