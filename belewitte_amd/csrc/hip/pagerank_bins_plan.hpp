@@ -34,7 +34,7 @@
 namespace bw {
 namespace bins {
 
-// Scatter block limits (measured on R-MAT scale 22: 2048 / 32768 beat
+// Largest scatter block (measured on R-MAT scale 22: 2048 / 32768 beat
 // 512 / 8192, 1024 / 16384, 4096 / 65536 and 8192 / 131072).
 #ifndef BW_BINS_BLOCK_VERTS
 #define BW_BINS_BLOCK_VERTS 2048
@@ -45,9 +45,25 @@ namespace bins {
 constexpr uint32_t kTaskEdges = 2048;    // unit of the chunk size (chunk_tasks x kTaskEdges edges at most)
 constexpr uint32_t kChunkWaves = 16;     // tasks per chunk: one per wave of the accumulate workgroup
 constexpr uint32_t kMaxRuns = 2048;      // partitions one scatter block may point into
-constexpr uint32_t kBlockVerts = BW_BINS_BLOCK_VERTS;  // vertices of one scatter block at most
+constexpr uint32_t kBlockVerts = BW_BINS_BLOCK_VERTS;  // vertices of one scatter block at most (block_verts)
 constexpr uint32_t kBlockWork = BW_BINS_BLOCK_WORK;    // vertices x chunks of their partition + pairs, per block
 constexpr uint16_t kNewPair = 0x8000;    // edge code flag: the edge opens a new pair
+
+// Scatter block limits of a graph of V vertices.  One workgroup finalises a
+// block, and the block with the most work ends last, so smaller graphs take
+// smaller blocks: the vertices halved, down to 256, until there are two blocks
+// per compute unit, the work in proportion to V.  The finalise at 150001
+// vertices (undirected R-MAT, edge factor 16): 14.6 us with the largest
+// blocks, 6.7 with these; the iteration at 2^20 vertices 68 us with a work
+// limit of 32768, 62 with 16384, 58 with 8192; at 2^21 74, 66, 67; at 2^22
+// 93.5, 98, 106.
+inline uint32_t block_verts(uint32_t V)
+{
+    uint32_t n = kBlockVerts;
+    while (n > 256 && V / n < 512) n /= 2;
+    return n;
+}
+inline uint32_t block_work(uint32_t V) { return std::min(std::max(V / 128, 2048u), kBlockWork); }
 
 struct Quad {
     uint32_t x, y, z, w;
@@ -165,11 +181,12 @@ inline bool build_plan(const uint32_t *off, const uint32_t *cols, uint32_t V, ui
     P.slots = P.chunk_base[K];
 
     // Scatter blocks: consecutive vertices of one partition, cut so that
-    // vertices x chunks of the partition + pairs stays within kBlockWork,
-    // at most kBlockVerts vertices and kMaxRuns runs.
+    // vertices x chunks of the partition + pairs stays within block_work(V),
+    // at most block_verts(V) vertices and kMaxRuns runs.
     std::vector<uint32_t> stamp(K, UINT32_MAX), blen(K, 0), done(K, 0), touched;
     std::vector<uint32_t> blockOf(V), runPart;
     uint32_t flat = 0;
+    const uint32_t maxVerts = block_verts(V), maxWork = block_work(V);
     for (uint32_t k = 0; k < K; k++) {
         const uint32_t vEnd = std::min<uint64_t>((static_cast<uint64_t>(k) << L) + D, V);
         const uint64_t perVertex = std::max<uint32_t>(1, P.chunk_base[k + 1] - P.chunk_base[k]);
@@ -178,7 +195,7 @@ inline bool build_plan(const uint32_t *off, const uint32_t *cols, uint32_t V, ui
             const uint32_t id = static_cast<uint32_t>(P.blocks.size()), v0 = s;
             uint64_t work = 0;
             touched.clear();
-            while (s < vEnd && s - v0 < kBlockVerts) {
+            while (s < vEnd && s - v0 < maxVerts) {
                 uint32_t fresh = 0, prev = UINT32_MAX;
                 for (uint32_t e = foff[s]; e < foff[s + 1]; e++) {
                     const uint32_t kk = frow[e] >> L;
@@ -186,7 +203,7 @@ inline bool build_plan(const uint32_t *off, const uint32_t *cols, uint32_t V, ui
                     prev = kk;
                 }
                 const uint64_t w = perVertex + pairsS[s];
-                if (s > v0 && (work + w > kBlockWork || touched.size() + fresh > kMaxRuns)) break;
+                if (s > v0 && (work + w > maxWork || touched.size() + fresh > kMaxRuns)) break;
                 prev = UINT32_MAX;
                 for (uint32_t e = foff[s]; e < foff[s + 1]; e++) {
                     const uint32_t kk = frow[e] >> L;

@@ -471,6 +471,9 @@ struct BinArgs {
     uint32_t npairs;            // length of bins (at least 1)
     float *bins;                // one contribution per pair, times pair_scale
     float *partials;            // [slot][rows per partition]
+    uint32_t split;             // workgroups per chunk (1: the chunk's whole sums become its partial)
+    const uint4 *pieces;        // split > 1: per task its `split` pieces
+    unsigned long long *sums;   // split > 1: [slot][piece][rows per partition] fixed-point sums
     const uint32_t *chunk_base; // per partition: its first slot (K + 1)
     const uint4 *blocks;        // (first vertex, end vertex, run begin, run count)
     uint32_t nblocks;
@@ -580,18 +583,21 @@ __global__ __launch_bounds__(kThreads, kRowsLog == 13 ? 8 : 4) void pr_bins_accu
                 reinterpret_cast<const u32x4 *>(reinterpret_cast<const char *>(a.codes) + off));
         }
     };
-    for (uint32_t c = blockIdx.x; c < a.nchunks; c += gridDim.x - 1) {
-        const uint4 ch = a.chunks[c];
+    for (uint32_t c = blockIdx.x; c < a.nchunks * a.split; c += gridDim.x - 1) {
+        const uint32_t piece = c % a.split;
+        const uint4 ch = a.chunks[c / a.split];
         for (uint32_t i = threadIdx.x; i < kRows; i += kThreads) acc[i] = 0ull;
         // Task records come from LDS in the loop: a global load there would
         // make every wait for it a wait for all the loads in flight.
-        for (uint32_t i = threadIdx.x; i < ch.y - ch.x; i += kThreads) stask[i] = a.tasks[ch.x + i];
+        for (uint32_t i = threadIdx.x; i < ch.y - ch.x; i += kThreads)
+            stask[i] = a.split == 1 ? a.tasks[ch.x + i] : a.pieces[static_cast<size_t>(ch.x + i) * a.split + piece];
         __syncthreads();
         // The wave's rounds, over its tasks of the chunk (t = ch.x + wid,
         // t + kWaves, ...: one task per wave with the plan's even splits),
         // are software-pipelined as set out above the loop below.
         uint32_t t = __builtin_amdgcn_readfirstlane(ch.x + wid);
-        if (t < ch.y) {
+        // (A short task has fewer pieces than workgroups: an empty one is skipped.)
+        if (t < ch.y && stask[t - ch.x].x < stask[t - ch.x].y) {
             uint4 tk = stask[t - ch.x];   // task of the round being staged
             uint32_t base = tk.z;
             uint32_t le = tk.x;           // edge of the round whose codes are loaded next
@@ -781,9 +787,17 @@ __global__ __launch_bounds__(kThreads, kRowsLog == 13 ? 8 : 4) void pr_bins_accu
         wave_done:;
         }
         __syncthreads();
-        float *out = a.partials + static_cast<size_t>(ch.w) * kRows;
-        for (uint32_t i = threadIdx.x; i < kRows; i += kThreads)
-            out[i] = static_cast<float>(acc[i]) * a.partial_scale;
+        if (a.split == 1) {
+            float *out = a.partials + static_cast<size_t>(ch.w) * kRows;
+            for (uint32_t i = threadIdx.x; i < kRows; i += kThreads)
+                out[i] = static_cast<float>(acc[i]) * a.partial_scale;
+        } else {
+            // The rows that exist; the finalise adds the pieces' sums (exact)
+            // before it rounds them to the partial.
+            const uint32_t n = min(kRows, a.V - (ch.z << kRowsLog));
+            unsigned long long *out = a.sums + (static_cast<size_t>(ch.w) * a.split + piece) * kRows;
+            for (uint32_t i = threadIdx.x; i < n; i += kThreads) out[i] = acc[i];
+        }
         __syncthreads();  // acc is cleared for the next chunk
     }
 }
@@ -798,7 +812,7 @@ __global__ __launch_bounds__(kThreads, kRowsLog == 13 ? 8 : 4) void pr_bins_accu
 #ifndef BW_BINS_SCATTER_UNROLL
 #define BW_BINS_SCATTER_UNROLL 8  // pair stores per lane and step of the scatter
 #endif
-template<int kRowsLog, int kThreads>
+template<int kRowsLog, int kThreads, bool kSplit>
 __global__ __launch_bounds__(kThreads) void pr_bins_finalise_kernel(BinArgs a)
 {
     constexpr int kScatterUnroll = BW_BINS_SCATTER_UNROLL;
@@ -823,7 +837,25 @@ __global__ __launch_bounds__(kThreads) void pr_bins_finalise_kernel(BinArgs a)
             const uint32_t vi = v0 + threadIdx.x / G;
             const bool live = vi < nv;
             double s = 0.0;
-            if (live && a.phase) {
+            if (kSplit && live && a.phase) {
+                // Slot c0 + q's pieces, eight loads in flight; their sum is
+                // rounded as the whole chunk's is.
+                for (uint32_t q = sub; q < ns; q += G) {
+                    const unsigned long long *pv =
+                        a.sums + (static_cast<size_t>(c0 + q) * a.split << kRowsLog) + (bl.x - rbase) + vi;
+                    unsigned long long sum = 0;
+                    for (uint32_t j = 0; j < a.split; j += 8) {
+                        unsigned long long t[8];
+#pragma unroll
+                        for (uint32_t i = 0; i < 8; i++)
+                            t[i] = j + i < a.split ? pv[static_cast<size_t>(j + i) << kRowsLog] : 0ull;
+#pragma unroll
+                        for (uint32_t i = 0; i < 8; i++) sum += t[i];
+                    }
+                    s += static_cast<double>(static_cast<float>(sum) * a.partial_scale);
+                }
+            }
+            if (!kSplit && live && a.phase) {
                 // partial of slot c0 + q for vertex bl.x + vi: [c0 + q][bl.x + vi - rbase]
                 const float *pv = a.partials + (static_cast<size_t>(c0) << kRowsLog) + (bl.x - rbase) + vi;
                 uint32_t q = sub;
@@ -909,6 +941,33 @@ __global__ __launch_bounds__(kThreads) void pr_bins_finalise_kernel(BinArgs a)
     write_partial<kThreads>(a.part, resid, dangl, red);
 }
 
+// The pieces of each task, one wave per task: whole 64-edge lines split
+// evenly (as many lines a piece as the task has, rounded), each with the pair
+// of its first edge from a count of the new-pair flags before it.
+constexpr uint32_t kMaxSplit = 16;
+
+__global__ __launch_bounds__(256) void pr_split_tasks_kernel(uint32_t ntasks, const uint4 *tasks,
+                                                             const uint16_t *codes, uint32_t split, uint4 *pieces)
+{
+    const uint32_t t = blockIdx.x * (256 / kWave) + threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+    if (t >= ntasks) return;
+    const uint4 tk = tasks[t];
+    const uint32_t lines = (tk.y - tk.x + 63) / 64;
+    uint32_t base = tk.z, at = 0;
+    for (uint32_t j = 0; j < split; j++) {
+        const uint32_t l1 = static_cast<uint32_t>(static_cast<uint64_t>(lines) * (j + 1) / split);
+        const uint32_t b = tk.x + at * 64, e = min(tk.x + l1 * 64, tk.y);
+        if (lane == 0) pieces[static_cast<size_t>(t) * split + j] = make_uint4(b, max(b, e), base, tk.w);
+        uint32_t flags = 0;
+        for (uint32_t l = at; l < l1; l++) {
+            const uint32_t i = tk.x + l * 64 + lane;
+            flags += i < tk.y ? codes[i] >> 15 : 0u;
+        }
+        base += wave_sum_u32(flags);
+        at = l1;
+    }
+}
+
 // Reduction of the last launch's partials (after the loop).
 __global__ __launch_bounds__(kBlock) void pr_reduce_kernel(const double2 *p, uint32_t n, double *resid_out,
                                                            double *dangl_out)
@@ -980,8 +1039,12 @@ struct bw_pr_plan {
         float *vals = nullptr, *partials = nullptr;
         double2 *part = nullptr;
         void *slab = nullptr;  // the one allocation behind the arrays (device build)
+        uint32_t split = 1;    // workgroups per chunk of the accumulate (split_chunks)
+        uint4 *pieces = nullptr;             // [task][split]
+        unsigned long long *sums = nullptr;  // [slot][split][rows], in the allocation of `pieces`
         void release()
         {
+            if (pieces) (void)hipFree(pieces);
             if (slab) (void)hipFree(slab);
             else for (void *p : {static_cast<void *>(codes), static_cast<void *>(tasks), static_cast<void *>(chunks),
                             static_cast<void *>(blocks), static_cast<void *>(chunk_base),
@@ -1299,6 +1362,41 @@ int bin_device(bw_pr_plan *plan, uint32_t rows_log2, uint32_t chunk_tasks, bw_pr
     return BW_HIP_OK;
 }
 
+// A graph of few chunks leaves most CUs idle in the accumulate, and a chunk
+// cannot be smaller without changing the partials.  Its tasks are cut into
+// `split` pieces instead, one workgroup per piece, whose fixed-point sums the
+// finalise adds exactly: the ranks are the same bit for bit.  The pieces' sums
+// (8 bytes a row each) cost the finalise what they save the accumulate beyond
+// about half the CUs, so up to 64 chunks are cut into 128 workgroups' worth,
+// up to 128 in two, and no piece is shorter than 8192 edges.  us per
+// iteration, whole chunks / pieces: 50021 vertices (4 chunks) 40.7 / 18,
+// 150001 (21) 44.9 / 28 (192 or 256 workgroups: 32), 300007 (42) 47.7 / 34,
+// 600011 (65) 53 / 35, 2^20 (117) 58 / 46.
+constexpr uint32_t kSplitChunks = 128;
+constexpr uint64_t kMinPiece = 8192;
+
+int split_chunks(bw_pr_plan::Bins &nb)
+{
+    nb.split = 1;
+    if (nb.nchunks == 0 || nb.nchunks > kSplitChunks) return BW_HIP_OK;
+    const uint64_t want = std::max(kSplitChunks / nb.nchunks, 2u), most = nb.ncodes / nb.nchunks / kMinPiece;
+    const uint32_t split = static_cast<uint32_t>(std::min<uint64_t>({want, kMaxSplit, most}));
+    if (split < 2) return BW_HIP_OK;
+    const size_t pieces = (sizeof(uint4) * nb.ntasks * split + 255) & ~size_t{255};
+    const size_t sums = (sizeof(unsigned long long) << nb.log2) * nb.slots * split;
+    if (hipMalloc(&nb.pieces, pieces + sums) != hipSuccess) {
+        nb.pieces = nullptr;
+        return fail(BW_HIP_ERR_NOMEM, "device allocation of the binned PageRank buffers failed");
+    }
+    nb.sums = reinterpret_cast<unsigned long long *>(reinterpret_cast<char *>(nb.pieces) + pieces);
+    hipLaunchKernelGGL(pr_split_tasks_kernel, dim3((nb.ntasks + 3) / 4), dim3(256), 0, nullptr, nb.ntasks, nb.tasks,
+                       nb.codes, split, nb.pieces);
+    BW_LAUNCH_CHECK();
+    BW_HIP_CHECK(hipStreamSynchronize(nullptr));
+    nb.split = split;
+    return BW_HIP_OK;
+}
+
 int bin_impl(bw_pr_plan *plan, int32_t rows_log2, int32_t chunk_tasks, int32_t lane_edges, bool on_host)
 {
     BW_TRY(check_bin_args(plan, rows_log2, chunk_tasks, lane_edges));
@@ -1324,6 +1422,11 @@ int bin_impl(bw_pr_plan *plan, int32_t rows_log2, int32_t chunk_tasks, int32_t l
     nb.log2 = static_cast<uint32_t>(rows_log2);
     nb.chunk_tasks = static_cast<uint32_t>(chunk_tasks);
     nb.lane_edges = static_cast<uint32_t>(lane_edges);
+    const int ss = split_chunks(nb);
+    if (ss != BW_HIP_OK) {
+        nb.release();
+        return ss;
+    }
     B.release();
     B = nb;
     plan->binned = true;
@@ -1413,8 +1516,11 @@ int run_binned(const bw_pr_plan *plan, int32_t iterations, int32_t mode, int32_t
                                             : pr_bins_accumulate_kernel<13, kBinAccThreads, 8, 2>)
                                      : (l16 ? pr_bins_accumulate_kernel<14, kBinAccThreads, 16, 2>
                                             : pr_bins_accumulate_kernel<14, kBinAccThreads, 8, BW_BINS_DEPTH14>);
-    const Kernel finK = B.log2 == 13 ? pr_bins_finalise_kernel<13, kBinFinThreads>
-                                     : pr_bins_finalise_kernel<14, kBinFinThreads>;
+    const bool sp = B.split > 1;
+    const Kernel finK = B.log2 == 13 ? (sp ? pr_bins_finalise_kernel<13, kBinFinThreads, true>
+                                           : pr_bins_finalise_kernel<13, kBinFinThreads, false>)
+                                     : (sp ? pr_bins_finalise_kernel<14, kBinFinThreads, true>
+                                           : pr_bins_finalise_kernel<14, kBinFinThreads, false>);
     BinArgs a;
     a.V = plan->V;
     a.codes = B.codes;
@@ -1424,6 +1530,9 @@ int run_binned(const bw_pr_plan *plan, int32_t iterations, int32_t mode, int32_t
     a.npairs = std::max<uint32_t>(B.pairs, 1);
     a.bins = B.vals;
     a.partials = B.partials;
+    a.split = B.split;
+    a.pieces = B.pieces;
+    a.sums = B.sums;
     a.chunk_base = B.chunk_base;
     a.blocks = B.blocks;
     a.nblocks = B.nblocks;
@@ -1445,7 +1554,7 @@ int run_binned(const bw_pr_plan *plan, int32_t iterations, int32_t mode, int32_t
     const int S = bins_fixed_shift(plan->V, plan->E, !a.divide);
     a.pair_scale = std::ldexp(1.0f, S - 32);
     a.partial_scale = std::ldexp(1.0f, -S);
-    const uint32_t finGrid = B.nblocks, accGrid = B.nchunks + 1;
+    const uint32_t finGrid = B.nblocks, accGrid = B.nchunks * B.split + 1;
     hipLaunchKernelGGL(finK, dim3(finGrid), dim3(kBinFinThreads), 0, s, a);
     BW_LAUNCH_CHECK();
     hipEvent_t ev0 = nullptr, ev1 = nullptr;

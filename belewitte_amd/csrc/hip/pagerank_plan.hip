@@ -189,8 +189,8 @@ __global__ void plan_bounds_kernel(uint32_t V, uint32_t L, uint32_t K, const uin
 
 // The scatter blocks of partition k = blockIdx.x, cut like the host
 // builder: consecutive vertices, a new block when the current one holds
-// kBlockVerts vertices or when adding the vertex would take the block's
-// work (vertices x chunks of the partition + pairs) past kBlockWork.  (The
+// maxVerts vertices or when adding the vertex would take the block's
+// work (vertices x chunks of the partition + pairs) past maxWork.  (The
 // host builder also closes a block whose distinct target partitions would
 // pass kMaxRuns; that never happens, since a plan has at most kMaxRuns
 // partitions.)  A block's work is perVertex x vertices + pairs, and pbase
@@ -201,8 +201,8 @@ __global__ void plan_bounds_kernel(uint32_t V, uint32_t L, uint32_t K, const uin
 // block b's (first vertex, end vertex, pairs, 0); plan_block_runs_kernel
 // fills in the runs.
 __global__ __launch_bounds__(64) void plan_cut_kernel(uint32_t V, uint32_t L, const uint32_t *pbase,
-                                                      const uint32_t *chunk_base, uint32_t *block_local,
-                                                      uint4 *pblocks, uint32_t *nblocks)
+                                                      const uint32_t *chunk_base, uint32_t maxVerts, uint32_t maxWork,
+                                                      uint32_t *block_local, uint4 *pblocks, uint32_t *nblocks)
 {
     const uint32_t k = blockIdx.x, lane = threadIdx.x;
     const uint32_t vBeg = k << L;
@@ -212,11 +212,11 @@ __global__ __launch_bounds__(64) void plan_cut_kernel(uint32_t V, uint32_t L, co
     for (uint32_t v0 = vBeg; v0 < vEnd; nb++) {
         const uint32_t p0 = pbase[v0];
         auto fits = [&](uint32_t e) {
-            return e - v0 <= 1 || perVertex * (e - v0) + (pbase[e] - p0) <= kBlockWork;
+            return e - v0 <= 1 || perVertex * (e - v0) + (pbase[e] - p0) <= maxWork;
         };
         // The largest e in [lo, hi] that fits; lo = v0 + 1 does.  The work
         // grows with e, so the lanes that fit are the first ones.
-        uint32_t lo = v0 + 1, hi = std::min(v0 + kBlockVerts, vEnd);
+        uint32_t lo = v0 + 1, hi = std::min(v0 + maxVerts, vEnd);
         while (lo < hi) {
             const uint32_t step = (hi - lo + 63) / 64;
             const uint32_t e = std::min(lo + (lane + 1) * step, hi);
@@ -673,8 +673,8 @@ int build_plan_device(const uint32_t *roff, const uint32_t *rcols, uint32_t V, u
     PLAN_ALLOC(pblocks, uint4, V);
     PLAN_ALLOC(nblocksK, uint32_t, K);
     PLAN_TRY(hipMemcpyAsync(dchunk_base, chunk_base.data(), sizeof(uint32_t) * (K + 1), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(plan_cut_kernel, dim3(K), dim3(64), 0, s, V, L, pbase, dchunk_base, block_local, pblocks,
-                       nblocksK);
+    hipLaunchKernelGGL(plan_cut_kernel, dim3(K), dim3(64), 0, s, V, L, pbase, dchunk_base, block_verts(V),
+                       block_work(V), block_local, pblocks, nblocksK);
     PLAN_TRY(hipGetLastError());
     std::vector<uint32_t> hnb(K), block_base(K + 1, 0);
     PLAN_TRY(hipMemcpyAsync(hnb.data(), nblocksK, sizeof(uint32_t) * K, hipMemcpyDeviceToHost, s));
