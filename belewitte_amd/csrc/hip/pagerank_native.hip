@@ -941,6 +941,138 @@ __global__ __launch_bounds__(kThreads) void pr_bins_finalise_kernel(BinArgs a)
     write_partial<kThreads>(a.part, resid, dangl, red);
 }
 
+// ------------------------------------------------------ small graphs
+
+// A whole run in one launch of one workgroup, for a graph whose run is
+// launches and latency (1000 vertices, 6600 edges, 30 iterations: 62 launches,
+// 376 us, now 130; 3.2 us per iteration, of 10.9; at 2000 and 13600 4.3 of
+// 13.1, at 8000 and 30000 9.0 of 15.9).  Past kSmallEdges per thread the LDS
+// adds of one CU catch up with the launches saved.  Ranks and degrees stay in registers (a
+// thread's rows are t, t + 1024, ...), the contributions and the row sums in
+// LDS, and each thread keeps kEdges consecutive in-edges in registers,
+// adding a row's run of them to its LDS sum once.  The sums are the binned
+// iteration's fixed-point ones, exact in any order, so the ranks of a plan
+// whose partitions are one chunk each are the same bit for bit.
+constexpr uint32_t kSmallThreads = 1024;
+constexpr uint32_t kSmallRows = 8;    // rows per thread at most
+constexpr uint32_t kSmallVerts = kSmallThreads * kSmallRows;
+constexpr uint32_t kSmallEdges = 32;  // edges per thread at most
+
+struct SmallArgs {
+    uint32_t V, E;
+    const uint32_t *roff, *rcols, *deg;
+    float *rank;
+    double *dangl;  // [iterations + 1]
+    double *resid;  // [iterations]
+    int iterations, mode, divide;
+    float pair_scale, partial_scale;  // see BinArgs
+};
+
+template<int kEdges>
+__global__ __launch_bounds__(kSmallThreads) void pr_small_kernel(SmallArgs a)
+{
+    extern __shared__ unsigned long long acc[];  // V row sums, then V contributions
+    float *contrib = reinterpret_cast<float *>(acc + a.V);
+    __shared__ double red[2][kSmallThreads / kWave][2];
+    const uint32_t t = threadIdx.x;
+    // An edge: its source, its row << 13, and 1 << 26 when it is the row's
+    // last of this thread; no edge: bit 31.
+    constexpr uint32_t kFlush = 1u << 26, kNone = 1u << 31, kMask = kSmallVerts - 1;
+    static_assert(kSmallVerts == 1u << 13, "13 bits per vertex");
+    uint32_t edge[kEdges];
+    {
+        const uint32_t e0 = t * kEdges;
+        uint32_t row = 0;
+        if (e0 < a.E) {
+            uint32_t hi = a.V - 1;  // the largest row starting at or before e0
+            while (row < hi) {
+                const uint32_t mid = row + (hi - row + 1) / 2;
+                if (a.roff[mid] <= e0) row = mid;
+                else hi = mid - 1;
+            }
+        }
+        uint32_t end = a.roff[row + 1];
+#pragma unroll
+        for (int k = 0; k < kEdges; k++) {
+            const uint32_t e = e0 + k;
+            edge[k] = kNone;
+            if (e >= a.E) continue;
+            while (end <= e) end = a.roff[++row + 1];
+            edge[k] = a.rcols[e] | row << 13 | (e + 1 == end || k + 1 == kEdges ? kFlush : 0u);
+        }
+    }
+    float rank[kSmallRows];
+    uint32_t deg[kSmallRows];
+    double resid = 0.0, dangl = 0.0;
+    const float init = 1.0f / static_cast<float>(a.V);
+#pragma unroll
+    for (uint32_t i = 0; i < kSmallRows; i++) {
+        const uint32_t v = t + i * kSmallThreads;
+        rank[i] = init;
+        deg[i] = 0;
+        if (v >= a.V) continue;
+        deg[i] = a.deg[v];
+        const float c = (a.divide && deg[i] != 0) ? init / static_cast<float>(deg[i]) : init;
+        contrib[v] = c * a.pair_scale;
+        acc[v] = 0ull;
+        if (deg[i] == 0) dangl += static_cast<double>(init);
+    }
+    // The workgroup's (residual, dangling mass) in a fixed order, the same in
+    // every thread; the two copies of red[] alternate, so a barrier per pass
+    // is enough.
+    auto reduce = [&](int copy) {
+        const double r = wave_sum_f64(resid), g = wave_sum_f64(dangl);
+        if ((t & (kWave - 1)) == 0) {
+            red[copy][t / kWave][0] = r;
+            red[copy][t / kWave][1] = g;
+        }
+        __syncthreads();
+        resid = dangl = 0.0;
+        double R = 0.0, G = 0.0;
+        for (uint32_t w = 0; w < kSmallThreads / kWave; w++) {
+            R += red[copy][w][0];
+            G += red[copy][w][1];
+        }
+        return make_double2(R, G);
+    };
+    double2 total = reduce(0);
+    if (t == 0) a.dangl[0] = total.y;
+    for (int it = 1; it <= a.iterations; it++) {
+        unsigned long long sum = 0;
+#pragma unroll
+        for (int k = 0; k < kEdges; k++) {
+            if (edge[k] & kNone) continue;
+            sum += bin_fixed(contrib[edge[k] & kMask]);
+            if (edge[k] & kFlush) {
+                atomicAdd(&acc[(edge[k] >> 13) & kMask], sum);
+                sum = 0;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t i = 0; i < kSmallRows; i++) {
+            const uint32_t v = t + i * kSmallThreads;
+            if (v >= a.V) continue;
+            const float nr = new_rank(a.mode, a.V, static_cast<float>(acc[v]) * a.partial_scale, total.y);
+            resid += fabs(static_cast<double>(nr) - static_cast<double>(rank[i]));
+            if (deg[i] == 0) dangl += static_cast<double>(nr);
+            rank[i] = nr;
+            contrib[v] = (deg[i] != 0 ? nr / static_cast<float>(deg[i]) : 0.0f) * a.pair_scale;
+            acc[v] = 0ull;
+        }
+        total = reduce(it & 1);
+        if (t == 0) {
+            a.resid[it - 1] = total.x;
+            a.dangl[it] = total.y;
+        }
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kSmallRows; i++) {
+        const uint32_t v = t + i * kSmallThreads;
+        if (v < a.V) a.rank[v] = rank[i];
+    }
+}
+
 // The pieces of each task, one wave per task: whole 64-edge lines split
 // evenly (as many lines a piece as the task has, rounded), each with the pair
 // of its first edge from a count of the new-pair flags before it.
@@ -1504,6 +1636,57 @@ constexpr int kBinAccThreads = 1024;
 #endif
 constexpr int kBinFinThreads = BW_BINS_FIN_THREADS;
 
+bool small_graph(uint32_t V, uint32_t E) { return V <= kSmallVerts && E <= kSmallThreads * kSmallEdges; }
+
+int run_small(const bw_pr_plan *plan, const uint32_t *roff, const uint32_t *rcols, int32_t iterations, int32_t mode,
+              int32_t nodiv_quirk, float *ranks, double *dangl, double *resid, double *resid_host, float *kernel_ms,
+              hipStream_t s)
+{
+    SmallArgs a;
+    a.V = plan->V;
+    a.E = plan->E;
+    a.roff = roff;
+    a.rcols = rcols;
+    a.deg = plan->deg;
+    a.rank = ranks;
+    a.dangl = dangl;
+    a.resid = resid;
+    a.iterations = iterations;
+    a.mode = mode;
+    a.divide = !(nodiv_quirk && mode == BW_PR_DANGLING_DROP);
+    const int S = bins_fixed_shift(plan->V, plan->E, !a.divide);
+    a.pair_scale = std::ldexp(1.0f, S - 32);
+    a.partial_scale = std::ldexp(1.0f, -S);
+    using Kernel = void (*)(SmallArgs);
+    const uint32_t per = (plan->E + kSmallThreads - 1) / kSmallThreads;
+    const Kernel k = per <= 8 ? pr_small_kernel<8> : per <= 16 ? pr_small_kernel<16> : pr_small_kernel<kSmallEdges>;
+    // 12 bytes a vertex: 96 KB at most.
+    const uint32_t lds = 12 * plan->V;
+    if (lds > 64 * 1024)
+        BW_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         static_cast<int>(lds)));
+    hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    if (kernel_ms) {
+        BW_HIP_CHECK(hipEventCreate(&ev0));
+        BW_HIP_CHECK(hipEventCreate(&ev1));
+        BW_HIP_CHECK(hipEventRecord(ev0, s));
+    }
+    hipLaunchKernelGGL(k, dim3(1), dim3(kSmallThreads), lds, s, a);
+    BW_LAUNCH_CHECK();
+    if (kernel_ms) {
+        BW_HIP_CHECK(hipEventRecord(ev1, s));
+        BW_HIP_CHECK(hipEventSynchronize(ev1));
+        BW_HIP_CHECK(hipEventElapsedTime(kernel_ms, ev0, ev1));
+        (void)hipEventDestroy(ev0);
+        (void)hipEventDestroy(ev1);
+    }
+    if (resid_host) {
+        BW_HIP_CHECK(hipMemcpyAsync(resid_host, resid, sizeof(double) * iterations, hipMemcpyDeviceToHost, s));
+        BW_HIP_CHECK(hipStreamSynchronize(s));
+    }
+    return BW_HIP_OK;
+}
+
 // The binned iteration loop: initial ranks and bins, then per iteration one
 // accumulate and one finalise launch; ranks are updated in place.
 int run_binned(const bw_pr_plan *plan, int32_t iterations, int32_t mode, int32_t nodiv_quirk, float *ranks,
@@ -1607,6 +1790,9 @@ extern "C" int bw_pr_fused_run(const bw_graph_dev *g, const bw_pr_plan *plan, in
     hipStream_t s = stream_of(cfg);
     const uint32_t V = plan->V;
     double *dangl = acc, *resid = acc + iterations + 1, *spare = acc + 2 * iterations + 2;
+    if (small_graph(V, plan->E))
+        return run_small(plan, static_cast<const uint32_t *>(g->rev_offsets), g->rev_cols, iterations, mode, nodiv_quirk,
+                         ranks, dangl, resid, resid_host, kernel_ms, s);
     if (plan->binned) return run_binned(plan, iterations, mode, nodiv_quirk, ranks, dangl, resid, spare, resid_host,
                                         kernel_ms, s);
 
