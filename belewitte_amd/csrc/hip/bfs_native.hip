@@ -45,6 +45,9 @@ constexpr int kBlock = 256;
 // maxima (bw_bfs_engine_set_queues).
 constexpr uint32_t kLdsQueueMax = BW_BFS_MAX_LDS_QUEUE;
 constexpr uint32_t kHubCapMax = BW_BFS_MAX_HUB_CAP;
+constexpr uint32_t kSegment = BW_BFS_DEFAULT_LDS_QUEUE;  // a workgroup's segment of the frontier
+constexpr uint32_t kMaxGrid = 4096;    // workgroups of a level kernel at most
+constexpr uint32_t kSegGroup = 8;      // segments per coarse step of the search for a frontier index
 constexpr uint32_t kParentScan = 32;   // in-edges scanned for a vertex's likely parent
 constexpr uint32_t kNoParent = 0xFFFFFFFFu;
 constexpr int kFeatures = BW_BFS_FEATURES;
@@ -60,7 +63,8 @@ enum Policy : int32_t { FIXED = BW_POLICY_FIXED, SCHEDULE = BW_POLICY_SCHEDULE, 
 struct BfsState {
     uint32_t depth;     // level being processed: the frontier is at `depth`
     uint32_t done;
-    uint32_t qcount;    // normal frontier queue size
+    uint32_t qcount;    // normal frontier size: the queue, then the workgroups' segments
+    uint32_t qglobal;   // of it in the queue
     uint32_t hubcount;  // hub frontier queue size
     uint32_t qout;      // appended to the next normal queue during the level
     uint32_t hubout;    // appended to the next hub queue (may exceed the hub capacity)
@@ -108,6 +112,15 @@ __host__ __device__ inline bool variant_available(const Graph &g, int32_t c)
 struct Buffers {
     int32_t *levels;
     uint32_t *q[2];
+    // What a workgroup discovers and does not have to spill to the queue
+    // stays in a segment of its own; the epilogue's prefix sum of the
+    // segments' counts places them behind the queue.  Appending to the queue
+    // takes an atomic per workgroup on one counter, about 15 ns each one
+    // after the other: any level that found something in most of the 2048
+    // workgroups took 35 us (1 M-vertex grid), SEGNOTE with segments.
+    uint32_t *seg[2];      // [workgroup][kSegment]
+    uint32_t *segcount;    // per workgroup: discovered in this level
+    uint32_t *segbase;     // per workgroup and one more: frontier index of its segment's first vertex
     uint32_t *hubq[2];
     uint64_t *hub_prefix;  // hub_cap + 1
     uint32_t *bits[3];     // frontier bitmaps, level d reads bits[d % 3]
@@ -204,7 +217,49 @@ struct Emitter {
         if (threadIdx.x == 0) *lcount = 0;
         __syncthreads();
     }
+
+    // Block-uniform, at the level's end: what is staged becomes the
+    // workgroup's segment (what a segment cannot hold goes to the queue).
+    __device__ __forceinline__ void finish(const Buffers &b, uint32_t d)
+    {
+        __syncthreads();
+        const uint32_t staged = min(*lcount, cap), n = min(staged, kSegment);
+        const uint32_t nq = (d & 1) ^ 1;
+        uint32_t *s = b.seg[nq] + static_cast<size_t>(blockIdx.x) * kSegment;
+        for (uint32_t i = threadIdx.x; i < n; i += kBlock) s[i] = lbuf[i];
+        if (threadIdx.x == 0) {
+            b.segcount[blockIdx.x] = n;
+            if (staged > n) *lbase = atomicAdd(&b.st->qout, staged - n);
+        }
+        __syncthreads();
+        for (uint32_t i = n + threadIdx.x; i < staged; i += kBlock) b.q[nq][*lbase + i - n] = lbuf[i];
+    }
 };
+
+// The frontier's vertex i >= st.qglobal, in some workgroup's segment: coarse[]
+// (LDS) holds every kSegGroup-th of the segments' first indexes.
+__device__ __forceinline__ uint32_t segment_vertex(const Buffers &b, uint32_t cur, uint32_t nseg,
+                                                   const uint32_t *coarse, uint32_t i)
+{
+    uint32_t lo = 0, hi = (nseg + kSegGroup - 1) / kSegGroup;  // last group starting at or before i
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (coarse[mid] <= i) lo = mid;
+        else hi = mid;
+    }
+    // The group's segments, whose bases are padded past the last one.
+    const uint4 *g = reinterpret_cast<const uint4 *>(b.segbase + lo * kSegGroup);
+    const uint4 x = g[0], y = g[1];
+    uint32_t w = lo * kSegGroup, first = x.x;
+    const uint32_t base[kSegGroup] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+#pragma unroll
+    for (uint32_t k = 1; k < kSegGroup; k++)
+        if (base[k] <= i) {
+            w = lo * kSegGroup + k;
+            first = base[k];
+        }
+    return b.seg[cur][static_cast<size_t>(w) * kSegment + (i - first)];
+}
 
 // Top-down discovery of w: the thread whose fetch-or sets w's visited bit
 // owns w and records its depth (unless the level defers its depths).
@@ -232,7 +287,7 @@ __device__ __forceinline__ bool defer_depths(const BfsState &st, const Buffers &
 // ------------------------------------------------------------- variants
 
 __device__ void level_td(const Graph &g, const Buffers &b, uint32_t d, Emitter &em, uint32_t *sstart,
-                         uint64_t *sscan, uint64_t *stotal)
+                         uint64_t *sscan, uint64_t *stotal, uint32_t *coarse)
 {
     const int32_t nd = static_cast<int32_t>(d) + 1;
     const uint32_t cur = d & 1;
@@ -266,13 +321,17 @@ __device__ void level_td(const Graph &g, const Buffers &b, uint32_t d, Emitter &
     // 256 at a time with the owner found by binary search in the LDS degree
     // scan.  A small frontier is spread over all workgroups (batches down to
     // one vertex), so its edges never pile up on a few workgroups.
-    const uint32_t n = st.qcount;
+    const uint32_t n = st.qcount, ng = st.qglobal;
+    if (n > ng) {
+        for (uint32_t k = tid; k * kSegGroup < gridDim.x; k += kBlock) coarse[k] = b.segbase[k * kSegGroup];
+        __syncthreads();
+    }
     const uint32_t bs = max(1u, min(static_cast<uint32_t>(kBlock), (n + gridDim.x - 1) / gridDim.x));
     for (uint32_t base = blockIdx.x * bs; base < n; base += gridDim.x * bs) {
         const uint32_t i = base + tid;
         uint32_t deg = 0, start = 0;
         if (tid < bs && i < n) {
-            const uint32_t u = b.q[cur][i];
+            const uint32_t u = i < ng ? b.q[cur][i] : segment_vertex(b, cur, gridDim.x, coarse, i);
             start = g.off[u];
             deg = g.off[u + 1] - start;
         }
@@ -534,6 +593,7 @@ __global__ __launch_bounds__(kBlock) void bfs_engine_step(Graph g, Buffers b)
     __shared__ uint64_t stotal;
     __shared__ uint32_t sstart[kBlock];
     __shared__ uint64_t sscan[kBlock];
+    __shared__ uint32_t coarse[kMaxGrid / kSegGroup];
     __shared__ uint64_t rout[kBlock / kWave];
     __shared__ double rsq[kBlock / kWave];
 
@@ -564,7 +624,7 @@ __global__ __launch_bounds__(kBlock) void bfs_engine_step(Graph g, Buffers b)
     if constexpr (!REF) {
         if (variant == TD) {
             fill_depths();
-            level_td(g, b, d, em, sstart, sscan, &stotal);
+            level_td(g, b, d, em, sstart, sscan, &stotal, coarse);
         } else {
             level_bu<true>(g, b, d, em, variant == BU_WAVE, fill);
         }
@@ -584,7 +644,7 @@ __global__ __launch_bounds__(kBlock) void bfs_engine_step(Graph g, Buffers b)
             }
         }
     }
-    em.flush(b, d, em.cap);  // reserve everything: moves all that is staged
+    em.finish(b, d);
 
     // Workgroup partials of the discovered vertices' out-degrees.
     uint64_t os = em.outsum;
@@ -823,6 +883,7 @@ __global__ __launch_bounds__(kBlock) void bfs_engine_epilogue(Graph g, Buffers b
     __shared__ uint64_t rout[kBlock / kWave];
     __shared__ double rsq[kBlock / kWave];
     __shared__ uint64_t hscan[kBlock];
+    __shared__ uint32_t sscan[kBlock / kWave];
 
     BfsState &st = *b.st;
     if (st.done) return;
@@ -867,9 +928,44 @@ __global__ __launch_bounds__(kBlock) void bfs_engine_epilogue(Graph g, Buffers b
     }
     const uint32_t d = st.depth;
     const uint32_t nhub = min(st.hubout, b.hub_cap);
-    const uint32_t nnew = nhub + st.qout;
     const bool deferred = defer_depths(st, b, g.V);  // this level's, before the state moves on
     __syncthreads();
+
+    // The segments' first frontier indexes, behind the queue's vertices:
+    // rounds of kSegGroup consecutive segments per thread.
+    const uint32_t qout = st.qout;
+    uint32_t segend = qout;
+    for (uint32_t r0 = 0; r0 < nparts; r0 += kBlock * kSegGroup) {
+        const uint32_t w0 = r0 + tid * kSegGroup;
+        uint32_t c[kSegGroup] = {}, sum = 0;
+        if (w0 < nparts) {  // segcount is padded to whole groups (with zeros)
+            const uint4 x = reinterpret_cast<const uint4 *>(b.segcount + w0)[0];
+            const uint4 y = reinterpret_cast<const uint4 *>(b.segcount + w0)[1];
+            c[0] = x.x, c[1] = x.y, c[2] = x.z, c[3] = x.w, c[4] = y.x, c[5] = y.y, c[6] = y.z, c[7] = y.w;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kSegGroup; k++) sum += c[k];
+        const uint32_t incl = wave_prefix_sum(sum);
+        if (lane == kWave - 1) sscan[wid] = incl;
+        __syncthreads();
+        uint32_t at = segend + incl - sum;
+        for (int w = 0; w < kBlock / kWave; w++) {
+            if (w < wid) at += sscan[w];
+            segend += sscan[w];
+        }
+        if (w0 < nparts) {
+#pragma unroll
+            for (uint32_t k = 0; k < kSegGroup; k++) {
+                const uint32_t x = c[k];
+                c[k] = at;
+                at += x;
+            }
+            reinterpret_cast<uint4 *>(b.segbase + w0)[0] = make_uint4(c[0], c[1], c[2], c[3]);
+            reinterpret_cast<uint4 *>(b.segbase + w0)[1] = make_uint4(c[4], c[5], c[6], c[7]);
+        }
+        __syncthreads();  // sscan is rewritten by the next round
+    }
+    const uint32_t nnew = nhub + segend;
 
     // Hub degree prefix of the next frontier, read by the next top-down
     // level: rounds of kBlock consecutive hubs, one per thread, each an
@@ -943,7 +1039,8 @@ __global__ __launch_bounds__(kBlock) void bfs_engine_epilogue(Graph g, Buffers b
             st.prev_time_ns = ns;
             st.prev_frontier = static_cast<uint64_t>(st.qcount) + st.hubcount;
             st.depth = d + 1;
-            st.qcount = st.qout;
+            st.qcount = segend;
+            st.qglobal = qout;
             st.hubcount = nhub;
             st.qout = 0;
             st.hubout = 0;
@@ -1004,6 +1101,7 @@ __global__ __launch_bounds__(kBlock) void bfs_engine_init(Graph g, Buffers b, Po
         st.stalled = 0;
         st.fill_levels = 0;
         st.qcount = nq;
+        st.qglobal = nq;
         st.hubcount = nh;
         st.choice = p.fixed;
     }
@@ -1065,6 +1163,7 @@ struct bw_bfs_engine {
     // Snapshot of levels, queues, bitmaps and state, for timing every
     // variant on the same level.
     int32_t *snap_levels = nullptr;
+    uint32_t *snap_seg = nullptr, *snap_segbase = nullptr;
     uint32_t *snap_q = nullptr, *snap_hub = nullptr, *snap_bits = nullptr;
     uint64_t *snap_prefix = nullptr;
     BfsState *snap_st = nullptr;
@@ -1093,6 +1192,7 @@ struct bw_bfs_engine {
         drop_exec();
         void *bufs[] = {own_levels, b.q[0], b.q[1], b.hubq[0], b.hubq[1], b.hub_prefix, b.bits[0], b.bits[1],
                         b.bits[2], b.vis, b.st, b.part, b.counts, b.times, b.choices, snap_levels, snap_q, snap_hub,
+                        b.seg[0], b.seg[1], b.segcount, b.segbase, snap_seg, snap_segbase,
                         snap_bits, snap_prefix, snap_st, mlp, schedule, roots, no_in, parent};
         for (void *p : bufs)
             if (p) (void)hipFree(p);
@@ -1184,7 +1284,8 @@ extern "C" int bw_bfs_engine_create(bw_bfs_engine **out, const bw_graph_dev *g, 
     e->g = Graph{V,       g->edge_count, static_cast<const uint32_t *>(g->offsets), g->cols,
                  static_cast<const uint32_t *>(g->rev_offsets), g->rev_cols, g->el_in, g->el_out, g->rel_in,
                  g->rel_out, g->sel, g->rsel};
-    e->grid = static_cast<uint32_t>(device_cus()) * 8;
+    e->grid = std::min(static_cast<uint32_t>(device_cus()) * 8, kMaxGrid);
+    const uint32_t segs = (e->grid + kSegGroup - 1) / kSegGroup * kSegGroup;  // whole groups
     const uint32_t words = static_cast<uint32_t>((V + 31) / 32);
     bool ok = true;
     auto alloc = [&](auto **p, size_t bytes) {
@@ -1197,6 +1298,9 @@ extern "C" int bw_bfs_engine_create(bw_bfs_engine **out, const bw_graph_dev *g, 
     e->b.levels = levels;
     alloc(&e->b.q[0], sizeof(uint32_t) * V);
     alloc(&e->b.q[1], sizeof(uint32_t) * V);
+    for (auto &x : e->b.seg) alloc(&x, sizeof(uint32_t) * kSegment * e->grid);
+    alloc(&e->b.segcount, sizeof(uint32_t) * segs);
+    alloc(&e->b.segbase, sizeof(uint32_t) * segs);
     alloc(&e->b.hubq[0], sizeof(uint32_t) * kHubCapMax);
     alloc(&e->b.hubq[1], sizeof(uint32_t) * kHubCapMax);
     alloc(&e->b.hub_prefix, sizeof(uint64_t) * (kHubCapMax + 1));
@@ -1221,6 +1325,10 @@ extern "C" int bw_bfs_engine_create(bw_bfs_engine **out, const bw_graph_dev *g, 
         return fail(BW_HIP_ERR_NOMEM, "device allocation of the BFS engine failed");
     }
     e->b.parent = e->parent;
+    if (bw_hip_fill_u32(e->b.segcount, 0u, segs, nullptr) != BW_HIP_OK) {
+        delete e;
+        return BW_HIP_ERR_RUNTIME;
+    }
     hipLaunchKernelGGL(no_in_edges_kernel, dim3(e->grid), dim3(kBlock), 0, nullptr, e->g, e->no_in);
     hipLaunchKernelGGL(likely_parent_kernel, dim3(e->grid), dim3(kBlock), 0, nullptr, e->g, e->parent);
     if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
@@ -1413,6 +1521,8 @@ extern "C" int bw_bfs_engine_snapshot(bw_bfs_engine *e, int32_t restore, void *s
         if (restore) return fail(BW_HIP_ERR_ARG, "no snapshot to restore");
         BW_HIP_CHECK(hipMalloc(&e->snap_levels, sizeof(int32_t) * V));
         BW_HIP_CHECK(hipMalloc(&e->snap_q, sizeof(uint32_t) * V));
+        BW_HIP_CHECK(hipMalloc(&e->snap_seg, sizeof(uint32_t) * kSegment * e->grid));
+        BW_HIP_CHECK(hipMalloc(&e->snap_segbase, sizeof(uint32_t) * e->grid));
         BW_HIP_CHECK(hipMalloc(&e->snap_hub, sizeof(uint32_t) * kHubCapMax));
         BW_HIP_CHECK(hipMalloc(&e->snap_bits, sizeof(uint32_t) * 4 * words));
         BW_HIP_CHECK(hipMalloc(&e->snap_prefix, sizeof(uint64_t) * (kHubCapMax + 1)));
@@ -1422,13 +1532,15 @@ extern "C" int bw_bfs_engine_snapshot(bw_bfs_engine *e, int32_t restore, void *s
     BW_HIP_CHECK(hipMemcpyAsync(&st, restore ? e->snap_st : e->b.st, sizeof st, hipMemcpyDeviceToHost, s));
     BW_HIP_CHECK(hipStreamSynchronize(s));
     const uint32_t cur = st.depth & 1;
-    const size_t nq = std::max<size_t>(st.qcount, 1), nh = std::max<size_t>(std::min(st.hubcount, e->b.hub_cap), 1);
+    const size_t nq = std::max<size_t>(st.qglobal, 1), nh = std::max<size_t>(std::min(st.hubcount, e->b.hub_cap), 1);
     auto copy = [&](void *saved, void *live, size_t bytes) {
         return restore ? hipMemcpyAsync(live, saved, bytes, hipMemcpyDeviceToDevice, s)
                        : hipMemcpyAsync(saved, live, bytes, hipMemcpyDeviceToDevice, s);
     };
     BW_HIP_CHECK(copy(e->snap_levels, e->b.levels, sizeof(int32_t) * V));
     BW_HIP_CHECK(copy(e->snap_q, e->b.q[cur], sizeof(uint32_t) * nq));
+    BW_HIP_CHECK(copy(e->snap_seg, e->b.seg[cur], sizeof(uint32_t) * kSegment * e->grid));
+    BW_HIP_CHECK(copy(e->snap_segbase, e->b.segbase, sizeof(uint32_t) * e->grid));
     BW_HIP_CHECK(copy(e->snap_hub, e->b.hubq[cur], sizeof(uint32_t) * nh));
     BW_HIP_CHECK(copy(e->snap_prefix, e->b.hub_prefix, sizeof(uint64_t) * (e->b.hub_cap + 1)));
     for (int i = 0; i < 3; i++) BW_HIP_CHECK(copy(e->snap_bits + i * words, e->b.bits[i], sizeof(uint32_t) * words));
