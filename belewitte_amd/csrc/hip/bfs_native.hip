@@ -77,10 +77,22 @@ struct BfsState {
     double frontier_sq;         // sum of squared out-degrees of the frontier
     uint64_t t_step;            // wall clock at the start of the level's step kernel
     uint32_t fill_levels;       // the previous level left its depths to this one (dense top-down)
-    uint32_t stalled;           // a level's variant was of a kind that was not launched (see run_impl)
+    uint32_t rot;               // level d reads frontier bitmap (d + rot) % 3
     uint64_t explored_edges;    // out-degree sum of every vertex discovered so far
     uint64_t prev_frontier;     // frontier size of the previous level (0 at level 0)
 };
+
+// What a search reports of each level.
+struct LevelOut {
+    uint64_t ns;      // device time
+    uint32_t count;   // discovered vertices
+    int32_t choice;   // variant
+};
+
+// The state and the levels' reports share one allocation, so that the host
+// reads the state and the first kOutFirst reports in one copy.
+constexpr size_t kOutOffset = 256, kOutFirst = 64;
+static_assert(sizeof(BfsState) <= kOutOffset, "the reports follow the state");
 
 struct Graph {
     uint64_t V;
@@ -117,21 +129,19 @@ struct Buffers {
     // segments' counts places them behind the queue.  Appending to the queue
     // takes an atomic per workgroup on one counter, about 15 ns each one
     // after the other: any level that found something in most of the 2048
-    // workgroups took 35 us (1 M-vertex grid), SEGNOTE with segments.
+    // workgroups took 35 us (1 M-vertex grid), 12 to 20 with segments.
     uint32_t *seg[2];      // [workgroup][kSegment]
     uint32_t *segcount;    // per workgroup: discovered in this level
     uint32_t *segbase;     // per workgroup and one more: frontier index of its segment's first vertex
     uint32_t *hubq[2];
     uint64_t *hub_prefix;  // hub_cap + 1
-    uint32_t *bits[3];     // frontier bitmaps, level d reads bits[d % 3]
+    uint32_t *bits[3];     // frontier bitmaps, level d reads bits[(d + rot) % 3]
     uint32_t *vis;         // visited bitmap
     const uint32_t *parent;  // per vertex: its likely parent (in-neighbour of largest out-degree among
                              // its first kParentScan in-edges), kNoParent without in-edges
     BfsState *st;
     uint64_t *part;        // per workgroup: out-degree sum, (double) sum of squares
-    uint32_t *counts;      // per level: discovered vertices
-    uint64_t *times;       // per level: device time in ns
-    int32_t *choices;      // per level: variant
+    LevelOut *out;         // per level, in the state's allocation (see kOutOffset)
     uint32_t max_levels;
     uint32_t words;        // bitmap words
     float ns_per_tick;
@@ -148,6 +158,7 @@ struct PolicyArgs {
     int32_t schedule_len;
     const float *mlp;  // packed weights, see mlp_len
     int32_t nout;
+    int32_t fuse;      // small levels run inside the epilogue (tiny_levels)
 };
 
 __device__ __forceinline__ uint32_t out_degree(const Graph &g, uint32_t v) { return g.off[v + 1] - g.off[v]; }
@@ -160,6 +171,7 @@ struct Emitter {
     uint32_t *lcount;
     uint32_t *lbase;
     uint32_t cap;  // lbuf's size
+    uint32_t rot;  // of the frontier bitmaps
     uint64_t outsum = 0;
     double sq = 0.0;
 
@@ -174,7 +186,7 @@ struct Emitter {
         const uint32_t dw = out_degree(g, w);
         outsum += dw;
         sq += static_cast<double>(dw) * static_cast<double>(dw);
-        if (mark) atomicOr(&b.bits[(d + 1) % 3][w >> 5], 1u << (w & 31));
+        if (mark) atomicOr(&b.bits[(d + 1 + rot) % 3][w >> 5], 1u << (w & 31));
         if (dw > b.hub_degree) {
             // Slots are handed out by a counter that only grows, so every
             // slot below min(count, hub_cap) is written exactly once.
@@ -326,9 +338,20 @@ __device__ void level_td(const Graph &g, const Buffers &b, uint32_t d, Emitter &
         for (uint32_t k = tid; k * kSegGroup < gridDim.x; k += kBlock) coarse[k] = b.segbase[k * kSegGroup];
         __syncthreads();
     }
-    const uint32_t bs = max(1u, min(static_cast<uint32_t>(kBlock), (n + gridDim.x - 1) / gridDim.x));
-    for (uint32_t base = blockIdx.x * bs; base < n; base += gridDim.x * bs) {
-        const uint32_t i = base + tid;
+    // A small frontier goes to the workgroups in contiguous pieces, whose
+    // vertices share cache lines.  Of a large one they take runs in turn:
+    // vertices near each other in it tend to be alike in degree too, and the
+    // level lasts as long as the piece with the most edges.
+    constexpr uint32_t kRun = 8, kRunsFrom = 32;
+    uint32_t bs = max(1u, min(static_cast<uint32_t>(kBlock), (n + gridDim.x - 1) / gridDim.x));
+    uint32_t first = blockIdx.x * bs, at = tid;
+    if (bs >= kRunsFrom) {
+        bs = (bs + kRun - 1) / kRun * kRun;
+        first = blockIdx.x * kRun;
+        at = tid / kRun * (gridDim.x * kRun) + tid % kRun;
+    }
+    for (uint32_t base = first; base < n; base += gridDim.x * bs) {
+        const uint32_t i = base + at;
         uint32_t deg = 0, start = 0;
         if (tid < bs && i < n) {
             const uint32_t u = i < ng ? b.q[cur][i] : segment_vertex(b, cur, gridDim.x, coarse, i);
@@ -371,7 +394,7 @@ template<bool USE_PARENT>
 __device__ void level_bu(const Graph &g, const Buffers &b, uint32_t d, Emitter &em, bool wave, bool fill)
 {
     const int32_t nd = static_cast<int32_t>(d) + 1;
-    const uint32_t *front = b.bits[d % 3];
+    const uint32_t *front = b.bits[(d + em.rot) % 3];
     const uint64_t V = g.V;
     const int lane = __lane_id();
     for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * kBlock; base < V;
@@ -438,7 +461,7 @@ __device__ void level_bu(const Graph &g, const Buffers &b, uint32_t d, Emitter &
             const uint32_t half = lane == 0 ? static_cast<uint32_t>(fm) : static_cast<uint32_t>(fm >> 32);
             if ((lane == 0 || lane == 32) && half) {
                 const uint64_t wi = w0 + (lane >> 5);
-                b.bits[(d + 1) % 3][wi] = half;
+                b.bits[(d + 1 + em.rot) % 3][wi] = half;
                 b.vis[wi] |= half;
             }
         }
@@ -462,7 +485,7 @@ template<int FAMILY>
 __device__ void level_ref_edges(const Graph &g, const Buffers &b, uint32_t d, Emitter &em)
 {
     const int32_t nd = static_cast<int32_t>(d) + 1;
-    const uint32_t *front = b.bits[d % 3];
+    const uint32_t *front = b.bits[(d + em.rot) % 3];
     const uint64_t E = g.E;
     for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * kBlock * 4; base < E;
          base += static_cast<uint64_t>(gridDim.x) * kBlock * 4) {
@@ -495,7 +518,7 @@ __device__ void level_ref_edges(const Graph &g, const Buffers &b, uint32_t d, Em
 __device__ void level_ref_push(const Graph &g, const Buffers &b, uint32_t d, Emitter &em)
 {
     const int32_t nd = static_cast<int32_t>(d) + 1;
-    const uint32_t *front = b.bits[d % 3];
+    const uint32_t *front = b.bits[(d + em.rot) % 3];
     for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * kBlock; base < g.V;
          base += static_cast<uint64_t>(gridDim.x) * kBlock) {
         const uint64_t v = base + threadIdx.x;
@@ -517,7 +540,7 @@ constexpr uint32_t kRefWarp = 32;
 __device__ void level_ref_push_warp(const Graph &g, const Buffers &b, uint32_t d, Emitter &em)
 {
     const int32_t nd = static_cast<int32_t>(d) + 1;
-    const uint32_t *front = b.bits[d % 3];
+    const uint32_t *front = b.bits[(d + em.rot) % 3];
     const uint32_t lane = threadIdx.x % kRefWarp;
     for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * kBlock; base < g.V;
          base += static_cast<uint64_t>(gridDim.x) * kBlock) {
@@ -542,7 +565,7 @@ __device__ void level_ref_push_warp(const Graph &g, const Buffers &b, uint32_t d
 __device__ void level_ref_pull_warp(const Graph &g, const Buffers &b, uint32_t d, Emitter &em)
 {
     const int32_t nd = static_cast<int32_t>(d) + 1;
-    const uint32_t *front = b.bits[d % 3];
+    const uint32_t *front = b.bits[(d + em.rot) % 3];
     const uint32_t lane = threadIdx.x % kRefWarp;
     const uint64_t half = (threadIdx.x & kRefWarp) ? ~0ull << 32 : 0xFFFFFFFFull;
     for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * kBlock; base < g.V;
@@ -571,7 +594,7 @@ __device__ void level_ref_pull_warp(const Graph &g, const Buffers &b, uint32_t d
         }
         if (lane == 0 && found_mask) {
             const uint64_t wi = c0 >> 5;
-            b.bits[(d + 1) % 3][wi] = found_mask;
+            b.bits[(d + 1 + em.rot) % 3][wi] = found_mask;
             b.vis[wi] |= found_mask;
         }
         em.flush(b, d, kBlock);
@@ -580,13 +603,13 @@ __device__ void level_ref_pull_warp(const Graph &g, const Buffers &b, uint32_t d
 
 // ---------------------------------------------------------- level kernel
 
-// The level kernel in two instantiations: REF = false runs the native
-// variants, REF = true the reference's families; each returns at once when
-// the level's variant is the other kind.  Kept apart so that the native
-// kernel's code is compiled on its own (with the reference families in the
-// same kernel its levels ran about 1.5x slower on MI355X).
-template<bool REF>
-__global__ __launch_bounds__(kBlock) void bfs_engine_step(Graph g, Buffers b)
+// The level kernel: whichever variant the state names.  The grid is eight
+// workgroups per CU, all in flight at once, which takes eight waves per SIMD:
+// at most 64 VGPRs, 20 KiB of LDS and 80 SGPRs.  Above 80 the trap handler's
+// 16 leave room for seven, the last eighth of the grid waits for a whole
+// round, and a bottom-up level that finds 950 K vertices takes 41 us instead
+// of 28 (82 or 88 SGPRs against 80, the same code otherwise).
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_num_sgpr(80))) void bfs_engine_step(Graph g, Buffers b)
 {
     extern __shared__ uint32_t lbuf[];  // b.lds_queue entries
     __shared__ uint32_t lcount, lbase;
@@ -599,49 +622,44 @@ __global__ __launch_bounds__(kBlock) void bfs_engine_step(Graph g, Buffers b)
 
     BfsState &st = *b.st;
     if (st.done) return;
-    const uint32_t d = st.depth;
-    const int32_t variant = st.choice;
-    if ((variant >= kRef) != REF) return;
+    // Wave-uniform, and said to be: the bitmaps they select are then
+    // addressed from scalar registers.
+    const uint32_t d = __builtin_amdgcn_readfirstlane(st.depth);
+    const uint32_t rot = __builtin_amdgcn_readfirstlane(st.rot);
+    const int32_t variant = __builtin_amdgcn_readfirstlane(st.choice);
     if (blockIdx.x == 0 && threadIdx.x == 0) st.t_step = wall_clock64();
 
     // Clear the bitmap that the next level will write.
-    uint32_t *clear = b.bits[(d + 2) % 3];
+    uint32_t *clear = b.bits[(d + 2 + rot) % 3];
     for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < b.words; i += gridDim.x * kBlock) clear[i] = 0;
 
     if (threadIdx.x == 0) lcount = 0;
     __syncthreads();
-    Emitter em{lbuf, &lcount, &lbase, b.lds_queue};
+    Emitter em{lbuf, &lcount, &lbase, b.lds_queue, rot};
     const bool fill = st.fill_levels != 0;
     // Bottom-up forms write the deferred depths in their vertex loop; the
     // others first write them from this level's frontier bitmap.
     auto fill_depths = [&] {
         if (!fill) return;
-        const uint32_t *front = b.bits[d % 3];
+        const uint32_t *front = b.bits[(d + em.rot) % 3];
         for (uint64_t v = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; v < g.V;
              v += static_cast<uint64_t>(gridDim.x) * kBlock)
             if (test_bit(front, static_cast<uint32_t>(v))) b.levels[v] = static_cast<int32_t>(d);
     };
-    if constexpr (!REF) {
-        if (variant == TD) {
-            fill_depths();
-            level_td(g, b, d, em, sstart, sscan, &stotal, coarse);
-        } else {
-            level_bu<true>(g, b, d, em, variant == BU_WAVE, fill);
-        }
+    if (variant == BU || variant == BU_WAVE || variant == kRef + BW_BFS_VERTEX_PULL) {
+        if (variant == kRef + BW_BFS_VERTEX_PULL) level_bu<false>(g, b, d, em, false, fill);
+        else level_bu<true>(g, b, d, em, variant == BU_WAVE, fill);
     } else {
-        if (variant == kRef + BW_BFS_VERTEX_PULL) {
-            level_bu<false>(g, b, d, em, false, fill);
-        } else {
-            fill_depths();
-            switch (variant - kRef) {
-            case BW_BFS_EDGE_LIST: level_ref_edges<BW_BFS_EDGE_LIST>(g, b, d, em); break;
-            case BW_BFS_REV_EDGE_LIST: level_ref_edges<BW_BFS_REV_EDGE_LIST>(g, b, d, em); break;
-            case BW_BFS_STRUCT_EDGE_LIST: level_ref_edges<BW_BFS_STRUCT_EDGE_LIST>(g, b, d, em); break;
-            case BW_BFS_REV_STRUCT_EDGE_LIST: level_ref_edges<BW_BFS_REV_STRUCT_EDGE_LIST>(g, b, d, em); break;
-            case BW_BFS_VERTEX_PUSH: level_ref_push(g, b, d, em); break;
-            case BW_BFS_VERTEX_PUSH_WARP: level_ref_push_warp(g, b, d, em); break;
-            default: level_ref_pull_warp(g, b, d, em); break;
-            }
+        fill_depths();
+        switch (variant) {
+        case TD: level_td(g, b, d, em, sstart, sscan, &stotal, coarse); break;
+        case kRef + BW_BFS_EDGE_LIST: level_ref_edges<BW_BFS_EDGE_LIST>(g, b, d, em); break;
+        case kRef + BW_BFS_REV_EDGE_LIST: level_ref_edges<BW_BFS_REV_EDGE_LIST>(g, b, d, em); break;
+        case kRef + BW_BFS_STRUCT_EDGE_LIST: level_ref_edges<BW_BFS_STRUCT_EDGE_LIST>(g, b, d, em); break;
+        case kRef + BW_BFS_REV_STRUCT_EDGE_LIST: level_ref_edges<BW_BFS_REV_STRUCT_EDGE_LIST>(g, b, d, em); break;
+        case kRef + BW_BFS_VERTEX_PUSH: level_ref_push(g, b, d, em); break;
+        case kRef + BW_BFS_VERTEX_PUSH_WARP: level_ref_push_warp(g, b, d, em); break;
+        default: level_ref_pull_warp(g, b, d, em); break;
         }
     }
     em.finish(b, d);
@@ -876,190 +894,379 @@ __device__ __forceinline__ void choose_next(const PolicyArgs &p, BfsState &st, c
     if (lane == 0) st.choice = c;
 }
 
-// The per-level epilogue: one workgroup.  Records the finished level,
-// advances the state to the next frontier and picks its variant.
-__global__ __launch_bounds__(kBlock) void bfs_engine_epilogue(Graph g, Buffers b, PolicyArgs p, uint32_t nparts)
-{
-    __shared__ uint64_t rout[kBlock / kWave];
-    __shared__ double rsq[kBlock / kWave];
-    __shared__ uint64_t hscan[kBlock];
-    __shared__ uint32_t sscan[kBlock / kWave];
+// ------------------------------------------------------- small levels
 
-    BfsState &st = *b.st;
-    if (st.done) return;
-    const uint64_t now = wall_clock64();
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
-    // The step kernel that ran the level stamped t_step; none did when the
-    // level's variant is of a kind this launch left out.  Then the level is
-    // still pending: the state stays as it is, and the host relaunches it
-    // with both kinds.
-    if (st.t_step == 0) {
-        if (tid == 0) st.stalled = 1;
+constexpr int kEpi = 512;          // threads of the epilogue and the init kernel
+constexpr uint32_t kTiny = 2048;   // vertices and out-edges of a level run inside them at most
+constexpr uint32_t kTinyLevels = 1024;  // levels one launch runs at most
+
+// The level time that the learned policy's features see is at least what a
+// level of its own launch takes, which is what its trees and networks were
+// fitted to: shown 2 us, the bundled model left top-down on a 1 M-vertex grid.
+constexpr float kLaunchNs = 8000.0f;
+
+struct EpiLds {
+    uint64_t rout[kEpi / kWave];
+    double rsq[kEpi / kWave];
+    uint64_t hscan[kEpi / kWave];
+    uint32_t wsum[kEpi / kWave];
+    uint32_t found;
+    uint32_t vid[2][kTiny];              // the frontier, and the next one
+    uint32_t start[kTiny], before[kTiny];  // per frontier vertex: its first edge, the edges of those before it
+};
+
+// The finished level's report and the state of the next one (thread 0).
+__device__ __forceinline__ void advance(BfsState &st, const Buffers &b, float ns, uint32_t nnew, uint32_t qcount,
+                                        uint32_t qglobal, uint32_t nhub, uint64_t edges, double sq, bool deferred)
+{
+    const uint32_t d = st.depth;
+    if (d < b.max_levels) b.out[d] = LevelOut{static_cast<uint64_t>(ns), nnew, st.choice};
+    st.num_levels = d + 1;
+    if (nnew == 0 || d + 1 >= b.max_levels) {
+        st.done = 1;
         return;
     }
+    st.prev_choice = st.choice;
+    st.prev_time_ns = ns;
+    st.prev_frontier = static_cast<uint64_t>(st.qcount) + st.hubcount;
+    st.depth = d + 1;
+    st.qcount = qcount;
+    st.qglobal = qglobal;
+    st.hubcount = nhub;
+    st.qout = 0;
+    st.hubout = 0;
+    st.visited += nnew;
+    st.explored_edges += edges;
+    st.frontier_edges = edges;
+    st.frontier_sq = sq;
+    st.fill_levels = deferred ? 1u : 0u;
+}
+
+// Whether the pending level is one for tiny_levels.
+__device__ __forceinline__ bool tiny(const PolicyArgs &p, const BfsState &st)
+{
+    return p.fuse && !st.done && st.choice == TD && st.hubcount == 0 && st.qcount <= kTiny &&
+           st.frontier_edges <= kTiny && !st.fill_levels;
+}
+
+// Runs the pending top-down level and those after it in this workgroup while
+// they stay small: a level of a few hundred vertices costs about 20 us as two
+// launches (8 us each even when they find nothing to do, and their gaps) and
+// 2 to 10 us here.  Expects the frontier in L.vid[0], tiny(p, st), and a
+// barrier behind both.  The frontier bitmaps are not touched in between:
+// the first frontier's words are cleared, and the last frontier goes to that
+// bitmap, so the one after it is clean as level_td expects and only the
+// level's index of the bitmap moves (rot).
+__device__ void tiny_levels(const Graph &g, const Buffers &b, const PolicyArgs &p, const LaneModel &lm, BfsState &st,
+                            EpiLds &L)
+{
+    const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
+    constexpr uint32_t kPer = kTiny / kEpi;
+    const uint32_t d0 = st.depth, rot0 = st.rot;
+    uint32_t *bits = b.bits[(d0 + rot0) % 3];
+    uint32_t n = st.qcount, cur = 0, left = kTinyLevels;
+    for (uint32_t i = tid; i < n; i += kEpi) atomicExch(&bits[L.vid[0][i] >> 5], 0u);
+    for (;;) {
+        const uint64_t t0 = wall_clock64();
+        const int32_t nd = static_cast<int32_t>(st.depth) + 1;
+        uint32_t deg[kPer], sum = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < kPer; k++) {
+            const uint32_t i = tid * kPer + k;
+            deg[k] = 0;
+            if (i < n) {
+                const uint32_t v = L.vid[cur][i], s = g.off[v];
+                deg[k] = g.off[v + 1] - s;
+                L.start[i] = s;
+            }
+            sum += deg[k];
+        }
+        const uint32_t incl = wave_prefix_sum(sum);
+        if (lane == kWave - 1) L.wsum[wid] = incl;
+        if (tid == 0) L.found = 0;
+        __syncthreads();
+        uint32_t at = incl - sum, total = 0;
+        for (uint32_t w = 0; w < kEpi / kWave; w++) {
+            if (w < wid) at += L.wsum[w];
+            total += L.wsum[w];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kPer; k++) {
+            if (tid * kPer + k < n) L.before[tid * kPer + k] = at;
+            at += deg[k];
+        }
+        __syncthreads();
+        // total <= kTiny: kPer edges per thread.
+        uint32_t nb[kPer];
+#pragma unroll
+        for (uint32_t k = 0; k < kPer; k++) {
+            const uint32_t e = tid + k * kEpi;
+            nb[k] = kNoParent;
+            if (e < total) {
+                uint32_t lo = 0, hi = n;  // the last vertex whose edges start at or before e
+                while (hi - lo > 1) {
+                    const uint32_t mid = (lo + hi) / 2;
+                    if (L.before[mid] <= e) lo = mid;
+                    else hi = mid;
+                }
+                nb[k] = g.col[L.start[lo] + (e - L.before[lo])];
+            }
+        }
+        uint64_t os = 0;
+        double sq = 0.0;
+#pragma unroll
+        for (uint32_t k = 0; k < kPer; k++) {
+            if (nb[k] == kNoParent || !try_discover(b, nb[k], nd, true)) continue;
+            L.vid[cur ^ 1][atomicAdd(&L.found, 1u)] = nb[k];
+            const uint32_t dw = out_degree(g, nb[k]);
+            os += dw;
+            sq += static_cast<double>(dw) * static_cast<double>(dw);
+        }
+        for (int o = kWave / 2; o > 0; o >>= 1) {
+            os += __shfl_xor(os, o, kWave);
+            sq += __shfl_xor(sq, o, kWave);
+        }
+        if (lane == 0) {
+            L.rout[wid] = os;
+            L.rsq[wid] = sq;
+        }
+        __syncthreads();
+        n = L.found;
+        cur ^= 1;
+        if (tid == 0) {
+            uint64_t a = 0;
+            double q = 0.0;
+            for (uint32_t w = 0; w < kEpi / kWave; w++) {
+                a += L.rout[w];
+                q += L.rsq[w];
+            }
+            advance(st, b, static_cast<float>(wall_clock64() - t0) * b.ns_per_tick, n, n, n, 0, a, q, false);
+            st.prev_time_ns = fmaxf(st.prev_time_ns, kLaunchNs);
+        }
+        if (wid == 0) choose_next(p, st, g, lm);
+        __syncthreads();
+        if (st.done) return;
+        if (--left == 0 || !tiny(p, st)) break;
+    }
+
+    // The next level is not for here: its frontier goes to the queue (a few
+    // hubs to the hub queue) and to the bitmap.
+    const uint32_t dn = st.depth, nq = dn & 1;
+    constexpr uint32_t kHubs = kWave;
+    __syncthreads();  // every thread has read the state and n
+    if (tid == 0) {
+        L.found = 0;
+        L.wsum[0] = 0;
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < n; i += kEpi) {
+        const uint32_t v = L.vid[cur][i], dv = out_degree(g, v);
+        atomicOr(&bits[v >> 5], 1u << (v & 31));
+        if (dv > b.hub_degree) {
+            const uint32_t h = atomicAdd(&L.wsum[0], 1u);
+            if (h < min(kHubs, b.hub_cap)) {
+                b.hubq[nq][h] = v;
+                L.start[h] = dv;
+                continue;
+            }
+        }
+        b.q[nq][atomicAdd(&L.found, 1u)] = v;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        const uint32_t nh = min(L.wsum[0], min(kHubs, b.hub_cap));
+        uint64_t sum = 0;
+        for (uint32_t h = 0; h < nh; h++) {
+            b.hub_prefix[h] = sum;
+            sum += L.start[h];
+        }
+        b.hub_prefix[nh] = sum;
+        st.qcount = st.qglobal = L.found;
+        st.hubcount = nh;
+        st.rot = (rot0 + 2 * (dn - d0)) % 3;
+    }
+}
+
+// The state, back to device memory.
+__device__ __forceinline__ void store_state(const BfsState &st, BfsState *to)
+{
+    static_assert(sizeof(BfsState) % 4 == 0 && sizeof(BfsState) / 4 <= kEpi, "one word per thread");
+    __syncthreads();
+    if (threadIdx.x < sizeof(BfsState) / 4)
+        reinterpret_cast<uint32_t *>(to)[threadIdx.x] = reinterpret_cast<const uint32_t *>(&st)[threadIdx.x];
+}
+
+// The per-level epilogue: one workgroup.  Records the finished level,
+// advances the state to the next frontier, picks its variant, and runs the
+// levels that are small enough.  The loads of its inputs are all issued
+// before the first wait.
+__global__ __launch_bounds__(kEpi) void bfs_engine_epilogue(Graph g, Buffers b, PolicyArgs p, uint32_t nparts)
+{
+    __shared__ EpiLds L;
+    __shared__ BfsState st;
+    __shared__ uint32_t coarse[kMaxGrid / kSegGroup];
+    const uint64_t now = wall_clock64();
+    asm volatile("" ::"s"(now) : "memory");  // read here, not at its use
+    const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
+    uint32_t word = 0;
+    if (tid < sizeof(BfsState) / 4) word = reinterpret_cast<const uint32_t *>(b.st)[tid];
     LaneModel lm;
     if (wid == 0) load_lane_model(p, lm);
+    // This thread's partials and its group of segment counts (padded to
+    // whole groups with zeros).
+    constexpr uint32_t kParts = kMaxGrid / kEpi;
+    static_assert(kParts == kSegGroup, "a thread takes one group of segments");
+    uint64_t pa[kParts], pq[kParts];
+#pragma unroll
+    for (uint32_t j = 0; j < kParts; j++) {
+        const uint32_t i = tid + j * kEpi;
+        pa[j] = i < nparts ? b.part[2 * i] : 0;
+        pq[j] = i < nparts ? b.part[2 * i + 1] : 0;
+    }
+    const uint32_t w0 = tid * kSegGroup;
+    uint4 c0 = make_uint4(0, 0, 0, 0), c1 = c0;
+    if (w0 < nparts) {
+        c0 = reinterpret_cast<const uint4 *>(b.segcount + w0)[0];
+        c1 = reinterpret_cast<const uint4 *>(b.segcount + w0)[1];
+    }
+    if (tid < sizeof(BfsState) / 4) reinterpret_cast<uint32_t *>(&st)[tid] = word;
+    __syncthreads();
+    if (st.done) return;
+    const uint32_t d = st.depth, nq = (d & 1) ^ 1;
+    const uint32_t nhub = min(st.hubout, b.hub_cap);
+    const bool deferred = defer_depths(st, b, g.V);  // this level's, before the state moves on
     uint64_t os = 0;
     double sq = 0.0;
-    // Four partials per thread in flight, added in the order of a plain
-    // stride loop.
-    for (uint32_t i0 = tid; i0 < nparts; i0 += 4 * kBlock) {
-        uint64_t pa[4], pq[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const uint32_t i = i0 + j * kBlock;
-            pa[j] = i < nparts ? b.part[2 * i] : 0;
-            pq[j] = i < nparts ? b.part[2 * i + 1] : 0;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            if (i0 + j * kBlock >= nparts) break;
-            os += pa[j];
-            sq += __longlong_as_double(static_cast<long long>(pq[j]));
-        }
+    for (uint32_t j = 0; j < kParts; j++) {
+        os += pa[j];
+        sq += __longlong_as_double(static_cast<long long>(pq[j]));
     }
     for (int o = kWave / 2; o > 0; o >>= 1) {
         os += __shfl_xor(os, o, kWave);
         sq += __shfl_xor(sq, o, kWave);
     }
+    // The segments' first frontier indexes, behind the queue's vertices.
+    uint32_t c[kSegGroup] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w}, sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kSegGroup; k++) sum += c[k];
+    const uint32_t incl = wave_prefix_sum(sum);
     if (lane == 0) {
-        rout[wid] = os;
-        rsq[wid] = sq;
+        L.rout[wid] = os;
+        L.rsq[wid] = sq;
     }
-    const uint32_t d = st.depth;
-    const uint32_t nhub = min(st.hubout, b.hub_cap);
-    const bool deferred = defer_depths(st, b, g.V);  // this level's, before the state moves on
+    if (lane == kWave - 1) L.wsum[wid] = incl;
     __syncthreads();
-
-    // The segments' first frontier indexes, behind the queue's vertices:
-    // rounds of kSegGroup consecutive segments per thread.
-    const uint32_t qout = st.qout;
-    uint32_t segend = qout;
-    for (uint32_t r0 = 0; r0 < nparts; r0 += kBlock * kSegGroup) {
-        const uint32_t w0 = r0 + tid * kSegGroup;
-        uint32_t c[kSegGroup] = {}, sum = 0;
-        if (w0 < nparts) {  // segcount is padded to whole groups (with zeros)
-            const uint4 x = reinterpret_cast<const uint4 *>(b.segcount + w0)[0];
-            const uint4 y = reinterpret_cast<const uint4 *>(b.segcount + w0)[1];
-            c[0] = x.x, c[1] = x.y, c[2] = x.z, c[3] = x.w, c[4] = y.x, c[5] = y.y, c[6] = y.z, c[7] = y.w;
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < kSegGroup; k++) sum += c[k];
-        const uint32_t incl = wave_prefix_sum(sum);
-        if (lane == kWave - 1) sscan[wid] = incl;
-        __syncthreads();
-        uint32_t at = segend + incl - sum;
-        for (int w = 0; w < kBlock / kWave; w++) {
-            if (w < wid) at += sscan[w];
-            segend += sscan[w];
-        }
-        if (w0 < nparts) {
-#pragma unroll
-            for (uint32_t k = 0; k < kSegGroup; k++) {
-                const uint32_t x = c[k];
-                c[k] = at;
-                at += x;
-            }
-            reinterpret_cast<uint4 *>(b.segbase + w0)[0] = make_uint4(c[0], c[1], c[2], c[3]);
-            reinterpret_cast<uint4 *>(b.segbase + w0)[1] = make_uint4(c[4], c[5], c[6], c[7]);
-        }
-        __syncthreads();  // sscan is rewritten by the next round
+    uint32_t at = st.qout + incl - sum, segend = st.qout;
+    for (uint32_t w = 0; w < kEpi / kWave; w++) {
+        if (w < wid) at += L.wsum[w];
+        segend += L.wsum[w];
     }
-    const uint32_t nnew = nhub + segend;
+    if (w0 < nparts) {
+        coarse[tid] = at;
+#pragma unroll
+        for (uint32_t k = 0; k < kSegGroup; k++) {
+            const uint32_t x = c[k];
+            c[k] = at;
+            at += x;
+        }
+        reinterpret_cast<uint4 *>(b.segbase + w0)[0] = make_uint4(c[0], c[1], c[2], c[3]);
+        reinterpret_cast<uint4 *>(b.segbase + w0)[1] = make_uint4(c[4], c[5], c[6], c[7]);
+    }
 
     // Hub degree prefix of the next frontier, read by the next top-down
-    // level: rounds of kBlock consecutive hubs, one per thread, each an
+    // level: rounds of kEpi consecutive hubs, one per thread, each an
     // exclusive block scan added to the previous rounds' total (a level
     // with few hubs takes one round of two dependent loads).
-    {
-        const uint32_t nq = (d & 1) ^ 1;
+    if (nhub) {
         // The degrees of the first kPreRounds rounds are loaded before any
         // scan, so those rounds wait on memory once.
-        constexpr int kPreRounds = 16;
+        constexpr int kPreRounds = 8;
         uint32_t ids[kPreRounds];
         uint64_t degs[kPreRounds];
 #pragma unroll
         for (int r = 0; r < kPreRounds; r++) {
-            const uint32_t h = r * kBlock + tid;
+            const uint32_t h = r * kEpi + tid;
             ids[r] = h < nhub ? b.hubq[nq][h] : 0u;
         }
 #pragma unroll
         for (int r = 0; r < kPreRounds; r++)
-            degs[r] = r * kBlock + tid < nhub ? out_degree(g, ids[r]) : 0;
+            degs[r] = r * kEpi + tid < nhub ? out_degree(g, ids[r]) : 0;
         uint64_t carry = 0;
         auto round = [&](uint32_t r0, uint64_t deg) {
             const uint32_t h = r0 + tid;
-            uint64_t incl = deg;
-            for (int o = 1; o < kWave; o <<= 1) {
-                const uint64_t y = __shfl_up(incl, static_cast<unsigned>(o), kWave);
-                if (lane >= o) incl += y;
-            }
-            if (lane == kWave - 1) hscan[wid] = incl;
+            const uint64_t to = wave_prefix_sum(deg);
+            if (lane == kWave - 1) L.hscan[wid] = to;
             __syncthreads();
             uint64_t before = carry, total = carry;
-            for (int w = 0; w < kBlock / kWave; w++) {
-                if (w < wid) before += hscan[w];
-                total += hscan[w];
+            for (uint32_t w = 0; w < kEpi / kWave; w++) {
+                if (w < wid) before += L.hscan[w];
+                total += L.hscan[w];
             }
-            if (h < nhub) b.hub_prefix[h] = before + incl - deg;
+            if (h < nhub) b.hub_prefix[h] = before + to - deg;
             carry = total;
             __syncthreads();  // hscan is rewritten by the next round
         };
 #pragma unroll
         for (int r = 0; r < kPreRounds; r++)
-            if (r * kBlock < nhub) round(r * kBlock, degs[r]);
-        for (uint32_t r0 = kPreRounds * kBlock; r0 < nhub; r0 += kBlock) {
+            if (r * kEpi < static_cast<int>(nhub)) round(r * kEpi, degs[r]);
+        for (uint32_t r0 = kPreRounds * kEpi; r0 < nhub; r0 += kEpi) {
             const uint32_t h = r0 + tid;
             round(r0, h < nhub ? out_degree(g, b.hubq[nq][h]) : 0);
         }
         if (tid == 0) b.hub_prefix[nhub] = carry;
+    } else if (tid == 0) {
+        b.hub_prefix[0] = 0;
     }
 
+    __syncthreads();  // the state has been read
     if (tid == 0) {
         uint64_t a = 0;
         double q = 0.0;
-        for (int w = 0; w < kBlock / kWave; w++) {
-            a += rout[w];
-            q += rsq[w];
+        for (uint32_t w = 0; w < kEpi / kWave; w++) {
+            a += L.rout[w];
+            q += L.rsq[w];
         }
         // Level time: from the start of the step kernel's first workgroup
         // to the start of this epilogue.
         const float ns = static_cast<float>(now - st.t_step) * b.ns_per_tick;
-        st.t_step = 0;  // read above by every thread, before the barriers
-        if (d < b.max_levels) {
-            b.counts[d] = nnew;
-            b.times[d] = static_cast<uint64_t>(ns);
-            b.choices[d] = st.choice;
-        }
-        st.num_levels = d + 1;
-        if (nnew == 0 || d + 1 >= b.max_levels) {
-            st.done = 1;
-        } else {
-            st.prev_choice = st.choice;
-            st.prev_time_ns = ns;
-            st.prev_frontier = static_cast<uint64_t>(st.qcount) + st.hubcount;
-            st.depth = d + 1;
-            st.qcount = segend;
-            st.qglobal = qout;
-            st.hubcount = nhub;
-            st.qout = 0;
-            st.hubout = 0;
-            st.visited += nnew;
-            st.explored_edges += a;
-            st.frontier_edges = a;
-            st.frontier_sq = q;
-            st.fill_levels = deferred ? 1u : 0u;
-        }
+        st.t_step = 0;
+        advance(st, b, ns, nhub + segend, segend, st.qout, nhub, a, q, deferred);
     }
     if (wid == 0) choose_next(p, st, g, lm);
+    __syncthreads();
+    if (tiny(p, st)) {
+        const uint32_t n = st.qcount, ng = st.qglobal;
+        for (uint32_t i = tid; i < n; i += kEpi)
+            L.vid[0][i] = i < ng ? b.q[nq][i] : segment_vertex(b, nq, nparts, coarse, i);
+        __syncthreads();
+        tiny_levels(g, b, p, lm, st, L);
+    }
+    store_state(st, b.st);
+}
+
+// Every level unvisited, the frontier bitmaps empty, and the vertices
+// without in-edges visited.
+__global__ __launch_bounds__(kBlock) void bfs_engine_reset(uint64_t V, Buffers b, const uint32_t *no_in)
+{
+    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
+    const uint64_t t = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    for (uint64_t i = t; i < b.words; i += stride) {
+        b.bits[0][i] = 0;
+        b.bits[1][i] = 0;
+        b.bits[2][i] = 0;
+        b.vis[i] = no_in[i];
+    }
+    for (uint64_t v = t; v < V; v += stride) b.levels[v] = kUnvisited;
 }
 
 // Level 0: the roots (roots[0..nroots), or just `root` when roots is NULL)
 // are the whole frontier; a repeated root counts once.
-__global__ __launch_bounds__(kBlock) void bfs_engine_init(Graph g, Buffers b, PolicyArgs p, uint32_t root,
-                                                          const uint32_t *roots, uint32_t nroots)
+__global__ __launch_bounds__(kEpi) void bfs_engine_init(Graph g, Buffers b, PolicyArgs p, uint32_t root,
+                                                        const uint32_t *roots, uint32_t nroots)
 {
-    BfsState &st = *b.st;
+    __shared__ EpiLds L;
+    __shared__ BfsState st;
     LaneModel lm;
     if (threadIdx.x < kWave) load_lane_model(p, lm);
     if (threadIdx.x == 0) {
@@ -1098,7 +1305,7 @@ __global__ __launch_bounds__(kBlock) void bfs_engine_init(Graph g, Buffers b, Po
         st.prev_choice = -1;
         st.prev_time_ns = 0.0f;
         st.t_step = 0;
-        st.stalled = 0;
+        st.rot = 0;
         st.fill_levels = 0;
         st.qcount = nq;
         st.qglobal = nq;
@@ -1106,6 +1313,13 @@ __global__ __launch_bounds__(kBlock) void bfs_engine_init(Graph g, Buffers b, Po
         st.choice = p.fixed;
     }
     if (threadIdx.x < kWave) choose_next(p, st, g, lm);
+    __syncthreads();
+    if (tiny(p, st)) {
+        for (uint32_t i = threadIdx.x; i < st.qcount; i += kEpi) L.vid[0][i] = b.q[0][i];
+        __syncthreads();
+        tiny_levels(g, b, p, lm, st, L);
+    }
+    store_state(st, b.st);
 }
 
 __global__ void set_choice(BfsState *st, int32_t c) { st->choice = c; }
@@ -1171,7 +1385,6 @@ struct bw_bfs_engine {
     int32_t mlp_out = 0;
     int32_t *schedule = nullptr;
     int32_t schedule_cap = 0;
-    uint32_t schedule_kinds = 1;  // level kernels the schedule needs (see policy_kinds)
     uint32_t *roots = nullptr;
     uint32_t roots_cap = 0;
     uint32_t *no_in = nullptr;  // vertices without in-edges (bitmap)
@@ -1191,7 +1404,7 @@ struct bw_bfs_engine {
     {
         drop_exec();
         void *bufs[] = {own_levels, b.q[0], b.q[1], b.hubq[0], b.hubq[1], b.hub_prefix, b.bits[0], b.bits[1],
-                        b.bits[2], b.vis, b.st, b.part, b.counts, b.times, b.choices, snap_levels, snap_q, snap_hub,
+                        b.bits[2], b.vis, b.st, b.part, snap_levels, snap_q, snap_hub,
                         b.seg[0], b.seg[1], b.segcount, b.segbase, snap_seg, snap_segbase,
                         snap_bits, snap_prefix, snap_st, mlp, schedule, roots, no_in, parent};
         for (void *p : bufs)
@@ -1202,7 +1415,8 @@ struct bw_bfs_engine {
 
 namespace {
 
-PolicyArgs make_policy(const bw_bfs_engine *e, int32_t policy, int32_t fixed, int32_t schedule_len)
+// fuse: the epilogues may run small levels themselves (whole searches).
+PolicyArgs make_policy(const bw_bfs_engine *e, int32_t policy, int32_t fixed, int32_t schedule_len, bool fuse = false)
 {
     PolicyArgs p;
     p.policy = policy;
@@ -1211,6 +1425,7 @@ PolicyArgs make_policy(const bw_bfs_engine *e, int32_t policy, int32_t fixed, in
     p.schedule_len = std::max(schedule_len, 1);
     p.mlp = e->mlp;
     p.nout = e->mlp_out;
+    p.fuse = fuse && policy != HOST;
     return p;
 }
 
@@ -1233,34 +1448,17 @@ int check_policy(const bw_bfs_engine *e, int32_t policy, int32_t fixed, int32_t 
     return BW_HIP_OK;
 }
 
-// Which level kernels a policy may need: bit 0 the native one, bit 1 the
-// reference families' (a level launches each it may need; the one whose
-// kind the level's variant is not returns at once).
-uint32_t policy_kinds(const bw_bfs_engine *e, const PolicyArgs &p)
+int launch_step(bw_bfs_engine *e, hipStream_t s)
 {
-    switch (p.policy) {
-    case FIXED: return p.fixed < kRef ? 1u : 2u;
-    case SCHEDULE: return e->schedule_kinds;
-    case LEARNED: return p.nout > kRef ? 3u : 1u;
-    case BEAMER: return 1u;
-    default: return 3u;  // HOST: the variant is set on the device
-    }
-}
-
-int launch_step(bw_bfs_engine *e, bool ref, hipStream_t s)
-{
-    const size_t lds = sizeof(uint32_t) * e->b.lds_queue;
-    if (ref) hipLaunchKernelGGL(bfs_engine_step<true>, dim3(e->grid), dim3(kBlock), lds, s, e->g, e->b);
-    else hipLaunchKernelGGL(bfs_engine_step<false>, dim3(e->grid), dim3(kBlock), lds, s, e->g, e->b);
+    hipLaunchKernelGGL(bfs_engine_step, dim3(e->grid), dim3(kBlock), sizeof(uint32_t) * e->b.lds_queue, s, e->g, e->b);
     BW_LAUNCH_CHECK();
     return BW_HIP_OK;
 }
 
-int launch_level(bw_bfs_engine *e, const PolicyArgs &p, hipStream_t s, uint32_t kinds)
+int launch_level(bw_bfs_engine *e, const PolicyArgs &p, hipStream_t s)
 {
-    if (kinds & 1u) BW_TRY(launch_step(e, false, s));
-    if (kinds & 2u) BW_TRY(launch_step(e, true, s));
-    hipLaunchKernelGGL(bfs_engine_epilogue, dim3(1), dim3(kBlock), 0, s, e->g, e->b, p, e->grid);
+    BW_TRY(launch_step(e, s));
+    hipLaunchKernelGGL(bfs_engine_epilogue, dim3(1), dim3(kEpi), 0, s, e->g, e->b, p, e->grid);
     BW_LAUNCH_CHECK();
     return BW_HIP_OK;
 }
@@ -1308,11 +1506,8 @@ extern "C" int bw_bfs_engine_create(bw_bfs_engine **out, const bw_graph_dev *g, 
     alloc(&e->b.vis, sizeof(uint32_t) * words);
     alloc(&e->no_in, sizeof(uint32_t) * words);
     alloc(&e->parent, sizeof(uint32_t) * V);
-    alloc(&e->b.st, sizeof(BfsState));
+    alloc(&e->b.st, kOutOffset + sizeof(LevelOut) * std::max<size_t>(max_levels, kOutFirst));
     alloc(&e->b.part, sizeof(uint64_t) * 2 * e->grid);
-    alloc(&e->b.counts, sizeof(uint32_t) * max_levels);
-    alloc(&e->b.times, sizeof(uint64_t) * max_levels);
-    alloc(&e->b.choices, sizeof(int32_t) * max_levels);
     e->b.max_levels = max_levels;
     e->b.words = words;
     e->b.ns_per_tick = 1e6f / static_cast<float>(rate_khz);
@@ -1325,6 +1520,7 @@ extern "C" int bw_bfs_engine_create(bw_bfs_engine **out, const bw_graph_dev *g, 
         return fail(BW_HIP_ERR_NOMEM, "device allocation of the BFS engine failed");
     }
     e->b.parent = e->parent;
+    e->b.out = reinterpret_cast<LevelOut *>(reinterpret_cast<char *>(e->b.st) + kOutOffset);
     if (bw_hip_fill_u32(e->b.segcount, 0u, segs, nullptr) != BW_HIP_OK) {
         delete e;
         return BW_HIP_ERR_RUNTIME;
@@ -1369,13 +1565,7 @@ extern "C" int bw_bfs_engine_set_model(bw_bfs_engine *e, const float *weights, i
 extern "C" int bw_bfs_engine_set_schedule(bw_bfs_engine *e, const int32_t *schedule, int32_t len)
 {
     if (!e || !schedule || len < 1) return fail(BW_HIP_ERR_ARG, "invalid schedule");
-    uint32_t kinds = 0;
-    for (int32_t i = 0; i < len; i++) {
-        BW_TRY(check_variant(e, schedule[i]));
-        kinds |= schedule[i] < kRef ? 1u : 2u;
-    }
-    if (kinds != e->schedule_kinds) e->drop_exec();  // the captured batch launches per the kinds
-    e->schedule_kinds = kinds;
+    for (int32_t i = 0; i < len; i++) BW_TRY(check_variant(e, schedule[i]));
     if (len > e->schedule_cap) {
         e->drop_exec();  // the captured batch holds the old schedule pointer
         if (e->schedule) (void)hipFree(e->schedule);
@@ -1417,14 +1607,13 @@ namespace {
 // Resets levels, bitmaps and state; roots_dev (device, n entries) or the
 // single `root` form the depth-0 frontier.
 int begin_impl(bw_bfs_engine *e, uint32_t root, const uint32_t *roots_dev, uint32_t nroots, int32_t policy,
-               int32_t fixed, int32_t schedule_len, hipStream_t s)
+               int32_t fixed, int32_t schedule_len, hipStream_t s, bool fuse)
 {
     BW_TRY(check_policy(e, policy, fixed, schedule_len));
-    BW_TRY(bw_hip_fill_u32(e->b.levels, static_cast<uint32_t>(kUnvisited), e->g.V, s));
-    for (uint32_t *bm : e->b.bits) BW_TRY(bw_hip_fill_u32(bm, 0u, e->b.words, s));
-    BW_HIP_CHECK(hipMemcpyAsync(e->b.vis, e->no_in, sizeof(uint32_t) * e->b.words, hipMemcpyDeviceToDevice, s));
-    hipLaunchKernelGGL(bfs_engine_init, dim3(1), dim3(kBlock), 0, s, e->g, e->b,
-                       make_policy(e, policy, fixed, schedule_len), root, roots_dev, nroots);
+    hipLaunchKernelGGL(bfs_engine_reset, dim3(e->grid), dim3(kBlock), 0, s, e->g.V, e->b, e->no_in);
+    BW_LAUNCH_CHECK();
+    hipLaunchKernelGGL(bfs_engine_init, dim3(1), dim3(kEpi), 0, s, e->g, e->b,
+                       make_policy(e, policy, fixed, schedule_len, fuse), root, roots_dev, nroots);
     BW_LAUNCH_CHECK();
     return BW_HIP_OK;
 }
@@ -1457,7 +1646,8 @@ extern "C" int bw_bfs_engine_begin(bw_bfs_engine *e, uint32_t root, int32_t poli
 {
     if (!e) return fail(BW_HIP_ERR_ARG, "engine is NULL");
     if (root >= e->g.V) return fail(BW_HIP_ERR_ARG, "root out of range");
-    return begin_impl(e, root, nullptr, 0, policy, fixed, schedule_len, static_cast<hipStream_t>(stream));
+    return begin_impl(e, root, nullptr, 0, policy, fixed, schedule_len, static_cast<hipStream_t>(stream),
+                      false);
 }
 
 extern "C" int bw_bfs_engine_begin_multi(bw_bfs_engine *e, const uint32_t *roots_host, uint32_t nroots,
@@ -1466,7 +1656,7 @@ extern "C" int bw_bfs_engine_begin_multi(bw_bfs_engine *e, const uint32_t *roots
     if (!e) return fail(BW_HIP_ERR_ARG, "engine is NULL");
     hipStream_t s = static_cast<hipStream_t>(stream);
     BW_TRY(upload_roots(e, roots_host, nroots, s));
-    return begin_impl(e, 0, e->roots, nroots, policy, fixed, schedule_len, s);
+    return begin_impl(e, 0, e->roots, nroots, policy, fixed, schedule_len, s, false);
 }
 
 // One level (step kernel + epilogue) with the given policy choosing the
@@ -1477,7 +1667,7 @@ extern "C" int bw_bfs_engine_level(bw_bfs_engine *e, int32_t policy, int32_t fix
     if (!e) return fail(BW_HIP_ERR_ARG, "engine is NULL");
     BW_TRY(check_policy(e, policy, fixed, schedule_len));
     const PolicyArgs p = make_policy(e, policy, fixed, schedule_len);
-    return launch_level(e, p, static_cast<hipStream_t>(stream), policy_kinds(e, p));
+    return launch_level(e, p, static_cast<hipStream_t>(stream));
 }
 
 // Overrides the variant of the pending level.
@@ -1569,10 +1759,10 @@ extern "C" int bw_bfs_engine_step_forced(bw_bfs_engine *e, int32_t variant, floa
     BW_HIP_CHECK(hipEventCreate(&ev1));
     int st = BW_HIP_OK;
     if (hipEventRecord(ev0, s) != hipSuccess) st = fail(BW_HIP_ERR_RUNTIME, "event record failed");
-    if (st == BW_HIP_OK) st = launch_step(e, variant >= kRef, s);
+    if (st == BW_HIP_OK) st = launch_step(e, s);
     if (st == BW_HIP_OK && hipEventRecord(ev1, s) != hipSuccess) st = fail(BW_HIP_ERR_RUNTIME, "event record failed");
     if (st == BW_HIP_OK) {
-        hipLaunchKernelGGL(bfs_engine_epilogue, dim3(1), dim3(kBlock), 0, s, e->g, e->b,
+        hipLaunchKernelGGL(bfs_engine_epilogue, dim3(1), dim3(kEpi), 0, s, e->g, e->b,
                            make_policy(e, HOST, variant, 1), e->grid);
         hipError_t le = hipGetLastError();
         if (le != hipSuccess) st = hip_fail(le, "bfs_engine_epilogue", __FILE__, __LINE__);
@@ -1586,7 +1776,8 @@ extern "C" int bw_bfs_engine_step_forced(bw_bfs_engine *e, int32_t variant, floa
     BfsState after;
     BW_HIP_CHECK(hipMemcpy(&after, e->b.st, sizeof after, hipMemcpyDeviceToHost));
     if (ms) *ms = t;
-    if (count) BW_HIP_CHECK(hipMemcpy(count, e->b.counts + before.depth, sizeof(uint32_t), hipMemcpyDeviceToHost));
+    if (count)
+        BW_HIP_CHECK(hipMemcpy(count, &e->b.out[before.depth].count, sizeof(uint32_t), hipMemcpyDeviceToHost));
     if (done) *done = after.done;
     return BW_HIP_OK;
 }
@@ -1610,15 +1801,7 @@ int run_impl(bw_bfs_engine *e, uint32_t root, const uint32_t *roots_host, uint32
         s = e->own_stream;
     }
     if (roots_host) BW_TRY(upload_roots(e, roots_host, nroots, s));
-    const PolicyArgs p = make_policy(e, policy, fixed, schedule_len);
-    // A learned policy over both kinds launches only the native level kernel
-    // (the reference families' kernel would mostly return at once, a fixed
-    // cost per level) until a level picks a reference family.  That level's
-    // epilogue leaves it pending and flags the state as stalled, and from the
-    // next batch on the search launches both kinds.
-    const uint32_t all_kinds = policy_kinds(e, p);
-    const uint32_t graph_kinds = (policy == LEARNED && all_kinds == 3u) ? 1u : all_kinds;
-    uint32_t kinds = graph_kinds;
+    const PolicyArgs p = make_policy(e, policy, fixed, schedule_len, true);
     if (use_graph) {
         const int32_t key[4] = {policy, fixed, std::max(schedule_len, 1), levels_per_sync};
         if (e->exec && (std::memcmp(key, e->exec_key, sizeof key) != 0 || e->exec_stream != s)) {
@@ -1631,7 +1814,7 @@ int run_impl(bw_bfs_engine *e, uint32_t root, const uint32_t *roots_host, uint32
             BW_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
             int cst = BW_HIP_OK;
             for (int32_t i = 0; cst == BW_HIP_OK && i < levels_per_sync; i++)
-                cst = launch_level(e, p, s, graph_kinds);
+                cst = launch_level(e, p, s);
             hipError_t ce = hipStreamEndCapture(s, &graph);
             if (cst != BW_HIP_OK) {
                 if (graph) (void)hipGraphDestroy(graph);
@@ -1654,28 +1837,31 @@ int run_impl(bw_bfs_engine *e, uint32_t root, const uint32_t *roots_host, uint32
     int st = BW_HIP_OK;
     if (hipEventRecord(ev0, s) != hipSuccess) st = fail(BW_HIP_ERR_RUNTIME, "event record failed");
     if (st == BW_HIP_OK)
-        st = begin_impl(e, root, roots_host ? e->roots : nullptr, nroots, policy, fixed, schedule_len, s);
-    BfsState bs{};
+        st = begin_impl(e, root, roots_host ? e->roots : nullptr, nroots, policy, fixed, schedule_len, s, true);
+    struct {
+        BfsState st;
+        char pad[kOutOffset - sizeof(BfsState)];
+        LevelOut out[kOutFirst];
+    } host{};
+    static_assert(offsetof(decltype(host), out) == kOutOffset, "as on the device");
+    BfsState &bs = host.st;
     uint32_t batches = 0;
-    // One more batch than the levels need: the one a stall leaves unfinished.
-    const uint32_t max_batches = e->b.max_levels / static_cast<uint32_t>(levels_per_sync) + 3;
+    const uint32_t max_batches = e->b.max_levels / static_cast<uint32_t>(levels_per_sync) + 2;
     while (st == BW_HIP_OK && !bs.done) {
         if (batches++ > max_batches) {
             st = fail(BW_HIP_ERR_LIMIT, "BFS engine exceeded its level bound");
             break;
         }
-        if (use_graph && kinds == graph_kinds) {
+        if (use_graph) {
             hipError_t le = hipGraphLaunch(e->exec, s);
             if (le != hipSuccess) st = hip_fail(le, "hipGraphLaunch", __FILE__, __LINE__);
         } else {
-            for (int32_t i = 0; st == BW_HIP_OK && i < levels_per_sync; i++) st = launch_level(e, p, s, kinds);
+            for (int32_t i = 0; st == BW_HIP_OK && i < levels_per_sync; i++) st = launch_level(e, p, s);
         }
         if (st != BW_HIP_OK) break;
-        if (hipMemcpyAsync(&bs, e->b.st, sizeof bs, hipMemcpyDeviceToHost, s) != hipSuccess ||
+        if (hipMemcpyAsync(&host, e->b.st, sizeof host, hipMemcpyDeviceToHost, s) != hipSuccess ||
             hipStreamSynchronize(s) != hipSuccess)
             st = fail(BW_HIP_ERR_RUNTIME, "reading the BFS state failed");
-        else if (bs.stalled)
-            kinds = all_kinds;
     }
     if (st == BW_HIP_OK) {
         if (hipEventRecord(ev1, s) != hipSuccess || hipEventSynchronize(ev1) != hipSuccess)
@@ -1686,22 +1872,23 @@ int run_impl(bw_bfs_engine *e, uint32_t root, const uint32_t *roots_host, uint32
     (void)hipEventDestroy(ev0);
     (void)hipEventDestroy(ev1);
     if (st != BW_HIP_OK) return st;
-    BfsState hs;
-    BW_HIP_CHECK(hipMemcpy(&hs, e->b.st, sizeof hs, hipMemcpyDeviceToHost));
-    *num_levels = hs.num_levels;
-    if (hs.num_levels >= e->b.max_levels) {
-        uint32_t last = 0;
-        BW_HIP_CHECK(hipMemcpy(&last, e->b.counts + e->b.max_levels - 1, sizeof last, hipMemcpyDeviceToHost));
-        if (last != 0)
-            return fail(BW_HIP_ERR_LIMIT, "BFS reached max_levels = " + std::to_string(e->b.max_levels) +
-                                              " with a non-empty frontier");
+    *num_levels = bs.num_levels;
+    const size_t n = std::min<uint32_t>(bs.num_levels, e->b.max_levels);
+    std::vector<LevelOut> more;
+    const LevelOut *out = host.out;
+    if (n > kOutFirst) {
+        more.resize(n);
+        BW_HIP_CHECK(hipMemcpy(more.data(), e->b.out, sizeof(LevelOut) * n, hipMemcpyDeviceToHost));
+        out = more.data();
     }
-    const size_t n = std::min<uint32_t>(hs.num_levels, e->b.max_levels);
-    if (counts_host && n) BW_HIP_CHECK(hipMemcpy(counts_host, e->b.counts, sizeof(uint32_t) * n, hipMemcpyDeviceToHost));
-    if (times_ns_host && n)
-        BW_HIP_CHECK(hipMemcpy(times_ns_host, e->b.times, sizeof(uint64_t) * n, hipMemcpyDeviceToHost));
-    if (choices_host && n)
-        BW_HIP_CHECK(hipMemcpy(choices_host, e->b.choices, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
+    if (bs.num_levels >= e->b.max_levels && out[e->b.max_levels - 1].count != 0)
+        return fail(BW_HIP_ERR_LIMIT, "BFS reached max_levels = " + std::to_string(e->b.max_levels) +
+                                          " with a non-empty frontier");
+    for (size_t i = 0; i < n; i++) {
+        if (counts_host) counts_host[i] = out[i].count;
+        if (times_ns_host) times_ns_host[i] = out[i].ns;
+        if (choices_host) choices_host[i] = out[i].choice;
+    }
     return BW_HIP_OK;
 }
 

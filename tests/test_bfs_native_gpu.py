@@ -282,10 +282,9 @@ def _depth_model(ref_variant: str, from_depth: int) -> np.ndarray:
 @pytest.mark.parametrize("use_graph", [True, False])
 @pytest.mark.parametrize("ref_variant,from_depth", [("vertex-push", 2), ("edge-list", 3), ("vertex-pull-warp", 1)])
 def test_learned_launches_reference_kernel_when_picked(cases, use_graph, ref_variant, from_depth):
-    """The learned policy launches only the native level kernel until a level
-    picks a reference family; that level stalls and the search goes on with
-    both kinds.  Depths and counts match the oracle, and every level ran the
-    variant the model picked for it."""
+    """A learned policy that goes over to a reference family at some depth.
+    Depths and counts match the oracle, and every level ran the variant the
+    model picked for it."""
     eng_model = _depth_model(ref_variant, from_depth)
     for g, csr, dg, eng, roots in cases[:4]:
         eng.set_model(eng_model)
