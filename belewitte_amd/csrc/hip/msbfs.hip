@@ -13,10 +13,11 @@
 //    tunable wave threshold; a vertex above the tunable hub degree is cut
 //    into chunks of in-edges, one wave each, that OR into next[] with
 //    atomics (msbfs_bu_hubs);
-//  - top-down: the frontier vertices are queued with their out-edge ranges
-//    reserved in one counter, then every frontier edge u -> w ORs u's mask
-//    into next[w] (edge-parallel, so a hub's edges spread over the grid).
-//    OR is order-independent, so the result is the same bit for bit.
+//  - top-down: the frontier's out-edges are numbered in vertex order (the
+//    level before left their prefix sums, per 64 vertices and within), then
+//    every frontier edge u -> w ORs u's mask into next[w] (edge-parallel,
+//    so a hub's edges spread over the grid).  OR is order-independent, so
+//    the result is the same bit for bit.
 // Either way the new bits give depth + 1 in those searches.  The level loop
 // runs on the device (a done flag read by every kernel), launched in
 // hipGraph batches.
@@ -24,7 +25,7 @@
 #include "common.hpp"
 
 #include <algorithm>
-#include <cstring>
+#include <cstddef>
 #include <vector>
 
 namespace bw {
@@ -32,7 +33,8 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kUnroll = 4;       // bottom-up wave path: chunks of 64 in-edges per round trip
-constexpr uint32_t kSlots = 8;   // top-down expand: consecutive edge slots per thread
+constexpr uint32_t kSlots = 2;   // top-down expand: edges per thread at a time
+constexpr int kEpi = 1024;       // threads of the epilogue and the init kernel
 // Bottom-up: vertices with more in-edges than the tunable hub degree are
 // split into chunks of kHubChunk in-edges, one wave each (msbfs_bu_hubs),
 // so that a few waves holding many such vertices do not hold up the level.
@@ -44,8 +46,16 @@ struct MsState {
     uint32_t done;
     uint32_t num_levels;
     uint32_t topdown;                // direction of the current level (1: top-down)
-    unsigned long long queue;        // top-down: (queued vertices << 32) | out-edges reserved
-    unsigned long long next_edges;   // out-edges of the vertices reached at this level
+    uint64_t edges;                  // out-edges of the frontier
+};
+
+// The state and the levels' counts share one allocation, so that the host
+// reads the state and the first kOutFirst counts in one copy.
+constexpr size_t kOutOffset = 64, kOutFirst = 64;
+static_assert(sizeof(MsState) <= kOutOffset, "the counts follow the state");
+
+struct Sources {
+    uint32_t v[64];
 };
 
 struct MsArgs {
@@ -59,13 +69,20 @@ struct MsArgs {
     uint64_t *front[2];  // level d reads front[d & 1], writes front[(d & 1) ^ 1]
     uint64_t *next;      // ORed frontier masks per vertex from the top-down edges or the hub
                          // chunks (zero between levels)
-    uint2 *queue;        // top-down: (vertex, first reserved edge) per frontier vertex
+    // The frontier's out-edges in vertex order: per vertex of a tile of 64
+    // (one wave of msbfs_level) the edges of the frontier vertices before it
+    // in the tile (only written where the tile has any), per tile its edges
+    // and, on top-down levels, those of the tiles before it.
+    uint32_t *before;
+    uint32_t *tile_edges, *tile_first;
+    uint32_t tiles;
+    uint64_t *part;      // per workgroup of msbfs_level: newly set bits, out-edges
     const uint4 *hubs;   // bottom-up: (vertex, first in-edge, end) per hub chunk
     uint32_t nhubs;
     uint32_t hub_degree; // in-degree above which a vertex is covered by hub chunks
     int32_t *depths;     // [nsrc][V]
     uint64_t all;        // mask of the nsrc searches
-    unsigned long long *level_bits;  // per level: newly set bits
+    uint64_t *level_bits;  // per level: newly set bits
     MsState *st;
     uint32_t max_levels;
     uint32_t wave_degree;
@@ -91,29 +108,19 @@ __device__ __forceinline__ void record(const MsArgs &a, uint64_t v, uint64_t nb,
     }
 }
 
-__device__ __forceinline__ void block_add(unsigned long long x, unsigned long long *dst,
-                                          unsigned long long (*part)[kBlock / kWave])
-{
-    for (int o = kWave / 2; o > 0; o >>= 1) x += __shfl_xor(x, o, kWave);
-    if (__lane_id() == 0) (*part)[threadIdx.x / kWave] = x;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned long long t = 0;
-        for (int w = 0; w < kBlock / kWave; w++) t += (*part)[w];
-        if (t) atomicAdd(dst, t);
-    }
-    __syncthreads();
-}
-
 // One level over all vertices.  Bottom-up: pulls the frontier masks of the
 // in-neighbours.  Top-down: takes the masks ORed into next[] by
-// msbfs_td_expand (and clears them).  Then the new bits update the visit
-// mask, the next frontier and the depths, and the block adds its new bits
-// and the next frontier's out-edges to the level's counters.
+// the expansion (and clears them).  Then the new bits update the visit mask,
+// the next frontier, the depths and the numbering of the frontier's edges;
+// the workgroup's new bits and out-edges go to part[] (the epilogue adds
+// them up: an atomic per workgroup on one counter would take about 3 ns
+// each, one after the other, 12 us a level for the two).  Tiles go to the
+// workgroups spread over the XCDs (spread_block): in generated order the
+// low-numbered vertices have most of the edges.
 __global__ __launch_bounds__(kBlock) void msbfs_level(MsArgs a)
 {
-    __shared__ unsigned long long part[kBlock / kWave];
-    MsState &st = *a.st;
+    __shared__ uint64_t wfound[kBlock / kWave], wedges[kBlock / kWave];
+    const MsState &st = *a.st;
     if (st.done) return;
     const uint32_t d = st.depth;
     const bool td = st.topdown != 0;
@@ -122,8 +129,8 @@ __global__ __launch_bounds__(kBlock) void msbfs_level(MsArgs a)
     const uint64_t *fin = (d & 1) ? a.front[1] : a.front[0];
     uint64_t *fout = (d & 1) ? a.front[0] : a.front[1];
     const int lane = __lane_id();
-    unsigned long long found = 0, nedges = 0;
-    for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * kBlock; base < a.V;
+    uint64_t found = 0, nedges = 0;
+    for (uint64_t base = static_cast<uint64_t>(spread_block(blockIdx.x, gridDim.x)) * kBlock; base < a.V;
          base += static_cast<uint64_t>(gridDim.x) * kBlock) {
         const uint64_t v64 = base + threadIdx.x;
         const uint32_t v = static_cast<uint32_t>(v64);
@@ -182,117 +189,111 @@ __global__ __launch_bounds__(kBlock) void msbfs_level(MsArgs a)
             }
         }
         const uint64_t nb = acc & ~vis;
+        uint32_t deg = 0;
         if (live) {
             fout[v] = nb;
             if (nb) {
                 a.visit[v] = vis | nb;
                 found += __popcll(nb);
-                nedges += a.off[v + 1] - a.off[v];
+                deg = a.off[v + 1] - a.off[v];
             }
+        }
+        if (base + (threadIdx.x & ~(kWave - 1u)) < a.V) {
+            const uint32_t incl = wave_prefix_sum(deg), all = __shfl(incl, kWave - 1, kWave);
+            if (all) a.before[v] = incl - deg;  // past the last vertex too
+            if (lane == 0) a.tile_edges[v / kWave] = all;
+            nedges += deg;
         }
         record(a, v64, nb, nd);
     }
-    block_add(found, &a.level_bits[d], &part);
-    block_add(nedges, &st.next_edges, &part);
-}
-
-// Top-down, step 1: queues the frontier vertices with out-edges, reserving
-// a contiguous range of edge slots for each.  Workgroup b takes a
-// contiguous chunk of vertices: it counts its entries and edges, reserves
-// them with one atomic, then writes them, so within the queue the reserved
-// ranges increase with the entry.
-__device__ __forceinline__ void td_scan(const MsArgs &a, MsState &st)
-{
-    __shared__ uint32_t wcnt[kBlock / kWave], wdeg[kBlock / kWave];
-    __shared__ unsigned long long base_slot;
-    const uint64_t *fin = (st.depth & 1) ? a.front[1] : a.front[0];
-    const int lane = __lane_id(), wid = threadIdx.x / kWave;
-    const uint64_t chunk = (a.V + gridDim.x - 1) / gridDim.x;
-    const uint64_t v0 = blockIdx.x * chunk, v1 = min(a.V, v0 + chunk);
-    // Pass 1: this thread's entries and edges.
-    uint32_t cnt = 0, deg = 0;
-    for (uint64_t v = v0 + threadIdx.x; v < v1; v += kBlock)
-        if (fin[v]) {
-            const uint32_t d = a.off[v + 1] - a.off[v];
-            cnt += d != 0;
-            deg += d;
-        }
-    // Exclusive prefixes over the workgroup (threads in order).
-    uint32_t pc = cnt, pd = deg;
-    for (int o = 1; o < kWave; o <<= 1) {
-        const uint32_t yc = __shfl_up(pc, static_cast<unsigned>(o), kWave);
-        const uint32_t yd = __shfl_up(pd, static_cast<unsigned>(o), kWave);
-        if (lane >= o) {
-            pc += yc;
-            pd += yd;
-        }
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        found += __shfl_xor(found, o, kWave);
+        nedges += __shfl_xor(nedges, o, kWave);
     }
-    if (lane == kWave - 1) {
-        wcnt[wid] = pc;
-        wdeg[wid] = pd;
+    if (lane == 0) {
+        wfound[threadIdx.x / kWave] = found;
+        wedges[threadIdx.x / kWave] = nedges;
     }
     __syncthreads();
-    uint32_t bc = 0, bd = 0, tc = 0, td = 0;
-    for (int w = 0; w < kBlock / kWave; w++) {
-        if (w < wid) {
-            bc += wcnt[w];
-            bd += wdeg[w];
+    if (threadIdx.x == 0) {
+        uint64_t f = 0, n = 0;
+        for (int w = 0; w < kBlock / kWave; w++) {
+            f += wfound[w];
+            n += wedges[w];
         }
-        tc += wcnt[w];
-        td += wdeg[w];
+        a.part[2 * blockIdx.x] = f;
+        a.part[2 * blockIdx.x + 1] = n;
     }
-    if (threadIdx.x == 0)
-        base_slot = tc ? atomicAdd(&st.queue, (static_cast<unsigned long long>(tc) << 32) | td) : 0ull;
-    __syncthreads();
-    if (tc == 0) return;
-    uint32_t idx = static_cast<uint32_t>(base_slot >> 32) + bc + pc - cnt;
-    uint32_t pos = static_cast<uint32_t>(base_slot) + bd + pd - deg;
-    // Pass 2: the same vertices in the same order, written out.
-    for (uint64_t v = v0 + threadIdx.x; v < v1; v += kBlock)
-        if (fin[v]) {
-            const uint32_t d = a.off[v + 1] - a.off[v];
-            if (d) {
-                a.queue[idx++] = make_uint2(static_cast<uint32_t>(v), pos);
-                pos += d;
-            }
-        }
 }
 
-// Top-down, step 2: each thread takes kSlots consecutive reserved edge
-// slots.  The queue entry holding the first is found by binary search, the
-// next ones by stepping forward; the edge u -> w in a slot ORs u's frontier
-// bits that w has not reached yet into next[w].
-__global__ __launch_bounds__(kBlock) void msbfs_td_expand(MsArgs a)
+// The last i of [0, n) with x[i] <= t (x ascending, x[0] <= t), for kSlots t
+// at once: their loads are in flight together.
+__device__ __forceinline__ void last_at_most(const uint32_t *const (&x)[kSlots], uint32_t n,
+                                             const uint32_t (&t)[kSlots], uint32_t (&at)[kSlots])
 {
-    const MsState &st = *a.st;
-    if (st.done || !st.topdown) return;
+#pragma unroll
+    for (uint32_t k = 0; k < kSlots; k++) at[k] = 0;
+    while (n > 1) {
+        const uint32_t half = n >> 1;
+#pragma unroll
+        for (uint32_t k = 0; k < kSlots; k++)
+            if (x[k][at[k] + half] <= t[k]) at[k] += half;
+        n -= half;
+    }
+}
+
+// Top-down: each frontier edge u -> w ORs u's frontier bits that w has not
+// reached yet into next[w].  A workgroup takes kSlots times 256 consecutive
+// edges at a time, neighbouring lanes neighbouring edges, and finds each
+// one's tile and vertex by binary search.  What bounds it is the chain of
+// dependent loads per edge, so every thread has kSlots of them in flight: a
+// level of 3.3 M edges (R-MAT scale 19) took 237 us with eight consecutive
+// edges per thread one after the other, 124 us so; with plain stores in the
+// atomics' place it would take 70.  Four slots leave small levels too few
+// workgroups (R-MAT scale 19: 0.66 ms a search against 0.64).
+__device__ __forceinline__ void td_expand(const MsArgs &a, const MsState &st)
+{
     const uint64_t *fin = (st.depth & 1) ? a.front[1] : a.front[0];
-    const unsigned long long q = st.queue;
-    const uint32_t n = static_cast<uint32_t>(q >> 32), T = static_cast<uint32_t>(q);
-    const uint64_t nchunks = (static_cast<uint64_t>(T) + kSlots - 1) / kSlots;
-    for (uint64_t c = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; c < nchunks;
-         c += static_cast<uint64_t>(gridDim.x) * kBlock) {
-        const uint32_t t0 = static_cast<uint32_t>(c * kSlots);
-        const uint32_t t1 = static_cast<uint32_t>(min(static_cast<uint64_t>(T), c * kSlots + kSlots));
-        uint32_t lo = 0, hi = n;  // queue[lo].y <= t0 < queue[hi].y, with queue[n].y taken as T
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (a.queue[mid].y <= t0) lo = mid;
-            else hi = mid;
+    const uint64_t T = st.edges;
+    constexpr uint32_t kWindow = kBlock * kSlots;
+    for (uint64_t c = static_cast<uint64_t>(blockIdx.x) * kWindow; c < T;
+         c += static_cast<uint64_t>(gridDim.x) * kWindow) {
+        uint32_t t[kSlots], at[kSlots], w[kSlots];
+        const uint32_t *x[kSlots];
+        uint64_t m[kSlots], seen[kSlots], next[kSlots];
+#pragma unroll
+        for (uint32_t k = 0; k < kSlots; k++) {
+            t[k] = static_cast<uint32_t>(min(c + k * kBlock + threadIdx.x, T - 1));
+            x[k] = a.tile_first;
         }
-        uint2 e = a.queue[lo];
-        uint32_t end = lo + 1 < n ? a.queue[lo + 1].y : T;
-        uint64_t m = fin[e.x];
-        for (uint32_t t = t0; t < t1; t++) {
-            while (t >= end) {  // next entry (entries have at least one edge)
-                lo++;
-                e = a.queue[lo];
-                end = lo + 1 < n ? a.queue[lo + 1].y : T;
-                m = fin[e.x];
-            }
-            const uint32_t w = a.col[a.off[e.x] + (t - e.y)];
-            const uint64_t nw = m & ~a.visit[w];
-            if (nw && (nw & ~a.next[w])) atomicOr(reinterpret_cast<unsigned long long *>(&a.next[w]), nw);
+        last_at_most(x, a.tiles, t, at);
+        uint32_t base[kSlots];
+#pragma unroll
+        for (uint32_t k = 0; k < kSlots; k++) {
+            base[k] = at[k] * kWave;
+            t[k] -= a.tile_first[at[k]];
+            x[k] = a.before + base[k];
+        }
+        // The last tile may hold fewer vertices: a.before has room for all.
+        last_at_most(x, kWave, t, at);
+#pragma unroll
+        for (uint32_t k = 0; k < kSlots; k++) {
+            const uint32_t u = base[k] + at[k];
+            m[k] = fin[u];
+            w[k] = a.col[a.off[u] + (t[k] - a.before[u])];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kSlots; k++) {
+            seen[k] = a.visit[w[k]];
+            // Past the L1, which would show what the word was when the CU
+            // first read it: fewer atomics that add nothing.
+            next[k] = __hip_atomic_load(&a.next[w[k]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kSlots; k++) {
+            const uint64_t nw = m[k] & ~seen[k];
+            if (c + k * kBlock + threadIdx.x < T && (nw & ~next[k]))
+                atomicOr(reinterpret_cast<unsigned long long *>(&a.next[w[k]]), nw);
         }
     }
 }
@@ -326,53 +327,174 @@ __device__ __forceinline__ void bu_hubs(const MsArgs &a, const MsState &st)
 }
 
 // The first kernel of a level, whichever its direction: the top-down
-// queue (td_scan) or the bottom-up hub chunks (bu_hubs).  One launch, where
-// two kernels would each return at once on the levels of the other
-// direction.
-__global__ __launch_bounds__(kBlock) void msbfs_scan_or_hubs(MsArgs a)
+// expansion or the bottom-up hub chunks.
+__global__ __launch_bounds__(kBlock) void msbfs_expand_or_hubs(MsArgs a)
 {
-    MsState &st = *a.st;
+    const MsState &st = *a.st;
     if (st.done) return;
-    if (st.topdown) td_scan(a, st);
+    if (st.topdown) td_expand(a, st);
     else if (a.nhubs) bu_hubs(a, st);
 }
 
-// Closes level d; picks the direction of level d + 1 from its frontier's
-// out-edges.
-__global__ void msbfs_epilogue(MsArgs a)
+// The edges of the tiles before each tile, by one workgroup: kPer consecutive
+// tiles per thread and round, the next round's loads in flight behind this
+// round's barriers.
+__device__ __forceinline__ void number_edges(const MsArgs &a, uint32_t *wsum)
 {
+    constexpr uint32_t kPer = 8;
+    const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
+    uint32_t carry = 0;
+    uint32_t x[kPer], y[kPer];
+    auto load = [&](uint32_t r0) {
+#pragma unroll
+        for (uint32_t k = 0; k < kPer; k++) {
+            const uint32_t i = r0 + tid * kPer + k;
+            y[k] = i < a.tiles ? a.tile_edges[i] : 0;
+        }
+    };
+    load(0);
+    for (uint32_t r0 = 0; r0 < a.tiles; r0 += kEpi * kPer) {
+        uint32_t sum = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < kPer; k++) {
+            x[k] = y[k];
+            sum += x[k];
+        }
+        load(r0 + kEpi * kPer);
+        const uint32_t incl = wave_prefix_sum(sum);
+        if (lane == kWave - 1) wsum[wid] = incl;
+        __syncthreads();
+        uint32_t at = carry + incl - sum;
+        for (uint32_t w = 0; w < kEpi / kWave; w++) {
+            if (w < wid) at += wsum[w];
+            carry += wsum[w];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kPer; k++) {
+            const uint32_t i = r0 + tid * kPer + k;
+            if (i < a.tiles) a.tile_first[i] = at;
+            at += x[k];
+        }
+        __syncthreads();  // wsum is rewritten
+    }
+}
+
+// Closes level d; picks the direction of level d + 1 from its frontier's
+// out-edges and numbers them if it is top-down.
+__global__ __launch_bounds__(kEpi) void msbfs_epilogue(MsArgs a, uint32_t nparts)
+{
+    __shared__ uint64_t wfound[kEpi / kWave], wedges[kEpi / kWave];
+    __shared__ uint32_t wsum[kEpi / kWave];
     MsState &st = *a.st;
     if (st.done) return;
-    const uint32_t d = st.depth;
-    st.num_levels = d + 1;
-    if (a.level_bits[d] == 0 || d + 1 >= a.max_levels) {
-        st.done = 1;
-    } else {
-        st.depth = d + 1;
-        st.topdown = a.td_div != 0 && st.next_edges * a.td_div <= a.E;
+    const uint32_t tid = threadIdx.x, d = st.depth;
+    uint64_t found = 0, edges = 0;
+    for (uint32_t i = tid; i < nparts; i += kEpi) {
+        found += a.part[2 * i];
+        edges += a.part[2 * i + 1];
     }
-    st.queue = 0;
-    st.next_edges = 0;
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        found += __shfl_xor(found, o, kWave);
+        edges += __shfl_xor(edges, o, kWave);
+    }
+    if (tid % kWave == 0) {
+        wfound[tid / kWave] = found;
+        wedges[tid / kWave] = edges;
+    }
+    __syncthreads();  // every thread has read the state too
+    found = edges = 0;
+    for (uint32_t w = 0; w < kEpi / kWave; w++) {
+        found += wfound[w];
+        edges += wedges[w];
+    }
+    const bool done = found == 0 || d + 1 >= a.max_levels;
+    const bool td = a.td_div != 0 && edges * a.td_div <= a.E;
+    if (tid == 0) {
+        a.level_bits[d] = found;
+        st.num_levels = d + 1;
+        st.done = done;
+        if (!done) st.depth = d + 1;
+        st.topdown = td;
+        st.edges = edges;
+    }
+    if (!done && td) number_edges(a, wsum);
+}
+
+// Nothing reached, no masks, no frontier edges.
+__global__ __launch_bounds__(kBlock) void msbfs_reset(MsArgs a, uint64_t ndepths)
+{
+    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
+    const uint64_t t = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    for (uint64_t i = t; i < a.V; i += stride) {
+        a.visit[i] = 0;
+        a.front[0][i] = 0;
+        a.next[i] = 0;
+    }
+    for (uint64_t i = t; i < a.tiles; i += stride) a.tile_edges[i] = 0;
+    // The rows start at any multiple of four bytes: whole 16-byte stores from
+    // the first aligned entry on.
+    const uint64_t head = min(ndepths, ((16 - (reinterpret_cast<uintptr_t>(a.depths) & 15)) & 15) / 4);
+    int4 *quads = reinterpret_cast<int4 *>(a.depths + head);
+    const uint64_t nquads = (ndepths - head) / 4;
+    for (uint64_t i = t; i < nquads; i += stride) quads[i] = make_int4(kUnvisited, kUnvisited, kUnvisited, kUnvisited);
+    if (t < head) a.depths[t] = kUnvisited;
+    const uint64_t tail = head + nquads * 4;
+    if (t < ndepths - tail) a.depths[tail + t] = kUnvisited;
 }
 
 // Depth 0: source i gets bit i (a repeated source vertex gets several).
-__global__ void msbfs_init(MsArgs a, const uint32_t *src, uint32_t n)
+__global__ __launch_bounds__(kEpi) void msbfs_init(MsArgs a, Sources src, uint32_t n)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    unsigned long long edges = 0;
-    for (uint32_t i = 0; i < n; i++) {
-        const uint32_t v = src[i];
-        a.visit[v] |= 1ull << i;
-        a.front[0][v] |= 1ull << i;
+    __shared__ uint32_t vert[64], degree[64];
+    __shared__ unsigned long long all;
+    __shared__ uint32_t wsum[kEpi / kWave];
+    const uint32_t i = threadIdx.x;
+    uint32_t own = 0;
+    if (i == 0) all = 0;
+    if (i < n) {
+        const uint32_t v = src.v[i];
+        vert[i] = v;
+        own = a.off[v + 1] - a.off[v];
+        atomicOr(reinterpret_cast<unsigned long long *>(&a.visit[v]), 1ull << i);
+        atomicOr(reinterpret_cast<unsigned long long *>(&a.front[0][v]), 1ull << i);
         a.depths[static_cast<uint64_t>(i) * a.V + v] = 0;
-        edges += a.off[v + 1] - a.off[v];
     }
-    a.st->depth = 0;
-    a.st->done = 0;
-    a.st->num_levels = 0;
-    a.st->topdown = a.td_div != 0 && edges * a.td_div <= a.E;
-    a.st->queue = 0;
-    a.st->next_edges = 0;
+    __syncthreads();
+    // The frontier's edges: every vertex once, in vertex order.  A wave per
+    // source numbers its tile, if no source before it has the same tile.
+    if (i < n) {
+        for (uint32_t j = 0; j < i; j++)
+            if (vert[j] == vert[i]) own = 0;
+        degree[i] = own;
+        atomicAdd(&all, static_cast<unsigned long long>(own));
+    }
+    __syncthreads();
+    const uint32_t lane = i % kWave;
+    const uint32_t lv = lane < n ? vert[lane] : 0xFFFFFFFFu, ld = lane < n ? degree[lane] : 0;
+    for (uint32_t j = i / kWave; j < n; j += kEpi / kWave) {
+        const uint32_t tile = vert[j] / kWave, v = tile * kWave + lane;
+        uint64_t same = __ballot(lv / kWave == tile);  // sources past n: a tile no vertex has
+        if (static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(same))) - 1 < j) continue;
+        uint32_t before = 0, edges = 0;
+        for (; same; same &= same - 1) {
+            const int k = __ffsll(static_cast<unsigned long long>(same)) - 1;
+            const uint32_t kv = __shfl(lv, k, kWave), kd = __shfl(ld, k, kWave);
+            edges += kd;
+            before += kv < v ? kd : 0;
+        }
+        a.before[v] = before;
+        if (lane == 0) a.tile_edges[tile] = edges;
+    }
+    __syncthreads();
+    const bool td = a.td_div != 0 && all * a.td_div <= a.E;
+    if (i == 0) {
+        a.st->depth = 0;
+        a.st->done = 0;
+        a.st->num_levels = 0;
+        a.st->topdown = td;
+        a.st->edges = all;
+    }
+    if (td) number_edges(a, wsum);
 }
 
 }  // namespace
@@ -386,13 +508,12 @@ struct bw_msbfs {
     const uint32_t *off = nullptr, *col = nullptr;
     uint64_t *visit = nullptr, *front[2] = {nullptr, nullptr};
     uint64_t *next = nullptr;
-    uint2 *queue = nullptr;
+    uint32_t *before = nullptr, *tile_edges = nullptr, *tile_first = nullptr;
+    uint64_t *part = nullptr;
     uint4 *hubs = nullptr;
     uint32_t nhubs = 0;
     uint32_t hub_degree = 0;  // the hub chunks are built for this degree (0: none yet)
-    unsigned long long *level_bits = nullptr;
-    MsState *st = nullptr;
-    uint32_t *src = nullptr;
+    MsState *st = nullptr;  // and the levels' counts behind it
     uint32_t max_levels = 0;
     uint32_t wave_degree = BW_MSBFS_DEFAULT_WAVE_DEGREE;
     uint32_t td_div = BW_MSBFS_DEFAULT_TOPDOWN_DIVISOR;
@@ -411,7 +532,7 @@ struct bw_msbfs {
     ~bw_msbfs()
     {
         if (exec) (void)hipGraphExecDestroy(exec);
-        void *bufs[] = {visit, front[0], front[1], next, queue, hubs, level_bits, st, src};
+        void *bufs[] = {visit, front[0], front[1], next, before, tile_edges, tile_first, part, hubs, st};
         for (void *p : bufs)
             if (p) (void)hipFree(p);
         if (own_stream) (void)hipStreamDestroy(own_stream);
@@ -433,13 +554,17 @@ MsArgs make_args(const bw_msbfs *m, int32_t *depths, uint32_t n)
     a.front[0] = m->front[0];
     a.front[1] = m->front[1];
     a.next = m->next;
-    a.queue = m->queue;
+    a.before = m->before;
+    a.tile_edges = m->tile_edges;
+    a.tile_first = m->tile_first;
+    a.tiles = static_cast<uint32_t>((m->V + kWave - 1) / kWave);
+    a.part = m->part;
     a.hubs = m->hubs;
     a.nhubs = m->nhubs;
     a.hub_degree = m->hub_degree;
     a.depths = depths;
     a.all = n >= 64 ? ~0ull : ((1ull << n) - 1ull);
-    a.level_bits = m->level_bits;
+    a.level_bits = reinterpret_cast<uint64_t *>(reinterpret_cast<char *>(m->st) + kOutOffset);
     a.st = m->st;
     a.max_levels = m->max_levels;
     a.wave_degree = m->wave_degree;
@@ -474,13 +599,11 @@ int build_hubs(bw_msbfs *m, uint32_t hub_degree)
 int launch_levels(const bw_msbfs *m, const MsArgs &a, int32_t count, hipStream_t s)
 {
     for (int32_t i = 0; i < count; i++) {
-        hipLaunchKernelGGL(msbfs_scan_or_hubs, dim3(m->grid), dim3(kBlock), 0, s, a);
-        BW_LAUNCH_CHECK();
-        hipLaunchKernelGGL(msbfs_td_expand, dim3(m->grid), dim3(kBlock), 0, s, a);
+        hipLaunchKernelGGL(msbfs_expand_or_hubs, dim3(m->grid), dim3(kBlock), 0, s, a);
         BW_LAUNCH_CHECK();
         hipLaunchKernelGGL(msbfs_level, dim3(m->grid), dim3(kBlock), 0, s, a);
         BW_LAUNCH_CHECK();
-        hipLaunchKernelGGL(msbfs_epilogue, dim3(1), dim3(1), 0, s, a);
+        hipLaunchKernelGGL(msbfs_epilogue, dim3(1), dim3(kEpi), 0, s, a, m->grid);
         BW_LAUNCH_CHECK();
     }
     return BW_HIP_OK;
@@ -506,11 +629,14 @@ extern "C" int bw_msbfs_create(bw_msbfs **out, const bw_graph_dev *g, uint32_t m
     m->col = g->cols;
     m->max_levels = max_levels;
     m->grid = static_cast<uint32_t>(device_cus()) * 8;
+    const uint64_t tiles = (m->V + kWave - 1) / kWave;
     bool ok = hipMalloc(&m->visit, 8 * m->V) == hipSuccess && hipMalloc(&m->front[0], 8 * m->V) == hipSuccess &&
               hipMalloc(&m->front[1], 8 * m->V) == hipSuccess && hipMalloc(&m->next, 8 * m->V) == hipSuccess &&
-              hipMalloc(&m->queue, sizeof(uint2) * m->V) == hipSuccess &&
-              hipMalloc(&m->level_bits, 8ull * max_levels) == hipSuccess &&
-              hipMalloc(&m->st, sizeof(MsState)) == hipSuccess && hipMalloc(&m->src, 4 * 64) == hipSuccess;
+              hipMalloc(&m->before, 4ull * kWave * tiles) == hipSuccess &&
+              hipMalloc(&m->tile_edges, 4ull * tiles) == hipSuccess &&
+              hipMalloc(&m->tile_first, 4ull * tiles) == hipSuccess &&
+              hipMalloc(&m->part, 16ull * m->grid) == hipSuccess &&
+              hipMalloc(&m->st, kOutOffset + 8 * std::max<size_t>(max_levels, kOutFirst)) == hipSuccess;
     if (!ok) {
         delete m;
         return fail(BW_HIP_ERR_NOMEM, "device allocation of the multi-source BFS failed");
@@ -590,25 +716,27 @@ extern "C" int bw_msbfs_run(bw_msbfs *m, const uint32_t *sources, uint32_t n, in
     BW_HIP_CHECK(hipEventCreate(&ev0));
     BW_HIP_CHECK(hipEventCreate(&ev1));
     int st = BW_HIP_OK;
-    auto step = [&](int rc) {
-        if (st == BW_HIP_OK && rc != BW_HIP_OK) st = rc;
-    };
     if (hipEventRecord(ev0, s) != hipSuccess) st = fail(BW_HIP_ERR_RUNTIME, "event record failed");
-    step(bw_hip_fill_u32(depths, static_cast<uint32_t>(kUnvisited), static_cast<uint64_t>(n) * m->V, s));
-    step(bw_hip_fill_u32(m->visit, 0u, 2 * m->V, s));
-    step(bw_hip_fill_u32(m->front[0], 0u, 2 * m->V, s));
-    step(bw_hip_fill_u32(m->next, 0u, 2 * m->V, s));
-    step(bw_hip_fill_u32(m->level_bits, 0u, 2ull * m->max_levels, s));
-    if (st == BW_HIP_OK && hipMemcpyAsync(m->src, sources, 4 * n, hipMemcpyHostToDevice, s) != hipSuccess)
-        st = fail(BW_HIP_ERR_RUNTIME, "copying the sources failed");
     if (st == BW_HIP_OK) {
-        hipLaunchKernelGGL(msbfs_init, dim3(1), dim3(64), 0, s, a, m->src, n);
-        const hipError_t le = hipGetLastError();
+        Sources src{};
+        std::copy(sources, sources + n, src.v);
+        hipLaunchKernelGGL(msbfs_reset, dim3(m->grid), dim3(kBlock), 0, s, a, n * m->V);
+        hipError_t le = hipGetLastError();
+        if (le == hipSuccess) {
+            hipLaunchKernelGGL(msbfs_init, dim3(1), dim3(kEpi), 0, s, a, src, n);
+            le = hipGetLastError();
+        }
         if (le != hipSuccess) st = hip_fail(le, "msbfs_init", __FILE__, __LINE__);
     }
-    uint32_t done = 0, batches = 0;
+    struct {
+        MsState st;
+        char pad[kOutOffset - sizeof(MsState)];
+        uint64_t bits[kOutFirst];
+    } host{};
+    static_assert(offsetof(decltype(host), bits) == kOutOffset, "as on the device");
+    uint32_t batches = 0;
     const uint32_t max_batches = m->max_levels / static_cast<uint32_t>(levels_per_sync) + 2;
-    while (st == BW_HIP_OK && !done) {
+    while (st == BW_HIP_OK && !host.st.done) {
         if (batches++ > max_batches) {
             st = fail(BW_HIP_ERR_LIMIT, "multi-source BFS exceeded its level bound");
             break;
@@ -620,7 +748,7 @@ extern "C" int bw_msbfs_run(bw_msbfs *m, const uint32_t *sources, uint32_t n, in
             st = launch_levels(m, a, levels_per_sync, s);
         }
         if (st != BW_HIP_OK) break;
-        if (hipMemcpyAsync(&done, &m->st->done, sizeof done, hipMemcpyDeviceToHost, s) != hipSuccess ||
+        if (hipMemcpyAsync(&host, m->st, sizeof host, hipMemcpyDeviceToHost, s) != hipSuccess ||
             hipStreamSynchronize(s) != hipSuccess)
             st = fail(BW_HIP_ERR_RUNTIME, "reading the multi-source BFS state failed");
     }
@@ -633,15 +761,16 @@ extern "C" int bw_msbfs_run(bw_msbfs *m, const uint32_t *sources, uint32_t n, in
     (void)hipEventDestroy(ev0);
     (void)hipEventDestroy(ev1);
     if (st != BW_HIP_OK) return st;
-    MsState hs;
-    BW_HIP_CHECK(hipMemcpy(&hs, m->st, sizeof hs, hipMemcpyDeviceToHost));
-    *num_levels = hs.num_levels;
-    const size_t k = std::min(hs.num_levels, m->max_levels);
-    if (k) {
-        unsigned long long last = 0;
-        BW_HIP_CHECK(hipMemcpy(&last, m->level_bits + k - 1, sizeof last, hipMemcpyDeviceToHost));
-        if (last != 0) return fail(BW_HIP_ERR_LIMIT, "multi-source BFS reached max_levels with work left");
+    *num_levels = host.st.num_levels;
+    const size_t k = std::min(host.st.num_levels, m->max_levels);
+    std::vector<uint64_t> more;
+    const uint64_t *bits = host.bits;
+    if (k > kOutFirst) {
+        more.resize(k);
+        BW_HIP_CHECK(hipMemcpy(more.data(), a.level_bits, 8 * k, hipMemcpyDeviceToHost));
+        bits = more.data();
     }
-    if (level_bits_host && k) BW_HIP_CHECK(hipMemcpy(level_bits_host, m->level_bits, 8 * k, hipMemcpyDeviceToHost));
+    if (k && bits[k - 1] != 0) return fail(BW_HIP_ERR_LIMIT, "multi-source BFS reached max_levels with work left");
+    if (level_bits_host) std::copy(bits, bits + k, level_bits_host);
     return BW_HIP_OK;
 }
