@@ -1049,10 +1049,10 @@ __device__ void tiny_levels(const Graph &g, const Buffers &b, const PolicyArgs &
         if (--left == 0 || !tiny(p, st)) break;
     }
 
-    // The next level is not for here: its frontier goes to the queue (a few
-    // hubs to the hub queue) and to the bitmap.
+    // The next level is not for here: its frontier goes to the queue (hubs
+    // to the hub queue) and to the bitmap.
     const uint32_t dn = st.depth, nq = dn & 1;
-    constexpr uint32_t kHubs = kWave;
+    const uint32_t hubs = min(kTiny, b.hub_cap);
     __syncthreads();  // every thread has read the state and n
     if (tid == 0) {
         L.found = 0;
@@ -1064,7 +1064,7 @@ __device__ void tiny_levels(const Graph &g, const Buffers &b, const PolicyArgs &
         atomicOr(&bits[v >> 5], 1u << (v & 31));
         if (dv > b.hub_degree) {
             const uint32_t h = atomicAdd(&L.wsum[0], 1u);
-            if (h < min(kHubs, b.hub_cap)) {
+            if (h < hubs) {
                 b.hubq[nq][h] = v;
                 L.start[h] = dv;
                 continue;
@@ -1073,14 +1073,28 @@ __device__ void tiny_levels(const Graph &g, const Buffers &b, const PolicyArgs &
         b.q[nq][atomicAdd(&L.found, 1u)] = v;
     }
     __syncthreads();
+    // The hubs' degree prefix, kPer consecutive hubs per thread.
+    const uint32_t nh = min(L.wsum[0], hubs);
+    uint64_t hd[kPer], hsum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; k++) {
+        const uint32_t h = tid * kPer + k;
+        hd[k] = h < nh ? L.start[h] : 0;
+        hsum += hd[k];
+    }
+    const uint64_t hincl = wave_prefix_sum(hsum);
+    if (lane == kWave - 1) L.hscan[wid] = hincl;
+    __syncthreads();
+    uint64_t hat = hincl - hsum;
+    for (uint32_t w = 0; w < wid; w++) hat += L.hscan[w];
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; k++) {
+        const uint32_t h = tid * kPer + k;
+        if (h < nh) b.hub_prefix[h] = hat;
+        hat += hd[k];
+    }
+    if (tid == kEpi - 1) b.hub_prefix[nh] = hat;
     if (tid == 0) {
-        const uint32_t nh = min(L.wsum[0], min(kHubs, b.hub_cap));
-        uint64_t sum = 0;
-        for (uint32_t h = 0; h < nh; h++) {
-            b.hub_prefix[h] = sum;
-            sum += L.start[h];
-        }
-        b.hub_prefix[nh] = sum;
         st.qcount = st.qglobal = L.found;
         st.hubcount = nh;
         st.rot = (rot0 + 2 * (dn - d0)) % 3;

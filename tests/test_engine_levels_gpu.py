@@ -26,10 +26,18 @@ def _layers(*sizes):
                             np.concatenate(dst).astype(np.uint32))
 
 
+def _hubs(hubs, degree):
+    """A vertex with `hubs` children of `degree` leaves each."""
+    src = np.concatenate([np.zeros(hubs, int), np.repeat(np.arange(1, 1 + hubs), degree)])
+    dst = np.concatenate([np.arange(1, 1 + hubs), np.arange(1 + hubs, 1 + hubs + hubs * degree)])
+    return graph.from_edges(1 + hubs * (degree + 1), src.astype(np.uint32), dst.astype(np.uint32))
+
+
 CASES = {
     "edges at the limit": _layers(1, 2048, 2048, 1, 2049, 3, 2047, 5),
     "out of it and back": _layers(1, 1, 3000, 2, 2, 4100, 1, 9000, 40, 40, 1),   # hubs of 4100 and 9000 edges too
     "more levels than a launch": graph.chain(3 * 1024 + 7),
+    "many hubs out of it": _hubs(300, 257),
     "segments": _layers(1, 65535, 65535, 65536, 65537, 70000, 300, 300, 200000, 1),
     "one vertex": graph.from_edges(1, np.zeros(0, np.uint32), np.zeros(0, np.uint32)),
 }
@@ -41,6 +49,9 @@ def test_level_forms(gpu, name, use_graph):
     g = CASES[name]
     csr, dg = O.CSR.from_graph(g), device.DeviceGraph(g)
     eng = bfs_native.BFSEngine(dg, edge_lists=True)
+    if "hubs" in name:
+        eng.set_tuning(hub_degree=256)  # every child is a hub, 256 of them in the hub queue at most
+        eng.set_queues(hub_cap=256)
     roots = sorted({0, g.vertex_count // 2, g.vertex_count - 1})
     depths = {r: O.bfs_queue(csr, r)[0] for r in roots}
     runs = [("fixed", "td", None), ("fixed", "bu-wave", None), ("beamer", "td", None),
