@@ -23,7 +23,7 @@ def _want(V, off, cols, perm):
 
 
 @pytest.mark.parametrize("V,E", [(1, 3), (2, 1), (63, 500), (5000, 3), (5000, 40000), (70000, 4097)])
-@pytest.mark.parametrize("reverse", ["transpose", "other", "none"])
+@pytest.mark.parametrize("reverse", ["transpose", "other", "columns", "none"])
 def test_relabel_directions(gpu, V, E, reverse):
     rng = np.random.default_rng(V * 7 + E)
     src = np.minimum(rng.integers(0, V, E), rng.integers(0, V, E))  # skewed, with repeated edges
@@ -31,6 +31,8 @@ def test_relabel_directions(gpu, V, E, reverse):
     off, cols = _csr(V, src, dst)
     if reverse == "transpose":
         roff, rcols = _csr(V, dst, src)
+    elif reverse == "columns":  # the transpose's in-degrees, but other columns
+        roff, rcols = _csr(V, dst, rng.permutation(src))
     else:  # not the transpose: other in-degrees
         roff, rcols = _csr(V, (dst + 1) % V, src)
     order = np.argsort(-np.diff(off.astype(np.int64)), kind="stable")
