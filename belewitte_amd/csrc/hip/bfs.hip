@@ -185,11 +185,12 @@ __global__ __launch_bounds__(1024) void bfs_vertex_push_kernel(
             before[at] = e0;
         }
         __syncthreads();
-        for (Off c = 0; c < total; c += static_cast<Off>(blockDim.x) * kPushBatch) {
+        // 64 bits: the step past a total near 2^32 must not wrap.
+        for (uint64_t c = 0; c < total; c += blockDim.x * kPushBatch) {
             uint32_t w[kPushBatch];
 #pragma unroll
             for (int u = 0; u < kPushBatch; u++) {
-                const uint64_t k = static_cast<uint64_t>(c) + u * blockDim.x + t;
+                const uint64_t k = c + u * blockDim.x + t;
                 w[u] = kNoVertex;
                 if (k < total) {
                     uint32_t lo = 0, hi = na;  // the last active vertex with before <= k
