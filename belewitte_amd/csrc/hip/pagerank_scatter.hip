@@ -388,8 +388,10 @@ __global__ __launch_bounds__(kAccThreads) void scatter_accumulate_kernel(const C
     const Chunk ch = chunks[blockIdx.x];
     for (uint32_t i = threadIdx.x; i < kRows; i += kAccThreads) acc[i] = 0.0;
     __syncthreads();
-    for (uint32_t j = ch.begin + threadIdx.x; j < ch.end; j += kAccThreads)
-        atomicAdd(&acc[row[j]], static_cast<double>(val[j]));
+    // Counted from the chunk's start: slots go up to 2^32 - 1, past which a
+    // slot counter's last step would wrap to the first one.
+    for (uint32_t i = threadIdx.x, len = ch.end - ch.begin; i < len; i += kAccThreads)
+        atomicAdd(&acc[row[ch.begin + i]], static_cast<double>(val[ch.begin + i]));
     __syncthreads();
     const uint64_t r0 = static_cast<uint64_t>(ch.part) << kRowsLog;
     const uint32_t n = static_cast<uint32_t>(V - r0 < kRows ? V - r0 : kRows);
@@ -470,13 +472,15 @@ __global__ __launch_bounds__(kGatherThreads) void scatter_gather_kernel(GatherAr
     const Chunk ch = a.chunks[blockIdx.x];
     for (uint32_t i = threadIdx.x; i < a.rows; i += kGatherThreads) acc[i] = 0.0;
     __syncthreads();
-    for (uint32_t j0 = ch.begin + threadIdx.x; j0 < ch.end; j0 += kGatherBatch * kGatherThreads) {
+    // Counted from the chunk's start, as in scatter_accumulate_kernel.
+    const uint32_t len = ch.end - ch.begin;
+    for (uint32_t i0 = threadIdx.x; i0 < len; i0 += kGatherBatch * kGatherThreads) {
         uint32_t s[kGatherBatch];
         uint32_t r[kGatherBatch];
         float c[kGatherBatch];
 #pragma unroll
         for (uint32_t k = 0; k < kGatherBatch; k++) {
-            const uint32_t j = min(j0 + k * kGatherThreads, ch.end - 1);
+            const uint32_t j = ch.begin + min(i0 + k * kGatherThreads, len - 1);
             s[k] = a.src[j];
             r[k] = a.row[j];
         }
@@ -484,7 +488,7 @@ __global__ __launch_bounds__(kGatherThreads) void scatter_gather_kernel(GatherAr
         for (uint32_t k = 0; k < kGatherBatch; k++) c[k] = a.contrib[s[k]];
 #pragma unroll
         for (uint32_t k = 0; k < kGatherBatch; k++)
-            if (j0 + k * kGatherThreads < ch.end) atomicAdd(&acc[r[k]], static_cast<double>(c[k]));
+            if (i0 + k * kGatherThreads < len) atomicAdd(&acc[r[k]], static_cast<double>(c[k]));
     }
     __syncthreads();
     double *out = a.partials + static_cast<uint64_t>(blockIdx.x) * a.rows;
