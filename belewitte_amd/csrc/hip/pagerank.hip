@@ -1719,7 +1719,7 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
         ~PullGuard() { bw_pr_pull_plan_destroy(p); }
     } pull_guard{pull};
     if (pull_variant(variant)) {
-        if (!g->rev_cols) return fail(BW_HIP_ERR_ARG, "NULL device pointer");
+        if (iterations > 0 && !g->rev_cols) return fail(BW_HIP_ERR_ARG, "NULL device pointer");
         BW_TRY(bw_pr_pull_plan_create(&pull, V, g->rev_offsets, g->offset_bytes, s));
     }
 
