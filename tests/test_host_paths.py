@@ -56,3 +56,45 @@ def test_pull_run_without_edges_or_iterations(fake):
             assert run(0) == 0, lib.bw_hip_last_error()
             assert run(1) == 1 and b"NULL device pointer" in lib.bw_hip_last_error()
     """)
+
+
+PLAN = """
+def binned(V, E):
+    # the host's plan: nothing runs on the device
+    rng = np.random.default_rng(V)
+    rows = np.sort(rng.integers(0, V, E))
+    off = np.searchsorted(rows, np.arange(V + 1)).astype(np.uint32)
+    g = N.BwGraphDev()
+    g.vertex_count, g.edge_count, g.offset_bytes = V, E, 4
+    keep = [device.DeviceArray.from_host(x) for x in (off, rng.integers(0, V, E).astype(np.uint32))]
+    g.rev_offsets, g.rev_cols = keep[0].ptr, keep[1].ptr
+    plan = C.c_void_p()
+    N.check_hip(lib.bw_pr_plan_create(C.byref(plan), V, E, g.rev_offsets, 4, g.rev_cols))
+    return g, plan, keep
+
+def run(g, plan, iterations=2):
+    V = g.vertex_count
+    bufs = [device.DeviceArray(V, np.float32), device.DeviceArray(V, np.float32),
+            device.DeviceArray(int(lib.bw_pr_fused_acc_len(iterations)), np.float64)]
+    fake.fake_clear()
+    return lib.bw_pr_fused_run(C.byref(g), plan, iterations, 0, 0, *(b.ptr for b in bufs), None, None, None)
+"""
+
+
+def test_binned_plan_without_room_for_pieces(fake):
+    """The pieces of a small graph's chunks need a buffer; without it the
+    plan keeps whole chunks."""
+    _run(fake, PLAN + """
+grids = []
+for limit in (2**64 - 1, 3 << 20):
+    g, plan, keep = binned(20000, 300000)
+    fake.fake_fail_from(limit)
+    assert lib.bw_pr_plan_bin_host(plan, 14, 128, 8) == 0, lib.bw_hip_last_error()
+    fake.fake_fail_from(2**64 - 1)
+    assert run(g, plan) == 0, lib.bw_hip_last_error()
+    grids.append({c[2] for c in calls("launch") if "accumulate" in c[0]})
+    lib.bw_pr_plan_destroy(plan)
+assert [len(x) for x in grids] == [1, 1]
+whole = int(grids[1].pop()) - 1  # and one workgroup for the reduction
+assert whole < 8 and int(grids[0].pop()) - 1 == 16 * whole, whole
+    """)
