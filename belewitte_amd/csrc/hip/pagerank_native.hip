@@ -1661,11 +1661,14 @@ int run_small(const bw_pr_plan *plan, const uint32_t *roff, const uint32_t *rcol
     using Kernel = void (*)(SmallArgs);
     const uint32_t per = (plan->E + kSmallThreads - 1) / kSmallThreads;
     const Kernel k = per <= 8 ? pr_small_kernel<8> : per <= 16 ? pr_small_kernel<16> : pr_small_kernel<kSmallEdges>;
-    // 12 bytes a vertex: 96 KB at most.
-    const uint32_t lds = 12 * plan->V;
+    // 12 bytes a vertex.  The kernel's limit is set to what the largest graph
+    // needs: all threads of the process share it, and one that set its own
+    // graph's size could lower it between another's setting and launch.
+    constexpr uint32_t kBytes = 12, kMost = kBytes * kSmallVerts;
+    const uint32_t lds = kBytes * plan->V;
     if (lds > 64 * 1024)
         BW_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         static_cast<int>(lds)));
+                                         static_cast<int>(kMost)));
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     if (kernel_ms) {
         BW_HIP_CHECK(hipEventCreate(&ev0));

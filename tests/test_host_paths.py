@@ -98,3 +98,20 @@ assert [len(x) for x in grids] == [1, 1]
 whole = int(grids[1].pop()) - 1  # and one workgroup for the reduction
 assert whole < 8 and int(grids[0].pop()) - 1 == 16 * whole, whole
     """)
+
+
+def test_small_run_lds_limit(fake):
+    """The LDS limit of a small graph's kernel is an attribute that all
+    threads share: whatever the graph's size it is set to one value, which
+    no launch exceeds."""
+    _run(fake, PLAN + """
+limits, needs = set(), set()
+for V in (5400, 6000, 8192):
+    g, plan, keep = binned(V, 30000)
+    assert run(g, plan) == 0, lib.bw_hip_last_error()
+    limits |= {(name, int(value)) for name, value in calls("attribute")}
+    needs |= {(c[0], int(c[6])) for c in calls("launch") if "pr_small_kernel" in c[0]}
+assert len(needs) == 3 and len(limits) == 1, (needs, limits)
+name, limit = limits.pop()
+assert all(n == name and lds <= limit for n, lds in needs), (needs, name, limit)
+    """)
