@@ -45,7 +45,7 @@ constexpr int kBlock = 256;
 // maxima (bw_bfs_engine_set_queues).
 constexpr uint32_t kLdsQueueMax = BW_BFS_MAX_LDS_QUEUE;
 constexpr uint32_t kHubCapMax = BW_BFS_MAX_HUB_CAP;
-constexpr uint32_t kSegment = BW_BFS_DEFAULT_LDS_QUEUE;  // a workgroup's segment of the frontier
+constexpr uint32_t kSegmentMax = BW_BFS_DEFAULT_LDS_QUEUE;  // a workgroup's segment of the frontier at most
 constexpr uint32_t kMaxGrid = 4096;    // workgroups of a level kernel at most
 constexpr uint32_t kSegGroup = 8;      // segments per coarse step of the search for a frontier index
 constexpr uint32_t kParentScan = 32;   // in-edges scanned for a vertex's likely parent
@@ -130,7 +130,8 @@ struct Buffers {
     // takes an atomic per workgroup on one counter, about 15 ns each one
     // after the other: any level that found something in most of the 2048
     // workgroups took 35 us (1 M-vertex grid), 12 to 20 with segments.
-    uint32_t *seg[2];      // [workgroup][kSegment]
+    uint32_t *seg[2];      // [workgroup][seg_size], in one allocation
+    uint32_t seg_size;
     uint32_t *segcount;    // per workgroup: discovered in this level
     uint32_t *segbase;     // per workgroup and one more: frontier index of its segment's first vertex
     uint32_t *hubq[2];
@@ -235,9 +236,9 @@ struct Emitter {
     __device__ __forceinline__ void finish(const Buffers &b, uint32_t d)
     {
         __syncthreads();
-        const uint32_t staged = min(*lcount, cap), n = min(staged, kSegment);
+        const uint32_t staged = min(*lcount, cap), n = min(staged, b.seg_size);
         const uint32_t nq = (d & 1) ^ 1;
-        uint32_t *s = b.seg[nq] + static_cast<size_t>(blockIdx.x) * kSegment;
+        uint32_t *s = b.seg[nq] + static_cast<size_t>(blockIdx.x) * b.seg_size;
         for (uint32_t i = threadIdx.x; i < n; i += kBlock) s[i] = lbuf[i];
         if (threadIdx.x == 0) {
             b.segcount[blockIdx.x] = n;
@@ -270,7 +271,7 @@ __device__ __forceinline__ uint32_t segment_vertex(const Buffers &b, uint32_t cu
             w = lo * kSegGroup + k;
             first = base[k];
         }
-    return b.seg[cur][static_cast<size_t>(w) * kSegment + (i - first)];
+    return b.seg[cur][static_cast<size_t>(w) * b.seg_size + (i - first)];
 }
 
 // Top-down discovery of w: the thread whose fetch-or sets w's visited bit
@@ -1419,7 +1420,7 @@ struct bw_bfs_engine {
         drop_exec();
         void *bufs[] = {own_levels, b.q[0], b.q[1], b.hubq[0], b.hubq[1], b.hub_prefix, b.bits[0], b.bits[1],
                         b.bits[2], b.vis, b.st, b.part, snap_levels, snap_q, snap_hub,
-                        b.seg[0], b.seg[1], b.segcount, b.segbase, snap_seg, snap_segbase,
+                        b.seg[0], b.segcount, b.segbase, snap_seg, snap_segbase,
                         snap_bits, snap_prefix, snap_st, mlp, schedule, roots, no_in, parent};
         for (void *p : bufs)
             if (p) (void)hipFree(p);
@@ -1477,6 +1478,13 @@ int launch_level(bw_bfs_engine *e, const PolicyArgs &p, hipStream_t s)
     return BW_HIP_OK;
 }
 
+// Entries of a workgroup's segment, whole waves of them.
+uint32_t segment_size(uint64_t V, uint32_t grid)
+{
+    const uint64_t want = (8 * V / grid + kWave - 1) / kWave * kWave;
+    return static_cast<uint32_t>(std::min<uint64_t>(std::max<uint64_t>(want, kWave), kSegmentMax));
+}
+
 }  // namespace
 
 extern "C" int bw_bfs_engine_create(bw_bfs_engine **out, const bw_graph_dev *g, int32_t *levels, uint32_t max_levels)
@@ -1510,7 +1518,14 @@ extern "C" int bw_bfs_engine_create(bw_bfs_engine **out, const bw_graph_dev *g, 
     e->b.levels = levels;
     alloc(&e->b.q[0], sizeof(uint32_t) * V);
     alloc(&e->b.q[1], sizeof(uint32_t) * V);
-    for (auto &x : e->b.seg) alloc(&x, sizeof(uint32_t) * kSegment * e->grid);
+    // Room for eight times a workgroup's share of the vertices: what a level
+    // leaves more in one place goes to the queue, and an engine on a small
+    // graph does not hold the 32 MiB that segments of 2048 take (2000
+    // vertices: 1 MiB).
+    e->b.seg_size = segment_size(V, e->grid);
+    const size_t seg = static_cast<size_t>(e->b.seg_size) * e->grid;
+    alloc(&e->b.seg[0], sizeof(uint32_t) * 2 * seg);
+    if (ok) e->b.seg[1] = e->b.seg[0] + seg;
     alloc(&e->b.segcount, sizeof(uint32_t) * segs);
     alloc(&e->b.segbase, sizeof(uint32_t) * segs);
     alloc(&e->b.hubq[0], sizeof(uint32_t) * kHubCapMax);
@@ -1725,7 +1740,7 @@ extern "C" int bw_bfs_engine_snapshot(bw_bfs_engine *e, int32_t restore, void *s
         if (restore) return fail(BW_HIP_ERR_ARG, "no snapshot to restore");
         BW_HIP_CHECK(hipMalloc(&e->snap_levels, sizeof(int32_t) * V));
         BW_HIP_CHECK(hipMalloc(&e->snap_q, sizeof(uint32_t) * V));
-        BW_HIP_CHECK(hipMalloc(&e->snap_seg, sizeof(uint32_t) * kSegment * e->grid));
+        BW_HIP_CHECK(hipMalloc(&e->snap_seg, sizeof(uint32_t) * e->b.seg_size * e->grid));
         BW_HIP_CHECK(hipMalloc(&e->snap_segbase, sizeof(uint32_t) * e->grid));
         BW_HIP_CHECK(hipMalloc(&e->snap_hub, sizeof(uint32_t) * kHubCapMax));
         BW_HIP_CHECK(hipMalloc(&e->snap_bits, sizeof(uint32_t) * 4 * words));
@@ -1743,7 +1758,7 @@ extern "C" int bw_bfs_engine_snapshot(bw_bfs_engine *e, int32_t restore, void *s
     };
     BW_HIP_CHECK(copy(e->snap_levels, e->b.levels, sizeof(int32_t) * V));
     BW_HIP_CHECK(copy(e->snap_q, e->b.q[cur], sizeof(uint32_t) * nq));
-    BW_HIP_CHECK(copy(e->snap_seg, e->b.seg[cur], sizeof(uint32_t) * kSegment * e->grid));
+    BW_HIP_CHECK(copy(e->snap_seg, e->b.seg[cur], sizeof(uint32_t) * e->b.seg_size * e->grid));
     BW_HIP_CHECK(copy(e->snap_segbase, e->b.segbase, sizeof(uint32_t) * e->grid));
     BW_HIP_CHECK(copy(e->snap_hub, e->b.hubq[cur], sizeof(uint32_t) * nh));
     BW_HIP_CHECK(copy(e->snap_prefix, e->b.hub_prefix, sizeof(uint64_t) * (e->b.hub_cap + 1)));

@@ -115,3 +115,22 @@ assert len(needs) == 3 and len(limits) == 1, (needs, limits)
 name, limit = limits.pop()
 assert all(n == name and lds <= limit for n, lds in needs), (needs, name, limit)
     """)
+
+
+def test_engine_memory_follows_the_graph(fake):
+    """An engine on a graph of a few thousand vertices holds what such a
+    graph needs, and gives it back."""
+    _run(fake, """
+        g = N.BwGraphDev()
+        g.vertex_count, g.edge_count, g.offset_bytes = 2000, 0, 4
+        off = device.DeviceArray.from_host(np.zeros(2001, np.uint32))
+        g.offsets = g.rev_offsets = off.ptr
+        before = fake.fake_live()
+        fake.fake_clear()
+        e = C.c_void_p()
+        N.check_hip(lib.bw_bfs_engine_create(C.byref(e), C.byref(g), None, 2001))
+        held = sum(int(c[0]) for c in calls("alloc"))
+        lib.bw_bfs_engine_destroy(e)
+        assert held < 2 << 20, held
+        assert fake.fake_live() == before
+    """)
