@@ -39,6 +39,7 @@ constexpr int kEpi = 1024;       // threads of the epilogue and the init kernel
 // split into chunks of kHubChunk in-edges, one wave each (msbfs_bu_hubs),
 // so that a few waves holding many such vertices do not hold up the level.
 constexpr uint32_t kHubChunk = 512;
+constexpr uint32_t kGroup = 4;   // tiles (64 vertices) per entry of the numbering of the frontier's edges
 constexpr int kLaneUnroll = 4;   // bottom-up lane path: in-edges per round trip
 
 struct MsState {
@@ -72,10 +73,12 @@ struct MsArgs {
     // The frontier's out-edges in vertex order: per vertex of a tile of 64
     // (one wave of msbfs_level) the edges of the frontier vertices before it
     // in the tile (only written where the tile has any), per tile its edges
-    // and, on top-down levels, those of the tiles before it.
+    // (groups of four tiles, the last one filled up with zeros) and, on
+    // top-down levels, per group the edges of the groups before it.
     uint32_t *before;
-    uint32_t *tile_edges, *tile_first;
-    uint32_t tiles;
+    uint4 *tile_edges;
+    uint32_t *group_first;
+    uint32_t groups;
     uint64_t *part;      // per workgroup of msbfs_level: newly set bits, out-edges
     const uint4 *hubs;   // bottom-up: (vertex, first in-edge, end) per hub chunk
     uint32_t nhubs;
@@ -201,7 +204,7 @@ __global__ __launch_bounds__(kBlock) void msbfs_level(MsArgs a)
         if (base + (threadIdx.x & ~(kWave - 1u)) < a.V) {
             const uint32_t incl = wave_prefix_sum(deg), all = __shfl(incl, kWave - 1, kWave);
             if (all) a.before[v] = incl - deg;  // past the last vertex too
-            if (lane == 0) a.tile_edges[v / kWave] = all;
+            if (lane == 0) reinterpret_cast<uint32_t *>(a.tile_edges)[v / kWave] = all;
             nedges += deg;
         }
         record(a, v64, nb, nd);
@@ -245,11 +248,11 @@ __device__ __forceinline__ void last_at_most(const uint32_t *const (&x)[kSlots],
 // Top-down: each frontier edge u -> w ORs u's frontier bits that w has not
 // reached yet into next[w].  A workgroup takes kSlots times 256 consecutive
 // edges at a time, neighbouring lanes neighbouring edges, and finds each
-// one's tile and vertex by binary search.  What bounds it is the chain of
-// dependent loads per edge, so every thread has kSlots of them in flight: a
-// level of 3.3 M edges (R-MAT scale 19) took 237 us with eight consecutive
-// edges per thread one after the other, 124 us so; with plain stores in the
-// atomics' place it would take 70.  Four slots leave small levels too few
+// one's group of tiles and vertex by binary search.  What bounds it is the
+// chain of dependent loads per edge, so every thread has kSlots of them in
+// flight: a level of 3.3 M edges (R-MAT scale 19) took 237 us with eight
+// consecutive edges per thread one after the other, 124 us so; with plain
+// stores in the atomics' place it would take 70.  Four slots leave small levels too few
 // workgroups (R-MAT scale 19: 0.66 ms a search against 0.64).
 __device__ __forceinline__ void td_expand(const MsArgs &a, const MsState &st)
 {
@@ -264,14 +267,19 @@ __device__ __forceinline__ void td_expand(const MsArgs &a, const MsState &st)
 #pragma unroll
         for (uint32_t k = 0; k < kSlots; k++) {
             t[k] = static_cast<uint32_t>(min(c + k * kBlock + threadIdx.x, T - 1));
-            x[k] = a.tile_first;
+            x[k] = a.group_first;
         }
-        last_at_most(x, a.tiles, t, at);
+        last_at_most(x, a.groups, t, at);
         uint32_t base[kSlots];
 #pragma unroll
         for (uint32_t k = 0; k < kSlots; k++) {
-            base[k] = at[k] * kWave;
-            t[k] -= a.tile_first[at[k]];
+            // The tile of the group: the first whose edges, added to those
+            // before it, pass t.
+            const uint4 e = a.tile_edges[at[k]];
+            const uint32_t r = t[k] - a.group_first[at[k]], e2 = e.x + e.y, e3 = e2 + e.z;
+            const uint32_t tile = (r >= e.x) + (r >= e2) + (r >= e3);
+            t[k] = r - (tile == 0 ? 0 : tile == 1 ? e.x : tile == 2 ? e2 : e3);
+            base[k] = (at[k] * kGroup + tile) * kWave;
             x[k] = a.before + base[k];
         }
         // The last tile may hold fewer vertices: a.before has room for all.
@@ -336,46 +344,48 @@ __global__ __launch_bounds__(kBlock) void msbfs_expand_or_hubs(MsArgs a)
     else if (a.nhubs) bu_hubs(a, st);
 }
 
-// The edges of the tiles before each tile, by one workgroup: kPer consecutive
-// tiles per thread and round, the next round's loads in flight behind this
-// round's barriers.
-__device__ __forceinline__ void number_edges(const MsArgs &a, uint32_t *wsum)
+// The edges of the groups before each group of tiles, by one workgroup: kPer
+// times 64 consecutive groups per wave and round, read and written in whole
+// lines, the next round's loads in flight behind this round's barrier.  One
+// CU's rate bounds it: the epilogue of 131072 tiles (2^23 vertices) takes 14
+// us, 4 of them for a level without numbers; tile by tile, eight consecutive
+// tiles per thread, it took 121, more than every workgroup's scan of the
+// frontier would have.
+__device__ __forceinline__ void number_edges(const MsArgs &a, uint32_t (*wsum)[kEpi / kWave])
 {
-    constexpr uint32_t kPer = 8;
-    const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
-    uint32_t carry = 0;
-    uint32_t x[kPer], y[kPer];
+    constexpr uint32_t kPer = 4;
+    const uint32_t lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+    uint32_t carry = 0, buf = 0;
+    uint4 y[kPer];
     auto load = [&](uint32_t r0) {
 #pragma unroll
         for (uint32_t k = 0; k < kPer; k++) {
-            const uint32_t i = r0 + tid * kPer + k;
-            y[k] = i < a.tiles ? a.tile_edges[i] : 0;
+            const uint32_t i = r0 + (wid * kPer + k) * kWave + lane;
+            y[k] = i < a.groups ? a.tile_edges[i] : make_uint4(0, 0, 0, 0);
         }
     };
     load(0);
-    for (uint32_t r0 = 0; r0 < a.tiles; r0 += kEpi * kPer) {
-        uint32_t sum = 0;
+    for (uint32_t r0 = 0; r0 < a.groups; r0 += kEpi * kPer, buf ^= 1) {
+        uint32_t first[kPer], sum = 0;
 #pragma unroll
         for (uint32_t k = 0; k < kPer; k++) {
-            x[k] = y[k];
-            sum += x[k];
+            const uint32_t x = y[k].x + y[k].y + y[k].z + y[k].w, incl = wave_prefix_sum(x);
+            first[k] = sum + incl - x;
+            sum += __builtin_amdgcn_readlane(static_cast<int>(incl), kWave - 1);
         }
         load(r0 + kEpi * kPer);
-        const uint32_t incl = wave_prefix_sum(sum);
-        if (lane == kWave - 1) wsum[wid] = incl;
-        __syncthreads();
-        uint32_t at = carry + incl - sum;
+        if (lane == 0) wsum[buf][wid] = sum;
+        __syncthreads();  // the other half of wsum is read until the next round's barrier
+        uint32_t at = carry;
         for (uint32_t w = 0; w < kEpi / kWave; w++) {
-            if (w < wid) at += wsum[w];
-            carry += wsum[w];
+            if (w < wid) at += wsum[buf][w];
+            carry += wsum[buf][w];
         }
 #pragma unroll
         for (uint32_t k = 0; k < kPer; k++) {
-            const uint32_t i = r0 + tid * kPer + k;
-            if (i < a.tiles) a.tile_first[i] = at;
-            at += x[k];
+            const uint32_t i = r0 + (wid * kPer + k) * kWave + lane;
+            if (i < a.groups) a.group_first[i] = at + first[k];
         }
-        __syncthreads();  // wsum is rewritten
     }
 }
 
@@ -384,7 +394,7 @@ __device__ __forceinline__ void number_edges(const MsArgs &a, uint32_t *wsum)
 __global__ __launch_bounds__(kEpi) void msbfs_epilogue(MsArgs a, uint32_t nparts)
 {
     __shared__ uint64_t wfound[kEpi / kWave], wedges[kEpi / kWave];
-    __shared__ uint32_t wsum[kEpi / kWave];
+    __shared__ uint32_t wsum[2][kEpi / kWave];
     MsState &st = *a.st;
     if (st.done) return;
     const uint32_t tid = threadIdx.x, d = st.depth;
@@ -430,7 +440,7 @@ __global__ __launch_bounds__(kBlock) void msbfs_reset(MsArgs a, uint64_t ndepths
         a.front[0][i] = 0;
         a.next[i] = 0;
     }
-    for (uint64_t i = t; i < a.tiles; i += stride) a.tile_edges[i] = 0;
+    for (uint64_t i = t; i < a.groups; i += stride) a.tile_edges[i] = make_uint4(0, 0, 0, 0);
     // The rows start at any multiple of four bytes: whole 16-byte stores from
     // the first aligned entry on.
     const uint64_t head = min(ndepths, ((16 - (reinterpret_cast<uintptr_t>(a.depths) & 15)) & 15) / 4);
@@ -447,7 +457,7 @@ __global__ __launch_bounds__(kEpi) void msbfs_init(MsArgs a, Sources src, uint32
 {
     __shared__ uint32_t vert[64], degree[64];
     __shared__ unsigned long long all;
-    __shared__ uint32_t wsum[kEpi / kWave];
+    __shared__ uint32_t wsum[2][kEpi / kWave];
     const uint32_t i = threadIdx.x;
     uint32_t own = 0;
     if (i == 0) all = 0;
@@ -483,7 +493,7 @@ __global__ __launch_bounds__(kEpi) void msbfs_init(MsArgs a, Sources src, uint32
             before += kv < v ? kd : 0;
         }
         a.before[v] = before;
-        if (lane == 0) a.tile_edges[tile] = edges;
+        if (lane == 0) reinterpret_cast<uint32_t *>(a.tile_edges)[tile] = edges;
     }
     __syncthreads();
     const bool td = a.td_div != 0 && all * a.td_div <= a.E;
@@ -508,7 +518,9 @@ struct bw_msbfs {
     const uint32_t *off = nullptr, *col = nullptr;
     uint64_t *visit = nullptr, *front[2] = {nullptr, nullptr};
     uint64_t *next = nullptr;
-    uint32_t *before = nullptr, *tile_edges = nullptr, *tile_first = nullptr;
+    uint32_t *before = nullptr, *group_first = nullptr;
+    uint4 *tile_edges = nullptr;
+    uint32_t groups = 0;
     uint64_t *part = nullptr;
     uint4 *hubs = nullptr;
     uint32_t nhubs = 0;
@@ -532,7 +544,7 @@ struct bw_msbfs {
     ~bw_msbfs()
     {
         if (exec) (void)hipGraphExecDestroy(exec);
-        void *bufs[] = {visit, front[0], front[1], next, before, tile_edges, tile_first, part, hubs, st};
+        void *bufs[] = {visit, front[0], front[1], next, before, tile_edges, group_first, part, hubs, st};
         for (void *p : bufs)
             if (p) (void)hipFree(p);
         if (own_stream) (void)hipStreamDestroy(own_stream);
@@ -556,8 +568,8 @@ MsArgs make_args(const bw_msbfs *m, int32_t *depths, uint32_t n)
     a.next = m->next;
     a.before = m->before;
     a.tile_edges = m->tile_edges;
-    a.tile_first = m->tile_first;
-    a.tiles = static_cast<uint32_t>((m->V + kWave - 1) / kWave);
+    a.group_first = m->group_first;
+    a.groups = m->groups;
     a.part = m->part;
     a.hubs = m->hubs;
     a.nhubs = m->nhubs;
@@ -629,12 +641,12 @@ extern "C" int bw_msbfs_create(bw_msbfs **out, const bw_graph_dev *g, uint32_t m
     m->col = g->cols;
     m->max_levels = max_levels;
     m->grid = static_cast<uint32_t>(device_cus()) * 8;
-    const uint64_t tiles = (m->V + kWave - 1) / kWave;
+    m->groups = static_cast<uint32_t>((m->V + kGroup * kWave - 1) / (kGroup * kWave));
     bool ok = hipMalloc(&m->visit, 8 * m->V) == hipSuccess && hipMalloc(&m->front[0], 8 * m->V) == hipSuccess &&
               hipMalloc(&m->front[1], 8 * m->V) == hipSuccess && hipMalloc(&m->next, 8 * m->V) == hipSuccess &&
-              hipMalloc(&m->before, 4ull * kWave * tiles) == hipSuccess &&
-              hipMalloc(&m->tile_edges, 4ull * tiles) == hipSuccess &&
-              hipMalloc(&m->tile_first, 4ull * tiles) == hipSuccess &&
+              hipMalloc(&m->before, 4ull * kWave * kGroup * m->groups) == hipSuccess &&
+              hipMalloc(&m->tile_edges, sizeof(uint4) * m->groups) == hipSuccess &&
+              hipMalloc(&m->group_first, 4ull * m->groups) == hipSuccess &&
               hipMalloc(&m->part, 16ull * m->grid) == hipSuccess &&
               hipMalloc(&m->st, kOutOffset + 8 * std::max<size_t>(max_levels, kOutFirst)) == hipSuccess;
     if (!ok) {

@@ -1,6 +1,6 @@
 """Multi-source search at the edges of its numbering of the frontier's edges
-(tiles of 64 vertices, windows of 512 edges, the epilogue's rounds of 8192
-tiles) and of its reset: depths equal the oracle's for every source and the
+(tiles of 64 vertices, groups of four tiles, windows of 512 edges, the
+epilogue's rounds of 4096 groups) and of its reset: depths equal the oracle's for every source and the
 levels' new bits are their counts."""
 import numpy as np
 import pytest
@@ -18,8 +18,9 @@ def _random(V, E, seed):
     return graph.from_edges(V, s.astype(np.uint32), d.astype(np.uint32))
 
 
-@pytest.mark.parametrize("V,E", [(1, 0), (63, 100), (64, 511), (65, 600), (129, 20), (8191, 30000), (8192 * 64, 700000),
-                                 (8192 * 64 + 1, 600000), (8192 * 64 * 2 + 63, 900000)])
+@pytest.mark.parametrize("V,E", [(1, 0), (63, 100), (64, 511), (65, 600), (129, 20), (255, 900), (257, 3),
+                                 (8191, 30000), (8192 * 64, 700000), (8192 * 64 + 1, 600000),
+                                 (8192 * 64 * 2 + 63, 900000), (8192 * 64 * 4 + 1, 700000)])
 @pytest.mark.parametrize("n", [1, 3, 64])
 def test_levels(gpu, V, E, n):
     g = _random(V, E, V + n)
