@@ -57,13 +57,35 @@ constexpr uint16_t kNewPair = 0x8000;    // edge code flag: the edge opens a new
 // blocks, 6.7 with these; the iteration at 2^20 vertices 68 us with a work
 // limit of 32768, 62 with 16384, 58 with 8192; at 2^21 74, 66, 67; at 2^22
 // 93.5, 98, 106.
+// Where partitions have many chunks each vertex adds up many partials, and
+// blocks of that little work would be thousands of a few vertices each: the
+// limit is at least a 350th of all vertices' partials then (partial_reads).
+// In chunks of 32768 edges, us per iteration with a limit from V alone, with
+// this one, and with 32768: 2^18 vertices, R-MAT, edge factor 80 89.5, 50.8,
+// 52.5; 2^19, 32 58, 43.5, 47; 2^20, 16 57.6, 51.8, 53.9; Erdos-Renyi 2^20, 40
+// 186, 161, 161.
 inline uint32_t block_verts(uint32_t V)
 {
     uint32_t n = kBlockVerts;
     while (n > 256 && V / n < 512) n /= 2;
     return n;
 }
-inline uint32_t block_work(uint32_t V) { return std::min(std::max(V / 128, 2048u), kBlockWork); }
+inline uint32_t block_work(uint32_t V, uint64_t reads)
+{
+    const uint64_t want = std::max<uint64_t>(V / 128, reads / 350);
+    return static_cast<uint32_t>(std::min<uint64_t>(std::max<uint64_t>(want, 2048), kBlockWork));
+}
+
+// The vertices of each partition times its chunks.
+inline uint64_t partial_reads(uint32_t V, uint32_t rows_log2, const std::vector<uint32_t> &chunk_base)
+{
+    uint64_t n = 0;
+    for (size_t k = 0; k + 1 < chunk_base.size(); k++) {
+        const uint64_t first = static_cast<uint64_t>(k) << rows_log2;
+        n += std::min<uint64_t>(V - first, 1ull << rows_log2) * (chunk_base[k + 1] - chunk_base[k]);
+    }
+    return n;
+}
 
 struct Quad {
     uint32_t x, y, z, w;
@@ -181,12 +203,12 @@ inline bool build_plan(const uint32_t *off, const uint32_t *cols, uint32_t V, ui
     P.slots = P.chunk_base[K];
 
     // Scatter blocks: consecutive vertices of one partition, cut so that
-    // vertices x chunks of the partition + pairs stays within block_work(V),
+    // vertices x chunks of the partition + pairs stays within block_work,
     // at most block_verts(V) vertices and kMaxRuns runs.
     std::vector<uint32_t> stamp(K, UINT32_MAX), blen(K, 0), done(K, 0), touched;
     std::vector<uint32_t> blockOf(V), runPart;
     uint32_t flat = 0;
-    const uint32_t maxVerts = block_verts(V), maxWork = block_work(V);
+    const uint32_t maxVerts = block_verts(V), maxWork = block_work(V, partial_reads(V, L, P.chunk_base));
     for (uint32_t k = 0; k < K; k++) {
         const uint32_t vEnd = std::min<uint64_t>((static_cast<uint64_t>(k) << L) + D, V);
         const uint64_t perVertex = std::max<uint32_t>(1, P.chunk_base[k + 1] - P.chunk_base[k]);

@@ -674,7 +674,7 @@ int build_plan_device(const uint32_t *roff, const uint32_t *rcols, uint32_t V, u
     PLAN_ALLOC(nblocksK, uint32_t, K);
     PLAN_TRY(hipMemcpyAsync(dchunk_base, chunk_base.data(), sizeof(uint32_t) * (K + 1), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(plan_cut_kernel, dim3(K), dim3(64), 0, s, V, L, pbase, dchunk_base, block_verts(V),
-                       block_work(V), block_local, pblocks, nblocksK);
+                       block_work(V, partial_reads(V, L, chunk_base)), block_local, pblocks, nblocksK);
     PLAN_TRY(hipGetLastError());
     std::vector<uint32_t> hnb(K), block_base(K + 1, 0);
     PLAN_TRY(hipMemcpyAsync(hnb.data(), nblocksK, sizeof(uint32_t) * K, hipMemcpyDeviceToHost, s));

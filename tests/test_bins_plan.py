@@ -81,3 +81,18 @@ def test_plan_rejects_too_many_partitions(checker, tmp_path):
     off, cols = _write_rev_csr(g, tmp_path / "long")
     r = subprocess.run([str(checker), off, cols, "8", "1", "1", "0"], capture_output=True, text=True, timeout=120)
     assert r.returncode == 4 and "too many partitions" in r.stdout
+
+
+def test_blocks_of_many_chunks(checker, tmp_path):
+    """A partition of many chunks gives each vertex many partials to add:
+    the blocks get the work of a 350th of them all, not a few vertices each."""
+    g = graph.rmat(15, 64, seed=5)
+    off, cols = _write_rev_csr(g, tmp_path / "dense")
+    r = subprocess.run([str(checker), off, cols, "13", "1", "1", "1"], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr + r.stdout
+    fields = r.stdout.split()
+    slots, blocks = (int(fields[fields.index(x) + 1]) for x in ("slots", "blocks"))
+    # 4 partitions of 8192 vertices: 8192 x slots partials in all.  A vertex of
+    # the longest partition may exceed half the limit, so up to two blocks for
+    # every 500th, and those cut at 256 vertices.
+    assert 8192 * slots // 350 > 2048 and blocks <= 2 * 350 + g.vertex_count // 256, (slots, blocks)
