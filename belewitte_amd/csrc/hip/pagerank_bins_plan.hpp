@@ -91,6 +91,18 @@ struct Quad {
     uint32_t x, y, z, w;
 };
 
+// Edges of the longest chunk.
+inline uint32_t longest_chunk(const std::vector<Quad> &chunks, const std::vector<Quad> &tasks)
+{
+    uint32_t most = 0;
+    for (const Quad &c : chunks) {
+        uint32_t n = 0;
+        for (uint32_t t = c.x; t < c.y; t++) n += tasks[t].y - tasks[t].x;
+        most = std::max(most, n);
+    }
+    return most;
+}
+
 struct Plan {
     uint32_t V = 0, E = 0, rows_log2 = 0, K = 0;
     uint32_t pairs = 0;                  // U, the number of (source, partition) pairs

@@ -1162,6 +1162,7 @@ struct bw_pr_plan {
     struct Bins {
         uint32_t log2 = 0, chunk_tasks = 0, nchunks = 0, nblocks = 0, pairs = 0, slots = 0, K = 0;
         uint32_t ntasks = 0, nruns = 0;  // task records; run entries (terminators included)
+        uint32_t longest = 0;            // edges of the longest chunk
         uint64_t ncodes = 0;             // edge codes, padding included
         uint32_t lane_edges = 8;  // edge codes per lane and round of the accumulate kernel
         uint16_t *codes = nullptr;
@@ -1460,6 +1461,7 @@ int bin_host(bw_pr_plan *plan, uint32_t rows_log2, uint32_t chunk_tasks, bw_pr_p
     nb.ntasks = static_cast<uint32_t>(P.tasks.size());
     nb.nruns = static_cast<uint32_t>(P.run_flat.size());
     nb.ncodes = P.codes.size();
+    nb.longest = bins::longest_chunk(P.chunks, P.tasks);
     return BW_HIP_OK;
 }
 
@@ -1491,6 +1493,7 @@ int bin_device(bw_pr_plan *plan, uint32_t rows_log2, uint32_t chunk_tasks, bw_pr
     nb.ntasks = d.ntasks;
     nb.nruns = d.nruns;
     nb.ncodes = d.ncodes;
+    nb.longest = d.longest;
     return BW_HIP_OK;
 }
 
@@ -1503,14 +1506,22 @@ int bin_device(bw_pr_plan *plan, uint32_t rows_log2, uint32_t chunk_tasks, bw_pr
 // up to 128 in two, and no piece is shorter than 8192 edges.  us per
 // iteration, whole chunks / pieces: 50021 vertices (4 chunks) 40.7 / 18,
 // 150001 (21) 44.9 / 28 (192 or 256 workgroups: 32), 300007 (42) 47.7 / 34,
-// 600011 (65) 53 / 35, 2^20 (117) 58 / 46.
+// 600011 (65) 53 / 35, 2^20 (117) 58 / 46.  With more than 64 chunks there are
+// CUs enough for them, and what is saved is half of the longest one: at most
+// 81920 edges are left whole (us per iteration, whole / pieces: longest 32768,
+// 1024 x 1024 grid in 128 chunks 27.5 / 29.4; 65536, R-MAT 600000 vertices in
+// 66 25.3 / 27.8 and 300000 in 98 28.3 / 30.4, Erdos-Renyi 2^21 in 128 41.1 /
+// 43.1; 98000, Erdos-Renyi 1.7 M in 104 44.8 / 41.6; 131072, R-MAT 600000 in
+// 82 35.8 / 31.5).
 constexpr uint32_t kSplitChunks = 128;
 constexpr uint64_t kMinPiece = 8192;
+constexpr uint32_t kWholeChunk = 81920;
 
 int split_chunks(bw_pr_plan::Bins &nb)
 {
     nb.split = 1;
     if (nb.nchunks == 0 || nb.nchunks > kSplitChunks) return BW_HIP_OK;
+    if (nb.nchunks > kSplitChunks / 2 && nb.longest <= kWholeChunk) return BW_HIP_OK;
     const uint64_t want = std::max(kSplitChunks / nb.nchunks, 2u), most = nb.ncodes / nb.nchunks / kMinPiece;
     const uint32_t split = static_cast<uint32_t>(std::min<uint64_t>({want, kMaxSplit, most}));
     if (split < 2) return BW_HIP_OK;

@@ -852,6 +852,7 @@ int build_plan_device(const uint32_t *roff, const uint32_t *rcols, uint32_t V, u
 #undef PLAN_TRY
 #undef PLAN_ALLOC
     made.ntasks = static_cast<uint32_t>(tasks.size());
+    made.longest = longest_chunk(chunks, tasks);
     out = made;
     made = DeviceBins();  // the caller's now
     return BW_HIP_OK;

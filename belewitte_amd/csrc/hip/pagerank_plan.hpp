@@ -24,6 +24,7 @@ struct DeviceBins {
     float *vals = nullptr, *partials = nullptr;
     double2 *part = nullptr;
     uint32_t K = 0, pairs = 0, slots = 0, nchunks = 0, nblocks = 0, ntasks = 0, nruns = 0;
+    uint32_t longest = 0;  // edges of the longest chunk
     uint64_t ncodes = 0;
 };
 

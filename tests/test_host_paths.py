@@ -134,3 +134,20 @@ def test_engine_memory_follows_the_graph(fake):
         assert held < 2 << 20, held
         assert fake.fake_live() == before
     """)
+
+
+def test_short_chunks_stay_whole(fake):
+    """More than 64 chunks are cut in two only if the longest one has more
+    than 81920 edges."""
+    _run(fake, PLAN + """
+for chunk_tasks, V, E in ((16, 20000, 2400000), (64, 200000, 9000000)):
+    g, plan, keep = binned(V, E)
+    N.check_hip(lib.bw_pr_plan_bin_host(plan, 13, chunk_tasks, 8))
+    chunks = C.c_uint32()
+    N.check_hip(lib.bw_pr_plan_bin_info(plan, None, C.byref(chunks), None))
+    assert 64 < chunks.value <= 128, chunks.value
+    N.check_hip(run(g, plan))
+    (grid,) = {int(c[2]) for c in calls("launch") if "accumulate" in c[0]}
+    assert grid - 1 == chunks.value * (1 if chunk_tasks == 16 else 2), (chunk_tasks, grid, chunks.value)
+    lib.bw_pr_plan_destroy(plan)
+    """)
