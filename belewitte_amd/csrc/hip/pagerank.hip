@@ -1040,7 +1040,7 @@ __global__ __launch_bounds__(1024) void pr_dangling_kernel(uint64_t V, const uin
 // together; 20 bytes per vertex are 4.3 us of HBM).
 struct FinishArgs {
     uint64_t V;
-    const uint32_t *deg;      // out-degrees
+    const uint32_t *deg;      // out-degrees; NULL: nothing reads the dangling mass or the contributions
     float *pr;
     float *np;                // the sums
     float *contrib;           // NULL: nothing gathers contributions
@@ -1104,7 +1104,7 @@ __global__ __launch_bounds__(kFinishThreads) void pr_finish_kernel(FinishArgs a,
             const uint64_t v = b0 + k * kFinishThreads + threadIdx.x;
             const uint64_t w = v < a.V ? v : a.V - 1;
             old[k] = a.pr[w];
-            dv[k] = a.deg[w];
+            dv[k] = a.deg ? a.deg[w] : 1u;
             acc[k] = GATHERED ? sums.row_sum(static_cast<uint32_t>(w)) : a.np[w];
         }
 #pragma unroll
@@ -1140,7 +1140,7 @@ __global__ __launch_bounds__(kFinishThreads) void pr_start_kernel(FinishArgs a, 
     double dangl = 0.0;
     for (uint64_t v = static_cast<uint64_t>(blockIdx.x) * kFinishThreads + threadIdx.x; v < a.V;
          v += static_cast<uint64_t>(gridDim.x) * kFinishThreads) {
-        const uint32_t d = a.deg[v];
+        const uint32_t d = a.deg ? a.deg[v] : 1u;
         a.pr[v] = (predivide && d != 0) ? init / static_cast<float>(d) : init;
         if (a.contrib) a.contrib[v] = contribution_of(init, d, a.int_degree);
         a.np[v] = 0.0f;
@@ -1619,7 +1619,7 @@ namespace {
 struct RunBuffers {
     uint32_t *deg = nullptr;
     float *np = nullptr;
-    float *contrib = nullptr;  // per-vertex contributions (the variants that gather them)
+    float *contrib = nullptr;  // per-vertex contributions (the variants that gather them without a pull plan)
     double *acc = nullptr;     // [iterations] residuals, [iterations + 1] dangling masses, one spare
     double2 *part = nullptr;   // per workgroup of a pass over the vertices: (residual, dangling mass)
     ~RunBuffers()
@@ -1672,25 +1672,7 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
     BW_HIP_CHECK(hipMalloc(&buf.np, sizeof(float) * V));
     BW_HIP_CHECK(hipMalloc(&buf.acc, sizeof(double) * (2 * iters + 2)));
     BW_HIP_CHECK(hipMalloc(&buf.part, sizeof(double2) * kFinishGrid));
-    if (!nodiv) BW_HIP_CHECK(hipMalloc(&buf.contrib, sizeof(float) * V));
     double *resid = buf.acc, *dang = buf.acc + iters, *spare = buf.acc + 2 * iters + 1;
-
-    // Degrees once per run (pagerank/pagerank.cpp:102-112).  With the forward
-    // CSR resident, every variant's out-degrees come from its offsets: the
-    // same integers the variant's own degree kernel counts
-    // (pagerank/pagerank.cu:40-123), without an atomic per edge; the push
-    // variants, which have no degree kernel, read the same offsets.
-    BW_TRY(bw_pr_zero_degrees(V, buf.deg, &cfg));
-    if (g->offsets) {
-        BW_TRY(bw_pr_degrees_csr(V, g->offsets, g->offset_bytes, buf.deg, &cfg));
-    } else switch (variant) {
-    case BW_PR_EDGE_LIST: BW_TRY(bw_pr_degrees_edge_list(E, g->el_in, buf.deg, &cfg)); break;
-    case BW_PR_REV_EDGE_LIST: BW_TRY(bw_pr_degrees_edge_list(E, g->rel_out, buf.deg, &cfg)); break;
-    case BW_PR_STRUCT_EDGE_LIST: BW_TRY(bw_pr_degrees_struct_edge_list(E, g->sel, 0, buf.deg, &cfg)); break;
-    case BW_PR_REV_STRUCT_EDGE_LIST: BW_TRY(bw_pr_degrees_struct_edge_list(E, g->rsel, 1, buf.deg, &cfg)); break;
-    default:
-        BW_TRY(bw_pr_degrees_rev_csr(V, g->rev_offsets, g->offset_bytes, g->rev_cols, buf.deg, &cfg));
-    }
 
     // The push forms scatter through a binned layout (propagation blocking)
     // instead of one global atomic per edge; a graph the layout refuses
@@ -1723,16 +1705,41 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
         BW_TRY(bw_pr_pull_plan_create(&pull, V, g->rev_offsets, g->offset_bytes, s));
     }
 
+    const bool gathered = scatter && scatter_gathers(scatter);
+    // Degrees once per run (pagerank/pagerank.cpp:102-112).  With the forward
+    // CSR resident, every variant's out-degrees come from its offsets: the
+    // same integers the variant's own degree kernel counts
+    // (pagerank/pagerank.cu:40-123), without an atomic per edge; the push
+    // variants, which have no degree kernel, read the same offsets, and only for
+    // the contributions or the dangling mass.
+    BW_TRY(bw_pr_zero_degrees(V, buf.deg, &cfg));
+    const bool degrees = gathered || mode == BW_PR_DANGLING_UNIFORM ||
+                         !(variant == BW_PR_VERTEX_PUSH || variant == BW_PR_VERTEX_PUSH_WARP);
+    if (!degrees) {
+        // nothing to count
+    } else if (g->offsets) {
+        BW_TRY(bw_pr_degrees_csr(V, g->offsets, g->offset_bytes, buf.deg, &cfg));
+    } else switch (variant) {
+    case BW_PR_EDGE_LIST: BW_TRY(bw_pr_degrees_edge_list(E, g->el_in, buf.deg, &cfg)); break;
+    case BW_PR_REV_EDGE_LIST: BW_TRY(bw_pr_degrees_edge_list(E, g->rel_out, buf.deg, &cfg)); break;
+    case BW_PR_STRUCT_EDGE_LIST: BW_TRY(bw_pr_degrees_struct_edge_list(E, g->sel, 0, buf.deg, &cfg)); break;
+    case BW_PR_REV_STRUCT_EDGE_LIST: BW_TRY(bw_pr_degrees_struct_edge_list(E, g->rsel, 1, buf.deg, &cfg)); break;
+    default:
+        BW_TRY(bw_pr_degrees_rev_csr(V, g->rev_offsets, g->offset_bytes, g->rev_cols, buf.deg, &cfg));
+    }
+
     FinishArgs fin{};
     fin.V = V;
-    fin.deg = buf.deg;
+    fin.deg = degrees ? buf.deg : nullptr;
     fin.pr = ranks;
     fin.np = buf.np;
-    fin.contrib = buf.contrib;
     fin.part = buf.part;
     fin.nodiv = nodiv;
     fin.mode = mode;
-    const bool gathered = scatter && scatter_gathers(scatter);
+    // The binned scatter and the atomic kernels divide for themselves.
+    if (gathered || variant == BW_PR_REV_EDGE_LIST || variant == BW_PR_REV_STRUCT_EDGE_LIST)
+        BW_HIP_CHECK(hipMalloc(&buf.contrib, sizeof(float) * V));
+    fin.contrib = pull && !nodiv ? pull->contrib : buf.contrib;
     const uint64_t passVerts = static_cast<uint64_t>(finish_per_thread(gathered)) * kFinishThreads;
     const uint32_t passGrid = static_cast<uint32_t>(std::min<uint64_t>((V + passVerts - 1) / passVerts, kFinishGrid));
     fin.zero_np = !pull && !gathered;  // these store every row's sum
@@ -1747,7 +1754,7 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
         const ReducePrev prev{buf.part, passGrid, it > 1 ? &resid[it - 2] : spare, &dang[it - 1]};
         bool reduced = false;  // the sums' launch reduced `prev`
         if (pull) {
-            BW_TRY(pull_sums(pull, variant, g->rev_cols, nodiv ? ranks : buf.contrib, buf.np, &cfg, prev));
+            BW_TRY(pull_sums(pull, variant, g->rev_cols, nodiv ? ranks : fin.contrib, buf.np, &cfg, prev));
             reduced = true;
         } else if (E && variant == BW_PR_REV_EDGE_LIST) {
             BW_TRY((launch_rev_segmented<false, true>(E, g->rel_in, g->rel_out, nullptr, buf.contrib, buf.np, s,
@@ -1760,7 +1767,8 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
             BW_TRY(scatter_gather(scatter, buf.contrib, prev, s));
             reduced = true;
         } else if (scatter) {
-            BW_TRY(bw_pr_scatter_iteration(scatter, buf.deg, ranks, buf.np, s));
+            BW_TRY(scatter_bins(scatter, buf.deg, ranks, buf.np, prev, s));
+            reduced = true;
         } else if (variant == BW_PR_EDGE_LIST) {
             BW_TRY(bw_pr_edge_list(E, g->el_in, g->el_out, buf.deg, ranks, buf.np, &cfg));
         } else if (variant == BW_PR_STRUCT_EDGE_LIST) {

@@ -275,8 +275,11 @@ constexpr uint32_t kBinBatch = 8;
 template<typename Src>
 __global__ __launch_bounds__(kBinThreads) void scatter_bin_kernel(Src src, uint64_t E,
                                                                   const uint32_t *__restrict__ deg,
-                                                                  const float *__restrict__ pr, BinOut o)
+                                                                  const float *__restrict__ pr, BinOut o,
+                                                                  ReducePrev prev)
 {
+    __shared__ ReduceLds red;
+    if (reduce_prev<kBinThreads>(prev, red)) return;
     __shared__ uint32_t cursor[kMaxParts];
     bin_setup(o, cursor);
     const uint64_t b0 = static_cast<uint64_t>(blockIdx.x) * o.per_block;
@@ -308,8 +311,11 @@ constexpr uint32_t kStagedPerThread = kBinBaseEdges / kStagedThreads;
 template<typename Src>
 __global__ __launch_bounds__(kStagedThreads) void scatter_bin_staged_kernel(Src src, uint64_t E,
                                                                            const uint32_t *__restrict__ deg,
-                                                                           const float *__restrict__ pr, BinOut o)
+                                                                           const float *__restrict__ pr, BinOut o,
+                                                                           ReducePrev prev)
 {
+    __shared__ ReduceLds red;
+    if (reduce_prev<kStagedThreads>(prev, red)) return;
     __shared__ uint32_t counts[kMaxParts], starts[kMaxParts], gbase[kMaxParts];
     __shared__ uint16_t stRow[kBinBaseEdges], stPart[kBinBaseEdges];
     __shared__ float stVal[kBinBaseEdges];
@@ -749,6 +755,31 @@ int scatter_gather(const bw_pr_scatter *sc, const float *contrib, const ReducePr
     return BW_HIP_OK;
 }
 
+// One iteration of the binned layout; prev is reduced by the bin launch.
+int scatter_bins(const bw_pr_scatter *sc, const uint32_t *deg, const float *pr, float *np, const ReducePrev &prev,
+                 hipStream_t s)
+{
+    BinOut o{sc->base, sc->row, sc->val, sc->parts, sc->per_block};
+    const uint32_t grid = sc->nb + (prev.part ? 1u : 0u);
+    BW_TRY(with_source(sc->kind, sc->a, sc->b, sc->ob, sc->src, [&](auto src) {
+        using Src = decltype(src);
+        if (sc->per_block == kBinBaseEdges)
+            hipLaunchKernelGGL(scatter_bin_staged_kernel<Src>, dim3(grid), dim3(kStagedThreads), 0, s, src, sc->E, deg,
+                               pr, o, prev);
+        else
+            hipLaunchKernelGGL(scatter_bin_kernel<Src>, dim3(grid), dim3(kBinThreads), 0, s, src, sc->E, deg, pr, o,
+                               prev);
+        return BW_HIP_OK;
+    }));
+    BW_LAUNCH_CHECK();
+    if (sc->nchunks) {
+        hipLaunchKernelGGL(scatter_accumulate_kernel, dim3(sc->nchunks), dim3(kAccThreads), 0, s, sc->chunks, sc->row,
+                           sc->val, sc->V, np);
+        BW_LAUNCH_CHECK();
+    }
+    return BW_HIP_OK;
+}
+
 }  // namespace bw
 
 extern "C" int bw_pr_scatter_destroy(bw_pr_scatter *sc)
@@ -776,22 +807,5 @@ extern "C" int bw_pr_scatter_iteration(const bw_pr_scatter *sc, const uint32_t *
         BW_LAUNCH_CHECK();
         return BW_HIP_OK;
     }
-    BinOut o{sc->base, sc->row, sc->val, sc->parts, sc->per_block};
-    BW_TRY(with_source(sc->kind, sc->a, sc->b, sc->ob, sc->src, [&](auto src) {
-        using Src = decltype(src);
-        if (sc->per_block == kBinBaseEdges)
-            hipLaunchKernelGGL(scatter_bin_staged_kernel<Src>, dim3(sc->nb), dim3(kStagedThreads), 0, s, src, sc->E,
-                               deg, pr, o);
-        else
-            hipLaunchKernelGGL(scatter_bin_kernel<Src>, dim3(sc->nb), dim3(kBinThreads), 0, s, src, sc->E, deg, pr,
-                               o);
-        return BW_HIP_OK;
-    }));
-    BW_LAUNCH_CHECK();
-    if (sc->nchunks) {
-        hipLaunchKernelGGL(scatter_accumulate_kernel, dim3(sc->nchunks), dim3(kAccThreads), 0, s, sc->chunks, sc->row,
-                           sc->val, sc->V, np);
-        BW_LAUNCH_CHECK();
-    }
-    return BW_HIP_OK;
+    return scatter_bins(sc, deg, pr, np, ReducePrev{}, s);
 }

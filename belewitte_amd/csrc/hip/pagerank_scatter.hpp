@@ -69,5 +69,7 @@ struct ScatterSums {
 bool scatter_gathers(const bw_pr_scatter *sc);
 ScatterSums scatter_sums(const bw_pr_scatter *sc);
 int scatter_gather(const bw_pr_scatter *sc, const float *contrib, const ReducePrev &prev, hipStream_t s);
+int scatter_bins(const bw_pr_scatter *sc, const uint32_t *deg, const float *pr, float *np, const ReducePrev &prev,
+                 hipStream_t s);
 
 }  // namespace bw

@@ -151,3 +151,20 @@ for chunk_tasks, V, E in ((16, 20000, 2400000), (64, 200000, 9000000)):
     assert grid - 1 == chunks.value * (1 if chunk_tasks == 16 else 2), (chunk_tasks, grid, chunks.value)
     lib.bw_pr_plan_destroy(plan)
     """)
+
+
+def test_contributions_only_where_gathered(fake):
+    """bw_pr_run holds per-vertex contributions (the only array of 4 bytes a
+    vertex besides degrees and sums) for the variants that gather them."""
+    _run(fake, """
+        V, E = (1 << 20) + 1, 1000  # past the gathered scatter layout
+        dg = device.DeviceGraph(graph.from_edges(V, np.arange(E, dtype=np.uint32), np.arange(1, E + 1, dtype=np.uint32)))
+        for name in pagerank.VARIANTS:
+            dg.ensure(pagerank.REPRESENTATION[pagerank.variant_id(name)])
+            ranks = device.DeviceArray(V, np.float32)
+            fake.fake_clear()
+            cfg = N.launch(warp=32, chunk=32)
+            N.check_hip(lib.bw_pr_run(dg.ref, pagerank.variant_id(name), 2, 1, ranks.ptr, None, C.byref(cfg)))
+            held = sum(int(c[0]) == 4 * V for c in calls("alloc"))
+            assert held == 2 + (name.startswith("rev-") or "pull" in name), (name, held)
+    """)
