@@ -1648,7 +1648,13 @@ constexpr int kBinAccThreads = 1024;
 #endif
 constexpr int kBinFinThreads = BW_BINS_FIN_THREADS;
 
-bool small_graph(uint32_t V, uint32_t E) { return V <= kSmallVerts && E <= kSmallThreads * kSmallEdges; }
+// In-edges per thread of a small graph's kernel; 0: no small graph.
+uint32_t small_edges(uint32_t V, uint32_t E)
+{
+    if (V > kSmallVerts || E > kSmallThreads * kSmallEdges) return 0;
+    const uint32_t per = (E + kSmallThreads - 1) / kSmallThreads;
+    return per <= 8 ? 8 : per <= 16 ? 16 : kSmallEdges;
+}
 
 int run_small(const bw_pr_plan *plan, const uint32_t *roff, const uint32_t *rcols, int32_t iterations, int32_t mode,
               int32_t nodiv_quirk, float *ranks, double *dangl, double *resid, double *resid_host, float *kernel_ms,
@@ -1670,8 +1676,8 @@ int run_small(const bw_pr_plan *plan, const uint32_t *roff, const uint32_t *rcol
     a.pair_scale = std::ldexp(1.0f, S - 32);
     a.partial_scale = std::ldexp(1.0f, -S);
     using Kernel = void (*)(SmallArgs);
-    const uint32_t per = (plan->E + kSmallThreads - 1) / kSmallThreads;
-    const Kernel k = per <= 8 ? pr_small_kernel<8> : per <= 16 ? pr_small_kernel<16> : pr_small_kernel<kSmallEdges>;
+    const uint32_t per = small_edges(plan->V, plan->E);
+    const Kernel k = per == 8 ? pr_small_kernel<8> : per == 16 ? pr_small_kernel<16> : pr_small_kernel<kSmallEdges>;
     // 12 bytes a vertex.  The kernel's limit is set to what the largest graph
     // needs: all threads of the process share it, and one that set its own
     // graph's size could lower it between another's setting and launch.
@@ -1791,6 +1797,14 @@ int run_binned(const bw_pr_plan *plan, int32_t iterations, int32_t mode, int32_t
 
 }  // namespace
 
+extern "C" int bw_pr_plan_form(const bw_pr_plan *plan, uint32_t *small, uint32_t *pieces)
+{
+    if (!plan) return fail(BW_HIP_ERR_ARG, "plan is NULL");
+    if (small) *small = small_edges(plan->V, plan->E);
+    if (pieces) *pieces = plan->binned ? plan->bins.split : 0;
+    return BW_HIP_OK;
+}
+
 extern "C" int bw_pr_fused_run(const bw_graph_dev *g, const bw_pr_plan *plan, int32_t iterations, int32_t mode,
                                int32_t nodiv_quirk, float *ranks, float *scratch, double *acc,
                                double *resid_host, float *kernel_ms, const bw_launch *cfg)
@@ -1805,7 +1819,7 @@ extern "C" int bw_pr_fused_run(const bw_graph_dev *g, const bw_pr_plan *plan, in
     hipStream_t s = stream_of(cfg);
     const uint32_t V = plan->V;
     double *dangl = acc, *resid = acc + iterations + 1, *spare = acc + 2 * iterations + 2;
-    if (small_graph(V, plan->E))
+    if (small_edges(V, plan->E))
         return run_small(plan, static_cast<const uint32_t *>(g->rev_offsets), g->rev_cols, iterations, mode, nodiv_quirk,
                          ranks, dangl, resid, resid_host, kernel_ms, s);
     if (plan->binned) return run_binned(plan, iterations, mode, nodiv_quirk, ranks, dangl, resid, spare, resid_host,

@@ -196,8 +196,14 @@ class FusedPageRank:
         more than `margin`, so that run-to-run noise does not flip the
         choice.  A shape is ("bins", rows_log2, chunk_tasks, lane_edges)
         for the binned iteration, else the pull kernels' (hot, rows_grid,
-        tiles, sorted_windows, batch).  Returns {shape: ms}."""
+        tiles, sorted_windows, batch).  Returns {shape: ms}.  A small graph
+        runs the same kernel whatever the shape, so its present one is kept
+        and timed alone."""
         from .device import device_props
+        if self._form()[0]:
+            self.run(iterations, "uniform", download=False)
+            ms = min(self.run(iterations, "uniform", download=False)[2] for _ in range(3))
+            return {"small": round(ms, 4)}
         cus = device_props(0)["compute_units"]
         cands = candidates or [("bins", 14, 128, 8), ("bins", 13, 64, 8), ("bins", 13, 32, 8), ("bins", 14, 64, 8),
                                ("bins", 14, 80, 8), ("bins", 14, 96, 8),
@@ -231,16 +237,25 @@ class FusedPageRank:
         h, g, t, w, b = shape
         return f"hot{h}/grid{g}/tiles{t}" + (f"/sorted{w}/batch{b}" if w else "")
 
+    def _form(self):
+        """(in-edges per thread of the small-graph kernel or 0, pieces per chunk)."""
+        small, pieces = C.c_uint32(), C.c_uint32()
+        N.check_hip(N.hip_lib().bw_pr_plan_form(self._plan, C.byref(small), C.byref(pieces)))
+        return small.value, pieces.value
+
     def kernel_names(self) -> str:
-        """The kernels one iteration launches under the current shape (a
-        graph of at most 8192 vertices and 32768 edges runs all its
-        iterations in one launch of pr_small_kernel instead)."""
+        """The kernels one iteration launches under the current shape, or
+        the one that runs all iterations of a small graph."""
+        small, pieces = self._form()
+        if small:
+            return f"pr_small_kernel<{small}>"
         if self.binning:
             r, _, lanes = self.binning
-            return f"pr_bins_accumulate_kernel<{r}, 1024, {lanes}, 2> + pr_bins_finalise_kernel<{r}, 512>"
+            return (f"pr_bins_accumulate_kernel<{r}, 1024, {lanes}, 2> + "
+                    f"pr_bins_finalise_kernel<{r}, 512, {'true' if pieces > 1 else 'false'}>")
         hot, _, tiles, width, batch = self.tuning
         rows = f"pr_windows_kernel<{width}, {batch}>" if width else f"pr_rows_kernel<{hot}, {tiles}>"
-        return f"pr_pieces_kernel + {rows}"
+        return f"pr_pieces_kernel<{hot}> + {rows}"
 
     def info(self) -> dict:
         a, b, c = C.c_uint32(), C.c_uint32(), C.c_uint32()

@@ -527,6 +527,13 @@ int bw_pr_plan_bin_array(const bw_pr_plan *plan, int32_t which, void *host_dst,
 /* Pairs, chunks and scatter blocks of the binned plan (0 when off). */
 int bw_pr_plan_bin_info(const bw_pr_plan *plan, uint32_t *pairs,
                         uint32_t *chunks, uint32_t *blocks);
+/* Which kernels a run takes.  small_edges: 0, or, for a graph of at most
+ * 8192 vertices and 32768 edges, whose run is one launch of one workgroup
+ * whatever the shape asked for, the in-edges that launch keeps per thread
+ * (8, 16 or 32).  pieces: workgroups per chunk of the binned plan's
+ * accumulate (0 when off). */
+int bw_pr_plan_form(const bw_pr_plan *plan, uint32_t *small_edges,
+                    uint32_t *pieces);
 
 /* Number of doubles of the `acc` workspace of bw_pr_fused_run. */
 uint64_t bw_pr_fused_acc_len(int32_t iterations);

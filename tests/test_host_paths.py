@@ -168,3 +168,35 @@ def test_contributions_only_where_gathered(fake):
             held = sum(int(c[0]) == 4 * V for c in calls("alloc"))
             assert held == 2 + (name.startswith("rev-") or "pull" in name), (name, held)
     """)
+
+
+def test_kernel_names_are_launched(fake):
+    """kernel_names() names what an iteration launches: the small-graph
+    kernel, the pull kernels, the binned ones with whole and with cut chunks.
+    Nothing is timed against itself for a small graph."""
+    _run(fake, r"""
+        import re, subprocess
+        def launched():
+            names = "\n".join(c[0] for c in calls("launch"))
+            plain = subprocess.run(["c++filt"], input=names, capture_output=True, text=True, check=True).stdout
+            plain = re.sub(r"(\d)u\b", r"\1", re.sub(r"\(anonymous namespace\)::", "", plain))
+            return set(re.findall(r"bw::(\w+(?:<[^<>(]*>)?)\(", plain))
+        rng = np.random.default_rng(3)
+        for V, E in ((5000, 6000), (5000, 14000), (8192, 30000), (8193, 9000), (40000, 300000)):
+            g = graph.from_edges(V, rng.integers(0, V, E).astype(np.uint32), rng.integers(0, V, E).astype(np.uint32))
+            f = pagerank.FusedPageRank(device.DeviceGraph(g), 3)
+            for shape in (None, (13, 64, 8), (14, 3, 16)):
+                if shape:
+                    f.bin(*shape, on_host=True)
+                else:
+                    f.tune(8192, 0, 2)
+                fake.fake_clear()
+                f.run(3)
+                names = set(f.kernel_names().split(" + "))
+                # one-off launches beside an iteration's
+                assert names <= launched() <= names | {"pr_fused_init_kernel", "pr_reduce_kernel"}, (names, launched())
+            if V <= 8192:
+                fake.fake_clear()
+                table = f.autotune(3)
+                assert f.binning == (14, 3, 16) and list(table) == ["small"] and len(calls("launch")) == 4
+    """)
