@@ -30,6 +30,28 @@ def degenerate_graphs():
     yield g
 
 
+def degenerate_graphs_past_small():
+    """The same for the fused kernels past the small form (8192 vertices,
+    32768 edges): no edge, a single one, a partition and a tile of a few
+    rows, and few vertices with many edges."""
+    empty = np.zeros(0, np.uint32)
+    g = graph.from_edges(8193, empty, empty)
+    g.name = "8193-isolated"
+    yield g
+    g = graph.from_edges(8193, np.array([8192], np.uint32), np.array([0], np.uint32))
+    g.name = "one-edge-of-8193"
+    yield g
+    s = np.array(list(range(9)) + [8195] * 9, np.uint32)
+    d = np.array(list(range(1, 10)) + list(range(8196, 8205)), np.uint32)
+    g = graph.from_edges(16385, s, d)
+    g.name = "chain-and-star-of-16385"
+    yield g
+    v = np.arange(200, dtype=np.uint32)
+    g = graph.from_edges(200, np.repeat(v, 200), np.tile(v, 200))
+    g.name = "complete-200"
+    yield g
+
+
 @pytest.mark.parametrize("policy", ["td", "bu", "bu-wave", "learned"])
 def test_engine_degenerate(gpu, policy):
     model = switch.Model.load(switch.MODEL_PATH).w
@@ -65,10 +87,12 @@ def test_multi_source_degenerate(gpu, td):
 @pytest.mark.parametrize("mode", ["drop", "uniform"])
 @pytest.mark.parametrize("width", [0, 2])
 def test_fused_pagerank_degenerate(gpu, mode, width):
-    for g in degenerate_graphs():
+    for g in (*degenerate_graphs(), *degenerate_graphs_past_small()):
         csr = O.CSR.from_graph(g)
         fp = pagerank.FusedPageRank.for_graph(g, max_iterations=10, reorder=True)
         fp.tune(0, 0, 1, width, 16)
+        small = g.vertex_count <= 8192 and g.edge_count <= 32768
+        assert ("pr_small_kernel" in fp.kernel_names()) == small, g.name
         ranks, resid, _ = fp.run(10, mode)
         want = O.pagerank_f64(csr, 10, mode)
         assert float(np.max(np.abs(ranks - want))) <= 1e-6, (g.name, mode, width)

@@ -14,7 +14,7 @@ import pytest
 
 from belewitte_amd import device, graph, pagerank
 from oracle import binding as O
-from test_degenerate_gpu import degenerate_graphs
+from test_degenerate_gpu import degenerate_graphs, degenerate_graphs_past_small
 
 pytestmark = pytest.mark.gpu
 
@@ -34,7 +34,10 @@ def _hub_graph():
 def cases(gpu):
     out = []
     for g in (graph.rmat(12, 16, seed=31), graph.erdos_renyi(2000, 9000, seed=3, undirected=False),
-              graph.rmat(11, 8, seed=32, undirected=True), graph.star(300), graph.chain(50), _hub_graph()):
+              graph.rmat(11, 8, seed=32, undirected=True), graph.star(300), graph.chain(50),
+              # past the small graphs, which run in one kernel whatever the layout
+              graph.erdos_renyi(9001, 36000, seed=3, undirected=False), graph.rmat(14, 2, seed=32, undirected=True),
+              graph.star(8300), graph.chain(16400), _hub_graph()):
         out.append((g, O.CSR.from_graph(g), device.DeviceGraph(g)))
     yield out
     for _, _, dg in out:
@@ -101,11 +104,13 @@ def test_binned_degree_ordered(gpu, rows_log2, chunk_tasks, lanes):
 
 @pytest.mark.parametrize("mode", ["drop", "uniform"])
 def test_binned_degenerate(gpu, mode):
-    for g in degenerate_graphs():
+    for g in (*degenerate_graphs(), *degenerate_graphs_past_small()):
         csr = O.CSR.from_graph(g)
         dg = device.DeviceGraph(g)
         fp = pagerank.FusedPageRank(dg, max_iterations=10)
         fp.bin(13, 1, 8)
+        small = g.vertex_count <= 8192 and g.edge_count <= 32768
+        assert ("pr_small_kernel" in fp.kernel_names()) == small, g.name
         ranks, resid, _ = fp.run(10, mode)
         x = O.pagerank_f64(csr, 10, mode)
         assert float(np.max(np.abs(ranks - x))) <= TOL, g.name
@@ -201,6 +206,7 @@ def _plan_graphs():
     yield graph.star(70000)
     yield graph.chain(40000)
     yield from degenerate_graphs()
+    yield from degenerate_graphs_past_small()
 
 
 @pytest.mark.parametrize("shape", [(13, 1, 8), (13, 64, 8), (14, 3, 16), (14, 128, 8)])

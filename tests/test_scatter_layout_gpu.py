@@ -29,7 +29,7 @@ def _edges(V, E, rng):
 
 
 @pytest.mark.parametrize("V,E", [(1, 5), (255, 900), (256, 2048), (257, 2049), (70001, 300000), (1 << 18, 400001),
-                                 ((1 << 20) + 1, 60000)])
+                                 ((1 << 20) + 1, 60000), ((1 << 20) + 1, 700001), (3 << 20, 1500000)])
 @pytest.mark.parametrize("kind", [EDGE_LIST, STRUCT, CSR])
 @pytest.mark.parametrize("offset_bytes", [4, 8])
 def test_scatter_sums(gpu, V, E, kind, offset_bytes):

@@ -32,6 +32,7 @@ def test_small_run(gpu, V, E, layout):
         if layout == "bins":
             fp.bin(14, 4096, 8)
         small = V <= 8192 and g.edge_count <= 32768
+        assert ("pr_small_kernel" in fp.kernel_names()) == small
         for quirk in (False, True):
             for iters in (1, 30):
                 ranks, resid, _ = fp.run(iters, "drop", nodiv_quirk=quirk)
