@@ -25,8 +25,10 @@
 // Frontier membership for the bottom-up probes is a bitmap (V bits, three
 // rotating: read, written, cleared), visited-ness a fourth bitmap, so the
 // probes hit a few MiB instead of the 4-byte depth array.  Discovered
-// vertices are appended to the next frontier queue through an LDS buffer
-// (wave-aggregated LDS atomics, one global atomic per flush).
+// vertices are staged in LDS (wave-aggregated LDS atomics); what is staged at
+// the level's end becomes the workgroup's segment of the next frontier, and
+// what the buffer or the segment cannot hold goes to a shared queue before the
+// segments (one global atomic per flush).
 
 #include "common.hpp"
 

@@ -19,8 +19,10 @@
 //   - forward edge lists and push forms: propagation blocking
 //     (pagerank_scatter.hip) in bw_pr_run and the plugin; the per-call
 //     entry points keep one atomic per edge;
-//   - FP64 reductions of the residual and dangling mass, one atomic per
-//     workgroup on a grid of two workgroups per CU.
+//   - FP64 reductions of the residual and dangling mass: partials per
+//     workgroup that the next launch adds up in a fixed order in bw_pr_run;
+//     the per-call entry points add with one atomic per workgroup on a grid
+//     of two workgroups per CU.
 
 #include "common.hpp"
 #include "pagerank_scatter.hpp"
@@ -873,8 +875,8 @@ __global__ __launch_bounds__(256) void pr_contrib_kernel(uint64_t V, const uint3
 }
 
 // One launch of a pull iteration: workgroups [0, long_blocks) sum the long
-// rows (the longest first, so that they start at once), the others one block
-// of kPullRows rows each.
+// rows (those of a whole workgroup first, each class in any order), so that
+// they start at once; the others one block of kPullRows rows each.
 template<int DIV, int W, typename Off>
 __global__ __launch_bounds__(kPullRows) void pr_pull_kernel(uint64_t V, const Off *__restrict__ roff,
                                                              const uint32_t *__restrict__ rcols,

@@ -10,10 +10,10 @@
 //      source's rows come in increasing order;
 //   2. the pairs: the first edge of each (source, partition) run, compacted
 //      by an exclusive scan of the new-pair flags;
-//   3. the scatter blocks: the host's greedy cut, one wave per partition
-//      walking its vertices with wave-uniform state, then each block's runs
-//      (distinct target partitions) counted in an LDS bitmap, one
-//      workgroup per block;
+//   3. the scatter blocks: the host's greedy cut, one wave per partition that
+//      finds each block's end by search in the prefix sums of the pairs, then
+//      each block's runs (distinct target partitions) counted in an LDS
+//      bitmap, one workgroup per block;
 //   4. the bin index of each pair: a stable sort of the pairs by partition;
 //      the scatter (flat) order: a stable sort by (block, partition);
 //   5. the edge codes: the forward edges stably sorted by partition.
@@ -923,6 +923,18 @@ __global__ __launch_bounds__(kThreads) void relabel_edges_kernel(uint32_t V, uin
     }
 }
 
+// A 64-bit hash: two odd multiplications, by 2^64 / golden ratio and by the
+// fraction of sqrt(2), each followed by the high half folded onto the low one.
+__device__ __forceinline__ uint64_t mix64(uint64_t x)
+{
+    x *= 0x9E3779B97F4A7C15ull;
+    x ^= x >> 32;
+    x *= 0x6A09E667F3BCC909ull;
+    return x ^ (x >> 32);
+}
+
+constexpr int kCompareEdges = 4;  // edges per thread and step, their loads in flight together
+
 // Compares the reverse lists made from the forward lists (row scol[j] and
 // column nrcols[j] of each edge j, rows ascending) with the ones given.
 // check[1] becomes 1 unless every row has as many edges in both: edge j then
@@ -932,15 +944,6 @@ __global__ __launch_bounds__(kThreads) void relabel_edges_kernel(uint32_t V, uin
 // on the order within a row: 0 when the rows hold the same columns, and for
 // any other lists with a chance of 2^-64.  (Scale 20, edge factor 16, 16 M
 // edges: 0.13 ms of the 0.94 ms both directions take.)
-__device__ __forceinline__ uint64_t mix64(uint64_t x)
-{
-    x = (x ^ (x >> 32)) * 0xD6E8FEB86659FD93ull;
-    x = (x ^ (x >> 32)) * 0xD6E8FEB86659FD93ull;
-    return x ^ (x >> 32);
-}
-
-constexpr int kCompareEdges = 4;  // edges per thread and step, their loads in flight together
-
 __global__ __launch_bounds__(kThreads) void relabel_compare_kernel(uint32_t E, const uint32_t *scol,
                                                                    const uint32_t *nrcols, const uint32_t *roff,
                                                                    const uint32_t *rcols, const uint32_t *order,

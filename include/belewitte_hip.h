@@ -122,11 +122,14 @@ typedef struct bw_launch {
 } bw_launch;
 
 /* Frontier-count reductions of bfs/bfs.hpp:32-116 (name suffixes "",
- * "-bulk", "-warpreduce", "-blockreduce"). */
-#define BW_RED_NORMAL 0 /* one atomic per discovered vertex          */
-#define BW_RED_BULK 1   /* per-thread count, one atomic per thread    */
-#define BW_RED_WAVE 2   /* wave64 reduce, one atomic per wave         */
-#define BW_RED_BLOCK 3  /* wave reduce + LDS block reduce, one atomic */
+ * "-bulk", "-warpreduce", "-blockreduce"): how a workgroup forms its count.
+ * Each then adds it to the frontier counter once, where the reference's first
+ * three add there directly: atomics on one address run one after another, and
+ * with them there the reductions' differences were mostly that queue. */
+#define BW_RED_NORMAL 0 /* one LDS atomic per discovered vertex       */
+#define BW_RED_BULK 1   /* per-thread count, one LDS atomic per thread */
+#define BW_RED_WAVE 2   /* wave64 reduce, one LDS atomic per wave     */
+#define BW_RED_BLOCK 3  /* wave reduce + LDS block reduce             */
 
 /* --------------------------------------------------------------- BFS */
 
