@@ -1674,7 +1674,36 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
     BW_HIP_CHECK(hipMalloc(&buf.np, sizeof(float) * V));
     BW_HIP_CHECK(hipMalloc(&buf.acc, sizeof(double) * (2 * iters + 2)));
     BW_HIP_CHECK(hipMalloc(&buf.part, sizeof(double2) * kFinishGrid));
+    const bool push = variant == BW_PR_EDGE_LIST || variant == BW_PR_STRUCT_EDGE_LIST || variant == BW_PR_VERTEX_PUSH ||
+                      variant == BW_PR_VERTEX_PUSH_WARP;
+    // The binned scatter and the atomic kernels divide for themselves, and a
+    // pull plan holds contributions of its own.
+    const bool gathers = push && E > 0 && scatter_gathers(V);
+    if (gathers || variant == BW_PR_REV_EDGE_LIST || variant == BW_PR_REV_STRUCT_EDGE_LIST)
+        BW_HIP_CHECK(hipMalloc(&buf.contrib, sizeof(float) * V));
     double *resid = buf.acc, *dang = buf.acc + iters, *spare = buf.acc + 2 * iters + 1;
+
+    // Degrees once per run (pagerank/pagerank.cpp:102-112).  With the forward
+    // CSR resident, every variant's out-degrees come from its offsets: the
+    // same integers the variant's own degree kernel counts
+    // (pagerank/pagerank.cu:40-123), without an atomic per edge; the push
+    // variants, which have no degree kernel, read the same offsets, and only for
+    // the contributions or the dangling mass.
+    BW_TRY(bw_pr_zero_degrees(V, buf.deg, &cfg));
+    const bool degrees = gathers || mode == BW_PR_DANGLING_UNIFORM ||
+                         !(variant == BW_PR_VERTEX_PUSH || variant == BW_PR_VERTEX_PUSH_WARP);
+    if (!degrees) {
+        // nothing to count
+    } else if (g->offsets) {
+        BW_TRY(bw_pr_degrees_csr(V, g->offsets, g->offset_bytes, buf.deg, &cfg));
+    } else switch (variant) {
+    case BW_PR_EDGE_LIST: BW_TRY(bw_pr_degrees_edge_list(E, g->el_in, buf.deg, &cfg)); break;
+    case BW_PR_REV_EDGE_LIST: BW_TRY(bw_pr_degrees_edge_list(E, g->rel_out, buf.deg, &cfg)); break;
+    case BW_PR_STRUCT_EDGE_LIST: BW_TRY(bw_pr_degrees_struct_edge_list(E, g->sel, 0, buf.deg, &cfg)); break;
+    case BW_PR_REV_STRUCT_EDGE_LIST: BW_TRY(bw_pr_degrees_struct_edge_list(E, g->rsel, 1, buf.deg, &cfg)); break;
+    default:
+        BW_TRY(bw_pr_degrees_rev_csr(V, g->rev_offsets, g->offset_bytes, g->rev_cols, buf.deg, &cfg));
+    }
 
     // The push forms scatter through a binned layout (propagation blocking)
     // instead of one global atomic per edge; a graph the layout refuses
@@ -1684,8 +1713,7 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
         bw_pr_scatter *&p;
         ~ScatterGuard() { bw_pr_scatter_destroy(p); }
     } scatter_guard{scatter};
-    if (E > 0 && (variant == BW_PR_EDGE_LIST || variant == BW_PR_STRUCT_EDGE_LIST || variant == BW_PR_VERTEX_PUSH ||
-                  variant == BW_PR_VERTEX_PUSH_WARP)) {
+    if (E > 0 && push) {
         int st = BW_HIP_OK;
         if (variant == BW_PR_EDGE_LIST)
             st = bw_pr_scatter_create(&scatter, BW_PR_SCATTER_EDGE_LIST, V, E, g->el_in, g->el_out, 4, s);
@@ -1707,29 +1735,7 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
         BW_TRY(bw_pr_pull_plan_create(&pull, V, g->rev_offsets, g->offset_bytes, s));
     }
 
-    const bool gathered = scatter && scatter_gathers(scatter);
-    // Degrees once per run (pagerank/pagerank.cpp:102-112).  With the forward
-    // CSR resident, every variant's out-degrees come from its offsets: the
-    // same integers the variant's own degree kernel counts
-    // (pagerank/pagerank.cu:40-123), without an atomic per edge; the push
-    // variants, which have no degree kernel, read the same offsets, and only for
-    // the contributions or the dangling mass.
-    BW_TRY(bw_pr_zero_degrees(V, buf.deg, &cfg));
-    const bool degrees = gathered || mode == BW_PR_DANGLING_UNIFORM ||
-                         !(variant == BW_PR_VERTEX_PUSH || variant == BW_PR_VERTEX_PUSH_WARP);
-    if (!degrees) {
-        // nothing to count
-    } else if (g->offsets) {
-        BW_TRY(bw_pr_degrees_csr(V, g->offsets, g->offset_bytes, buf.deg, &cfg));
-    } else switch (variant) {
-    case BW_PR_EDGE_LIST: BW_TRY(bw_pr_degrees_edge_list(E, g->el_in, buf.deg, &cfg)); break;
-    case BW_PR_REV_EDGE_LIST: BW_TRY(bw_pr_degrees_edge_list(E, g->rel_out, buf.deg, &cfg)); break;
-    case BW_PR_STRUCT_EDGE_LIST: BW_TRY(bw_pr_degrees_struct_edge_list(E, g->sel, 0, buf.deg, &cfg)); break;
-    case BW_PR_REV_STRUCT_EDGE_LIST: BW_TRY(bw_pr_degrees_struct_edge_list(E, g->rsel, 1, buf.deg, &cfg)); break;
-    default:
-        BW_TRY(bw_pr_degrees_rev_csr(V, g->rev_offsets, g->offset_bytes, g->rev_cols, buf.deg, &cfg));
-    }
-
+    const bool gathered = scatter && gathers;
     FinishArgs fin{};
     fin.V = V;
     fin.deg = degrees ? buf.deg : nullptr;
@@ -1738,9 +1744,6 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
     fin.part = buf.part;
     fin.nodiv = nodiv;
     fin.mode = mode;
-    // The binned scatter and the atomic kernels divide for themselves.
-    if (gathered || variant == BW_PR_REV_EDGE_LIST || variant == BW_PR_REV_STRUCT_EDGE_LIST)
-        BW_HIP_CHECK(hipMalloc(&buf.contrib, sizeof(float) * V));
     fin.contrib = pull && !nodiv ? pull->contrib : buf.contrib;
     const uint64_t passVerts = static_cast<uint64_t>(finish_per_thread(gathered)) * kFinishThreads;
     const uint32_t passGrid = static_cast<uint32_t>(std::min<uint64_t>((V + passVerts - 1) / passVerts, kFinishGrid));

@@ -619,7 +619,7 @@ extern "C" int bw_pr_scatter_create(bw_pr_scatter **out, int32_t kind, uint64_t 
     if (!a || (kind != BW_PR_SCATTER_STRUCT && !b)) return fail(BW_HIP_ERR_ARG, "NULL device pointer");
     if (kind == BW_PR_SCATTER_CSR && offset_bytes != 4 && offset_bytes != 8)
         return fail(BW_HIP_ERR_ARG, "offset_bytes must be 4 or 8");
-    const bool gather = V <= kGatherMaxV;
+    const bool gather = scatter_gathers(V);
     uint32_t rows_log = kRowsLog;
     if (gather) {
         rows_log = kGatherMinLog;
@@ -740,7 +740,7 @@ extern "C" int bw_pr_scatter_create(bw_pr_scatter **out, int32_t kind, uint64_t 
 
 namespace bw {
 
-bool scatter_gathers(const bw_pr_scatter *sc) { return sc->gather; }
+bool scatter_gathers(uint64_t V) { return V <= kGatherMaxV; }
 
 ScatterSums scatter_sums(const bw_pr_scatter *sc) { return ScatterSums{sc->partials, sc->chunk_base, sc->rows_log}; }
 

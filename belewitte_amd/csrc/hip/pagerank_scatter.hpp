@@ -66,7 +66,7 @@ struct ScatterSums {
     }
 };
 
-bool scatter_gathers(const bw_pr_scatter *sc);
+bool scatter_gathers(uint64_t V);  // whether a layout of V vertices is a gathered one
 ScatterSums scatter_sums(const bw_pr_scatter *sc);
 int scatter_gather(const bw_pr_scatter *sc, const float *contrib, const ReducePrev &prev, hipStream_t s);
 int scatter_bins(const bw_pr_scatter *sc, const uint32_t *deg, const float *pr, float *np, const ReducePrev &prev,
