@@ -196,7 +196,7 @@ __global__ void plan_bounds_kernel(uint32_t V, uint32_t L, uint32_t K, const uin
 // partitions.)  A block's work is perVertex x vertices + pairs, and pbase
 // holds the prefix sums of the pairs, so the end of the block from v0 is the
 // last e whose work fits: one wave finds it by probing 64 vertices at a time
-// (a walk over the vertices took 1.54 ms at R-MAT scale 20, 30 us now).
+// (a walk over the vertices took 1.54 ms at R-MAT scale 20, 85 us now).
 // Writes each vertex's block (local to the partition) and, at k << L + b,
 // block b's (first vertex, end vertex, pairs, 0); plan_block_runs_kernel
 // fills in the runs.
