@@ -1668,6 +1668,11 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
             return fail(BW_HIP_ERR_ARG, "variant needs the reverse CSR representation");
     }
 
+    // The passes over the vertices have a geometry of their own; the caller's
+    // is held to the same bounds as in the per-call entries.
+    uint32_t block = 0, grid = 0;
+    if (iterations > 0) BW_TRY(resolve_geometry(&cfg, V, block, grid));
+
     RunBuffers buf;
     const uint64_t iters = static_cast<uint64_t>(std::max(iterations, 1));
     BW_HIP_CHECK(hipMalloc(&buf.deg, sizeof(uint32_t) * V));

@@ -200,3 +200,22 @@ def test_kernel_names_are_launched(fake):
                 table = f.autotune(3)
                 assert f.binning == (14, 3, 16) and list(table) == ["small"] and len(calls("launch")) == 4
     """)
+
+
+def test_run_refuses_what_its_kernels_would(fake):
+    """bw_pr_run refuses a block size that its passes over the vertices do not
+    take, whichever variant runs (when iterations do)."""
+    _run(fake, """
+        dg = device.DeviceGraph(graph.rmat_n(300, 2000, seed=1))
+        ranks = device.DeviceArray(dg.vertex_count, np.float32)
+        def run(variant, iterations, mode=0, **launch):
+            cfg = N.launch(warp=32, chunk=32, **launch)
+            return lib.bw_pr_run(dg.ref, variant, iterations, mode, ranks.ptr, None, C.byref(cfg))
+        for name in pagerank.VARIANTS:
+            v = pagerank.variant_id(name)
+            dg.ensure(pagerank.REPRESENTATION[v])
+            for mode in (0, 1):
+                assert run(v, 2, mode) == run(v, 2, mode, block=1024) == 0, lib.bw_hip_last_error()
+                for block in (100, 2048):
+                    assert run(v, 2, mode, block=block) == 1 and b"block size" in lib.bw_hip_last_error(), (name, block)
+    """)
