@@ -1683,7 +1683,7 @@ extern "C" int bw_pr_run(const bw_graph_dev *g, int32_t variant, int32_t iterati
                       variant == BW_PR_VERTEX_PUSH_WARP;
     // The binned scatter and the atomic kernels divide for themselves, and a
     // pull plan holds contributions of its own.
-    const bool gathers = push && E > 0 && scatter_gathers(V);
+    const bool gathers = push && E > 0 && iterations > 0 && scatter_gathers(V);
     if (gathers || variant == BW_PR_REV_EDGE_LIST || variant == BW_PR_REV_STRUCT_EDGE_LIST)
         BW_HIP_CHECK(hipMalloc(&buf.contrib, sizeof(float) * V));
     double *resid = buf.acc, *dang = buf.acc + iters, *spare = buf.acc + 2 * iters + 1;

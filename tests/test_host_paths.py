@@ -204,7 +204,8 @@ def test_kernel_names_are_launched(fake):
 
 def test_run_refuses_what_its_kernels_would(fake):
     """bw_pr_run refuses a block size that its passes over the vertices do not
-    take, whichever variant runs (when iterations do)."""
+    take, whichever variant runs (when iterations do), and asks nothing of the
+    offsets of a push variant that does not iterate."""
     _run(fake, """
         dg = device.DeviceGraph(graph.rmat_n(300, 2000, seed=1))
         ranks = device.DeviceArray(dg.vertex_count, np.float32)
@@ -218,4 +219,8 @@ def test_run_refuses_what_its_kernels_would(fake):
                 assert run(v, 2, mode) == run(v, 2, mode, block=1024) == 0, lib.bw_hip_last_error()
                 for block in (100, 2048):
                     assert run(v, 2, mode, block=block) == 1 and b"block size" in lib.bw_hip_last_error(), (name, block)
+        dg.desc.offset_bytes = 5
+        for name in ("vertex-push", "vertex-push-warp"):
+            v = pagerank.variant_id(name)
+            assert run(v, 0) == 0 and run(v, 1) == 1 and run(v, 0, 1) == 1
     """)
