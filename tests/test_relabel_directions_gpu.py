@@ -54,3 +54,29 @@ def test_relabel_directions(gpu, V, E, reverse):
         woff, wcols = _want(V, o, c, perm)
         assert np.array_equal(got[2 * k], woff), (V, E, reverse, k)
         assert np.array_equal(got[2 * k + 1], wcols), (V, E, reverse, k)
+
+
+# (row, row, column, column) whose swap an order-independent sum of hashes with
+# two rounds of multiplication does not see.
+@pytest.mark.parametrize("r1,r2,c1,c2", [(34456, 53208, 44788, 18958), (33183, 35060, 50385, 30693),
+                                         (1794, 31874, 44307, 32023)])
+def test_reverse_lists_with_two_columns_swapped(gpu, r1, r2, c1, c2):
+    V = 65536
+    src = np.arange(V)  # one edge each: the order stays
+    dst = np.arange(V)
+    dst[[c1, c2]] = r1, r2
+    off, cols = _csr(V, src, dst)
+    src[[c1, c2]] = c2, c1
+    roff, rcols = _csr(V, dst, src)
+    ins = [device.DeviceArray.from_host(x) for x in (off, cols, roff, rcols)]
+    outs = [device.DeviceArray(n, np.uint32) for n in (V + 1, V, V + 1, V, V)]
+    try:
+        N.check_hip(N.hip_lib().bw_graph_relabel_by_degree(V, V, *(x.ptr for x in ins + outs), None))
+        got = [o.download() for o in outs]
+    finally:
+        for x in ins + outs:
+            x.free()
+    for k, (o, c) in enumerate([(off, cols), (roff, rcols)]):
+        woff, wcols = _want(V, o, c, np.arange(V, dtype=np.uint32))
+        assert np.array_equal(got[2 * k], woff)
+        assert np.array_equal(got[2 * k + 1], wcols)
