@@ -1043,8 +1043,9 @@ int relabel_both(Scratch &sc, uint32_t V, uint32_t E, const uint32_t *off, const
         e = sort_pairs(sc, static_cast<const uint32_t *>(col), scol, static_cast<const uint32_t *>(row), nrcols, E,
                        bits, s);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(relabel_compare_kernel, dim3(std::min(grid_for(E, kCompareEdges * kThreads), 2048u)), dim3(kThreads), 0, s, E, scol,
-                           nrcols, roff, rcols, order, perm, nroff, check);
+        const uint32_t grid = std::min(grid_for(E, kCompareEdges * kThreads), 2048u);
+        hipLaunchKernelGGL(relabel_compare_kernel, dim3(grid), dim3(kThreads), 0, s, E, scol, nrcols, roff, rcols,
+                           order, perm, nroff, check);
         e = hipGetLastError();
     }
     if (e == hipSuccess)
